@@ -116,11 +116,11 @@ __device__ __forceinline__ void ax_pair(const StepStatic& P, const float* psi, i
   t.n1 = t.n2 = t.an = t.kn = 0.f;
   if (t.sn < 0) return;
   const bool h = t.sn == 1;
-  const int L = h ? B.L : A.L, dep = cn - (h ? B.lo : A.lo);
-  const long long cells = h ? B.cells : A.cells;
-  t.kapn = !(h ? B.kappa_one : A.kappa_one);
-  const long long q = ax_psi<AX>(P, h ? B.psi_off : A.psi_off, W, cells, L, dep, i, j, k);
-  const float* cf = (h ? B.coef : A.coef) + (W ? 3 * L : 0);
+  const int L = side_of(h, B.L, A.L), dep = cn - side_of(h, B.lo, A.lo);
+  const long long cells = side_of(h, B.cells, A.cells);
+  t.kapn = !side_of(h, B.kappa_one, A.kappa_one);
+  const long long q = ax_psi<AX>(P, side_of(h, B.psi_off, A.psi_off), W, cells, L, dep, i, j, k);
+  const float* cf = side_of(h, B.coef, A.coef) + (W ? 3 * L : 0);
   t.n1 = psi[q];
   t.n2 = psi[q + cells];
   t.an = cf[L + dep];
@@ -195,7 +195,8 @@ __device__ __forceinline__ float g_adj(const StepStatic& P, const AdjDyn& A, uin
   return lam_h(P, A, m, walls, r, oo, ii, jj, kk);
 }
 
-__global__ __launch_bounds__(kBlock) void k_adj_wT(const StepStatic P, const AdjDyn A, int field) {
+__global__ __launch_bounds__(kBlock) void k_adj_wT(const StepStatic* __restrict__ Pp, const AdjDyn A, int field) {
+  const StepStatic& P = as_const(Pp);
   int i, j, k;
   long long o;
   uint32_t m;
@@ -344,7 +345,8 @@ __device__ __forceinline__ void reverse_E_cell(const StepStatic& P, const AdjDyn
 }
 
 // K^{n+1/2} of every cell, for the off-diagonal permittivity gradient.
-__global__ __launch_bounds__(kBlock) void k_adj_K(const StepStatic P, const AdjDyn A) {
+__global__ __launch_bounds__(kBlock) void k_adj_K(const StepStatic* __restrict__ Pp, const AdjDyn A) {
+  const StepStatic& P = as_const(Pp);
   int i, j, k;
   long long o;
   uint32_t m;
@@ -360,7 +362,8 @@ __global__ __launch_bounds__(kBlock) void k_adj_K(const StepStatic P, const AdjD
 // reads, after which E holds E^n.
 // AXS: per-axis CPML (acax), the slab loads of all three axes issued first.
 template <int EC, int MC, bool REV, bool AXS>
-__global__ __launch_bounds__(kBlock) void k_adj_A(const StepStatic P, const AdjDyn A) {
+__global__ __launch_bounds__(kBlock) void k_adj_A(const StepStatic* __restrict__ Pp, const AdjDyn A) {
+  const StepStatic& P = as_const(Pp);
   int i, j, k;
   long long o;
   uint32_t m;
@@ -499,7 +502,8 @@ __global__ __launch_bounds__(kBlock) void k_adj_A(const StepStatic P, const AdjD
 }
 
 template <int EC, int MC, bool AXS>
-__global__ __launch_bounds__(kBlock) void k_adj_B(const StepStatic P, const AdjDyn A) {
+__global__ __launch_bounds__(kBlock) void k_adj_B(const StepStatic* __restrict__ Pp, const AdjDyn A) {
+  const StepStatic& P = as_const(Pp);
   int i, j, k;
   long long o;
   uint32_t m;
@@ -604,7 +608,8 @@ __global__ __launch_bounds__(kBlock) void k_adj_B(const StepStatic P, const AdjD
 // Pass C: lam_E^n = (1 - x) / (1 + x) * mu_E in the electric conductivity box, one thread per box
 // cell (pass B has read mu_E at every neighbour by now).
 template <int EC>
-__global__ __launch_bounds__(kBlock) void k_adj_C(const StepStatic P, const AdjDyn A) {
+__global__ __launch_bounds__(kBlock) void k_adj_C(const StepStatic* __restrict__ Pp, const AdjDyn A) {
+  const StepStatic& P = as_const(Pp);
   const LossK& L = P.loss[0];
   const long long q = (long long)blockIdx.x * kBlock + threadIdx.x;
   if (q >= L.cells) return;
@@ -623,7 +628,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_C(const StepStatic P, const AdjD
 hipError_t launch_adjoint(const StepStatic& P, const AdjDyn& A, int ec, int mc, hipStream_t s) {
   const dim3 g((unsigned)P.nblocks_pad);
   const dim3 gc((unsigned)((P.loss[0].cells + kBlock - 1) / kBlock));
-  using AdjKernel = void (*)(const StepStatic, const AdjDyn);
+  using AdjKernel = void (*)(const StepStatic*, const AdjDyn);
   AdjKernel ka = nullptr, kb = nullptr;
   const bool axs = P.acax != 0;
   if (ec == 9 || mc == 9) {  // full tensors: the slab loop
@@ -658,14 +663,14 @@ hipError_t launch_adjoint(const StepStatic& P, const AdjDyn& A, int ec, int mc, 
   if (!ka) return hipErrorInvalidValue;
   // full tensors: the transposed-tensor cotangent of the H half-step, and every cell's K for the
   // permittivity gradient, before pass A; that of the E half-step (from mu_E) before pass B
-  if (mc == 9) hipLaunchKernelGGL(k_adj_wT, g, dim3(kBlock), 0, s, P, A, 1);
-  if (ec == 9) hipLaunchKernelGGL(k_adj_K, g, dim3(kBlock), 0, s, P, A);
-  hipLaunchKernelGGL(ka, g, dim3(kBlock), 0, s, P, A);
-  if (ec == 9) hipLaunchKernelGGL(k_adj_wT, g, dim3(kBlock), 0, s, P, A, 0);
-  hipLaunchKernelGGL(kb, g, dim3(kBlock), 0, s, P, A);
+  if (mc == 9) hipLaunchKernelGGL(k_adj_wT, g, dim3(kBlock), 0, s, P.self, A, 1);
+  if (ec == 9) hipLaunchKernelGGL(k_adj_K, g, dim3(kBlock), 0, s, P.self, A);
+  hipLaunchKernelGGL(ka, g, dim3(kBlock), 0, s, P.self, A);
+  if (ec == 9) hipLaunchKernelGGL(k_adj_wT, g, dim3(kBlock), 0, s, P.self, A, 0);
+  hipLaunchKernelGGL(kb, g, dim3(kBlock), 0, s, P.self, A);
   if (P.loss[0].comps) {
-    if (ec == 3) hipLaunchKernelGGL(k_adj_C<3>, gc, dim3(kBlock), 0, s, P, A);
-    else hipLaunchKernelGGL(k_adj_C<1>, gc, dim3(kBlock), 0, s, P, A);
+    if (ec == 3) hipLaunchKernelGGL(k_adj_C<3>, gc, dim3(kBlock), 0, s, P.self, A);
+    else hipLaunchKernelGGL(k_adj_C<1>, gc, dim3(kBlock), 0, s, P.self, A);
   }
   return hipGetLastError();
 }

@@ -477,20 +477,23 @@ __device__ __forceinline__ float reduce_finalize_tile(const StepStatic& P, const
 }
 
 template <bool CX>
-__global__ __launch_bounds__(kBlock) void k_detector(const StepStatic P, const DetK K, const DetDyn D) {
+__global__ __launch_bounds__(kBlock) void k_detector(const StepStatic* __restrict__ Pp, const DetK K, const DetDyn D) {
+  const StepStatic& P = as_const(Pp);
   detector_tile<CX>(P, K, D, D.n, D.slot, blockIdx.x, gridDim.x);
 }
 
-__global__ __launch_bounds__(kBlock) void k_reduce_finalize(const StepStatic P, const DetK K, const double* partial,
+__global__ __launch_bounds__(kBlock) void k_reduce_finalize(const StepStatic* __restrict__ Pp, const DetK K, const double* partial,
                                                             int nparts, void* state, int slot, int n) {
+  const StepStatic& P = as_const(Pp);
   reduce_finalize_tile(P, K, partial, nparts, state, slot, n);
 }
 
-static_assert(sizeof(StepStatic) + sizeof(void*) + sizeof(DetGroup) <= 4096, "grouped detector kernel arguments exceed 4 KB");
+static_assert(2 * sizeof(void*) + sizeof(DetGroup) <= 4096, "grouped detector kernel arguments exceed 4 KB");
 
 template <bool CX>
-__global__ __launch_bounds__(kBlock) void k_detector_group(const StepStatic P, const DetK* __restrict__ Kd,
+__global__ __launch_bounds__(kBlock) void k_detector_group(const StepStatic* __restrict__ Pp, const DetK* __restrict__ Kd,
                                                            const DetGroup G) {
+  const StepStatic& P = as_const(Pp);
   int a = 0;
   while (a + 1 < G.count && (int)blockIdx.x >= G.start[a + 1]) ++a;
   const DetK& K = Kd[G.q[a]];
@@ -498,8 +501,9 @@ __global__ __launch_bounds__(kBlock) void k_detector_group(const StepStatic P, c
   detector_tile<CX>(P, K, D, D.n, G.slot[a], (int)blockIdx.x - G.start[a], G.start[a + 1] - G.start[a]);
 }
 
-__global__ __launch_bounds__(kBlock) void k_finalize_group(const StepStatic P, const DetK* __restrict__ Kd,
+__global__ __launch_bounds__(kBlock) void k_finalize_group(const StepStatic* __restrict__ Pp, const DetK* __restrict__ Kd,
                                                            const DetGroup G) {
+  const StepStatic& P = as_const(Pp);
   const int a0 = G.fin[blockIdx.x];
   for (int a = a0; a < G.count; ++a) {
     const DetK& K = Kd[G.q[a]];
@@ -583,27 +587,28 @@ int detector_blocks(const DetK& K) {
 }
 
 hipError_t launch_detector(const StepStatic& P, const DetK& K, const DetDyn& D, int nblocks, hipStream_t s) {
-  if (D.Ei) hipLaunchKernelGGL(k_detector<true>, dim3(nblocks), dim3(kBlock), 0, s, P, K, D);
-  else hipLaunchKernelGGL(k_detector<false>, dim3(nblocks), dim3(kBlock), 0, s, P, K, D);
+  if (D.Ei) hipLaunchKernelGGL(k_detector<true>, dim3(nblocks), dim3(kBlock), 0, s, P.self, K, D);
+  else hipLaunchKernelGGL(k_detector<false>, dim3(nblocks), dim3(kBlock), 0, s, P.self, K, D);
   if (reduced_values(K))
-    hipLaunchKernelGGL(k_reduce_finalize, dim3(1), dim3(kBlock), 0, s, P, K, (const double*)D.partial, nblocks,
+    hipLaunchKernelGGL(k_reduce_finalize, dim3(1), dim3(kBlock), 0, s, P.self, K, (const double*)D.partial, nblocks,
                        D.state, D.slot, D.n);
   return hipGetLastError();
 }
 
 hipError_t launch_detector_group(const StepStatic& P, const DetK* Kdev, const DetGroup& G, hipStream_t s) {
   if (G.count <= 0) return hipSuccess;
-  if (G.dd[0].Ei) hipLaunchKernelGGL(k_detector_group<true>, dim3(G.start[G.count]), dim3(kBlock), 0, s, P, Kdev, G);
-  else hipLaunchKernelGGL(k_detector_group<false>, dim3(G.start[G.count]), dim3(kBlock), 0, s, P, Kdev, G);
-  if (G.nfin > 0) hipLaunchKernelGGL(k_finalize_group, dim3(G.nfin), dim3(kBlock), 0, s, P, Kdev, G);
+  if (G.dd[0].Ei) hipLaunchKernelGGL(k_detector_group<true>, dim3(G.start[G.count]), dim3(kBlock), 0, s, P.self, Kdev, G);
+  else hipLaunchKernelGGL(k_detector_group<false>, dim3(G.start[G.count]), dim3(kBlock), 0, s, P.self, Kdev, G);
+  if (G.nfin > 0) hipLaunchKernelGGL(k_finalize_group, dim3(G.nfin), dim3(kBlock), 0, s, P.self, Kdev, G);
   return hipGetLastError();
 }
 
 // Copy of the three components of a field over box [lo, hi) into dst (3, box); blockIdx.y = 1
 // copies the second field (src1 into dst1) over the same box, so that two snapshots share a launch.
-__global__ __launch_bounds__(kBlock) void k_snapshot(const StepStatic P, const float* src0, float* dst0,
+__global__ __launch_bounds__(kBlock) void k_snapshot(const StepStatic* __restrict__ Pp, const float* src0, float* dst0,
                                                      const float* src1, float* dst1, int lo0, int lo1, int lo2,
                                                      int hi0, int hi1, int hi2) {
+  const StepStatic& P = as_const(Pp);
   const float* src = blockIdx.y ? src1 : src0;
   float* dst = blockIdx.y ? dst1 : dst0;
   const int sy = hi1 - lo1, sz = hi2 - lo2;
@@ -619,8 +624,9 @@ __global__ __launch_bounds__(kBlock) void k_snapshot(const StepStatic P, const f
   }
 }
 
-__global__ __launch_bounds__(kBlock) void k_zero_box(const StepStatic P, float* F, int lo0, int lo1, int lo2,
+__global__ __launch_bounds__(kBlock) void k_zero_box(const StepStatic* __restrict__ Pp, float* F, int lo0, int lo1, int lo2,
                                                      int hi0, int hi1, int hi2) {
+  const StepStatic& P = as_const(Pp);
   const int sy = hi1 - lo1, sz = hi2 - lo2;
   const long long cells = (long long)(hi0 - lo0) * sy * sz;
   for (long long q = (long long)blockIdx.x * kBlock + threadIdx.x; q < cells; q += (long long)gridDim.x * kBlock) {
@@ -640,7 +646,7 @@ hipError_t launch_zero_box(const StepStatic& P, float* F, const int* lo, const i
   long long b = (cells + kBlock - 1) / kBlock;
   if (b > 2048) b = 2048;
   if (b < 1) b = 1;
-  hipLaunchKernelGGL(k_zero_box, dim3((unsigned)b), dim3(kBlock), 0, s, P, F, lo[0], lo[1], lo[2], hi[0], hi[1],
+  hipLaunchKernelGGL(k_zero_box, dim3((unsigned)b), dim3(kBlock), 0, s, P.self, F, lo[0], lo[1], lo[2], hi[0], hi[1],
                      hi[2]);
   return hipGetLastError();
 }
@@ -651,7 +657,7 @@ hipError_t launch_snapshot(const StepStatic& P, const float* src, float* dst, co
   long long b = (cells + kBlock - 1) / kBlock;
   if (b > 2048) b = 2048;
   if (b < 1) b = 1;
-  hipLaunchKernelGGL(k_snapshot, dim3((unsigned)b, src1 ? 2u : 1u), dim3(kBlock), 0, s, P, src, dst, src1, dst1,
+  hipLaunchKernelGGL(k_snapshot, dim3((unsigned)b, src1 ? 2u : 1u), dim3(kBlock), 0, s, P.self, src, dst, src1, dst1,
                      lo[0], lo[1], lo[2], hi[0], hi[1], hi[2]);
   return hipGetLastError();
 }
@@ -659,7 +665,8 @@ hipError_t launch_snapshot(const StepStatic& P, const float* src, float* dst, co
 // ---------------------------------------------------------------- detector adjoint
 // Stage 1: cotangents in the interpolated space (6 per region cell), the transpose of each
 // detector's update() with respect to its co-located inputs.
-__global__ __launch_bounds__(kBlock) void k_det_adj_g(const StepStatic P, const DetK K, const DetAdjDyn D) {
+__global__ __launch_bounds__(kBlock) void k_det_adj_g(const StepStatic* __restrict__ Pp, const DetK K, const DetAdjDyn D) {
+  const StepStatic& P = as_const(Pp);
   const Src3 e = box3(D.E1, D.slo, D.shi, 0);
   const Src3 h1 = box3(D.H1, D.slo, D.shi, 1);
   const Src3 h0 = full3(P, D.H0, 1);
@@ -776,7 +783,8 @@ __device__ __forceinline__ void gather_T(const StepStatic& P, const DetK& K, con
 // after the adjoint sweeps (k_add_half_vH). Below an electric symmetry plane the stencils read the
 // mirror of rows 0 and 1 (mirror_fold), so the cotangent gathered at each halo position folds back
 // onto its mirror row with the component's sign, for every set of mirror axes the cell borders.
-__global__ __launch_bounds__(kBlock) void k_det_adj_scatter(const StepStatic P, const DetK K, const DetAdjDyn D) {
+__global__ __launch_bounds__(kBlock) void k_det_adj_scatter(const StepStatic* __restrict__ Pp, const DetK K, const DetAdjDyn D) {
+  const StepStatic& P = as_const(Pp);
   const int ey = D.ehi[1] - D.elo[1], ez = D.ehi[2] - D.elo[2];
   const long long cells = (long long)(D.ehi[0] - D.elo[0]) * ey * ez;
   for (long long q = (long long)blockIdx.x * kBlock + threadIdx.x; q < cells; q += (long long)gridDim.x * kBlock) {
@@ -830,7 +838,8 @@ __global__ __launch_bounds__(kBlock) void k_det_adj_scatter(const StepStatic P, 
   }
 }
 
-__global__ __launch_bounds__(kBlock) void k_add_half_vH(const StepStatic P, const DetAdjDyn D) {
+__global__ __launch_bounds__(kBlock) void k_add_half_vH(const StepStatic* __restrict__ Pp, const DetAdjDyn D) {
+  const StepStatic& P = as_const(Pp);
   const int ey = D.ehi[1] - D.elo[1], ez = D.ehi[2] - D.elo[2];
   const long long cells = (long long)(D.ehi[0] - D.elo[0]) * ey * ez;
   for (long long q = (long long)blockIdx.x * kBlock + threadIdx.x; q < cells; q += (long long)gridDim.x * kBlock) {
@@ -852,15 +861,15 @@ static int blocks_for(long long cells) {
 }
 
 hipError_t launch_detector_adjoint(const StepStatic& P, const DetK& K, const DetAdjDyn& D, hipStream_t s) {
-  hipLaunchKernelGGL(k_det_adj_g, dim3(blocks_for(K.cells)), dim3(kBlock), 0, s, P, K, D);
+  hipLaunchKernelGGL(k_det_adj_g, dim3(blocks_for(K.cells)), dim3(kBlock), 0, s, P.self, K, D);
   const long long ec = (long long)(D.ehi[0] - D.elo[0]) * (D.ehi[1] - D.elo[1]) * (D.ehi[2] - D.elo[2]);
-  hipLaunchKernelGGL(k_det_adj_scatter, dim3(blocks_for(ec)), dim3(kBlock), 0, s, P, K, D);
+  hipLaunchKernelGGL(k_det_adj_scatter, dim3(blocks_for(ec)), dim3(kBlock), 0, s, P.self, K, D);
   return hipGetLastError();
 }
 
 hipError_t launch_add_half_vH(const StepStatic& P, const DetAdjDyn& D, hipStream_t s) {
   const long long ec = (long long)(D.ehi[0] - D.elo[0]) * (D.ehi[1] - D.elo[1]) * (D.ehi[2] - D.elo[2]);
-  hipLaunchKernelGGL(k_add_half_vH, dim3(blocks_for(ec)), dim3(kBlock), 0, s, P, D);
+  hipLaunchKernelGGL(k_add_half_vH, dim3(blocks_for(ec)), dim3(kBlock), 0, s, P.self, D);
   return hipGetLastError();
 }
 

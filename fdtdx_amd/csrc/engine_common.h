@@ -71,6 +71,7 @@ struct LossK {             // conductivity box; zero conductivity outside it
 };
 
 struct StepStatic {
+  const StepStatic* self;  // this table in device memory (the kernels' argument)
   int nx, ny, nz;
   int T;
   long long plane;         // ny*nz
@@ -190,6 +191,27 @@ constexpr int kMaskSnap = 18;
 constexpr int kMaskWall = 19;  // bits [19, 25): PEC / PMC faces (footprint widened by one cell)
 constexpr int kMaskLoss = 25;  // bits 25, 26: conductivity boxes (footprint widened by one cell)
 constexpr uint32_t kMaskAll = 0xffffffffu;
+
+// The plan's table (about 2.5 KB) lives in device memory and a kernel takes its address: a launch
+// then writes 0.2 KB of arguments instead of 2.7 KB, and the table's scalar loads hit the caches the
+// previous launch filled instead of reading a fresh argument block. It is constant for the whole
+// kernel, so it is read through the constant address space (scalar loads, also after stores; the
+// integer cast keeps the compiler from folding the address space away). Measured on 400-step runs,
+// table by value -> by address: 64^3 dipole 52.5 -> 49.5 us per step, 128x128x64 plane wave
+// 48.2 -> 45.2, adjoint 64^3 92.8 -> 86.3, adjoint 200x200x100 402 -> 372; host time per launch
+// 4.6 -> 3.0 us; 200x200x100 and larger forwards unchanged (77.9 -> 77.7, 530 -> 529 us).
+template <class T>
+__device__ __forceinline__ const T& as_const(const T* p) {
+  return *(const T*)(const __attribute__((address_space(4))) T*)(uintptr_t)p;
+}
+
+// The value of a table entry for side 1 or 0 of an axis. Both are read (scalar loads), then selected
+// per lane: `h ? B.x : A.x` would select the address and read the table per lane (the 400x400x200
+// step measured 550 us that way against 529).
+template <class T>
+__device__ __forceinline__ T side_of(bool h, T b, T a) {
+  return h ? b : a;
+}
 
 struct StepDyn {
   float* E;

@@ -20,7 +20,8 @@
 namespace fdtdx {
 
 template <int EC, int MC, int M>
-__global__ __launch_bounds__(kFusedThreads) void k_fused(const StepStatic P, const FusedDyn D) {
+__global__ __launch_bounds__(kFusedThreads) void k_fused(const StepStatic* __restrict__ Pp, const FusedDyn D) {
+  const StepStatic& P = as_const(Pp);
   extern __shared__ float lds[];
   const long long lb = logical_block(0, D.nblocks_pad);
   if (lb >= D.nblocks) return;
@@ -266,13 +267,13 @@ hipError_t launch_fused(const StepStatic& P, const FusedDyn& D, int ec, int mc, 
   const dim3 g((unsigned)D.nblocks_pad), b(kFusedThreads);
   constexpr int M = kFusedM;
   if (ec == 3) {
-    if (mc == 3) hipLaunchKernelGGL((k_fused<3, 3, M>), g, b, lds, s, P, D);
-    else if (mc == 1) hipLaunchKernelGGL((k_fused<3, 1, M>), g, b, lds, s, P, D);
-    else hipLaunchKernelGGL((k_fused<3, 0, M>), g, b, lds, s, P, D);
+    if (mc == 3) hipLaunchKernelGGL((k_fused<3, 3, M>), g, b, lds, s, P.self, D);
+    else if (mc == 1) hipLaunchKernelGGL((k_fused<3, 1, M>), g, b, lds, s, P.self, D);
+    else hipLaunchKernelGGL((k_fused<3, 0, M>), g, b, lds, s, P.self, D);
   } else {
-    if (mc == 3) hipLaunchKernelGGL((k_fused<1, 3, M>), g, b, lds, s, P, D);
-    else if (mc == 1) hipLaunchKernelGGL((k_fused<1, 1, M>), g, b, lds, s, P, D);
-    else hipLaunchKernelGGL((k_fused<1, 0, M>), g, b, lds, s, P, D);
+    if (mc == 3) hipLaunchKernelGGL((k_fused<1, 3, M>), g, b, lds, s, P.self, D);
+    else if (mc == 1) hipLaunchKernelGGL((k_fused<1, 1, M>), g, b, lds, s, P.self, D);
+    else hipLaunchKernelGGL((k_fused<1, 0, M>), g, b, lds, s, P.self, D);
   }
   return hipGetLastError();
 }

@@ -418,8 +418,9 @@ __device__ __forceinline__ void tensor_ade(const StepStatic& P, const StepDyn& D
 // The curl sweep of a full-tensor half-step: K = curl (+ CPML, psi advanced when update = 1 or
 // frozen when 0) of H (E = 0) or of E (E = 1), written to D.K; the E sweep also snapshots H_prev.
 template <bool X>
-__global__ __launch_bounds__(kBlock) void k_tensor_curl(const StepStatic P, const StepDyn D, int field, int update,
+__global__ __launch_bounds__(kBlock) void k_tensor_curl(const StepStatic* __restrict__ Pp, const StepDyn D, int field, int update,
                                                         int perm) {
+  const StepStatic& P = as_const(Pp);
   int i, j, k;
   long long o;
   const long long lb = logical_block(P.xorder, P.nblocks_pad);
@@ -504,7 +505,8 @@ __device__ __forceinline__ bool tensor_sigma_rows(const StepStatic& P, const Ste
 // E' = E + B avg(K) with sources and PEC faces (forward), or E = (E + sources(inverse)) - B avg(K)
 // (update_E_reverse, update.py:611-683); A avg(E) +- B avg(K) in the conductivity box.
 template <bool X>
-__global__ __launch_bounds__(kBlock) void k_tensor_E(const StepStatic P, const StepDyn D, int reverse) {
+__global__ __launch_bounds__(kBlock) void k_tensor_E(const StepStatic* __restrict__ Pp, const StepDyn D, int reverse) {
+  const StepStatic& P = as_const(Pp);
   int i, j, k;
   long long o;
   const long long lb = logical_block(P.xorder, P.nblocks_pad);
@@ -531,7 +533,8 @@ __global__ __launch_bounds__(kBlock) void k_tensor_E(const StepStatic P, const S
 // H' = H - B avg(K) with sources, PMC faces and the float32 interface record (forward), or
 // H = (H + sources(inverse)) + B avg(K) (update_H_reverse, update.py:960-1004).
 template <bool X>
-__global__ __launch_bounds__(kBlock) void k_tensor_H(const StepStatic P, const StepDyn D, int reverse) {
+__global__ __launch_bounds__(kBlock) void k_tensor_H(const StepStatic* __restrict__ Pp, const StepDyn D, int reverse) {
+  const StepStatic& P = as_const(Pp);
   int i, j, k;
   long long o;
   const long long lb = logical_block(P.xorder, P.nblocks_pad);
@@ -558,12 +561,14 @@ __global__ __launch_bounds__(kBlock) void k_tensor_H(const StepStatic P, const S
 
 // X: the plan has periodic axes or conductivity (false compiles both out of the sweep).
 template <int EC, bool X>
-__global__ __launch_bounds__(kBlock) void k_update_E(const StepStatic P, const StepDyn D) {
+__global__ __launch_bounds__(kBlock) void k_update_E(const StepStatic* __restrict__ Pp, const StepDyn D) {
+  const StepStatic& P = as_const(Pp);
   update_E_tile<EC, false, X>(P, D, D.n, logical_block(P.xorder, P.nblocks_pad));
 }
 
 template <int MC, bool X>
-__global__ __launch_bounds__(kBlock) void k_update_H(const StepStatic P, const StepDyn D) {
+__global__ __launch_bounds__(kBlock) void k_update_H(const StepStatic* __restrict__ Pp, const StepDyn D) {
+  const StepStatic& P = as_const(Pp);
   update_H_tile<MC, false, X>(P, D, D.n, D.record, logical_block(P.xorder, P.nblocks_pad));
 }
 
@@ -690,14 +695,14 @@ __device__ __forceinline__ long long quad_psi_offset(const StepStatic& P, bool h
                                                      int& aligned) {
   const StepStatic::AxSlab& A = P.axd[AX][0];
   const StepStatic::AxSlab& B = P.axd[AX][1];
-  const int lo = hi ? B.lo : A.lo;
-  L = hi ? B.L : A.L;
-  cells = hi ? B.cells : A.cells;
-  cf = (hi ? B.coef : A.coef) + (W ? 3 * L : 0);
-  kap = hi ? B.kappa_one : A.kappa_one;
-  aligned = hi ? B.aligned : A.aligned;
+  const int lo = side_of(hi, B.lo, A.lo);
+  L = side_of(hi, B.L, A.L);
+  cells = side_of(hi, B.cells, A.cells);
+  cf = side_of(hi, B.coef, A.coef) + (W ? 3 * L : 0);
+  kap = side_of(hi, B.kappa_one, A.kappa_one);
+  aligned = side_of(hi, B.aligned, A.aligned);
   dep = (AX == 0 ? i : (AX == 1 ? j : k0)) - lo;
-  const long long base = (hi ? B.psi_off : A.psi_off) + (W ? 2 * cells : 0);
+  const long long base = side_of(hi, B.psi_off, A.psi_off) + (W ? 2 * cells : 0);
   if (AX == 0) return base + (long long)dep * P.plane + (long long)j * P.nz + k0;
   if (AX == 1) return base + ((long long)i * L + dep) * P.nz + k0;
   return base + ((long long)i * P.ny + j) * L + dep;
@@ -712,7 +717,7 @@ __device__ __forceinline__ void quad_slab_load(const StepStatic& P, const float*
     S.hi[AX] = k0 + 3 >= B.lo && B.lo < B.hi;
     S.in[AX] = S.hi[AX] || k0 < A.hi;
     if (!S.in[AX]) return;
-    const int lo = S.hi[AX] ? B.lo : A.lo, hi = S.hi[AX] ? B.hi : A.hi;
+    const int lo = side_of(S.hi[AX], B.lo, A.lo), hi = side_of(S.hi[AX], B.hi, A.hi);
     S.zm = 0u;
 #pragma unroll
     for (int e = 0; e < 4; ++e) S.zm |= (k0 + e >= lo && k0 + e < hi) ? (1u << e) : 0u;
@@ -851,7 +856,8 @@ __device__ __forceinline__ bool slow_cell(const StepStatic& P, const int* list, 
 // The listed quad tiles of the E (k_update_E4s) and H (k_update_H4s) sweeps, one cell per thread,
 // launched beside the quad kernels so that those keep a small register budget.
 template <int EC, bool X>
-__global__ __launch_bounds__(kBlock) void k_update_E4s(const StepStatic P, const StepDyn D) {
+__global__ __launch_bounds__(kBlock) void k_update_E4s(const StepStatic* __restrict__ Pp, const StepDyn D) {
+  const StepStatic& P = as_const(Pp);
   int i, j, k;
   long long o;
   uint32_t ms;
@@ -860,7 +866,8 @@ __global__ __launch_bounds__(kBlock) void k_update_E4s(const StepStatic P, const
 }
 
 template <int MC, bool X>
-__global__ __launch_bounds__(kBlock) void k_update_H4s(const StepStatic P, const StepDyn D) {
+__global__ __launch_bounds__(kBlock) void k_update_H4s(const StepStatic* __restrict__ Pp, const StepDyn D) {
+  const StepStatic& P = as_const(Pp);
   int i, j, k;
   long long o;
   uint32_t ms;
@@ -870,7 +877,8 @@ __global__ __launch_bounds__(kBlock) void k_update_H4s(const StepStatic P, const
 
 // CAX: the per-axis CPML (plans with StepStatic::cax), else the slab loop of cpml_quad.
 template <int EC, bool X, bool CAX>
-__global__ __launch_bounds__(kBlock) void k_update_E4(const StepStatic P, const StepDyn D) {
+__global__ __launch_bounds__(kBlock) void k_update_E4(const StepStatic* __restrict__ Pp, const StepDyn D) {
+  const StepStatic& P = as_const(Pp);
   int i, j, k0;
   long long o;
   const long long lb = logical_block(P.xorder, P.vnblocks_pad);
@@ -933,7 +941,8 @@ __global__ __launch_bounds__(kBlock) void k_update_E4(const StepStatic P, const 
 }
 
 template <int MC, bool X, bool CAX>
-__global__ __launch_bounds__(kBlock) void k_update_H4(const StepStatic P, const StepDyn D) {
+__global__ __launch_bounds__(kBlock) void k_update_H4(const StepStatic* __restrict__ Pp, const StepDyn D) {
+  const StepStatic& P = as_const(Pp);
   int i, j, k0;
   long long o;
   const long long lb = logical_block(P.xorder, P.vnblocks_pad);
@@ -998,7 +1007,8 @@ __global__ __launch_bounds__(kBlock) void k_update_H4(const StepStatic P, const 
 // multiplied by 1 + x and the result divided by 1 - x.
 // AXS: per-axis CPML (acax), the psi loads of all three axes issued ahead of the curl's.
 template <int MC, bool AXS>
-__global__ __launch_bounds__(kBlock) void k_reverse_H(const StepStatic P, const StepDyn D) {
+__global__ __launch_bounds__(kBlock) void k_reverse_H(const StepStatic* __restrict__ Pp, const StepDyn D) {
+  const StepStatic& P = as_const(Pp);
   int i, j, k;
   long long o;
   const long long lb = logical_block(P.xorder, P.nblocks_pad);
@@ -1044,7 +1054,8 @@ __global__ __launch_bounds__(kBlock) void k_reverse_H(const StepStatic P, const 
 }
 
 template <int EC>
-__global__ __launch_bounds__(kBlock) void k_reverse_E(const StepStatic P, const StepDyn D) {
+__global__ __launch_bounds__(kBlock) void k_reverse_E(const StepStatic* __restrict__ Pp, const StepDyn D) {
+  const StepStatic& P = as_const(Pp);
   int i, j, k;
   long long o;
   const long long lb = logical_block(P.xorder, P.nblocks_pad);
@@ -1086,7 +1097,8 @@ __global__ __launch_bounds__(kBlock) void k_reverse_E(const StepStatic P, const 
 // n's slot, or interpolate between the slots around it, and write it back into E and H. Where
 // interface planes of two slabs cross, the later slab's value is the one restored, as in the
 // reference's loop over PML objects.
-__global__ __launch_bounds__(kBlock) void k_restore(const StepStatic P, const StepDyn D) {
+__global__ __launch_bounds__(kBlock) void k_restore(const StepStatic* __restrict__ Pp, const StepDyn D) {
+  const StepStatic& P = as_const(Pp);
   const long long t = (long long)blockIdx.x * kBlock + threadIdx.x;
   long long acc = 0;
 #pragma unroll
@@ -1127,7 +1139,8 @@ __global__ __launch_bounds__(kBlock) void k_restore(const StepStatic P, const St
 // collect_interfaces + Recorder.compress (update.py:1140-1178, recorder.py:70-119) for records
 // with narrow layers: after step n's H sweep, encode the interface layers of E^{n+1} and H^{n+1}
 // into step n's slot, one thread per interface cell and slab.
-__global__ __launch_bounds__(kBlock) void k_record(const StepStatic P, const StepDyn D) {
+__global__ __launch_bounds__(kBlock) void k_record(const StepStatic* __restrict__ Pp, const StepDyn D) {
+  const StepStatic& P = as_const(Pp);
   const long long t = (long long)blockIdx.x * kBlock + threadIdx.x;
   long long acc = 0;
   for (int s = 0; s < P.nslab; ++s) {
@@ -1157,10 +1170,10 @@ static bool extras(const StepStatic& P) {
   return P.wrap[0] || P.wrap[1] || P.wrap[2] || P.loss[0].comps || P.loss[1].comps;
 }
 
-using SweepKernel = void (*)(const StepStatic, const StepDyn);
+using SweepKernel = void (*)(const StepStatic*, const StepDyn);
 
-using TensorCurl = void (*)(const StepStatic, const StepDyn, int, int, int);
-using TensorSweep = void (*)(const StepStatic, const StepDyn, int);
+using TensorCurl = void (*)(const StepStatic*, const StepDyn, int, int, int);
+using TensorSweep = void (*)(const StepStatic*, const StepDyn, int);
 
 // One full-tensor half-step: the curl sweep, then the tensor sweep (field 0: E, 1: H).
 // The per-cell matrices of a full-tensor half-step with conductivity (compute_anisotropic_update_
@@ -1181,7 +1194,8 @@ __device__ __forceinline__ void mul3(const double* X, const double* Y, double* Z
     for (int c = 0; c < 3; ++c) Z[3 * r + c] = X[3 * r] * Y[c] + X[3 * r + 1] * Y[3 + c] + X[3 * r + 2] * Y[6 + c];
 }
 
-__global__ __launch_bounds__(kBlock) void k_tensor_ab(const StepStatic P, const float* inv, int w, float* out) {
+__global__ __launch_bounds__(kBlock) void k_tensor_ab(const StepStatic* __restrict__ Pp, const float* inv, int w, float* out) {
+  const StepStatic& P = as_const(Pp);
   const LossK& L = P.loss[w];
   const long long q = (long long)blockIdx.x * kBlock + threadIdx.x;
   if (q >= L.cells) return;
@@ -1220,7 +1234,7 @@ hipError_t launch_tensor_ab(const StepStatic& P, const StepDyn& D, hipStream_t s
   for (int w = 0; w < 2; ++w) {
     if (!P.tsig[w]) continue;
     const unsigned g = (unsigned)((P.loss[w].cells + kBlock - 1) / kBlock);
-    hipLaunchKernelGGL(k_tensor_ab, dim3(g), dim3(kBlock), 0, s, P, w == 0 ? D.ie : D.im, w, (float*)D.ab[w]);
+    hipLaunchKernelGGL(k_tensor_ab, dim3(g), dim3(kBlock), 0, s, P.self, w == 0 ? D.ie : D.im, w, (float*)D.ab[w]);
   }
   return hipGetLastError();
 }
@@ -1230,8 +1244,8 @@ static hipError_t launch_tensor(const StepStatic& P, const StepDyn& D, int field
   const TensorCurl fc = x ? k_tensor_curl<true> : k_tensor_curl<false>;
   const TensorSweep ft = field == 0 ? (x ? k_tensor_E<true> : k_tensor_E<false>)
                                     : (x ? k_tensor_H<true> : k_tensor_H<false>);
-  hipLaunchKernelGGL(fc, grid_of(P), dim3(kBlock), 0, s, P, D, field, reverse ? 0 : 1, reverse ? 0 : 1);
-  hipLaunchKernelGGL(ft, grid_of(P), dim3(kBlock), 0, s, P, D, reverse);
+  hipLaunchKernelGGL(fc, grid_of(P), dim3(kBlock), 0, s, P.self, D, field, reverse ? 0 : 1, reverse ? 0 : 1);
+  hipLaunchKernelGGL(ft, grid_of(P), dim3(kBlock), 0, s, P.self, D, reverse);
   return hipGetLastError();
 }
 
@@ -1241,7 +1255,7 @@ hipError_t launch_update_E(const StepStatic& P, const StepDyn& D, int ec, hipStr
   SweepKernel f;
   if (ec == 3) f = x ? k_update_E<3, true> : k_update_E<3, false>;
   else f = x ? k_update_E<1, true> : k_update_E<1, false>;
-  hipLaunchKernelGGL(f, grid_of(P), dim3(kBlock), 0, s, P, D);
+  hipLaunchKernelGGL(f, grid_of(P), dim3(kBlock), 0, s, P.self, D);
   return hipGetLastError();
 }
 
@@ -1252,7 +1266,7 @@ hipError_t launch_update_H(const StepStatic& P, const StepDyn& D, int mc, hipStr
   if (mc == 3) f = x ? k_update_H<3, true> : k_update_H<3, false>;
   else if (mc == 1) f = x ? k_update_H<1, true> : k_update_H<1, false>;
   else f = x ? k_update_H<0, true> : k_update_H<0, false>;
-  hipLaunchKernelGGL(f, grid_of(P), dim3(kBlock), 0, s, P, D);
+  hipLaunchKernelGGL(f, grid_of(P), dim3(kBlock), 0, s, P.self, D);
   return hipGetLastError();
 }
 
@@ -1270,8 +1284,8 @@ hipError_t launch_update_E4(const StepStatic& P, const StepDyn& D, int ec, hipSt
           : (c ? k_update_E4<1, false, true> : k_update_E4<1, false, false>);
     fs = x ? k_update_E4s<1, true> : k_update_E4s<1, false>;
   }
-  hipLaunchKernelGGL(f, dim3((unsigned)P.vnblocks_pad), dim3(kBlock), 0, s, P, D);
-  if (P.vnslow) hipLaunchKernelGGL(fs, dim3((unsigned)(4 * P.vnslow)), dim3(kBlock), 0, s, P, D);
+  hipLaunchKernelGGL(f, dim3((unsigned)P.vnblocks_pad), dim3(kBlock), 0, s, P.self, D);
+  if (P.vnslow) hipLaunchKernelGGL(fs, dim3((unsigned)(4 * P.vnslow)), dim3(kBlock), 0, s, P.self, D);
   return hipGetLastError();
 }
 
@@ -1293,33 +1307,33 @@ hipError_t launch_update_H4(const StepStatic& P, const StepDyn& D, int mc, hipSt
           : (c ? k_update_H4<0, false, true> : k_update_H4<0, false, false>);
     fs = x ? k_update_H4s<0, true> : k_update_H4s<0, false>;
   }
-  hipLaunchKernelGGL(f, dim3((unsigned)P.vnblocks_pad), dim3(kBlock), 0, s, P, D);
-  if (P.vnslowH) hipLaunchKernelGGL(fs, dim3((unsigned)(4 * P.vnslowH)), dim3(kBlock), 0, s, P, D);
+  hipLaunchKernelGGL(f, dim3((unsigned)P.vnblocks_pad), dim3(kBlock), 0, s, P.self, D);
+  if (P.vnslowH) hipLaunchKernelGGL(fs, dim3((unsigned)(4 * P.vnslowH)), dim3(kBlock), 0, s, P.self, D);
   return hipGetLastError();
 }
 
 hipError_t launch_record(const StepStatic& P, const StepDyn& D, long long iface_cells, hipStream_t s) {
   if (iface_cells > 0) {
-    hipLaunchKernelGGL(k_record, dim3((unsigned)((iface_cells + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, P, D);
+    hipLaunchKernelGGL(k_record, dim3((unsigned)((iface_cells + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, P.self, D);
   }
   return hipGetLastError();
 }
 
 hipError_t launch_restore(const StepStatic& P, const StepDyn& D, long long iface_cells, hipStream_t s) {
   if (iface_cells > 0) {
-    hipLaunchKernelGGL(k_restore, dim3((unsigned)((iface_cells + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, P, D);
+    hipLaunchKernelGGL(k_restore, dim3((unsigned)((iface_cells + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, P.self, D);
   }
   return hipGetLastError();
 }
 
 // k_reverse_H for diagonal inverse permeability of mc components, per-axis CPML under acax
-static void (*reverse_H_kernel(const StepStatic& P, int mc))(const StepStatic, const StepDyn) {
+static void (*reverse_H_kernel(const StepStatic& P, int mc))(const StepStatic*, const StepDyn) {
   if (P.acax) return mc == 3 ? k_reverse_H<3, true> : (mc == 1 ? k_reverse_H<1, true> : k_reverse_H<0, true>);
   return mc == 3 ? k_reverse_H<3, false> : (mc == 1 ? k_reverse_H<1, false> : k_reverse_H<0, false>);
 }
 
 hipError_t launch_reverse_H(const StepStatic& P, const StepDyn& D, int mc, hipStream_t s) {
-  hipLaunchKernelGGL(reverse_H_kernel(P, mc), grid_of(P), dim3(kBlock), 0, s, P, D);
+  hipLaunchKernelGGL(reverse_H_kernel(P, mc), grid_of(P), dim3(kBlock), 0, s, P.self, D);
   return hipGetLastError();
 }
 
@@ -1328,11 +1342,11 @@ hipError_t launch_reverse(const StepStatic& P, const StepDyn& D, int ec, int mc,
     const hipError_t e = launch_tensor(P, D, 1, 1, s);
     if (e != hipSuccess) return e;
   } else {
-    hipLaunchKernelGGL(reverse_H_kernel(P, mc), grid_of(P), dim3(kBlock), 0, s, P, D);
+    hipLaunchKernelGGL(reverse_H_kernel(P, mc), grid_of(P), dim3(kBlock), 0, s, P.self, D);
   }
   if (ec == 9) return launch_tensor(P, D, 0, 1, s);
-  if (ec == 3) hipLaunchKernelGGL(k_reverse_E<3>, grid_of(P), dim3(kBlock), 0, s, P, D);
-  else hipLaunchKernelGGL(k_reverse_E<1>, grid_of(P), dim3(kBlock), 0, s, P, D);
+  if (ec == 3) hipLaunchKernelGGL(k_reverse_E<3>, grid_of(P), dim3(kBlock), 0, s, P.self, D);
+  else hipLaunchKernelGGL(k_reverse_E<1>, grid_of(P), dim3(kBlock), 0, s, P.self, D);
   return hipGetLastError();
 }
 

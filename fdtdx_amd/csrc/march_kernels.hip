@@ -89,7 +89,8 @@ __device__ __forceinline__ bool span_hits(int a0, int a1, const int lo, const in
 }
 
 template <int EC, int MC, int TY>
-__global__ __launch_bounds__(kMarchThreads) void k_march(const StepStatic P, const MarchDyn D) {
+__global__ __launch_bounds__(kMarchThreads) void k_march(const StepStatic* __restrict__ Pp, const MarchDyn D) {
+  const StepStatic& P = as_const(Pp);
   const int lane = threadIdx.x & 63;
   const long long lb = logical_block(0, D.nblocks_pad);
   const long long t = lb * (kMarchThreads / 64) + (threadIdx.x >> 6);
@@ -367,13 +368,13 @@ template <int TY>
 static void launch_march_ty(const StepStatic& P, const MarchDyn& D, int ec, int mc, hipStream_t s) {
   const dim3 g((unsigned)D.nblocks_pad), b(kMarchThreads);
   if (ec == 3) {
-    if (mc == 3) hipLaunchKernelGGL((k_march<3, 3, TY>), g, b, 0, s, P, D);
-    else if (mc == 1) hipLaunchKernelGGL((k_march<3, 1, TY>), g, b, 0, s, P, D);
-    else hipLaunchKernelGGL((k_march<3, 0, TY>), g, b, 0, s, P, D);
+    if (mc == 3) hipLaunchKernelGGL((k_march<3, 3, TY>), g, b, 0, s, P.self, D);
+    else if (mc == 1) hipLaunchKernelGGL((k_march<3, 1, TY>), g, b, 0, s, P.self, D);
+    else hipLaunchKernelGGL((k_march<3, 0, TY>), g, b, 0, s, P.self, D);
   } else {
-    if (mc == 3) hipLaunchKernelGGL((k_march<1, 3, TY>), g, b, 0, s, P, D);
-    else if (mc == 1) hipLaunchKernelGGL((k_march<1, 1, TY>), g, b, 0, s, P, D);
-    else hipLaunchKernelGGL((k_march<1, 0, TY>), g, b, 0, s, P, D);
+    if (mc == 3) hipLaunchKernelGGL((k_march<1, 3, TY>), g, b, 0, s, P.self, D);
+    else if (mc == 1) hipLaunchKernelGGL((k_march<1, 1, TY>), g, b, 0, s, P.self, D);
+    else hipLaunchKernelGGL((k_march<1, 0, TY>), g, b, 0, s, P.self, D);
   }
 }
 

@@ -741,6 +741,8 @@ static int plan_create(const fdtdx_plan_desc* d, fdtdx_plan** out) {
     }
   }
   pl->ws_bytes = off;
+  // the table last: every launch passes its device copy
+  if ((rc = pl->upload(&P, 1, &P.self))) return bail(rc);
   *out = pl;
   return FDTDX_OK;
 }

@@ -5,8 +5,8 @@
 #include "engine_common.h"
 
 // Descriptor loops (slabs, sources) are rolled or fully unrolled per kernel through the template
-// flag U. Measured on the 400x400x200 forward: the single-solve sweeps (descriptors in the kernel
-// argument block) run 0.66 ms/step rolled against 1.12 ms/step unrolled, while the batch sweeps
+// flag U. Measured on the 400x400x200 forward: the single-solve sweeps (descriptors then passed by
+// value) run 0.66 ms/step rolled against 1.12 ms/step unrolled, while the batch sweeps
 // (descriptors read from the device table) run 0.68 ms/step unrolled against 0.90 rolled.
 
 namespace fdtdx {
@@ -122,11 +122,11 @@ __device__ __forceinline__ void ax_cell(const StepStatic& P, const float* psi, i
   t.p1 = t.p2 = t.b = t.a = t.km1 = 0.f;
   if (t.s < 0) return;
   const bool h = t.s == 1;
-  const int L = h ? B.L : A.L, dep = c - (h ? B.lo : A.lo);
-  t.cells = h ? B.cells : A.cells;
-  t.kap = !(h ? B.kappa_one : A.kappa_one);
-  t.q = ax_psi<AX>(P, h ? B.psi_off : A.psi_off, W, t.cells, L, dep, i, j, k);
-  const float* cf = (h ? B.coef : A.coef) + (W ? 3 * L : 0);
+  const int L = side_of(h, B.L, A.L), dep = c - side_of(h, B.lo, A.lo);
+  t.cells = side_of(h, B.cells, A.cells);
+  t.kap = !side_of(h, B.kappa_one, A.kappa_one);
+  t.q = ax_psi<AX>(P, side_of(h, B.psi_off, A.psi_off), W, t.cells, L, dep, i, j, k);
+  const float* cf = side_of(h, B.coef, A.coef) + (W ? 3 * L : 0);
   t.p1 = psi[t.q];
   t.p2 = psi[t.q + t.cells];
   if (BA) {
