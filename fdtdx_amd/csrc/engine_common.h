@@ -120,20 +120,21 @@ struct StepStatic {
   // masks of that order. zlo = 0, zhi = nz is the plain row-major order.
   int zlo, zhi, zg;
   const uint32_t* fwd_mask;
-  // Quad sweeps (nz a multiple of 4): each lane updates 4 consecutive z cells with dwordx4 loads
-  // and stores; a quad tile is kBlock quads (4 kBlock cells) of one x-plane, visited in the same
-  // row-grouped order as above at quad granularity (vzlo, vzhi in quads; plain row-major when the
-  // z-slab edges are not multiples of 4). vq = 0: the one-cell sweeps run.
+  // Quad sweeps: each lane updates 4 consecutive z cells with dwordx4 loads and stores; a row has
+  // nzq quads, the last one starting at nz - 4 when nz is not a multiple of 4 (quad.h), a quad tile
+  // is kBlock quads of one x-plane, visited in the same row-grouped order as above at quad
+  // granularity (vzlo, vzhi in quads; plain row-major when the z-slab edges are not multiples of 4).
+  // vq = 0: the one-cell sweeps run.
   int vq;
+  int nzq;
   int vzlo, vzhi, vzg;
   int vbpp;                // quad tiles per x-plane
   long long vnblocks, vnblocks_pad;
   const uint32_t* vec_mask;  // per quad tile, as fwd_mask
   long long vnslow;          // quad tiles whose E half-step runs one cell per thread (vlistE bits) ...
   const int* vslow;          // ... and their indices
-  long long vnslowH;         // the same for the H half-step
-  const int* vslowH;
-  uint32_t vlistE, vlistH;   // the mask bits that list a quad tile for the E / H half-step
+  uint32_t vlistE;           // the mask bits that list a quad tile for the E half-step (ADE boxes)
+  uint32_t vpoint[2];        // the mask bits of E sources and PEC faces, of H sources and PMC faces
   // Per-axis CPML (acax = 1): every slab spans its face, at most one slab per side of an axis and
   // no two overlapping, and the x slabs before the y slabs before the z slabs in object order (the
   // order in which the corrections are added); the one-cell reverse and adjoint sweeps then find
@@ -178,11 +179,13 @@ __host__ __device__ __forceinline__ void perm_cell(const StepStatic& P, int p, i
   perm_pos(p, P.ny, P.nz, P.zlo, P.zhi, P.zg, j, k);
 }
 
-// Row j and first column k of quad p of an x-plane in the quad sweeps' order.
-__host__ __device__ __forceinline__ void perm_quad(const StepStatic& P, int p, int& j, int& k) {
+// Row j and first column k of quad p of an x-plane in the quad sweeps' order, and the number sm of
+// its leading cells that belong to the quad before it (the last quad of a row of nz % 4 != 0 cells).
+__host__ __device__ __forceinline__ void perm_quad(const StepStatic& P, int p, int& j, int& k, int& sm) {
   int kq;
-  perm_pos(p, P.ny, P.nz / 4, P.vzlo, P.vzhi, P.vzg, j, kq);
-  k = 4 * kq;
+  perm_pos(p, P.ny, P.nzq, P.vzlo, P.vzhi, P.vzg, j, kq);
+  k = 4 * kq <= P.nz - 4 ? 4 * kq : P.nz - 4;
+  sm = 4 * kq - k;
 }
 
 constexpr int kMaskSrc = 6;

@@ -12,6 +12,7 @@
 
 #include "engine_common.h"
 #include "kernels.h"
+#include "quad.h"
 #include "record_codec.h"
 #include "stencil.h"
 
@@ -215,26 +216,6 @@ __device__ __forceinline__ void update_E_tile(const StepStatic& P, const StepDyn
   uint32_t m = tile_mask<true>(P, lb);
   if (X && D.cpart < 0) m &= ~(0xffu << kMaskSrc);  // real sources drive the real part only
   update_E_cell<EC, U, X>(P, D, n, m, i, j, k, o);
-}
-
-// collect_interfaces (update.py:1140-1178, fdtd/misc.py:10-35): the float32 E and H of a cell on
-// a slab's interface plane into step n's record slot.
-__device__ __forceinline__ void record_iface(const StepStatic& P, uint32_t m, char* record, int i, int j, int k,
-                                             float ex, float ey, float ez, float hx, float hy, float hz) {
-#pragma unroll
-  for (int s = 0; s < FDTDX_MAX_CPML; ++s) {
-    if (s >= P.nslab) break;
-    if (!((m >> s) & 1u)) continue;
-    const SlabK& sl = P.slab[s];
-    const int coord = sl.axis == 0 ? i : (sl.axis == 1 ? j : k);
-    if (coord != sl.iface) continue;
-    const long long pc = (long long)sl.pn0 * sl.pn1;
-    const long long q = sl.axis == 0 ? (long long)j * P.nz + k : (sl.axis == 1 ? (long long)i * P.nz + k : (long long)i * P.ny + j);
-    float* fe = (float*)(record + sl.rec_off_E);
-    float* fh = (float*)(record + sl.rec_off_H);
-    fe[q] = ex; fe[pc + q] = ey; fe[2 * pc + q] = ez;
-    fh[q] = hx; fh[pc + q] = hy; fh[2 * pc + q] = hz;
-  }
 }
 
 // H half-step of step n for cell (i, j, k) at offset o (m: its tile's mask); record (step n's
@@ -573,35 +554,22 @@ __global__ __launch_bounds__(kBlock) void k_update_H(const StepStatic* __restric
 }
 
 // ---------------------------------------------------------------- quad sweeps
-// The forward sweeps with four consecutive z cells per lane (nz a multiple of 4): every field
-// array moves in dwordx4 loads and stores, the z neighbours inside the quad come from the lane's
-// own registers, and a quad tile covers 4 kBlock cells. Per cell the arithmetic is that of
-// update_E_cell / update_H_cell, in the same order, so the results are bit-identical.
-typedef float f4v __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ f4v ld4(const float* p) { return *reinterpret_cast<const f4v*>(p); }
-__device__ __forceinline__ void st4(float* p, f4v v) { *reinterpret_cast<f4v*>(p) = v; }
-
-constexpr uint32_t kSlabBits = (1u << FDTDX_MAX_CPML) - 1u;
-constexpr uint32_t kSnapBit = 1u << kMaskSnap;
-
-// Quad of this lane in quad tile lb: cells (i, j, k0 .. k0 + 3) at offsets o .. o + 3.
-__device__ __forceinline__ bool quad_of(const StepStatic& P, long long lb, int& i, int& j, int& k0, long long& o) {
+// The forward sweeps with four consecutive z cells per lane (quad.h); a quad tile covers kBlock
+// quads. RAG: rows of nz % 4 != 0 cells (a sweep with 4-byte aligned accesses). Measured on the
+// 301x277x150 plane wave: E / H sweep 119 / 113 us against 128 / 122 us one cell per lane (an aligned
+// grid of that many cells would take about 101 / 90).
+// Quad of this lane in quad tile lb: cells (i, j, k0 .. k0 + 3) at offsets o .. o + 3, the first sm
+// of which it leaves out of its stores.
+__device__ __forceinline__ bool quad_of(const StepStatic& P, long long lb, int& i, int& j, int& k0, int& sm,
+                                        long long& o) {
   if (lb >= P.vnblocks) return false;
   i = (int)(lb / P.vbpp);
   const int p = (int)(lb - (long long)i * P.vbpp) * kBlock + threadIdx.x;
-  if (p >= P.ny * (P.nz / 4)) return false;
-  perm_quad(P, p, j, k0);
+  if (p >= P.ny * P.nzq) return false;
+  perm_quad(P, p, j, k0, sm);
   o = (long long)i * P.plane + (long long)j * P.nz + k0;
   return true;
 }
-
-// One-sided derivatives of the four cells of a quad, one vector per (axis, component) pair that
-// feeds a CPML slab: curl H uses (dx Hz, dx Hy), (dy Hx, dy Hz), (dz Hy, dz Hx), curl E the same
-// pairs of E (the order of pml_pair).
-struct QuadDeriv {
-  f4v x1, x2, y1, y2, z1, z2;
-};
 
 // CPML of the four cells of a quad, slab by slab in object order (per cell the order of
 // apply_cpml, with cpml_slab's arithmetic). A slab holding all four cells with 16-byte aligned
@@ -673,223 +641,51 @@ __device__ __forceinline__ void cpml_quad(const StepStatic& P, uint32_t mask, fl
   }
 }
 
-// Per-axis CPML of a quad (StepStatic::cax): the quad meets at most one slab per axis, the x slab
-// fixed by i, the y slab by j and the z slab by k0 (a quad across a z-slab edge updates the cells
-// inside the slab one by one). Every
-// psi and coefficient load is issued before any is used (quad_slab_loads, ahead of the field
-// loads), then the corrections are added x, y, z, i.e. in slab order (quad_slab_apply) with cpml_slab's
-// arithmetic, so the results are bit-identical to cpml_quad. Descriptor fields are read for both
-// sides of an axis (wave-uniform) and selected per lane.
-struct QuadSlabs {
-  bool in[3], hi[3];  // the quad meets the axis's slab; of its max side
-  unsigned zm;        // cells of the quad inside its z slab (bit e: cell k0 + e)
-  f4v p1[3], p2[3];   // psi1, psi2 of the quad in that slab (zero for cells outside it)
-};
-
-// Descriptor fields of the slab of one side of axis AX (wave-uniform), and the float offset of psi1
-// of cell (i, j, k0) in it (for the z axis k0 - lo may be negative or reach past the slab when the
-// quad straddles a slab edge; only the cells inside are addressed).
-template <int W, int AX>
-__device__ __forceinline__ long long quad_psi_offset(const StepStatic& P, bool hi, int i, int j, int k0, int& dep,
-                                                     long long& cells, const float*& cf, int& L, int& kap,
-                                                     int& aligned) {
-  const StepStatic::AxSlab& A = P.axd[AX][0];
-  const StepStatic::AxSlab& B = P.axd[AX][1];
-  const int lo = side_of(hi, B.lo, A.lo);
-  L = side_of(hi, B.L, A.L);
-  cells = side_of(hi, B.cells, A.cells);
-  cf = side_of(hi, B.coef, A.coef) + (W ? 3 * L : 0);
-  kap = side_of(hi, B.kappa_one, A.kappa_one);
-  aligned = side_of(hi, B.aligned, A.aligned);
-  dep = (AX == 0 ? i : (AX == 1 ? j : k0)) - lo;
-  const long long base = side_of(hi, B.psi_off, A.psi_off) + (W ? 2 * cells : 0);
-  if (AX == 0) return base + (long long)dep * P.plane + (long long)j * P.nz + k0;
-  if (AX == 1) return base + ((long long)i * L + dep) * P.nz + k0;
-  return base + ((long long)i * P.ny + j) * L + dep;
-}
-
-template <int W, int AX>
-__device__ __forceinline__ void quad_slab_load(const StepStatic& P, const float* psi, int i, int j, int k0,
-                                               QuadSlabs& S) {
-  const StepStatic::AxSlab& A = P.axd[AX][0];
-  const StepStatic::AxSlab& B = P.axd[AX][1];
-  if (AX == 2) {  // a quad may straddle a z-slab edge (the plan keeps it off the other slab)
-    S.hi[AX] = k0 + 3 >= B.lo && B.lo < B.hi;
-    S.in[AX] = S.hi[AX] || k0 < A.hi;
-    if (!S.in[AX]) return;
-    const int lo = side_of(S.hi[AX], B.lo, A.lo), hi = side_of(S.hi[AX], B.hi, A.hi);
-    S.zm = 0u;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) S.zm |= (k0 + e >= lo && k0 + e < hi) ? (1u << e) : 0u;
-  } else {
-    const int c = AX == 0 ? i : j;
-    S.hi[AX] = c >= B.lo && c < B.hi;
-    S.in[AX] = S.hi[AX] || (c >= A.lo && c < A.hi);
-    if (!S.in[AX]) return;
-  }
-  int dep, L, kap, aligned;
-  long long cells;
-  const float* cf;
-  const long long q = quad_psi_offset<W, AX>(P, S.hi[AX], i, j, k0, dep, cells, cf, L, kap, aligned);
-  if (AX != 2 || (aligned && S.zm == 15u)) {
-    S.p1[AX] = ld4(psi + q);
-    S.p2[AX] = ld4(psi + q + cells);
-  } else {
-    f4v a = {0.f, 0.f, 0.f, 0.f}, b = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if ((S.zm >> e) & 1u) {
-        a[e] = psi[q + e];
-        b[e] = psi[q + e + cells];
-      }
-    S.p1[AX] = a;
-    S.p2[AX] = b;
-  }
-}
-
-template <int W>
-__device__ __forceinline__ void quad_slab_loads(const StepStatic& P, const float* psi, int i, int j, int k0,
-                                                QuadSlabs& S) {
-  quad_slab_load<W, 0>(P, psi, i, j, k0, S);
-  quad_slab_load<W, 1>(P, psi, i, j, k0, S);
-  quad_slab_load<W, 2>(P, psi, i, j, k0, S);
-}
-
-template <int W, int AX>
-__device__ __forceinline__ void quad_slab_axis(const StepStatic& P, const QuadSlabs& S, float* psi, int i, int j,
-                                               int k0, const QuadDeriv& d, f4v& cx, f4v& cy, f4v& cz) {
-  if (!S.in[AX]) return;
-  int dep, L, kap, aligned;
-  long long cells;
-  const float* cf;
-  const long long q = quad_psi_offset<W, AX>(P, S.hi[AX], i, j, k0, dep, cells, cf, L, kap, aligned);
-  const bool whole = AX != 2 || S.zm == 15u;
-  // depths of the four cells (z: clamped into the slab for the cells outside it)
-  int de[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) de[e] = AX != 2 ? dep : (dep + e < 0 ? 0 : (dep + e >= L ? L - 1 : dep + e));
-  // z slabs with edges on quad boundaries: the quad's four depths are dep .. dep + 3 with dep and L
-  // multiples of 4, so each coefficient vector is one aligned dwordx4
-  const bool zvec = AX == 2 && whole && aligned;
-  f4v b, a;
-  if (zvec) {
-    b = ld4(cf + dep);
-    a = ld4(cf + L + dep);
-  } else if (AX == 2) {
-    b = f4v{cf[de[0]], cf[de[1]], cf[de[2]], cf[de[3]]};
-    a = f4v{cf[L + de[0]], cf[L + de[1]], cf[L + de[2]], cf[L + de[3]]};
-  } else {
-    const float bv = cf[dep], av = cf[L + dep];
-    b = f4v{bv, bv, bv, bv};
-    a = f4v{av, av, av, av};
-  }
-  const f4v d1 = AX == 0 ? d.x1 : (AX == 1 ? d.y1 : d.z1);
-  const f4v d2 = AX == 0 ? d.x2 : (AX == 1 ? d.y2 : d.z2);
-  const f4v n1 = b * S.p1[AX] + a * d1;
-  const f4v n2 = b * S.p2[AX] + a * d2;
-  f4v r1 = n1, r2 = n2;
-  if (!kap) {  // 1/kappa - 1
-    const float* km = cf + 2 * L;
-    f4v k;
-    if (zvec) k = ld4(km + dep);
-    else k = f4v{km[de[0]], km[de[1]], km[de[2]], km[de[3]]};
-    r1 = k * d1 + n1;
-    r2 = k * d2 + n2;
-  }
-  if (whole && (AX != 2 || aligned)) {
-    st4(psi + q, n1);
-    st4(psi + q + cells, n2);
-  } else {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      if (!((S.zm >> e) & 1u)) {  // outside the slab: no correction (an exact zero)
-        r1[e] = 0.f;
-        r2[e] = 0.f;
-        continue;
-      }
-      psi[q + e] = n1[e];
-      psi[q + e + cells] = n2[e];
-    }
-  }
-  // curl[(a+1)%3] += -corr1, curl[(a+2)%3] += corr2
-  if (AX == 0) {
-    cy = cy + (-r1);
-    cz = cz + r2;
-  } else if (AX == 1) {
-    cz = cz + (-r1);
-    cx = cx + r2;
-  } else {
-    cx = cx + (-r1);
-    cy = cy + r2;
-  }
-}
-
-template <int W>
-__device__ __forceinline__ void quad_slab_apply(const StepStatic& P, const QuadSlabs& S, float* psi, int i, int j,
-                                                int k0, const QuadDeriv& d, f4v& cx, f4v& cy, f4v& cz) {
-  quad_slab_axis<W, 0>(P, S, psi, i, j, k0, d, cx, cy, cz);
-  quad_slab_axis<W, 1>(P, S, psi, i, j, k0, d, cx, cy, cz);
-  quad_slab_axis<W, 2>(P, S, psi, i, j, k0, d, cx, cy, cz);
-}
-
-// Quad tiles whose mask holds anything beyond CPML slabs and the detector snapshot (sources, ADE
-// boxes, PEC / PMC faces, conductivity) are listed in vslow and run one cell per thread in a
-// launch of their own, four blocks per listed tile. Cell of block b: false past the last listed
-// tile.
-__device__ __forceinline__ bool slow_cell(const StepStatic& P, const int* list, long long nlist, long long b, int& i,
-                                          int& j, int& k, long long& o, uint32_t& m) {
+// The E half-step of quad tiles that meet an ADE box (listed in vslow) runs one cell per thread in a
+// launch of its own, four blocks per listed tile: the polarisation update would cost the quad
+// kernel its register budget. Cell of block b: false past the last listed tile.
+__device__ __forceinline__ bool slow_cell(const StepStatic& P, long long b, int& i, int& j, int& k, long long& o,
+                                          uint32_t& m) {
   const long long s = b >> 2;
-  if (s >= nlist) return false;
-  const long long lb = list[s];
+  if (s >= P.vnslow) return false;
+  const long long lb = P.vslow[s];
   m = P.vec_mask[lb];
   i = (int)(lb / P.vbpp);
   const int c = (int)(b & 3) * kBlock + threadIdx.x;  // cell of the quad tile, four per quad
   const int p = (int)(lb - (long long)i * P.vbpp) * kBlock + (c >> 2);
-  if (p >= P.ny * (P.nz / 4)) return false;
-  int k0;
-  perm_quad(P, p, j, k0);
+  if (p >= P.ny * P.nzq) return false;
+  int k0, sm;
+  perm_quad(P, p, j, k0, sm);
+  if ((c & 3) < sm) return false;
   k = k0 + (c & 3);
   o = (long long)i * P.plane + (long long)j * P.nz + k;
   return true;
 }
 
-// The listed quad tiles of the E (k_update_E4s) and H (k_update_H4s) sweeps, one cell per thread,
-// launched beside the quad kernels so that those keep a small register budget.
 template <int EC, bool X>
 __global__ __launch_bounds__(kBlock) void k_update_E4s(const StepStatic* __restrict__ Pp, const StepDyn D) {
   const StepStatic& P = as_const(Pp);
   int i, j, k;
   long long o;
   uint32_t ms;
-  if (slow_cell(P, P.vslow, P.vnslow, (long long)blockIdx.x, i, j, k, o, ms))
-    update_E_cell<EC, false, X>(P, D, D.n, ms, i, j, k, o);
-}
-
-template <int MC, bool X>
-__global__ __launch_bounds__(kBlock) void k_update_H4s(const StepStatic* __restrict__ Pp, const StepDyn D) {
-  const StepStatic& P = as_const(Pp);
-  int i, j, k;
-  long long o;
-  uint32_t ms;
-  if (slow_cell(P, P.vslowH, P.vnslowH, (long long)blockIdx.x, i, j, k, o, ms))
-    update_H_cell<MC, false, X>(P, D, D.n, D.record, ms, i, j, k, o);
+  if (slow_cell(P, (long long)blockIdx.x, i, j, k, o, ms)) update_E_cell<EC, false, X>(P, D, D.n, ms, i, j, k, o);
 }
 
 // CAX: the per-axis CPML (plans with StepStatic::cax), else the slab loop of cpml_quad.
-template <int EC, bool X, bool CAX>
+template <int EC, bool X, bool CAX, bool RAG>
 __global__ __launch_bounds__(kBlock) void k_update_E4(const StepStatic* __restrict__ Pp, const StepDyn D) {
   const StepStatic& P = as_const(Pp);
-  int i, j, k0;
+  int i, j, k0, sm;
   long long o;
   const long long lb = logical_block(P.xorder, P.vnblocks_pad);
-  if (!quad_of(P, lb, i, j, k0, o)) return;
+  if (!quad_of(P, lb, i, j, k0, sm, o)) return;
   const uint32_t m = P.vec_mask[lb];
   if (m & P.vlistE) return;  // a listed tile: its cells run in k_update_E4s
   QuadSlabs S;
   S.in[0] = S.in[1] = S.in[2] = false;
   S.hi[0] = S.hi[1] = S.hi[2] = false;
   const bool fast_slabs = CAX && (m & kSlabBits);
-  if (fast_slabs) quad_slab_loads<0>(P, D.psi, i, j, k0, S);
+  if (fast_slabs) quad_slab_loads<0, RAG>(P, D.psi, i, j, k0, S);
   const long long N = P.N;
   const float* Hx = D.H;
   const float* Hy = D.H + N;
@@ -897,9 +693,9 @@ __global__ __launch_bounds__(kBlock) void k_update_E4(const StepStatic* __restri
   long long dj, di, dk;
   const bool vj = prev_off<X>(P, 1, j, dj), vi = prev_off<X>(P, 0, i, di), vk = prev_off<X>(P, 2, k0, dk);
   const f4v z4 = {0.f, 0.f, 0.f, 0.f};
-  const f4v hx = ld4(Hx + o), hy = ld4(Hy + o), hz = ld4(Hz + o);
-  const f4v hxj = vj ? ld4(Hx + o + dj) : z4, hzj = vj ? ld4(Hz + o + dj) : z4;
-  const f4v hyi = vi ? ld4(Hy + o + di) : z4, hzi = vi ? ld4(Hz + o + di) : z4;
+  const f4v hx = ld4<RAG>(Hx + o), hy = ld4<RAG>(Hy + o), hz = ld4<RAG>(Hz + o);
+  const f4v hxj = vj ? ld4<RAG>(Hx + o + dj) : z4, hzj = vj ? ld4<RAG>(Hz + o + dj) : z4;
+  const f4v hyi = vi ? ld4<RAG>(Hy + o + di) : z4, hzi = vi ? ld4<RAG>(Hz + o + di) : z4;
   const float hxk = vk ? Hx[o + dk] : 0.f, hyk = vk ? Hy[o + dk] : 0.f;
   // k - 1 neighbours of the four cells: the previous cell of the quad, the neighbour quad's last
   const f4v hxm = {hxk, hx[0], hx[1], hx[2]};
@@ -914,18 +710,26 @@ __global__ __launch_bounds__(kBlock) void k_update_E4(const StepStatic* __restri
   f4v cx = d.y2 - d.z1;  // dy Hz - dz Hy
   f4v cy = d.z2 - d.x1;  // dz Hx - dx Hz
   f4v cz = d.x2 - d.y1;  // dx Hy - dy Hx
-  if (fast_slabs) quad_slab_apply<0>(P, S, D.psi, i, j, k0, d, cx, cy, cz);
+  if (fast_slabs) quad_slab_apply<0, RAG>(P, S, D.psi, i, j, k0, sm, true, d, cx, cy, cz);
   else if (!CAX && (m & kSlabBits)) cpml_quad(P, m, D.psi, 0, i, j, k0, d, cx, cy, cz);
-  const f4v iex = ld4(D.ie + o);
-  const f4v iey = EC == 3 ? ld4(D.ie + N + o) : iex;
-  const f4v iez = EC == 3 ? ld4(D.ie + 2 * N + o) : iex;
+  const f4v iex = ld4<RAG>(D.ie + o);
+  const f4v iey = EC == 3 ? ld4<RAG>(D.ie + N + o) : iex;
+  const f4v iez = EC == 3 ? ld4<RAG>(D.ie + 2 * N + o) : iex;
   float* Ex = D.E;
   float* Ey = D.E + N;
   float* Ez = D.E + 2 * N;
   const f4v c = {P.c, P.c, P.c, P.c};
-  st4(Ex + o, ld4(Ex + o) + (c * cx) * iex);
-  st4(Ey + o, ld4(Ey + o) + (c * cy) * iey);
-  st4(Ez + o, ld4(Ez + o) + (c * cz) * iez);
+  const f4v eo[3] = {ld4<RAG>(Ex + o), ld4<RAG>(Ey + o), ld4<RAG>(Ez + o)};
+  const f4v t[3] = {(c * cx) * iex, (c * cy) * iey, (c * cz) * iez};
+  f4v en[3] = {eo[0] + t[0], eo[1] + t[1], eo[2] + t[2]};
+  if (X && ((m >> kMaskLoss) & 1u)) {
+    const f4v inv[3] = {iex, iey, iez};
+    quad_loss<0>(P, i, j, k0, inv, eo, t, en);
+  }
+  st4m<RAG>(Ex + o, en[0], sm);
+  st4m<RAG>(Ey + o, en[1], sm);
+  st4m<RAG>(Ez + o, en[2], sm);
+  if (m & P.vpoint[0]) quad_points<0>(P, m, D.ie, D.im, D.E, D.n, i, j, k0, sm, o, EC, 0);
   if ((m & kSnapBit) && D.snap) {  // H_prev of the detector boxes, as update_E_cell
     const long long sy = D.shi[1] - D.slo[1], sz = D.shi[2] - D.slo[2];
     const long long sc = (long long)(D.shi[0] - D.slo[0]) * sy * sz;
@@ -940,20 +744,19 @@ __global__ __launch_bounds__(kBlock) void k_update_E4(const StepStatic* __restri
   }
 }
 
-template <int MC, bool X, bool CAX>
+template <int MC, bool X, bool CAX, bool RAG>
 __global__ __launch_bounds__(kBlock) void k_update_H4(const StepStatic* __restrict__ Pp, const StepDyn D) {
   const StepStatic& P = as_const(Pp);
-  int i, j, k0;
+  int i, j, k0, sm;
   long long o;
   const long long lb = logical_block(P.xorder, P.vnblocks_pad);
-  if (!quad_of(P, lb, i, j, k0, o)) return;
+  if (!quad_of(P, lb, i, j, k0, sm, o)) return;
   const uint32_t m = P.vec_mask[lb];
-  if (m & P.vlistH) return;  // a listed tile: its cells run in k_update_H4s
   QuadSlabs S;
   S.in[0] = S.in[1] = S.in[2] = false;
   S.hi[0] = S.hi[1] = S.hi[2] = false;
   const bool fast_slabs = CAX && (m & kSlabBits);
-  if (fast_slabs) quad_slab_loads<1>(P, D.psi, i, j, k0, S);
+  if (fast_slabs) quad_slab_loads<1, RAG>(P, D.psi, i, j, k0, S);
   const long long N = P.N;
   const float* Ex = D.E;
   const float* Ey = D.E + N;
@@ -961,9 +764,9 @@ __global__ __launch_bounds__(kBlock) void k_update_H4(const StepStatic* __restri
   long long dj, di, dk;
   const bool vj = next_off<X>(P, 1, j, dj), vi = next_off<X>(P, 0, i, di), vk = next_off<X>(P, 2, k0 + 3, dk);
   const f4v z4 = {0.f, 0.f, 0.f, 0.f};
-  const f4v ex = ld4(Ex + o), ey = ld4(Ey + o), ez = ld4(Ez + o);
-  const f4v exj = vj ? ld4(Ex + o + dj) : z4, ezj = vj ? ld4(Ez + o + dj) : z4;
-  const f4v eyi = vi ? ld4(Ey + o + di) : z4, ezi = vi ? ld4(Ez + o + di) : z4;
+  const f4v ex = ld4<RAG>(Ex + o), ey = ld4<RAG>(Ey + o), ez = ld4<RAG>(Ez + o);
+  const f4v exj = vj ? ld4<RAG>(Ex + o + dj) : z4, ezj = vj ? ld4<RAG>(Ez + o + dj) : z4;
+  const f4v eyi = vi ? ld4<RAG>(Ey + o + di) : z4, ezi = vi ? ld4<RAG>(Ez + o + di) : z4;
   const float exk = vk ? Ex[o + 3 + dk] : 0.f, eyk = vk ? Ey[o + 3 + dk] : 0.f;
   // k + 1 neighbours: the next cell of the quad, the neighbour quad's first
   const f4v exp_ = {ex[1], ex[2], ex[3], exk};
@@ -978,25 +781,37 @@ __global__ __launch_bounds__(kBlock) void k_update_H4(const StepStatic* __restri
   f4v cx = d.y2 - d.z1;  // dy Ez - dz Ey
   f4v cy = d.z2 - d.x1;  // dz Ex - dx Ez
   f4v cz = d.x2 - d.y1;  // dx Ey - dy Ex
-  if (fast_slabs) quad_slab_apply<1>(P, S, D.psi, i, j, k0, d, cx, cy, cz);
+  if (fast_slabs) quad_slab_apply<1, RAG>(P, S, D.psi, i, j, k0, sm, true, d, cx, cy, cz);
   else if (!CAX && (m & kSlabBits)) cpml_quad(P, m, D.psi, 1, i, j, k0, d, cx, cy, cz);
   float* Hx = D.H;
   float* Hy = D.H + N;
   float* Hz = D.H + 2 * N;
   const f4v one4 = {1.f, 1.f, 1.f, 1.f};
-  const f4v imx = MC ? ld4(D.im + o) : one4;
-  const f4v imy = MC == 3 ? ld4(D.im + N + o) : imx;
-  const f4v imz = MC == 3 ? ld4(D.im + 2 * N + o) : imx;
+  const f4v imx = MC ? ld4<RAG>(D.im + o) : one4;
+  const f4v imy = MC == 3 ? ld4<RAG>(D.im + N + o) : imx;
+  const f4v imz = MC == 3 ? ld4<RAG>(D.im + 2 * N + o) : imx;
   const f4v c = {P.c, P.c, P.c, P.c};
-  const f4v hx = ld4(Hx + o) - (c * cx) * imx;
-  const f4v hy = ld4(Hy + o) - (c * cy) * imy;
-  const f4v hz = ld4(Hz + o) - (c * cz) * imz;
-  st4(Hx + o, hx);
-  st4(Hy + o, hy);
-  st4(Hz + o, hz);
+  const f4v ho[3] = {ld4<RAG>(Hx + o), ld4<RAG>(Hy + o), ld4<RAG>(Hz + o)};
+  const f4v t[3] = {(c * cx) * imx, (c * cy) * imy, (c * cz) * imz};
+  f4v hn[3] = {ho[0] - t[0], ho[1] - t[1], ho[2] - t[2]};
+  if (X && ((m >> (kMaskLoss + 1)) & 1u)) {
+    const f4v inv[3] = {imx, imy, imz};
+    quad_loss<1>(P, i, j, k0, inv, ho, t, hn);
+  }
+  st4m<RAG>(Hx + o, hn[0], sm);
+  st4m<RAG>(Hy + o, hn[1], sm);
+  st4m<RAG>(Hz + o, hn[2], sm);
+  if (m & P.vpoint[1]) {
+    quad_points<1>(P, m, D.ie, D.im, D.H, D.n, i, j, k0, sm, o, 1, MC);
+    if (D.record) {  // the recorded layers hold the sources
+      hn[0] = ld4<RAG>(Hx + o);
+      hn[1] = ld4<RAG>(Hy + o);
+      hn[2] = ld4<RAG>(Hz + o);
+    }
+  }
   if (D.record && (m & kSlabBits)) {
 #pragma unroll 1
-    for (int e = 0; e < 4; ++e) record_iface(P, m, D.record, i, j, k0 + e, ex[e], ey[e], ez[e], hx[e], hy[e], hz[e]);
+    for (int e = RAG ? sm : 0; e < 4; ++e) record_iface(P, m, D.record, i, j, k0 + e, ex[e], ey[e], ez[e], hn[0][e], hn[1][e], hn[2][e]);
   }
 }
 
@@ -1270,45 +1085,36 @@ hipError_t launch_update_H(const StepStatic& P, const StepDyn& D, int mc, hipStr
   return hipGetLastError();
 }
 
+// Kernel of a quad sweep: x (periodic axes or conductivity), the per-axis CPML c, rows of nz % 4 != 0
+// cells rag (which always have the per-axis CPML).
+template <int EC>
+static SweepKernel quad_E(bool x, bool c, bool rag) {
+  if (rag) return x ? k_update_E4<EC, true, true, true> : k_update_E4<EC, false, true, true>;
+  if (c) return x ? k_update_E4<EC, true, true, false> : k_update_E4<EC, false, true, false>;
+  return x ? k_update_E4<EC, true, false, false> : k_update_E4<EC, false, false, false>;
+}
+
+template <int MC>
+static SweepKernel quad_H(bool x, bool c, bool rag) {
+  if (rag) return x ? k_update_H4<MC, true, true, true> : k_update_H4<MC, false, true, true>;
+  if (c) return x ? k_update_H4<MC, true, true, false> : k_update_H4<MC, false, true, false>;
+  return x ? k_update_H4<MC, true, false, false> : k_update_H4<MC, false, false, false>;
+}
+
 hipError_t launch_update_E4(const StepStatic& P, const StepDyn& D, int ec, hipStream_t s) {
-  const bool x = extras(P);
-  SweepKernel f;
-  SweepKernel fs;
-  const bool c = P.cax != 0;
-  if (ec == 3) {
-    f = x ? (c ? k_update_E4<3, true, true> : k_update_E4<3, true, false>)
-          : (c ? k_update_E4<3, false, true> : k_update_E4<3, false, false>);
-    fs = x ? k_update_E4s<3, true> : k_update_E4s<3, false>;
-  } else {
-    f = x ? (c ? k_update_E4<1, true, true> : k_update_E4<1, true, false>)
-          : (c ? k_update_E4<1, false, true> : k_update_E4<1, false, false>);
-    fs = x ? k_update_E4s<1, true> : k_update_E4s<1, false>;
-  }
+  const bool x = extras(P), c = P.cax != 0, rag = P.nz % 4 != 0;
+  const SweepKernel f = ec == 3 ? quad_E<3>(x, c, rag) : quad_E<1>(x, c, rag);
+  const SweepKernel fs = ec == 3 ? (x ? k_update_E4s<3, true> : k_update_E4s<3, false>)
+                                 : (x ? k_update_E4s<1, true> : k_update_E4s<1, false>);
   hipLaunchKernelGGL(f, dim3((unsigned)P.vnblocks_pad), dim3(kBlock), 0, s, P.self, D);
   if (P.vnslow) hipLaunchKernelGGL(fs, dim3((unsigned)(4 * P.vnslow)), dim3(kBlock), 0, s, P.self, D);
   return hipGetLastError();
 }
 
 hipError_t launch_update_H4(const StepStatic& P, const StepDyn& D, int mc, hipStream_t s) {
-  const bool x = extras(P);
-  SweepKernel f;
-  SweepKernel fs;
-  const bool c = P.cax != 0;
-  if (mc == 3) {
-    f = x ? (c ? k_update_H4<3, true, true> : k_update_H4<3, true, false>)
-          : (c ? k_update_H4<3, false, true> : k_update_H4<3, false, false>);
-    fs = x ? k_update_H4s<3, true> : k_update_H4s<3, false>;
-  } else if (mc == 1) {
-    f = x ? (c ? k_update_H4<1, true, true> : k_update_H4<1, true, false>)
-          : (c ? k_update_H4<1, false, true> : k_update_H4<1, false, false>);
-    fs = x ? k_update_H4s<1, true> : k_update_H4s<1, false>;
-  } else {
-    f = x ? (c ? k_update_H4<0, true, true> : k_update_H4<0, true, false>)
-          : (c ? k_update_H4<0, false, true> : k_update_H4<0, false, false>);
-    fs = x ? k_update_H4s<0, true> : k_update_H4s<0, false>;
-  }
+  const bool x = extras(P), c = P.cax != 0, rag = P.nz % 4 != 0;
+  const SweepKernel f = mc == 3 ? quad_H<3>(x, c, rag) : (mc == 1 ? quad_H<1>(x, c, rag) : quad_H<0>(x, c, rag));
   hipLaunchKernelGGL(f, dim3((unsigned)P.vnblocks_pad), dim3(kBlock), 0, s, P.self, D);
-  if (P.vnslowH) hipLaunchKernelGGL(fs, dim3((unsigned)(4 * P.vnslowH)), dim3(kBlock), 0, s, P.self, D);
   return hipGetLastError();
 }
 

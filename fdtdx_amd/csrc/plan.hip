@@ -546,8 +546,8 @@ static int plan_create(const fdtdx_plan_desc* d, fdtdx_plan** out) {
     P.cax = 0;
     P.acax = 0;
     const char* qenv = getenv("FDTDX_SWEEP");
-    const bool quad_ok = P.nz % 4 == 0 && d->eps_comps <= 3 && d->mu_comps <= 3 && !pl->cplx &&
-                         !(qenv && strcmp(qenv, "quad") != 0 && strcmp(qenv, "default") != 0);
+    bool quad_ok = P.nz >= 4 && d->eps_comps <= 3 && d->mu_comps <= 3 && !pl->cplx &&
+                   !(qenv && strcmp(qenv, "quad") != 0 && strcmp(qenv, "default") != 0);
     // per-axis CPML: every slab spans its face, at most one slab per side of an axis, the two sides
     // apart, and the x slabs before the y slabs before the z slabs in object order (the order in
     // which the corrections are added). The one-cell adjoint sweeps use it as it is (acax); the
@@ -577,8 +577,14 @@ static int plan_create(const fdtdx_plan_desc* d, fdtdx_plan** out) {
       // results; for comparing the two paths)
       const char* renv = getenv("FDTDX_REVERSE_CPML");
       P.acax = xyz && !(renv && strcmp(renv, "loop") == 0) ? 1 : 0;
-      const bool zq = !(P.axs[2][0] >= 0 && P.axs[2][1] >= 0 &&
-                        (P.slab[P.axs[2][0]].hi - 1) / 4 >= P.slab[P.axs[2][1]].lo / 4);  // no quad meets both
+      bool zq = true;  // no quad meets both z slabs (a row's last quad starts at nz - 4 or above)
+      if (xyz && P.axs[2][0] >= 0 && P.axs[2][1] >= 0) {
+        const int zhi0 = P.slab[P.axs[2][0]].hi, zlo1 = P.slab[P.axs[2][1]].lo;
+        zq = (zhi0 - 1) / 4 < zlo1 / 4 && (P.nz % 4 == 0 || P.nz - 4 >= zhi0);
+      }
+      // rows of nz % 4 != 0 cells only with the per-axis CPML: the slab loop's vector path needs
+      // aligned quads
+      if (P.nz % 4 && !(xyz && zq)) quad_ok = false;
       P.cax = quad_ok && xyz && zq ? 1 : 0;
       for (int u = 0; u < 3; ++u) P.axord[u] = ord[u];
       for (int a = 0; a < 3; ++a)
@@ -601,7 +607,8 @@ static int plan_create(const fdtdx_plan_desc* d, fdtdx_plan** out) {
       // quads of a group of rows, then its z-slab quads) when the z-slab edges fall on quad
       // boundaries. With it they run row-major: the 400x400x200 forward measured 0.293 / 0.261 ms
       // per E / H sweep row-major against 0.313 / 0.283 ms in the row-grouped order.
-      const int nzq = P.nz / 4;
+      const int nzq = (P.nz + 3) / 4;
+      P.nzq = nzq;
       P.vzlo = 0;
       P.vzhi = nzq;
       if (!P.cax && perm && P.zlo % 4 == 0 && P.zhi % 4 == 0) {
@@ -626,10 +633,17 @@ static int plan_create(const fdtdx_plan_desc* d, fdtdx_plan** out) {
         const int i = (int)(lb / P.vbpp);
         const long long q0 = (lb - (long long)i * P.vbpp) * kBlock;
         const long long q1 = std::min(q0 + kBlock, nq) - 1;
+        if (!vperm) {  // row-major: the footprint from the first and the last quad
+          const int jlo = (int)(q0 / nzq), jhi = (int)(q1 / nzq);
+          const int klo = jlo == jhi ? std::min(4 * (int)(q0 % nzq), P.nz - 4) : 0;
+          const int khi = jlo == jhi ? std::min(4 * (int)(q1 % nzq), P.nz - 4) + 3 : P.nz - 1;
+          vm[(size_t)lb] = box_mask(i, jlo, jhi, klo, khi, false);
+          continue;
+        }
         int lo[2][2] = {{P.ny, P.nz}, {P.ny, P.nz}}, hi[2][2] = {{-1, -1}, {-1, -1}};
         for (long long q = q0; q <= q1; ++q) {
-          int j, k;
-          perm_quad(P, (int)q, j, k);
+          int j, k, sm;
+          perm_quad(P, (int)q, j, k, sm);
           const int c = (k < P.zlo || k >= P.zhi) ? 1 : 0;
           lo[c][0] = std::min(lo[c][0], j); hi[c][0] = std::max(hi[c][0], j);
           lo[c][1] = std::min(lo[c][1], k); hi[c][1] = std::max(hi[c][1], k + 3);
@@ -640,29 +654,20 @@ static int plan_create(const fdtdx_plan_desc* d, fdtdx_plan** out) {
         vm[(size_t)lb] = m;
       }
       if ((rc = pl->upload(vm.data(), vm.size(), &P.vec_mask))) return bail(rc);
-      // listed tiles, one cell per thread: those of the E half-step have descriptors beyond CPML
-      // slabs and the snapshot; those of the H half-step beyond these and ADE boxes, which only
-      // the E half-step reads (a quad-vectorised ADE sweep measured slower than the one-cell one:
-      // 0.245 against 0.236 ms per E sweep of the 256^3 dispersive case)
-      // The descriptors each half-step reads: E sources, PEC faces, ADE boxes and electric
-      // conductivity for E; H sources, PMC faces and magnetic conductivity for H.
-      uint32_t eb = ((1u << FDTDX_MAX_ADE) - 1u) << kMaskAde | (1u << kMaskLoss);
-      uint32_t hb = 1u << (kMaskLoss + 1);
-      for (int q = 0; q < P.nsrc; ++q) (P.src[q].field == 0 ? eb : hb) |= 1u << (kMaskSrc + q);
-      for (int w = 0; w < P.nwall; ++w) (P.wall[w].kind == FDTDX_WALL_PEC ? eb : hb) |= 1u << (kMaskWall + w);
-      P.vlistE = eb;
-      P.vlistH = hb;
-      std::vector<int> slow, slowH;
-      for (long long lb = 0; lb < P.vnblocks; ++lb) {
-        if (vm[(size_t)lb] & eb) slow.push_back((int)lb);
-        if (vm[(size_t)lb] & hb) slowH.push_back((int)lb);
-      }
+      // listed tiles, one cell per thread: those whose E half-step meets an ADE box (a
+      // quad-vectorised ADE sweep measured slower than the one-cell one: 0.245 against 0.236 ms per
+      // E sweep of the 256^3 dispersive case); conductivity, sources and conducting faces run in the
+      // quad sweeps
+      P.vlistE = ((1u << FDTDX_MAX_ADE) - 1u) << kMaskAde;
+      P.vpoint[0] = P.vpoint[1] = 0u;
+      for (int q = 0; q < P.nsrc; ++q) P.vpoint[P.src[q].field] |= 1u << (kMaskSrc + q);
+      for (int w = 0; w < P.nwall; ++w) P.vpoint[P.wall[w].kind == FDTDX_WALL_PEC ? 0 : 1] |= 1u << (kMaskWall + w);
+      std::vector<int> slow;
+      for (long long lb = 0; lb < P.vnblocks; ++lb)
+        if (vm[(size_t)lb] & P.vlistE) slow.push_back((int)lb);
       P.vnslow = (long long)slow.size();
       P.vslow = nullptr;
       if (!slow.empty() && (rc = pl->upload(slow.data(), slow.size(), &P.vslow))) return bail(rc);
-      P.vnslowH = (long long)slowH.size();
-      P.vslowH = nullptr;
-      if (!slowH.empty() && (rc = pl->upload(slowH.data(), slowH.size(), &P.vslowH))) return bail(rc);
       P.vq = 1;
     }
   }

@@ -1,0 +1,292 @@
+// Device helpers of the kernels that update four consecutive z cells (a quad) per lane: the two
+// sweeps of fwd_kernels.hip and the single-pass step of fused_kernels.hip. Every field array moves
+// as dwordx4, the z neighbours inside a quad come from the lane's own registers. Per cell the
+// arithmetic is that of the one-cell sweeps, in the same order, so results are bit-identical.
+//
+// Rows of nz cells with nz not a multiple of 4 (RAG): the row's last quad starts at nz - 4 and so
+// repeats up to 3 cells of the quad before it. Both lanes compute these cells from the same
+// inputs (a sweep reads only its own cells of the field it writes), only the first stores them:
+// `sm` is the number of leading cells a lane leaves out of its stores. Accesses are then aligned to
+// 4 bytes only, which global dwordx4 accesses allow.
+#pragma once
+#include "engine_common.h"
+#include "stencil.h"
+
+namespace fdtdx {
+
+typedef float f4v __attribute__((ext_vector_type(4)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+
+template <bool RAG = false>
+__device__ __forceinline__ f4v ld4(const float* p) {
+  if constexpr (RAG) return *reinterpret_cast<const f4u*>(p);
+  else return *reinterpret_cast<const f4v*>(p);
+}
+
+__device__ __forceinline__ void st4(float* p, f4v v) { *reinterpret_cast<f4v*>(p) = v; }
+
+// Store of the cells e >= sm of a quad.
+template <bool RAG>
+__device__ __forceinline__ void st4m(float* p, f4v v, int sm) {
+  if constexpr (!RAG) {
+    st4(p, v);
+  } else if (sm == 0) {
+    *reinterpret_cast<f4u*>(p) = v;
+  } else {
+#pragma unroll
+    for (int e = 1; e < 4; ++e)
+      if (e >= sm) p[e] = v[e];
+  }
+}
+
+constexpr uint32_t kSlabBits = (1u << FDTDX_MAX_CPML) - 1u;
+constexpr uint32_t kSnapBit = 1u << kMaskSnap;
+
+// One-sided derivatives of the four cells of a quad, one vector per (axis, component) pair that
+// feeds a CPML slab: curl H uses (dx Hz, dx Hy), (dy Hx, dy Hz), (dz Hy, dz Hx), curl E the same
+// pairs of E (the order of pml_pair).
+struct QuadDeriv {
+  f4v x1, x2, y1, y2, z1, z2;
+};
+
+// Per-axis CPML of a quad (StepStatic::cax): the quad meets at most one slab per axis, the x slab
+// fixed by i, the y slab by j and the z slab by k0 (a quad across a z-slab edge updates the cells
+// inside the slab one by one). Every psi load is issued before any is used (quad_slab_loads, ahead
+// of the field loads), then the corrections are added x, y, z, i.e. in slab order (quad_slab_apply)
+// with cpml_slab's arithmetic. Descriptor fields are read for both sides of an axis (wave-uniform)
+// and selected per lane.
+struct QuadSlabs {
+  bool in[3], hi[3];  // the quad meets the axis's slab; of its max side
+  unsigned zm;        // cells of the quad inside its z slab (bit e: cell k0 + e)
+  f4v p1[3], p2[3];   // psi1, psi2 of the quad in that slab (zero for cells outside it)
+};
+
+// Descriptor fields of the slab of one side of axis AX (wave-uniform), and the float offset of psi1
+// of cell (i, j, k0) in it (for the z axis k0 - lo may be negative or reach past the slab when the
+// quad straddles a slab edge; only the cells inside are addressed).
+template <int W, int AX>
+__device__ __forceinline__ long long quad_psi_offset(const StepStatic& P, bool hi, int i, int j, int k0, int& dep,
+                                                     long long& cells, const float*& cf, int& L, int& kap,
+                                                     int& aligned) {
+  const StepStatic::AxSlab& A = P.axd[AX][0];
+  const StepStatic::AxSlab& B = P.axd[AX][1];
+  const int lo = side_of(hi, B.lo, A.lo);
+  L = side_of(hi, B.L, A.L);
+  cells = side_of(hi, B.cells, A.cells);
+  cf = side_of(hi, B.coef, A.coef) + (W ? 3 * L : 0);
+  kap = side_of(hi, B.kappa_one, A.kappa_one);
+  aligned = side_of(hi, B.aligned, A.aligned);
+  dep = (AX == 0 ? i : (AX == 1 ? j : k0)) - lo;
+  const long long base = side_of(hi, B.psi_off, A.psi_off) + (W ? 2 * cells : 0);
+  if (AX == 0) return base + (long long)dep * P.plane + (long long)j * P.nz + k0;
+  if (AX == 1) return base + ((long long)i * L + dep) * P.nz + k0;
+  return base + ((long long)i * P.ny + j) * L + dep;
+}
+
+template <int W, int AX, bool RAG>
+__device__ __forceinline__ void quad_slab_load(const StepStatic& P, const float* psi, int i, int j, int k0,
+                                               QuadSlabs& S) {
+  const StepStatic::AxSlab& A = P.axd[AX][0];
+  const StepStatic::AxSlab& B = P.axd[AX][1];
+  if (AX == 2) {  // a quad may straddle a z-slab edge (the plan keeps it off the other slab)
+    S.hi[AX] = k0 + 3 >= B.lo && B.lo < B.hi;
+    S.in[AX] = S.hi[AX] || k0 < A.hi;
+    if (!S.in[AX]) return;
+    const int lo = side_of(S.hi[AX], B.lo, A.lo), hi = side_of(S.hi[AX], B.hi, A.hi);
+    S.zm = 0u;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) S.zm |= (k0 + e >= lo && k0 + e < hi) ? (1u << e) : 0u;
+  } else {
+    const int c = AX == 0 ? i : j;
+    S.hi[AX] = c >= B.lo && c < B.hi;
+    S.in[AX] = S.hi[AX] || (c >= A.lo && c < A.hi);
+    if (!S.in[AX]) return;
+  }
+  int dep, L, kap, aligned;
+  long long cells;
+  const float* cf;
+  const long long q = quad_psi_offset<W, AX>(P, S.hi[AX], i, j, k0, dep, cells, cf, L, kap, aligned);
+  if (AX != 2 || (S.zm == 15u && (RAG || aligned))) {
+    S.p1[AX] = ld4<RAG>(psi + q);
+    S.p2[AX] = ld4<RAG>(psi + q + cells);
+  } else {
+    f4v a = {0.f, 0.f, 0.f, 0.f}, b = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if ((S.zm >> e) & 1u) {
+        a[e] = psi[q + e];
+        b[e] = psi[q + e + cells];
+      }
+    S.p1[AX] = a;
+    S.p2[AX] = b;
+  }
+}
+
+template <int W, bool RAG>
+__device__ __forceinline__ void quad_slab_loads(const StepStatic& P, const float* psi, int i, int j, int k0,
+                                                QuadSlabs& S) {
+  quad_slab_load<W, 0, RAG>(P, psi, i, j, k0, S);
+  quad_slab_load<W, 1, RAG>(P, psi, i, j, k0, S);
+  quad_slab_load<W, 2, RAG>(P, psi, i, j, k0, S);
+}
+
+// store: write the advanced psi of the cells e >= sm to psi_out (false: a recomputed halo quad).
+template <int W, int AX, bool RAG>
+__device__ __forceinline__ void quad_slab_axis(const StepStatic& P, const QuadSlabs& S, float* psi_out, int i, int j,
+                                               int k0, int sm, bool store, const QuadDeriv& d, f4v& cx, f4v& cy,
+                                               f4v& cz) {
+  if (!S.in[AX]) return;
+  int dep, L, kap, aligned;
+  long long cells;
+  const float* cf;
+  const long long q = quad_psi_offset<W, AX>(P, S.hi[AX], i, j, k0, dep, cells, cf, L, kap, aligned);
+  const bool whole = AX != 2 || S.zm == 15u;
+  // depths of the four cells (z: clamped into the slab for the cells outside it)
+  int de[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) de[e] = AX != 2 ? dep : (dep + e < 0 ? 0 : (dep + e >= L ? L - 1 : dep + e));
+  // z slabs with edges on quad boundaries: the quad's four depths are dep .. dep + 3 with dep and L
+  // multiples of 4, so each coefficient vector is one aligned dwordx4 (unaligned rows: any whole quad)
+  const bool zvec = AX == 2 && whole && (RAG || aligned);
+  f4v b, a;
+  if (zvec) {
+    b = ld4<RAG>(cf + dep);
+    a = ld4<RAG>(cf + L + dep);
+  } else if (AX == 2) {
+    b = f4v{cf[de[0]], cf[de[1]], cf[de[2]], cf[de[3]]};
+    a = f4v{cf[L + de[0]], cf[L + de[1]], cf[L + de[2]], cf[L + de[3]]};
+  } else {
+    const float bv = cf[dep], av = cf[L + dep];
+    b = f4v{bv, bv, bv, bv};
+    a = f4v{av, av, av, av};
+  }
+  const f4v d1 = AX == 0 ? d.x1 : (AX == 1 ? d.y1 : d.z1);
+  const f4v d2 = AX == 0 ? d.x2 : (AX == 1 ? d.y2 : d.z2);
+  const f4v n1 = b * S.p1[AX] + a * d1;
+  const f4v n2 = b * S.p2[AX] + a * d2;
+  f4v r1 = n1, r2 = n2;
+  if (!kap) {  // 1/kappa - 1
+    const float* km = cf + 2 * L;
+    f4v k;
+    if (zvec) k = ld4<RAG>(km + dep);
+    else k = f4v{km[de[0]], km[de[1]], km[de[2]], km[de[3]]};
+    r1 = k * d1 + n1;
+    r2 = k * d2 + n2;
+  }
+  if (AX != 2 || zvec) {
+    if (store) {
+      st4m<RAG>(psi_out + q, n1, sm);
+      st4m<RAG>(psi_out + q + cells, n2, sm);
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (!((S.zm >> e) & 1u)) {  // outside the slab: no correction (an exact zero)
+        r1[e] = 0.f;
+        r2[e] = 0.f;
+        continue;
+      }
+      if (store && e >= sm) {
+        psi_out[q + e] = n1[e];
+        psi_out[q + e + cells] = n2[e];
+      }
+    }
+  }
+  // curl[(a+1)%3] += -corr1, curl[(a+2)%3] += corr2
+  if (AX == 0) {
+    cy = cy + (-r1);
+    cz = cz + r2;
+  } else if (AX == 1) {
+    cz = cz + (-r1);
+    cx = cx + r2;
+  } else {
+    cx = cx + (-r1);
+    cy = cy + r2;
+  }
+}
+
+template <int W, bool RAG>
+__device__ __forceinline__ void quad_slab_apply(const StepStatic& P, const QuadSlabs& S, float* psi_out, int i, int j,
+                                                int k0, int sm, bool store, const QuadDeriv& d, f4v& cx, f4v& cy,
+                                                f4v& cz) {
+  quad_slab_axis<W, 0, RAG>(P, S, psi_out, i, j, k0, sm, store, d, cx, cy, cz);
+  quad_slab_axis<W, 1, RAG>(P, S, psi_out, i, j, k0, sm, store, d, cx, cy, cz);
+  quad_slab_axis<W, 2, RAG>(P, S, psi_out, i, j, k0, sm, store, d, cx, cy, cz);
+}
+
+// Conductivity of a quad (loss_x and the update of update_E_cell / update_H_cell): f the field before
+// the step, t = (c curl) inv, n the lossless result, replaced for the cells inside the box.
+template <int W>
+__device__ __forceinline__ void quad_loss(const StepStatic& P, int i, int j, int k0, const f4v* inv, const f4v* f,
+                                          const f4v* t, f4v* n) {
+  const LossK& L = P.loss[W];
+  if (i < L.lo[0] || i >= L.hi[0] || j < L.lo[1] || j >= L.hi[1] || k0 + 3 < L.lo[2] || k0 >= L.hi[2]) return;
+  const long long q = ((long long)(i - L.lo[0]) * L.by + (j - L.lo[1])) * L.bz + (k0 - L.lo[2]);
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (k0 + e < L.lo[2] || k0 + e >= L.hi[2]) continue;
+      const float sg = L.sig[(L.comps == 3 ? a : 0) * L.cells + q + e];
+      const float x = W == 0 ? (((P.c * sg) * P.eta0) * inv[a][e]) / 2.0f : (((P.c * sg) / P.eta0) * inv[a][e]) / 2.0f;
+      const float g = (1.0f - x) * f[a][e];
+      n[a][e] = (W == 0 ? g + t[a][e] : g - t[a][e]) / (1.0f + x);
+    }
+  }
+}
+
+// Sources and conducting faces of field W (0: E, PEC; 1: H, PMC) over a quad, after its update has
+// been stored: the cells e >= sm are read back, changed and stored one by one (rolled, so that the
+// few quads that hold one cost the others no registers). m: the tile's mask. Before, such tiles
+// ran one cell per lane in launches of their own: 6 to 9 us each whatever the grid, against no
+// measurable time here (steps of the 64^3 dipole 49.5 -> 44.6 us, the 128x128x64 plane wave 45.2
+// -> 37.8, the 200x200x100 dipole 77.7 -> 70.4, the 400x400x200 plane wave 529 -> 511).
+template <int W>
+__device__ __forceinline__ void quad_points(const StepStatic& P, uint32_t m, const float* ie, const float* im,
+                                            float* F, int n, int i, int j, int k0, int sm, long long o, int ec,
+                                            int mc) {
+  bool hit = false;
+  for (uint32_t mm = (m >> kMaskSrc) & ((1u << P.nsrc) - 1u); mm; mm &= mm - 1u) {
+    const SrcK& sr = P.src[__builtin_ctz(mm)];
+    hit = hit || (sr.field == W && i >= sr.lo[0] && i < sr.hi[0] && j >= sr.lo[1] && j < sr.hi[1] &&
+                  k0 + 3 >= sr.lo[2] && k0 < sr.hi[2]);
+  }
+  for (uint32_t mm = (m >> kMaskWall) & ((1u << P.nwall) - 1u); mm; mm &= mm - 1u) {
+    const WallK& w = P.wall[__builtin_ctz(mm)];
+    const int c = w.axis == 0 ? i : (w.axis == 1 ? j : k0);
+    hit = hit || (w.kind == (W ? FDTDX_WALL_PMC : FDTDX_WALL_PEC) && w.index >= c && w.index <= (w.axis == 2 ? c + 3 : c));
+  }
+  if (!hit) return;
+  float* p = F + o;
+#pragma unroll 1
+  for (int e = sm; e < 4; ++e) {
+    float x = p[e], y = p[P.N + e], z = p[2 * P.N + e];
+    apply_sources<false>(P, m, ie, im, W, n, false, i, j, k0 + e, o + e, ec, mc, x, y, z);
+    apply_walls(P, m, W ? FDTDX_WALL_PMC : FDTDX_WALL_PEC, i, j, k0 + e, x, y, z);
+    p[e] = x;
+    p[P.N + e] = y;
+    p[2 * P.N + e] = z;
+  }
+}
+
+// collect_interfaces (update.py:1140-1178, fdtd/misc.py:10-35): the float32 E and H of a cell on
+// a slab's interface plane into step n's record slot.
+__device__ __forceinline__ void record_iface(const StepStatic& P, uint32_t m, char* record, int i, int j, int k,
+                                             float ex, float ey, float ez, float hx, float hy, float hz) {
+#pragma unroll
+  for (int s = 0; s < FDTDX_MAX_CPML; ++s) {
+    if (s >= P.nslab) break;
+    if (!((m >> s) & 1u)) continue;
+    const SlabK& sl = P.slab[s];
+    const int coord = sl.axis == 0 ? i : (sl.axis == 1 ? j : k);
+    if (coord != sl.iface) continue;
+    const long long pc = (long long)sl.pn0 * sl.pn1;
+    const long long q = sl.axis == 0 ? (long long)j * P.nz + k : (sl.axis == 1 ? (long long)i * P.nz + k : (long long)i * P.ny + j);
+    float* fe = (float*)(record + sl.rec_off_E);
+    float* fh = (float*)(record + sl.rec_off_H);
+    fe[q] = ex; fe[pc + q] = ey; fe[2 * pc + q] = ez;
+    fh[q] = hx; fh[pc + q] = hy; fh[2 * pc + q] = hz;
+  }
+}
+
+}  // namespace fdtdx

@@ -470,6 +470,57 @@ def test_quad_sweeps_equal_one_cell_sweeps_bitwise(case, monkeypatch):
         assert np.array_equal(a, b)
 
 
+def _ragged_cases():
+    """Rows of nz % 4 != 0 cells: the last quad of a row repeats cells of the quad before it."""
+    c1 = W.scenario_c1(T=60, n=29, pml=5, cube=6)                                  # nz % 4 = 1
+    c2 = W.scenario_c2(T=50, shape=(44, 36, 30), pml=6, slab=(12, 12, 8))          # nz % 4 = 2, H sources
+    c4 = W.scenario_c4(T=50, n=35, pml=8, slab=(12, 12, 8), cube=4)                # nz % 4 = 3, ADE tiles
+    lossy = W.scenario_c1(T=60, n=27, pml=4, cube=6)                               # conductivity, walls, mu
+    lossy["pml"] = dict(lossy["pml"], types={"max_x": "pec", "max_z": "pec"})
+    lossy["boxes"] = lossy["boxes"] + [
+        dict(slc=((14, 24), (8, 20), (18, 27)), eps=2.0, sigma_E=(3e4, 1e4, 2e4), sigma_H=2e9, mu=(1.5, 2.0, 2.5))]
+    per = W.scenario_c2(T=50, shape=(48, 24, 21), pml=6, slab=(16, 12, 8))        # periodic y, z
+    per["pml"] = dict(per["pml"], types={"min_y": "periodic", "max_y": "periodic", "min_z": "periodic",
+                                         "max_z": "periodic"})
+    thin = W.scenario_c1(T=40, n=24, pml=4, cube=4)                                # two quads per row, no z CPML
+    thin["shape"] = (24, 24, 5)
+    thin["pml"] = dict(thin["pml"], types={"min_z": "pec", "max_z": "pec"})
+    thin["boxes"] = [dict(slc=((8, 12), (8, 12), (1, 4)), eps=2.25)]
+    thin["sources"][0]["cell"] = (12, 12, 2)
+    thin["detectors"] = []
+    return {"mod1": c1, "mod2": c2, "mod3_ade": c4, "lossy_walls_mu": lossy, "periodic": per, "thin": thin}
+
+
+@pytest.mark.parametrize("case", ["mod1", "mod2", "mod3_ade", "lossy_walls_mu", "periodic", "thin"])
+def test_ragged_quad_sweeps_equal_one_cell_sweeps_bitwise(case, monkeypatch):
+    """The quad sweeps over rows whose length is no multiple of four against one cell per lane: the
+    same operations in the same order, so every state agrees bit for bit."""
+    import torch
+
+    from fdtdx_amd import fdtd as F
+    import scenarios
+
+    spec = _ragged_cases()[case]
+    assert spec["shape"][2] % 4 != 0
+    out = {}
+    for mode in ("two", "quad"):
+        _set_mode(monkeypatch, mode)
+        objects, arrays, params, config = scenarios.build(spec)
+        rec = 0 if case == "mod3_ade" else spec["T"]
+        s = F.Solve(objects, config, arrays, record_steps=rec)
+        assert s.plan.quad == (mode == "quad")
+        arrays.reset()
+        print(f"case {case} mode {mode}", flush=True)
+        s.forward(0, spec["T"], record=bool(rec))
+        torch.cuda.synchronize()
+        out[mode] = [arrays.fields.E.cpu().numpy(), arrays.fields.H.cpu().numpy(), arrays.psi.cpu().numpy()]
+        out[mode] += [s.record.cpu().numpy()] if s.record is not None else []
+        out[mode] += [t.cpu().numpy() for t in s.det_tensors()]
+    assert np.abs(out["two"][0]).max() > 0
+    for a, b in zip(out["quad"], out["two"]):
+        assert np.array_equal(a, b)
+
+
 def test_gaussian_mode_overlap_matches_oracle():
     """GaussianModeOverlapDetector (detectors/mode.py:666-798): the engine's 6-component phasor
     plane and the overlap with the diverging Gaussian reference at three frequencies against the
