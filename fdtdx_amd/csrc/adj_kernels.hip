@@ -17,6 +17,7 @@
 // becomes mu_E (c K - c sigma eta0 E^n) / (1 + x)^2; sigma is a constant (initialization.py:287).
 #include "engine_common.h"
 #include "kernels.h"
+#include "quad.h"
 #include "stencil.h"
 
 namespace fdtdx {
@@ -605,6 +606,324 @@ __global__ __launch_bounds__(kBlock) void k_adj_B(const StepStatic* __restrict__
   A.lamH[2 * P.N + o] = lh[2];
 }
 
+// ---------------------------------------------------------------- four z cells per lane (aquad)
+// Passes A and B over quads: the arithmetic of the one-cell passes per cell, in the same order, with
+// dwordx4 accesses and the z neighbours from the lane's own registers. A pass reads its neighbours'
+// values of fields it does not write, and its own cells of those it writes, so the cells that a row's
+// last quad repeats (quad.h) are safe.
+
+// One axis of the transposed CPML of a quad: lam_psi of the quad and of its neighbour at DIR along
+// the axis, both in the same slab if they are in one (the plan keeps the two slabs of an axis apart).
+struct QuadPair {
+  unsigned zm, nm;      // cells of the quad inside the slab; cells whose neighbour is inside it
+  f4v p1, p2, n1, n2;   // lam_psi of the cells and of their neighbours
+  f4v a, b, an;
+  f4v km, kn;           // 1/kappa - 1 (with kap only)
+  bool kap;
+  long long q, cells;
+  bool vec;             // the whole quad moves as dwordx4
+};
+
+template <int W, int AX, int DIR, bool RAG>
+__device__ __forceinline__ bool quad_pair(const StepStatic& P, const float* psi, int i, int j, int k0, QuadPair& t) {
+  const StepStatic::AxSlab& A = P.axd[AX][0];
+  const StepStatic::AxSlab& B = P.axd[AX][1];
+  const int c = AX == 0 ? i : (AX == 1 ? j : k0);
+  const int c0 = AX == 2 ? (DIR < 0 ? c - 1 : c) : (DIR < 0 ? c - 1 : c);  // first and last coordinate involved
+  const int c1 = AX == 2 ? (DIR < 0 ? c + 3 : c + 4) : (DIR < 0 ? c : c + 1);
+  const bool hi = c1 >= B.lo && c0 < B.hi && B.lo < B.hi;
+  if (!hi && !(c1 >= A.lo && c0 < A.hi && A.lo < A.hi)) return false;
+  const int lo = side_of(hi, B.lo, A.lo), up = side_of(hi, B.hi, A.hi), L = side_of(hi, B.L, A.L);
+  const int dep = c - lo;
+  t.cells = side_of(hi, B.cells, A.cells);
+  t.kap = !side_of(hi, B.kappa_one, A.kappa_one);
+  t.q = ax_psi<AX>(P, side_of(hi, B.psi_off, A.psi_off), W, t.cells, L, dep, i, j, k0);
+  const float* cf = side_of(hi, B.coef, A.coef) + (W ? 3 * L : 0);
+  const f4v z4 = {0.f, 0.f, 0.f, 0.f};
+  t.p1 = t.p2 = t.n1 = t.n2 = t.a = t.b = t.an = t.km = t.kn = z4;
+  if constexpr (AX != 2) {
+    const bool in = c >= lo && c < up, nin = c + DIR >= lo && c + DIR < up;
+    t.zm = in ? 15u : 0u;
+    t.nm = nin ? 15u : 0u;
+    t.vec = true;
+    const long long stride = AX == 0 ? P.plane : (long long)P.nz;
+    if (in) {
+      t.p1 = ld4<RAG>(psi + t.q);
+      t.p2 = ld4<RAG>(psi + t.q + t.cells);
+      const float b = cf[dep], a = cf[L + dep];
+      t.b = f4v{b, b, b, b};
+      t.a = f4v{a, a, a, a};
+      if (t.kap) {
+        const float km = cf[2 * L + dep];
+        t.km = f4v{km, km, km, km};
+      }
+    }
+    if (nin) {
+      t.n1 = ld4<RAG>(psi + t.q + DIR * stride);
+      t.n2 = ld4<RAG>(psi + t.q + t.cells + DIR * stride);
+      const float a = cf[L + dep + DIR];
+      t.an = f4v{a, a, a, a};
+      if (t.kap) {
+        const float km = cf[2 * L + dep + DIR];
+        t.kn = f4v{km, km, km, km};
+      }
+    }
+  } else {
+    const int ke = DIR < 0 ? -1 : 4;  // the cell beside the quad
+    const bool ein = c + ke >= lo && c + ke < up;
+    t.zm = 0u;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) t.zm |= (c + e >= lo && c + e < up) ? (1u << e) : 0u;
+    t.nm = DIR < 0 ? (((t.zm << 1) & 15u) | (ein ? 1u : 0u)) : ((t.zm >> 1) | (ein ? 8u : 0u));
+    t.vec = t.zm == 15u && (RAG || side_of(hi, B.aligned, A.aligned));
+    if (t.vec) {
+      t.p1 = ld4<RAG>(psi + t.q);
+      t.p2 = ld4<RAG>(psi + t.q + t.cells);
+      t.b = ld4<RAG>(cf + dep);
+      t.a = ld4<RAG>(cf + L + dep);
+      if (t.kap) t.km = ld4<RAG>(cf + 2 * L + dep);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if ((t.zm >> e) & 1u) {
+          t.p1[e] = psi[t.q + e];
+          t.p2[e] = psi[t.q + t.cells + e];
+          t.b[e] = cf[dep + e];
+          t.a[e] = cf[L + dep + e];
+          if (t.kap) t.km[e] = cf[2 * L + dep + e];
+        }
+    }
+    float e1 = 0.f, e2 = 0.f, ea = 0.f, ek = 0.f;
+    if (ein) {
+      e1 = psi[t.q + ke];
+      e2 = psi[t.q + t.cells + ke];
+      ea = cf[L + dep + ke];
+      if (t.kap) ek = cf[2 * L + dep + ke];
+    }
+    if (DIR < 0) {
+      t.n1 = f4v{e1, t.p1[0], t.p1[1], t.p1[2]};
+      t.n2 = f4v{e2, t.p2[0], t.p2[1], t.p2[2]};
+      t.an = f4v{ea, t.a[0], t.a[1], t.a[2]};
+      t.kn = f4v{ek, t.km[0], t.km[1], t.km[2]};
+    } else {
+      t.n1 = f4v{t.p1[1], t.p1[2], t.p1[3], e1};
+      t.n2 = f4v{t.p2[1], t.p2[2], t.p2[3], e2};
+      t.an = f4v{t.a[1], t.a[2], t.a[3], ea};
+      t.kn = f4v{t.km[1], t.km[2], t.km[3], ek};
+    }
+  }
+  return true;
+}
+
+// ax_transpose over a quad (PA: pass A).
+template <bool PA, int W, int AX, bool RAG>
+__device__ __forceinline__ void quad_transpose(const StepStatic& P, const float* psi, float* out, int i, int j, int k0,
+                                               int sm, f4v wi_m, f4v wj_m, f4v wi_p, f4v wj_p, f4v& x, f4v& y,
+                                               f4v& z) {
+  QuadPair t;
+  if (!quad_pair<W, AX, PA ? -1 : 1, RAG>(P, psi, i, j, k0, t)) return;
+  const f4v si_m = PA ? wi_m : -wi_m, sj_m = PA ? -wj_m : wj_m;
+  const f4v si_p = PA ? wi_p : -wi_p, sj_p = PA ? -wj_p : wj_p;
+  const f4v g1 = t.p1 + si_m, g2 = t.p2 + sj_m;
+  f4v u1m = t.a * g1, u2m = t.a * g2;
+  f4v u1p = t.an * (t.n1 + si_p), u2p = t.an * (t.n2 + sj_p);
+  if (t.kap) {
+    u1m = u1m + t.km * si_m;
+    u2m = u2m + t.km * sj_m;
+    u1p = u1p + t.kn * si_p;
+    u2p = u2p + t.kn * sj_p;
+  }
+  const f4v o1 = t.b * g1, o2 = t.b * g2;
+  if (t.vec && t.zm) {
+    st4m<RAG>(out + t.q, o1, sm);
+    st4m<RAG>(out + t.q + t.cells, o2, sm);
+  } else if (!t.vec) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (((t.zm >> e) & 1u) && e >= sm) {
+        out[t.q + e] = o1[e];
+        out[t.q + t.cells + e] = o2[e];
+      }
+  }
+  f4v v1, v2;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {  // cells outside the slab contribute an exact zero
+    const float a1 = ((t.zm >> e) & 1u) ? u1m[e] : 0.f, a2 = ((t.zm >> e) & 1u) ? u2m[e] : 0.f;
+    const float b1 = ((t.nm >> e) & 1u) ? u1p[e] : 0.f, b2 = ((t.nm >> e) & 1u) ? u2p[e] : 0.f;
+    v1[e] = PA ? b1 - a1 : a1 - b1;
+    v2[e] = PA ? b2 - a2 : a2 - b2;
+  }
+  if (AX == 0) {  // add_comp
+    y = y + v2;
+    z = z + v1;
+  } else if (AX == 1) {
+    z = z + v2;
+    x = x + v1;
+  } else {
+    x = x + v2;
+    y = y + v1;
+  }
+}
+
+// psi_E's correction of both curls of a quad on one axis: K with psi advanced, Kr with psi frozen.
+template <int AX, bool RAG>
+__device__ __forceinline__ void quad_two_curls(const StepStatic& P, const float* psi, int i, int j, int k0, f4v d1,
+                                               f4v d2, f4v* K, f4v* Kr) {
+  QuadSlabs S;
+  quad_slab_load<0, AX, RAG>(P, psi, i, j, k0, S);
+  if (!S.in[AX]) return;
+  int dep, L, kap, aligned;
+  long long cells;
+  const float* cf;
+  quad_psi_offset<0, AX>(P, S.hi[AX], i, j, k0, dep, cells, cf, L, kap, aligned);
+  const f4v s1 = S.p1[AX], s2 = S.p2[AX];
+  f4v c1, c2, r1 = s1, r2 = s2;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const bool in = AX != 2 || ((S.zm >> e) & 1u);
+    const int de = AX != 2 ? dep : (in ? dep + e : (dep + e < 0 ? 0 : L - 1));
+    const float b = cf[de], a = cf[L + de];
+    c1[e] = b * s1[e] + a * d1[e];
+    c2[e] = b * s2[e] + a * d2[e];
+    if (!kap) {
+      const float km = cf[2 * L + de];
+      c1[e] = km * d1[e] + c1[e];
+      c2[e] = km * d2[e] + c2[e];
+      r1[e] = km * d1[e] + s1[e];
+      r2[e] = km * d2[e] + s2[e];
+    }
+    if (!in) c1[e] = c2[e] = r1[e] = r2[e] = 0.f;
+  }
+  constexpr int u = (AX + 1) % 3, v = (AX + 2) % 3;
+  K[u] = K[u] + (-c1);
+  K[v] = K[v] + c2;
+  Kr[u] = Kr[u] + (-r1);
+  Kr[v] = Kr[v] + r2;
+}
+
+// w_H at a quad: (c inv_mu) lam_H of component C.
+template <int MC, bool RAG>
+__device__ __forceinline__ f4v w_h4(const StepStatic& P, const AdjDyn& A, int C, long long oo) {
+  const f4v c = {P.c, P.c, P.c, P.c};
+  const f4v l = ld4<RAG>(A.lamH + C * P.N + oo);
+  if constexpr (MC == 0) return c * l;
+  return (c * ld4<RAG>(A.im + (MC == 3 ? C : 0) * P.N + oo)) * l;
+}
+
+template <int MC>
+__device__ __forceinline__ float w_h1(const StepStatic& P, const AdjDyn& A, int C, long long oo) {
+  const float l = A.lamH[C * P.N + oo];
+  if constexpr (MC == 0) return P.c * l;
+  return (P.c * A.im[(MC == 3 ? C : 0) * P.N + oo]) * l;
+}
+
+// Pass A with the fused reverse E half-step.
+template <int EC, int MC, bool RAG>
+__global__ __launch_bounds__(kBlock) void k_adj_A4(const StepStatic* __restrict__ Pp, const AdjDyn A) {
+  const StepStatic& P = as_const(Pp);
+  int i, j, k0, sm;
+  long long o;
+  const long long lb = logical_block(P.xorder, P.vnblocks_pad);
+  if (!quad_of(P, lb, i, j, k0, sm, o)) return;
+  const uint32_t m = P.vec_mask[lb];
+  if (m & P.vpoint[0]) quad_points<0, true>(P, m, A.ie, A.im, A.Erev, A.n, i, j, k0, sm, o, EC, 0);
+  const long long N = P.N;
+  const bool vj = j > 0, vi = i > 0, vk = k0 > 0;
+  const f4v z4 = {0.f, 0.f, 0.f, 0.f}, c = {P.c, P.c, P.c, P.c};
+  f4v K[3];
+  {  // curl H^n, the reverse E half-step
+    const float *Hx = A.H + o, *Hy = Hx + N, *Hz = Hy + N;
+    const f4v hx = ld4<RAG>(Hx), hy = ld4<RAG>(Hy), hz = ld4<RAG>(Hz);
+    const f4v hxj = vj ? ld4<RAG>(Hx - P.nz) : z4, hzj = vj ? ld4<RAG>(Hz - P.nz) : z4;
+    const f4v hyi = vi ? ld4<RAG>(Hy - P.plane) : z4, hzi = vi ? ld4<RAG>(Hz - P.plane) : z4;
+    const float hxk = vk ? Hx[-1] : 0.f, hyk = vk ? Hy[-1] : 0.f;
+    const f4v hxm = {hxk, hx[0], hx[1], hx[2]}, hym = {hyk, hy[0], hy[1], hy[2]};
+    const f4v dxz = hz - hzi, dxy = hy - hyi, dyx = hx - hxj, dyz = hz - hzj, dzy = hy - hym, dzx = hx - hxm;
+    K[0] = dyz - dzy;
+    K[1] = dzx - dxz;
+    K[2] = dxy - dyx;
+    f4v Kr[3] = {K[0], K[1], K[2]};
+    if (m & kSlabBits) {
+      quad_two_curls<0, RAG>(P, A.psi, i, j, k0, dxz, dxy, K, Kr);
+      quad_two_curls<1, RAG>(P, A.psi, i, j, k0, dyx, dyz, K, Kr);
+      quad_two_curls<2, RAG>(P, A.psi, i, j, k0, dzy, dzx, K, Kr);
+    }
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      float* Ea = A.Erev + a * N + o;
+      st4m<RAG>(Ea, ld4<RAG>(Ea) - (c * Kr[a]) * ld4<RAG>(A.ie + (EC == 3 ? a : 0) * N + o), sm);
+    }
+  }
+  const f4v wx = w_h4<MC, RAG>(P, A, 0, o), wy = w_h4<MC, RAG>(P, A, 1, o), wz = w_h4<MC, RAG>(P, A, 2, o);
+  const f4v wx_jm = vj ? w_h4<MC, RAG>(P, A, 0, o - P.nz) : z4, wz_jm = vj ? w_h4<MC, RAG>(P, A, 2, o - P.nz) : z4;
+  const f4v wy_im = vi ? w_h4<MC, RAG>(P, A, 1, o - P.plane) : z4, wz_im = vi ? w_h4<MC, RAG>(P, A, 2, o - P.plane) : z4;
+  const float wxk = vk ? w_h1<MC>(P, A, 0, o - 1) : 0.f, wyk = vk ? w_h1<MC>(P, A, 1, o - 1) : 0.f;
+  const f4v wx_km = {wxk, wx[0], wx[1], wx[2]}, wy_km = {wyk, wy[0], wy[1], wy[2]};
+  f4v mu[3];
+  mu[0] = ld4<RAG>(A.lamE + o) - ((wz - wz_jm) - (wy - wy_km));
+  mu[1] = ld4<RAG>(A.lamE + N + o) - ((wx - wx_km) - (wz - wz_im));
+  mu[2] = ld4<RAG>(A.lamE + 2 * N + o) - ((wy - wy_im) - (wx - wx_jm));
+  quad_transpose<true, 1, 0, RAG>(P, A.lpsi_in, A.lpsi_out, i, j, k0, sm, wy, wz, wy_im, wz_im, mu[0], mu[1], mu[2]);
+  quad_transpose<true, 1, 1, RAG>(P, A.lpsi_in, A.lpsi_out, i, j, k0, sm, wz, wx, wz_jm, wx_jm, mu[0], mu[1], mu[2]);
+  quad_transpose<true, 1, 2, RAG>(P, A.lpsi_in, A.lpsi_out, i, j, k0, sm, wx, wy, wx_km, wy_km, mu[0], mu[1], mu[2]);
+  f4v g[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) g[a] = mu[a] * (c * K[a]);
+  if (EC == 3) {
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      float* G = A.grad + a * N + o;
+      st4m<RAG>(G, ld4<RAG>(G) + g[a], sm);
+    }
+  } else {
+    st4m<RAG>(A.grad + o, ld4<RAG>(A.grad + o) + ((g[0] + g[1]) + g[2]), sm);
+  }
+#pragma unroll
+  for (int a = 0; a < 3; ++a) st4m<RAG>(A.lamE + a * N + o, mu[a], sm);
+}
+
+template <int EC, bool RAG>
+__device__ __forceinline__ f4v w_e4(const StepStatic& P, const AdjDyn& A, int C, long long oo) {
+  const f4v c = {P.c, P.c, P.c, P.c};
+  return (c * ld4<RAG>(A.ie + (EC == 3 ? C : 0) * P.N + oo)) * ld4<RAG>(A.lamE + C * P.N + oo);
+}
+
+template <int EC>
+__device__ __forceinline__ float w_e1(const StepStatic& P, const AdjDyn& A, int C, long long oo) {
+  return (P.c * A.ie[(EC == 3 ? C : 0) * P.N + oo]) * A.lamE[C * P.N + oo];
+}
+
+template <int EC, bool RAG>
+__global__ __launch_bounds__(kBlock) void k_adj_B4(const StepStatic* __restrict__ Pp, const AdjDyn A) {
+  const StepStatic& P = as_const(Pp);
+  int i, j, k0, sm;
+  long long o;
+  const long long lb = logical_block(P.xorder, P.vnblocks_pad);
+  if (!quad_of(P, lb, i, j, k0, sm, o)) return;
+  const long long N = P.N;
+  const bool vj = j < P.ny - 1, vi = i < P.nx - 1, vk = k0 + 4 < P.nz;
+  const f4v z4 = {0.f, 0.f, 0.f, 0.f};
+  const f4v wx = w_e4<EC, RAG>(P, A, 0, o), wy = w_e4<EC, RAG>(P, A, 1, o), wz = w_e4<EC, RAG>(P, A, 2, o);
+  const f4v wx_jp = vj ? w_e4<EC, RAG>(P, A, 0, o + P.nz) : z4, wz_jp = vj ? w_e4<EC, RAG>(P, A, 2, o + P.nz) : z4;
+  const f4v wy_ip = vi ? w_e4<EC, RAG>(P, A, 1, o + P.plane) : z4, wz_ip = vi ? w_e4<EC, RAG>(P, A, 2, o + P.plane) : z4;
+  const float wxk = vk ? w_e1<EC>(P, A, 0, o + 4) : 0.f, wyk = vk ? w_e1<EC>(P, A, 1, o + 4) : 0.f;
+  const f4v wx_kp = {wx[1], wx[2], wx[3], wxk}, wy_kp = {wy[1], wy[2], wy[3], wyk};
+  f4v lh[3];
+  lh[0] = ld4<RAG>(A.lamH + o) + ((wz_jp - wz) - (wy_kp - wy));
+  lh[1] = ld4<RAG>(A.lamH + N + o) + ((wx_kp - wx) - (wz_ip - wz));
+  lh[2] = ld4<RAG>(A.lamH + 2 * N + o) + ((wy_ip - wy) - (wx_jp - wx));
+  quad_transpose<false, 0, 0, RAG>(P, A.lpsi_in, A.lpsi_out, i, j, k0, sm, wy, wz, wy_ip, wz_ip, lh[0], lh[1], lh[2]);
+  quad_transpose<false, 0, 1, RAG>(P, A.lpsi_in, A.lpsi_out, i, j, k0, sm, wz, wx, wz_jp, wx_jp, lh[0], lh[1], lh[2]);
+  quad_transpose<false, 0, 2, RAG>(P, A.lpsi_in, A.lpsi_out, i, j, k0, sm, wx, wy, wx_kp, wy_kp, lh[0], lh[1], lh[2]);
+#pragma unroll
+  for (int a = 0; a < 3; ++a) st4m<RAG>(A.lamH + a * N + o, lh[a], sm);
+}
+
+template <int EC, bool RAG>
+static void (*adj_A4(int mc))(const StepStatic*, const AdjDyn) {
+  return mc == 3 ? k_adj_A4<EC, 3, RAG> : (mc == 1 ? k_adj_A4<EC, 1, RAG> : k_adj_A4<EC, 0, RAG>);
+}
+
 // Pass C: lam_E^n = (1 - x) / (1 + x) * mu_E in the electric conductivity box, one thread per box
 // cell (pass B has read mu_E at every neighbour by now).
 template <int EC>
@@ -626,6 +945,17 @@ __global__ __launch_bounds__(kBlock) void k_adj_C(const StepStatic* __restrict__
 }
 
 hipError_t launch_adjoint(const StepStatic& P, const AdjDyn& A, int ec, int mc, hipStream_t s) {
+  if (P.aquad && A.Erev && ec != 9 && mc != 9) {
+    const bool rag = P.nz % 4 != 0;
+    const dim3 gq((unsigned)P.vnblocks_pad);
+    const auto a4 = ec == 3 ? (rag ? adj_A4<3, true>(mc) : adj_A4<3, false>(mc))
+                            : (rag ? adj_A4<1, true>(mc) : adj_A4<1, false>(mc));
+    const auto b4 = ec == 3 ? (rag ? k_adj_B4<3, true> : k_adj_B4<3, false>)
+                            : (rag ? k_adj_B4<1, true> : k_adj_B4<1, false>);
+    hipLaunchKernelGGL(a4, gq, dim3(kBlock), 0, s, P.self, A);
+    hipLaunchKernelGGL(b4, gq, dim3(kBlock), 0, s, P.self, A);
+    return hipGetLastError();
+  }
   const dim3 g((unsigned)P.nblocks_pad);
   const dim3 gc((unsigned)((P.loss[0].cells + kBlock - 1) / kBlock));
   using AdjKernel = void (*)(const StepStatic*, const AdjDyn);

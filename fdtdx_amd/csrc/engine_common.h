@@ -142,6 +142,11 @@ struct StepStatic {
   // meeting both z slabs. axs[a][side] is the slab index (-1: none); axord lists the axes in the
   // order of their slab indices.
   int cax, acax;
+  // Quad adjoint (aquad = 1): the reverse and adjoint sweeps of diagonal media run four z cells per
+  // lane; needs cax and acax, no conducting faces, conductivity or periodic axes, one cell between
+  // the two slabs of x and of y and five between those of z (so that a quad and the cell beside it meet
+  // one slab at most).
+  int aquad;
   int xorder;                // block order (logical_block): 0 per-XCD ranges, 1 XCD turns
   int axs[3][2];
   int axord[3];

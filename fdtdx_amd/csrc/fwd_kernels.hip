@@ -558,18 +558,6 @@ __global__ __launch_bounds__(kBlock) void k_update_H(const StepStatic* __restric
 // quads. RAG: rows of nz % 4 != 0 cells (a sweep with 4-byte aligned accesses). Measured on the
 // 301x277x150 plane wave: E / H sweep 119 / 113 us against 128 / 122 us one cell per lane (an aligned
 // grid of that many cells would take about 101 / 90).
-// Quad of this lane in quad tile lb: cells (i, j, k0 .. k0 + 3) at offsets o .. o + 3, the first sm
-// of which it leaves out of its stores.
-__device__ __forceinline__ bool quad_of(const StepStatic& P, long long lb, int& i, int& j, int& k0, int& sm,
-                                        long long& o) {
-  if (lb >= P.vnblocks) return false;
-  i = (int)(lb / P.vbpp);
-  const int p = (int)(lb - (long long)i * P.vbpp) * kBlock + threadIdx.x;
-  if (p >= P.ny * P.nzq) return false;
-  perm_quad(P, p, j, k0, sm);
-  o = (long long)i * P.plane + (long long)j * P.nz + k0;
-  return true;
-}
 
 // CPML of the four cells of a quad, slab by slab in object order (per cell the order of
 // apply_cpml, with cpml_slab's arithmetic). A slab holding all four cells with 16-byte aligned
@@ -868,6 +856,50 @@ __global__ __launch_bounds__(kBlock) void k_reverse_H(const StepStatic* __restri
   Hz[o] = rz;
 }
 
+// The same for four z cells per lane (plans with StepStatic::aquad: no conducting faces,
+// conductivity or periodic axes).
+template <int MC, bool RAG>
+__global__ __launch_bounds__(kBlock) void k_reverse_H4(const StepStatic* __restrict__ Pp, const StepDyn D) {
+  const StepStatic& P = as_const(Pp);
+  int i, j, k0, sm;
+  long long o;
+  const long long lb = logical_block(P.xorder, P.vnblocks_pad);
+  if (!quad_of(P, lb, i, j, k0, sm, o)) return;
+  const uint32_t m = P.vec_mask[lb];
+  if (m & P.vpoint[1]) quad_points<1, true>(P, m, D.ie, D.im, D.H, D.n, i, j, k0, sm, o, 1, MC);
+  const long long N = P.N;
+  QuadSlabs S;
+  S.in[0] = S.in[1] = S.in[2] = false;
+  S.hi[0] = S.hi[1] = S.hi[2] = false;
+  if (m & kSlabBits) quad_slab_loads<1, RAG>(P, D.psi, i, j, k0, S);
+  const float *Ex = D.E + o, *Ey = Ex + N, *Ez = Ey + N;
+  float *Hx = D.H + o, *Hy = Hx + N, *Hz = Hy + N;
+  const bool vj = j < P.ny - 1, vi = i < P.nx - 1, vk = k0 + 4 < P.nz;
+  const f4v z4 = {0.f, 0.f, 0.f, 0.f};
+  const f4v ex = ld4<RAG>(Ex), ey = ld4<RAG>(Ey), ez = ld4<RAG>(Ez);
+  const f4v exj = vj ? ld4<RAG>(Ex + P.nz) : z4, ezj = vj ? ld4<RAG>(Ez + P.nz) : z4;
+  const f4v eyi = vi ? ld4<RAG>(Ey + P.plane) : z4, ezi = vi ? ld4<RAG>(Ez + P.plane) : z4;
+  const float exk = vk ? Ex[4] : 0.f, eyk = vk ? Ey[4] : 0.f;
+  const f4v ho[3] = {ld4<RAG>(Hx), ld4<RAG>(Hy), ld4<RAG>(Hz)};
+  const f4v exn = {ex[1], ex[2], ex[3], exk}, eyn = {ey[1], ey[2], ey[3], eyk};
+  QuadDeriv d;
+  d.x1 = ezi - ez;
+  d.x2 = eyi - ey;
+  d.y1 = exj - ex;
+  d.y2 = ezj - ez;
+  d.z1 = eyn - ey;
+  d.z2 = exn - ex;
+  f4v cx = d.y2 - d.z1, cy = d.z2 - d.x1, cz = d.x2 - d.y1;
+  if (m & kSlabBits) quad_slab_frozen<1, RAG>(P, S, i, j, k0, d, cx, cy, cz);
+  const f4v one = {1.f, 1.f, 1.f, 1.f}, c = {P.c, P.c, P.c, P.c};
+  const f4v imx = MC ? ld4<RAG>(D.im + o) : one;
+  const f4v imy = MC == 3 ? ld4<RAG>(D.im + N + o) : imx;
+  const f4v imz = MC == 3 ? ld4<RAG>(D.im + 2 * N + o) : imx;
+  st4m<RAG>(Hx, ho[0] + (c * cx) * imx, sm);
+  st4m<RAG>(Hy, ho[1] + (c * cy) * imy, sm);
+  st4m<RAG>(Hz, ho[2] + (c * cz) * imz, sm);
+}
+
 template <int EC>
 __global__ __launch_bounds__(kBlock) void k_reverse_E(const StepStatic* __restrict__ Pp, const StepDyn D) {
   const StepStatic& P = as_const(Pp);
@@ -1139,6 +1171,14 @@ static void (*reverse_H_kernel(const StepStatic& P, int mc))(const StepStatic*, 
 }
 
 hipError_t launch_reverse_H(const StepStatic& P, const StepDyn& D, int mc, hipStream_t s) {
+  if (P.aquad) {
+    const bool rag = P.nz % 4 != 0;
+    const SweepKernel f = mc == 3 ? (rag ? k_reverse_H4<3, true> : k_reverse_H4<3, false>)
+                                  : (mc == 1 ? (rag ? k_reverse_H4<1, true> : k_reverse_H4<1, false>)
+                                             : (rag ? k_reverse_H4<0, true> : k_reverse_H4<0, false>));
+    hipLaunchKernelGGL(f, dim3((unsigned)P.vnblocks_pad), dim3(kBlock), 0, s, P.self, D);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(reverse_H_kernel(P, mc), grid_of(P), dim3(kBlock), 0, s, P.self, D);
   return hipGetLastError();
 }

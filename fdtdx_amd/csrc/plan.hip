@@ -574,7 +574,7 @@ static int plan_create(const fdtdx_plan_desc* d, fdtdx_plan** out) {
         for (int b2 = a + 1; b2 < 3; ++b2)
           if (hi_id[a] >= 0 && hi_id[b2] >= 0 && hi_id[a] > lo_id[b2]) xyz = false;
       // FDTDX_REVERSE_CPML=loop keeps the reverse and adjoint sweeps on the slab loop (the same
-      // results; for comparing the two paths)
+      // results; for comparing the two paths), =cell on one cell per lane
       const char* renv = getenv("FDTDX_REVERSE_CPML");
       P.acax = xyz && !(renv && strcmp(renv, "loop") == 0) ? 1 : 0;
       bool zq = true;  // no quad meets both z slabs (a row's last quad starts at nz - 4 or above)
@@ -586,6 +586,12 @@ static int plan_create(const fdtdx_plan_desc* d, fdtdx_plan** out) {
       // aligned quads
       if (P.nz % 4 && !(xyz && zq)) quad_ok = false;
       P.cax = quad_ok && xyz && zq ? 1 : 0;
+      bool gap = true;
+      for (int a = 0; a < 3; ++a)
+        if (ok && P.axs[a][0] >= 0 && P.axs[a][1] >= 0)
+          gap = gap && P.slab[P.axs[a][1]].lo - P.slab[P.axs[a][0]].hi >= (a == 2 ? 5 : 1);
+      P.aquad = P.cax && P.acax && gap && P.nwall == 0 && !P.loss[0].comps && !P.loss[1].comps && !P.wrap[0] &&
+                !P.wrap[1] && !P.wrap[2] && !(renv && strcmp(renv, "cell") == 0) ? 1 : 0;
       for (int u = 0; u < 3; ++u) P.axord[u] = ord[u];
       for (int a = 0; a < 3; ++a)
         for (int side = 0; side < 2; ++side) {

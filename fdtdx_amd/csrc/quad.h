@@ -42,6 +42,19 @@ __device__ __forceinline__ void st4m(float* p, f4v v, int sm) {
 constexpr uint32_t kSlabBits = (1u << FDTDX_MAX_CPML) - 1u;
 constexpr uint32_t kSnapBit = 1u << kMaskSnap;
 
+// Quad of this lane in quad tile lb: cells (i, j, k0 .. k0 + 3) at offsets o .. o + 3, the first sm
+// of which it leaves out of its stores.
+__device__ __forceinline__ bool quad_of(const StepStatic& P, long long lb, int& i, int& j, int& k0, int& sm,
+                                        long long& o) {
+  if (lb >= P.vnblocks) return false;
+  i = (int)(lb / P.vbpp);
+  const int p = (int)(lb - (long long)i * P.vbpp) * kBlock + threadIdx.x;
+  if (p >= P.ny * P.nzq) return false;
+  perm_quad(P, p, j, k0, sm);
+  o = (long long)i * P.plane + (long long)j * P.nz + k0;
+  return true;
+}
+
 // One-sided derivatives of the four cells of a quad, one vector per (axis, component) pair that
 // feeds a CPML slab: curl H uses (dx Hz, dx Hy), (dy Hx, dy Hz), (dz Hy, dz Hx), curl E the same
 // pairs of E (the order of pml_pair).
@@ -214,6 +227,47 @@ __device__ __forceinline__ void quad_slab_apply(const StepStatic& P, const QuadS
   quad_slab_axis<W, 2, RAG>(P, S, psi_out, i, j, k0, sm, store, d, cx, cy, cz);
 }
 
+// The correction with psi frozen (the reverse run, PML.py:181-182) of the preloaded slabs, x, y, z.
+template <int W, int AX, bool RAG>
+__device__ __forceinline__ void quad_frozen_axis(const StepStatic& P, const QuadSlabs& S, int i, int j, int k0,
+                                                 const QuadDeriv& d, f4v& cx, f4v& cy, f4v& cz) {
+  if (!S.in[AX]) return;
+  f4v r1 = S.p1[AX], r2 = S.p2[AX];  // zero for the cells outside a z slab
+  int dep, L, kap, aligned;
+  long long cells;
+  const float* cf;
+  quad_psi_offset<W, AX>(P, S.hi[AX], i, j, k0, dep, cells, cf, L, kap, aligned);
+  if (!kap) {
+    const f4v d1 = AX == 0 ? d.x1 : (AX == 1 ? d.y1 : d.z1);
+    const f4v d2 = AX == 0 ? d.x2 : (AX == 1 ? d.y2 : d.z2);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (AX == 2 && !((S.zm >> e) & 1u)) continue;
+      const float km = cf[2 * L + (AX == 2 ? dep + e : dep)];
+      r1[e] = km * d1[e] + r1[e];
+      r2[e] = km * d2[e] + r2[e];
+    }
+  }
+  if (AX == 0) {
+    cy = cy + (-r1);
+    cz = cz + r2;
+  } else if (AX == 1) {
+    cz = cz + (-r1);
+    cx = cx + r2;
+  } else {
+    cx = cx + (-r1);
+    cy = cy + r2;
+  }
+}
+
+template <int W, bool RAG>
+__device__ __forceinline__ void quad_slab_frozen(const StepStatic& P, const QuadSlabs& S, int i, int j, int k0,
+                                                 const QuadDeriv& d, f4v& cx, f4v& cy, f4v& cz) {
+  quad_frozen_axis<W, 0, RAG>(P, S, i, j, k0, d, cx, cy, cz);
+  quad_frozen_axis<W, 1, RAG>(P, S, i, j, k0, d, cx, cy, cz);
+  quad_frozen_axis<W, 2, RAG>(P, S, i, j, k0, d, cx, cy, cz);
+}
+
 // Conductivity of a quad (loss_x and the update of update_E_cell / update_H_cell): f the field before
 // the step, t = (c curl) inv, n the lossless result, replaced for the cells inside the box.
 template <int W>
@@ -241,7 +295,8 @@ __device__ __forceinline__ void quad_loss(const StepStatic& P, int i, int j, int
 // ran one cell per lane in launches of their own: 6 to 9 us each whatever the grid, against no
 // measurable time here (steps of the 64^3 dipole 49.5 -> 44.6 us, the 128x128x64 plane wave 45.2
 // -> 37.8, the 200x200x100 dipole 77.7 -> 70.4, the 400x400x200 plane wave 529 -> 511).
-template <int W>
+// INV: the reverse run's sources (negated), added before the half-step is undone.
+template <int W, bool INV = false>
 __device__ __forceinline__ void quad_points(const StepStatic& P, uint32_t m, const float* ie, const float* im,
                                             float* F, int n, int i, int j, int k0, int sm, long long o, int ec,
                                             int mc) {
@@ -261,8 +316,8 @@ __device__ __forceinline__ void quad_points(const StepStatic& P, uint32_t m, con
 #pragma unroll 1
   for (int e = sm; e < 4; ++e) {
     float x = p[e], y = p[P.N + e], z = p[2 * P.N + e];
-    apply_sources<false>(P, m, ie, im, W, n, false, i, j, k0 + e, o + e, ec, mc, x, y, z);
-    apply_walls(P, m, W ? FDTDX_WALL_PMC : FDTDX_WALL_PEC, i, j, k0 + e, x, y, z);
+    apply_sources<false>(P, m, ie, im, W, n, INV, i, j, k0 + e, o + e, ec, mc, x, y, z);
+    if (!INV) apply_walls(P, m, W ? FDTDX_WALL_PMC : FDTDX_WALL_PEC, i, j, k0 + e, x, y, z);
     p[e] = x;
     p[P.N + e] = y;
     p[2 * P.N + e] = z;

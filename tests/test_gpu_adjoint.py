@@ -163,6 +163,52 @@ def test_per_axis_reverse_cpml_equals_slab_loop_bitwise(case, monkeypatch):
     assert np.array_equal(out["loop"][0], out["axes"][0])
 
 
+def _quad_adjoint_cases():
+    def c3(shape, pml=5):
+        return W.scenario_c3(T=70, shape=shape, pml=pml, design=(8, 8, 4))
+
+    kap = c3((30, 28, 26))  # kappa > 1, diagonal permittivity and permeability
+    kap["pml"] = dict(kap["pml"], params=dict(kappa_start=1.0, kappa_end=3.0))
+    kap["boxes"] = [dict(slc=((4, 20), (6, 20), (3, 22)), eps=1.0, mu=(1.4, 2.2, 1.8))]
+    del kap["design"]
+    kap["boxes"].append(dict(slc=((12, 20), (8, 18), (9, 15)), eps=(2.0, 4.0, 3.0)))
+    plane = W.scenario_c2(T=60, shape=(40, 30, 27), pml=5, slab=(10, 12, 8))  # E and H source hooks, phasors
+    return {"aligned": c3((30, 28, 24), 4), "unaligned_slabs": c3((30, 28, 24)), "mod1": c3((30, 28, 25)),
+            "mod2": c3((30, 28, 22)), "mod3": c3((28, 30, 23), 4), "kappa_mu_diag": kap, "plane": plane}
+
+
+@pytest.mark.parametrize("case", ["aligned", "unaligned_slabs", "mod1", "mod2", "mod3", "kappa_mu_diag", "plane"])
+def test_quad_adjoint_equals_one_cell_adjoint_bitwise(case, monkeypatch):
+    """The reverse and adjoint sweeps with four z cells per lane against one (FDTDX_REVERSE_CPML=cell):
+    the same operations in the same order, so the gradient of the whole permittivity array and the
+    detector states agree bit for bit, with z slabs on and inside quads, rows of any length and
+    kappa > 1."""
+    import torch
+
+    import fdtdx_amd as fx
+    import scenarios
+
+    spec = _quad_adjoint_cases()[case]
+    out = {}
+    for mode in ("cell", "quad"):
+        if mode == "cell":
+            monkeypatch.setenv("FDTDX_REVERSE_CPML", "cell")
+        else:
+            monkeypatch.delenv("FDTDX_REVERSE_CPML", raising=False)
+        print("case", case, mode, spec["shape"], flush=True)
+        objects, arrays, params, config = scenarios.build(spec, gradient=True)
+        ie = arrays.inv_permittivities.detach().clone().requires_grad_(True)
+        arrays.inv_permittivities = ie
+        _, arrays = fx.run_fdtd(arrays, objects, config)
+        states = [v for st in arrays.detector_states.values() for v in st.values()]
+        sum((v.real.sum() + (0.5 * v.imag.sum() if v.is_complex() else 0.0)) for v in states).backward()
+        torch.cuda.synchronize()
+        out[mode] = [ie.grad.cpu().numpy()] + [v.detach().cpu().numpy() for v in states]
+    assert np.abs(out["cell"][0]).max() > 0
+    for a, b in zip(out["quad"], out["cell"]):
+        assert np.array_equal(a, b)
+
+
 @pytest.mark.parametrize("num_checkpoints", [0, 2])
 def test_gradient_with_conductivity_matches_oracle(num_checkpoints):
     """The lossy reverse update and the transposed loss factors (w_H, w_E, the pass-through of
