@@ -104,58 +104,63 @@ __device__ __forceinline__ float hc(const StepStatic& P, const Src3& hp, const S
   return (at(P, hp, c, i, j, k) + at(P, h, c, i, j, k)) / 2.0f;
 }
 
-// The stencil of interp at (i, j, k) reads i-1, j-1 and k+1: when that stays inside a source's box
-// (which lies inside the domain) no halo, wrap, mirror or Bloch phase applies and the reads are
-// plain offsets.
-__device__ __forceinline__ bool stencil_inside(const Src3& s, int i, int j, int k) {
-  return i - 1 >= s.lo[0] && j - 1 >= s.lo[1] && k + 1 < s.hi[2] && i < s.hi[0] && j < s.hi[1] && k >= s.lo[2];
-}
-
 __device__ __forceinline__ long long src_index(const Src3& s, int i, int j, int k) {
   return ((long long)(i - s.lo[0]) * s.sy + (j - s.lo[1])) * s.sz + (k - s.lo[2]);
 }
 
-// interp where stencil_inside holds for e, hp and h: the same expressions in the same order, so
-// the result is identical to the general path's.
-__device__ __forceinline__ void interp_inside(const Src3& e, const Src3& hp, const Src3& h, int i, int j, int k,
-                                              float* Ei, float* Hi) {
+// interp where no halo of a periodic axis or symmetry plane is needed (needs_halo): the stencil reads
+// i-1, j-1 and k+1, which a source's box holds unless they lie beyond the domain (the zero halo; then the cell itself is
+// read and dropped). Plain offsets and no branches: all loads are in flight together, and a wavefront
+// with one cell on a face costs no second pass. The expressions and their order are those of the
+// general path.
+__device__ __forceinline__ void interp_open(const StepStatic& P, const Src3& e, const Src3& hp, const Src3& h, int i,
+                                            int j, int k, float* Ei, float* Hi) {
+  const bool vi = i > 0, vj = j > 0, vk = k + 1 < P.nz;
   const long long oe = src_index(e, i, j, k);
-  const long long xe = (long long)e.sy * e.sz, ye = e.sz;
+  const long long xe = vi ? -(long long)e.sy * e.sz : 0, ye = vj ? -(long long)e.sz : 0, ze = vk ? 1 : 0;
+  auto z = [](bool v, float x) { return v ? x : 0.f; };
   const float* ex = e.p;
   const float* ey = e.p + e.stride;
   const float* ez = e.p + 2 * e.stride;
-  const float lo_x = 0.5f * (ex[oe] + ex[oe - xe]);
-  const float up_x = 0.5f * (ex[oe + 1] + ex[oe - xe + 1]);
+  const float lo_x = 0.5f * (ex[oe] + z(vi, ex[oe + xe]));
+  const float up_x = 0.5f * (z(vk, ex[oe + ze]) + z(vi && vk, ex[oe + xe + ze]));
   Ei[0] = (lo_x + up_x) / 2.0f;
-  const float lo_y = 0.5f * (ey[oe] + ey[oe - ye]);
-  const float up_y = 0.5f * (ey[oe + 1] + ey[oe - ye + 1]);
+  const float lo_y = 0.5f * (ey[oe] + z(vj, ey[oe + ye]));
+  const float up_y = 0.5f * (z(vk, ey[oe + ze]) + z(vj && vk, ey[oe + ye + ze]));
   Ei[1] = (lo_y + up_y) / 2.0f;
   Ei[2] = ez[oe];
   const long long op = src_index(hp, i, j, k), oh = src_index(h, i, j, k);
-  const long long xp = (long long)hp.sy * hp.sz, yp = hp.sz, xh = (long long)h.sy * h.sz, yh = h.sz;
-  // time-centred H at the offset (dx, dy, dz) in {-1, 0} x {-1, 0} x {0, 1}
+  const long long xp = vi ? -(long long)hp.sy * hp.sz : 0, yp = vj ? -(long long)hp.sz : 0;
+  const long long xh = vi ? -(long long)h.sy * h.sz : 0, yh = vj ? -(long long)h.sz : 0;
+  // time-centred H at the offset (-dx, -dy, +dz)
   auto hcq = [&](int c, int dx, int dy, int dz) {
-    const float a = hp.p[c * hp.stride + op + dx * xp + dy * yp + dz];
-    const float b = h.p[c * h.stride + oh + dx * xh + dy * yh + dz];
-    return (a + b) / 2.0f;
+    const float a = hp.p[c * hp.stride + op + dx * xp + dy * yp + dz * ze];
+    const float b = h.p[c * h.stride + oh + dx * xh + dy * yh + dz * ze];
+    return z((!dx || vi) && (!dy || vj) && (!dz || vk), (a + b) / 2.0f);
   };
-  Hi[0] = 0.5f * (hcq(0, 0, 0, 0) + hcq(0, 0, -1, 0));
-  Hi[1] = 0.5f * (hcq(1, 0, 0, 0) + hcq(1, -1, 0, 0));
+  Hi[0] = 0.5f * (hcq(0, 0, 0, 0) + hcq(0, 0, 1, 0));
+  Hi[1] = 0.5f * (hcq(1, 0, 0, 0) + hcq(1, 1, 0, 0));
   float zz[2];
 #pragma unroll
   for (int dz = 0; dz < 2; ++dz) {
-    const float a = 0.5f * (hcq(2, 0, 0, dz) + hcq(2, -1, 0, dz));
-    const float b = 0.5f * (hcq(2, 0, -1, dz) + hcq(2, -1, -1, dz));
+    const float a = 0.5f * (hcq(2, 0, 0, dz) + hcq(2, 1, 0, dz));
+    const float b = 0.5f * (hcq(2, 0, 1, dz) + hcq(2, 1, 1, dz));
     zz[dz] = 0.5f * (a + b);
   }
   Hi[2] = (zz[0] + zz[1]) / 2.0f;
 }
 
-// interpolate_fields (curl.py:86-224) at cell (i,j,k) on a uniform grid.
+// Where that halo is needed, cells whose stencil stays inside every source's box read plain offsets.
+__device__ __forceinline__ bool stencil_inside(const Src3& s, int i, int j, int k) {
+  return i - 1 >= s.lo[0] && j - 1 >= s.lo[1] && k + 1 < s.hi[2] && i < s.hi[0] && j < s.hi[1] && k >= s.lo[2];
+}
+
+// interpolate_fields (curl.py:86-224) at cell (i,j,k) on a uniform grid. HALO: see needs_halo.
+template <bool HALO>
 __device__ __forceinline__ void interp(const StepStatic& P, const Src3& e, const Src3& hp, const Src3& h, int i, int j, int k,
                        float* Ei, float* Hi) {
-  if (stencil_inside(e, i, j, k) && stencil_inside(hp, i, j, k) && stencil_inside(h, i, j, k)) {
-    interp_inside(e, hp, h, i, j, k, Ei, Hi);
+  if (!HALO || (stencil_inside(e, i, j, k) && stencil_inside(hp, i, j, k) && stencil_inside(h, i, j, k))) {
+    interp_open(P, e, hp, h, i, j, k, Ei, Hi);
     return;
   }
   const float lo_x = 0.5f * (at(P, e, 0, i, j, k) + at(P, e, 0, i - 1, j, k));
@@ -198,15 +203,20 @@ __device__ __forceinline__ void region_cell(const DetK& K, long long q, int& i, 
   i = (int)ii + K.lo[0];
 }
 
+// Sum of v over the block, as thread 0 sees it: a fixed binary tree, its last six levels by lane
+// shuffles within the first wavefront.
 __device__ __forceinline__ double block_sum(double v) {
   __shared__ double sh[kBlock];
   sh[threadIdx.x] = v;
   __syncthreads();
-  for (int s = kBlock / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
-    __syncthreads();
+  double r = 0.0;
+  if (threadIdx.x < 128) sh[threadIdx.x] += sh[threadIdx.x + 128];
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    r = sh[threadIdx.x] + sh[threadIdx.x + 64];
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) r += __shfl_down(r, s);
   }
-  const double r = sh[0];
   __syncthreads();  // sh may be reused by the next call of this block
   return r;
 }
@@ -254,7 +264,7 @@ __device__ __forceinline__ void plane_axes(int ax, int& b0, int& b1) {
 // EnergyDetector(as_slices) with a collapsed-axis mean (energy.py:107-114): thread per cell of the
 // plane normal to K.axis, the energy averaged along that axis (float64 sum, then divided), stored
 // as slot `slot` of the (n_rec, d0, d1) state.
-template <bool CX>
+template <bool CX, bool HALO>
 __device__ __forceinline__ void energy_mean_tile(const StepStatic& P, const DetK& K, const DetDyn& D, int slot,
                                                  int blk, int nblk, const Src3& e, const Src3& hp, const Src3& h,
                                                  const Src3& e2, const Src3& hp2, const Src3& h2) {
@@ -275,8 +285,8 @@ __device__ __forceinline__ void energy_mean_tile(const StepStatic& P, const DetK
       const long long o = ((long long)c[0] * P.ny + c[1]) * P.nz + c[2];
       float Ei[3], Hi[3], Ej[3] = {0.f, 0.f, 0.f}, Hj[3] = {0.f, 0.f, 0.f};
       if (K.exact) {
-        interp(P, e, hp, h, c[0], c[1], c[2], Ei, Hi);
-        if (cx) interp(P, e2, hp2, h2, c[0], c[1], c[2], Ej, Hj);
+        interp<HALO>(P, e, hp, h, c[0], c[1], c[2], Ei, Hi);
+        if (cx) interp<HALO>(P, e2, hp2, h2, c[0], c[1], c[2], Ej, Hj);
       } else {
         for (int cc = 0; cc < 3; ++cc) { Ei[cc] = D.E[cc * P.N + o]; Hi[cc] = D.H[cc * P.N + o]; }
         if (cx)
@@ -292,7 +302,11 @@ __device__ __forceinline__ void energy_mean_tile(const StepStatic& P, const DetK
 // that stride over the detector's cells. A reducing detector leaves one partial sum per block and
 // value: the weighted energy or flux, or the sum of each recorded component (field and phasor
 // detectors with reduce_volume, whose box mean is formed in reduce_finalize_tile).
-template <bool CX>
+// PH: the launch has a detector with per-cell phasors, HALO: one that needs_halo. Without them
+// the kernel takes 76 (119 with phasors) instead of 199 (232) registers and more blocks run at a time:
+// the full-volume energy of the 64^3 cube measured 6.2 us against 25.5, the flux and three-frequency
+// phasor planes of 400x400x200 13.5 against 17.2.
+template <bool CX, bool PH, bool HALO>
 __device__ __forceinline__ void detector_tile(const StepStatic& P, const DetK& K, const DetDyn& D, int n, int slot,
                                               int blk, int nblk) {
   // CX: a complex-field plan (D.Ei set): e, hp, h view the real part and e2, hp2, h2 the imaginary one
@@ -308,7 +322,7 @@ __device__ __forceinline__ void detector_tile(const StepStatic& P, const DetK& K
     e2 = e; h2 = h; hp2 = hp;
   }
   if (K.kind == FDTDX_DET_ENERGY && K.reduce == 2) {
-    energy_mean_tile<CX>(P, K, D, slot, blk, nblk, e, hp, h, e2, hp2, h2);
+    energy_mean_tile<CX, HALO>(P, K, D, slot, blk, nblk, e, hp, h, e2, hp2, h2);
     return;
   }
   const int nv = reduced_values(K);
@@ -318,9 +332,22 @@ __device__ __forceinline__ void detector_tile(const StepStatic& P, const DetK& K
     region_cell(K, q, i, j, k);
     const long long o = ((long long)i * P.ny + j) * P.nz + k;
     float Ei[3], Hi[3], Ej[3] = {0.f, 0.f, 0.f}, Hj[3] = {0.f, 0.f, 0.f};
+    // per-cell phasors: the state words of up to three frequencies are loaded before any is updated,
+    // those of the first three ahead of the field reads, so that all are in flight together (a plane
+    // detector launches too few waves to hide them one by one)
+    float2 old[3][6];
+    auto load_phasor = [&](int f0) {
+      const float2* st = (const float2*)D.state;
+#pragma unroll
+      for (int df = 0; df < 3; ++df)
+#pragma unroll
+        for (int c = 0; c < 6; ++c)
+          if (f0 + df < K.nfreq && c < K.ncomp) old[df][c] = st[((long long)(f0 + df) * K.ncomp + c) * K.cells + q];
+    };
+    if (PH && K.kind == FDTDX_DET_PHASOR && !nv) load_phasor(0);
     if (K.exact) {
-      interp(P, e, hp, h, i, j, k, Ei, Hi);
-      if (cx) interp(P, e2, hp2, h2, i, j, k, Ej, Hj);
+      interp<HALO>(P, e, hp, h, i, j, k, Ei, Hi);
+      if (cx) interp<HALO>(P, e2, hp2, h2, i, j, k, Ej, Hj);
     } else {
       for (int c = 0; c < 3; ++c) { Ei[c] = D.E[c * P.N + o]; Hi[c] = D.H[c * P.N + o]; }
       if (cx)
@@ -359,10 +386,7 @@ __device__ __forceinline__ void detector_tile(const StepStatic& P, const DetK& K
       for (int c = 0; c < K.ncomp; ++c) acc[c] += (double)pick6(K.comps[c], Ei, Hi);
       if (cx)  // the imaginary parts' sums follow the real parts'
         for (int c = 0; c < K.ncomp; ++c) acc[K.ncomp + c] += (double)pick6(K.comps[c], Ej, Hj);
-    } else {  // PHASOR (phasor.py:190-235): state += EH * exp(i w t) * scale * window
-      // the state words of up to three frequencies are all loaded before any is updated, so their
-      // reads are in flight together (a plane detector launches too few waves to hide them
-      // one by one)
+    } else if constexpr (PH) {  // PHASOR (phasor.py:190-235): state += EH * exp(i w t) * scale * window
       float2* st = (float2*)D.state;
       const float w = K.window[n];
       float v[6], vi[6];
@@ -372,12 +396,7 @@ __device__ __forceinline__ void detector_tile(const StepStatic& P, const DetK& K
         vi[c] = c < K.ncomp ? pick6(K.comps[c], Ej, Hj) : 0.f;
       }
       for (int f0 = 0; f0 < K.nfreq; f0 += 3) {
-        float2 old[3][6];
-#pragma unroll
-        for (int df = 0; df < 3; ++df)
-#pragma unroll
-          for (int c = 0; c < 6; ++c)
-            if (f0 + df < K.nfreq && c < K.ncomp) old[df][c] = st[((long long)(f0 + df) * K.ncomp + c) * K.cells + q];
+        if (f0) load_phasor(f0);
 #pragma unroll
         for (int df = 0; df < 3; ++df) {
           const int f = f0 + df;
@@ -479,7 +498,7 @@ __device__ __forceinline__ float reduce_finalize_tile(const StepStatic& P, const
 template <bool CX>
 __global__ __launch_bounds__(kBlock) void k_detector(const StepStatic* __restrict__ Pp, const DetK K, const DetDyn D) {
   const StepStatic& P = as_const(Pp);
-  detector_tile<CX>(P, K, D, D.n, D.slot, blockIdx.x, gridDim.x);
+  detector_tile<CX, true, true>(P, K, D, D.n, D.slot, blockIdx.x, gridDim.x);
 }
 
 __global__ __launch_bounds__(kBlock) void k_reduce_finalize(const StepStatic* __restrict__ Pp, const DetK K, const double* partial,
@@ -490,7 +509,7 @@ __global__ __launch_bounds__(kBlock) void k_reduce_finalize(const StepStatic* __
 
 static_assert(2 * sizeof(void*) + sizeof(DetGroup) <= 4096, "grouped detector kernel arguments exceed 4 KB");
 
-template <bool CX>
+template <bool CX, bool PH, bool HALO>
 __global__ __launch_bounds__(kBlock) void k_detector_group(const StepStatic* __restrict__ Pp, const DetK* __restrict__ Kd,
                                                            const DetGroup G) {
   const StepStatic& P = as_const(Pp);
@@ -498,7 +517,7 @@ __global__ __launch_bounds__(kBlock) void k_detector_group(const StepStatic* __r
   while (a + 1 < G.count && (int)blockIdx.x >= G.start[a + 1]) ++a;
   const DetK& K = Kd[G.q[a]];
   const DetDyn& D = G.dd[a];
-  detector_tile<CX>(P, K, D, D.n, G.slot[a], (int)blockIdx.x - G.start[a], G.start[a + 1] - G.start[a]);
+  detector_tile<CX, PH, HALO>(P, K, D, D.n, G.slot[a], (int)blockIdx.x - G.start[a], G.start[a + 1] - G.start[a]);
 }
 
 __global__ __launch_bounds__(kBlock) void k_finalize_group(const StepStatic* __restrict__ Pp, const DetK* __restrict__ Kd,
@@ -512,6 +531,30 @@ __global__ __launch_bounds__(kBlock) void k_finalize_group(const StepStatic* __r
     reduce_finalize_tile(P, K, D.partial, G.start[a + 1] - G.start[a], D.state, G.slot[a], D.n);
     __syncthreads();  // the next accumulating detector reads the value thread 0 just stored
   }
+}
+
+// The sums of up to kDetRing steps in one launch: block (b, t) finalizes step F.n0 + t of chain head
+// F.q[b] (an energy, flux or field detector) and of the detectors accumulating after it, from the
+// partial sums that step left in its part of the ring. A launch per step took 2.4 to 4.8 us.
+__global__ __launch_bounds__(kBlock) void k_finalize_ring(const StepStatic* __restrict__ Pp,
+                                                          const DetK* __restrict__ Kd, const DetRing F) {
+  const StepStatic& P = as_const(Pp);
+  const int n = F.n0 + (int)blockIdx.y;
+  const double* part = F.partial + (long long)blockIdx.y * F.ndet * kDetMaxValues * kDetMaxBlocks;
+  const int q0 = F.q[blockIdx.x];
+  const int slot = Kd[q0].tti[n];
+  if (slot < 0) return;
+  for (int q = q0; q < F.ndet && (q == q0 || Kd[q].accum); ++q) {
+    reduce_finalize_tile(P, Kd[q], part + (long long)q * kDetMaxValues * kDetMaxBlocks, detector_blocks(Kd[q]),
+                         F.state[q], slot, n);
+    __syncthreads();  // the next accumulating detector reads the value thread 0 just stored
+  }
+}
+
+hipError_t launch_finalize_ring(const StepStatic& P, const DetK* Kdev, const DetRing& F, int steps, hipStream_t s) {
+  if (F.count > 0 && steps > 0)
+    hipLaunchKernelGGL(k_finalize_ring, dim3((unsigned)F.count, (unsigned)steps), dim3(kBlock), 0, s, P.self, Kdev, F);
+  return hipGetLastError();
 }
 
 // Batch detectors: the blocks of every (entry, detector) pair are concatenated; a persistent grid
@@ -534,7 +577,7 @@ __global__ __launch_bounds__(kBlock) void k_batch_detector(const BatchTable* __r
     int slot = K.tti[n];
     if (slot < 0) continue;
     if (K.kind == FDTDX_DET_PHASOR) slot = 0;
-    detector_tile<false>(I.P, K, I.dd[q], n, slot, b, I.det_nb[q]);
+    detector_tile<false, true, true>(I.P, K, I.dd[q], n, slot, b, I.det_nb[q]);
   }
 }
 
@@ -579,13 +622,6 @@ hipError_t launch_batch_detectors(const BatchTable* tab, const int* base, int r,
   return hipGetLastError();
 }
 
-int detector_blocks(const DetK& K) {
-  long long b = (K.cells + kBlock - 1) / kBlock;
-  if (b > kDetMaxBlocks) b = kDetMaxBlocks;
-  if (b < 1) b = 1;
-  return (int)b;
-}
-
 hipError_t launch_detector(const StepStatic& P, const DetK& K, const DetDyn& D, int nblocks, hipStream_t s) {
   if (D.Ei) hipLaunchKernelGGL(k_detector<true>, dim3(nblocks), dim3(kBlock), 0, s, P.self, K, D);
   else hipLaunchKernelGGL(k_detector<false>, dim3(nblocks), dim3(kBlock), 0, s, P.self, K, D);
@@ -597,8 +633,13 @@ hipError_t launch_detector(const StepStatic& P, const DetK& K, const DetDyn& D, 
 
 hipError_t launch_detector_group(const StepStatic& P, const DetK* Kdev, const DetGroup& G, hipStream_t s) {
   if (G.count <= 0) return hipSuccess;
-  if (G.dd[0].Ei) hipLaunchKernelGGL(k_detector_group<true>, dim3(G.start[G.count]), dim3(kBlock), 0, s, P.self, Kdev, G);
-  else hipLaunchKernelGGL(k_detector_group<false>, dim3(G.start[G.count]), dim3(kBlock), 0, s, P.self, Kdev, G);
+  const dim3 g((unsigned)G.start[G.count]);
+  using GroupKernel = void (*)(const StepStatic*, const DetK*, const DetGroup);
+  const bool hl = G.halo != 0;
+  const GroupKernel f = G.dd[0].Ei ? (hl ? k_detector_group<true, true, true> : k_detector_group<true, true, false>)
+                        : G.phasor ? (hl ? k_detector_group<false, true, true> : k_detector_group<false, true, false>)
+                                   : (hl ? k_detector_group<false, false, true> : k_detector_group<false, false, false>);
+  hipLaunchKernelGGL(f, g, dim3(kBlock), 0, s, P.self, Kdev, G);
   if (G.nfin > 0) hipLaunchKernelGGL(k_finalize_group, dim3(G.nfin), dim3(kBlock), 0, s, P.self, Kdev, G);
   return hipGetLastError();
 }
@@ -665,6 +706,7 @@ hipError_t launch_snapshot(const StepStatic& P, const float* src, float* dst, co
 // ---------------------------------------------------------------- detector adjoint
 // Stage 1: cotangents in the interpolated space (6 per region cell), the transpose of each
 // detector's update() with respect to its co-located inputs.
+template <bool HALO>
 __global__ __launch_bounds__(kBlock) void k_det_adj_g(const StepStatic* __restrict__ Pp, const DetK K, const DetAdjDyn D) {
   const StepStatic& P = as_const(Pp);
   const Src3 e = box3(D.E1, D.slo, D.shi, 0);
@@ -676,7 +718,7 @@ __global__ __launch_bounds__(kBlock) void k_det_adj_g(const StepStatic* __restri
     const long long o = ((long long)i * P.ny + j) * P.nz + k;
     float Ei[3], Hi[3];
     if (K.exact) {
-      interp(P, e, h0, h1, i, j, k, Ei, Hi);
+      interp<HALO>(P, e, h0, h1, i, j, k, Ei, Hi);
     } else {
       for (int c = 0; c < 3; ++c) { Ei[c] = at(P, e, c, i, j, k); Hi[c] = at(P, h1, c, i, j, k); }
     }
@@ -861,7 +903,8 @@ static int blocks_for(long long cells) {
 }
 
 hipError_t launch_detector_adjoint(const StepStatic& P, const DetK& K, const DetAdjDyn& D, hipStream_t s) {
-  hipLaunchKernelGGL(k_det_adj_g, dim3(blocks_for(K.cells)), dim3(kBlock), 0, s, P.self, K, D);
+  hipLaunchKernelGGL(needs_halo(P, K) ? k_det_adj_g<true> : k_det_adj_g<false>, dim3(blocks_for(K.cells)), dim3(kBlock), 0, s,
+                     P.self, K, D);
   const long long ec = (long long)(D.ehi[0] - D.elo[0]) * (D.ehi[1] - D.elo[1]) * (D.ehi[2] - D.elo[2]);
   hipLaunchKernelGGL(k_det_adj_scatter, dim3(blocks_for(ec)), dim3(kBlock), 0, s, P.self, K, D);
   return hipGetLastError();

@@ -54,12 +54,39 @@ constexpr int kDetGroup = 8;         // detectors of one grouped launch (the ker
 // which then also finalizes the accumulating detectors that follow it.
 struct DetGroup {
   int count, nfin;
+  int phasor;  // some detector of the group keeps per-cell phasors
+  int halo;    // some detector of the group needs_halo
   int q[kDetGroup];
   int slot[kDetGroup];
   int start[kDetGroup + 1];
   int fin[kDetGroup];
   DetDyn dd[kDetGroup];
 };
+// Blocks of one detector's launch.
+__host__ __device__ inline int detector_blocks(const DetK& K) {
+  const long long b = (K.cells + kBlock - 1) / kBlock;
+  return (int)(b > kDetMaxBlocks ? kDetMaxBlocks : (b < 1 ? 1 : b));
+}
+
+// The interpolation stencil of some cell of the detector reads beyond a periodic face or below a
+// symmetry plane, whose halo is not zero.
+inline bool needs_halo(const StepStatic& P, const DetK& K) {
+  const int n[3] = {P.nx, P.ny, P.nz};
+  for (int a = 0; a < 3; ++a)
+    if ((P.wrap[a] && (K.lo[a] == 0 || K.hi[a] == n[a])) || (P.mirror[a] && K.lo[a] == 0)) return true;
+  return false;
+}
+
+// Deferred sums (k_finalize_ring): the partial sums of up to kDetRing steps, and the chain heads
+// (reducing energy, flux and field detectors that do not accumulate).
+constexpr int kDetRing = 16;
+struct DetRing {
+  int n0, ndet, count;
+  int q[FDTDX_MAX_DETECTORS];
+  void* state[FDTDX_MAX_DETECTORS];
+  const double* partial;  // step n0 + t, detector q: partial[(t * ndet + q) * kDetMaxValues * kDetMaxBlocks]
+};
+
 constexpr int kDetMaxValues = 6;     // reduced values per step: 1 (energy), 1 or 3 (flux), one per component
 
 // Reduced values a detector sums over its box per step, 0 when it keeps per-cell values.
@@ -183,7 +210,7 @@ hipError_t launch_record(const StepStatic& P, const StepDyn& D, long long iface_
 hipError_t launch_reverse(const StepStatic& P, const StepDyn& D, int ec, int mc, hipStream_t s);
 hipError_t launch_detector(const StepStatic& P, const DetK& K, const DetDyn& D, int nblocks, hipStream_t s);
 hipError_t launch_detector_group(const StepStatic& P, const DetK* Kdev, const DetGroup& G, hipStream_t s);
-int detector_blocks(const DetK& K);
+hipError_t launch_finalize_ring(const StepStatic& P, const DetK* Kdev, const DetRing& F, int steps, hipStream_t s);
 
 struct AdjDyn {
   float* lamE;

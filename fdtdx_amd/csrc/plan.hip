@@ -72,7 +72,8 @@ struct fdtdx_plan {
   size_t ws_snapH = 0, ws_snapE = 0, ws_partial = 0, ws_g = 0, ws_half = 0, ws_lpsi = 0, ws_bytes = 0;
   size_t ws_K = 0, ws_W = 0;  // full-tensor plans only
   size_t ws_Fo = 0, ws_ab[2] = {0, 0};  // full-tensor plans with conductivity
-  size_t ws_fwd_end = 0;       // workspace bytes the two-sweep forward uses
+  size_t ws_fwd_end = 0;       // workspace bytes the two-sweep forward without the ring uses
+  size_t ws_ring = 0;          // partial sums of kDetRing steps (0: no detector sums)
   size_t g_off[FDTDX_MAX_DETECTORS], half_off[FDTDX_MAX_DETECTORS];
   // single-pass paths (1: LDS-tiled fused kernel, 2: register-march kernel): tile configuration
   // and ping-pong copies of E, H and psi in the workspace
@@ -713,6 +714,9 @@ static int plan_create(const fdtdx_plan_desc* d, fdtdx_plan** out) {
   pl->ws_snapE = off; off = align256(off + 3 * (size_t)pl->snap_cells * 4);
   pl->ws_partial = off; off = align256(off + (size_t)pl->ndet * kDetMaxValues * kDetMaxBlocks * 8);
   pl->ws_fwd_end = off;  // the forward (two-sweep schedules) touches nothing past this offset
+  for (int q = 0; q < pl->ndet; ++q)
+    if (reduced_values(pl->det[q]) && pl->det[q].kind != FDTDX_DET_PHASOR) pl->ws_ring = off;
+  if (pl->ws_ring) off = align256(off + (size_t)kDetRing * pl->ndet * kDetMaxValues * kDetMaxBlocks * 8);
   for (int q = 0; q < pl->ndet; ++q) { pl->g_off[q] = off; off = align256(off + 6 * (size_t)pl->det[q].cells * 4); }
   for (int q = 0; q < pl->ndet; ++q) {
     const long long ec = (long long)(pl->ehi[q][0] - pl->elo[q][0]) * (pl->ehi[q][1] - pl->elo[q][1]) *
@@ -830,7 +834,7 @@ static StepDyn make_dyn(const fdtdx_plan* p, const fdtdx_buffers* b) {
 }
 
 static int forward_impl(const fdtdx_plan* p, const fdtdx_buffers* b, int32_t t0, int32_t t1, int32_t rec,
-                        void* stream, hipEvent_t* ev);
+                        void* stream, hipEvent_t* ev, bool ring = true);
 
 // ---------------------------------------------------------------- forward without allocation
 // fdtdx_forward_noalloc runs fdtdx_forward with its workspace (the H_prev snapshot of the detector
@@ -874,7 +878,7 @@ int fdtdx_forward_noalloc(const fdtdx_plan* p, const fdtdx_buffers* b, int32_t t
   if (rc) return rc;
   fdtdx_buffers b2 = *b;
   b2.workspace = ws;
-  return forward_impl(p, &b2, t0, t1, rec, stream, nullptr);
+  return forward_impl(p, &b2, t0, t1, rec, stream, nullptr, false);  // the ring lies past ws_fwd_end
 }
 
 int fdtdx_plan_schedule(const fdtdx_plan* p, int32_t* out) {
@@ -917,7 +921,7 @@ int fdtdx_forward_timed(const fdtdx_plan* p, const fdtdx_buffers* b, int32_t t0,
 }
 
 static int forward_impl(const fdtdx_plan* p, const fdtdx_buffers* b, int32_t t0, int32_t t1, int32_t rec,
-                        void* stream, hipEvent_t* ev) {
+                        void* stream, hipEvent_t* ev, bool ring) {
   if (!p) return fail(FDTDX_EINVAL, "null plan");
   int rc = check_buffers(p, b);
   if (rc) return rc;
@@ -941,6 +945,21 @@ static int forward_impl(const fdtdx_plan* p, const fdtdx_buffers* b, int32_t t0,
   float* Eb[2] = {b->E, p->use_fused ? (float*)(ws + p->ws_Ealt) : b->E};
   float* Hb[2] = {b->H, p->use_fused ? (float*)(ws + p->ws_Halt) : b->H};
   float* Pb[2] = {b->psi, p->use_fused ? (float*)(ws + p->ws_psialt) : b->psi};
+  // sums of energy, flux and field detectors: finalized for kDetRing steps at a time
+  DetRing F;
+  memset(&F, 0, sizeof(F));
+  ring = ring && p->ws_ring;
+  if (ring) {
+    F.n0 = t0;
+    F.ndet = p->ndet;
+    F.partial = (const double*)(ws + p->ws_ring);
+    for (int q = 0; q < p->ndet; ++q) {
+      F.state[q] = b->detector_state[q];
+      if (reduced_values(p->det[q]) && p->det[q].kind != FDTDX_DET_PHASOR && !p->det[q].accum && !p->det[q].inv)
+        F.q[F.count++] = q;
+    }
+  }
+  auto deferred = [&](int q) { return ring && p->det[q].kind != FDTDX_DET_PHASOR; };
   for (int n = t0; n < t1; ++n) {
     bool any = false;
     for (int q = 0; q < p->ndet; ++q) any = any || p->tti[q][n] >= 0;
@@ -994,11 +1013,11 @@ static int forward_impl(const fdtdx_plan* p, const fdtdx_buffers* b, int32_t t0,
     // the detectors of step n in grouped launches of up to kDetGroup (a chain of accumulating
     // detectors stays in one group); one finalize launch per group for the reduced values
     DetGroup G;
-    G.count = G.nfin = 0;
+    G.count = G.nfin = G.phasor = G.halo = 0;
     G.start[0] = 0;
     auto flush = [&]() -> int {
       const hipError_t e = launch_detector_group(p->P, p->det_dev, G, s);
-      G.count = G.nfin = 0;
+      G.count = G.nfin = G.phasor = G.halo = 0;
       return e == hipSuccess ? FDTDX_OK : fail(FDTDX_EHIP, "detector launch: %s", hipGetErrorString(e));
     };
     for (int q = 0; q < p->ndet; ++q) {
@@ -1014,6 +1033,8 @@ static int forward_impl(const fdtdx_plan* p, const fdtdx_buffers* b, int32_t t0,
         const int tail = G.count - h;
         DetGroup R;
         R.count = 0; R.nfin = 0; R.start[0] = 0;
+        R.phasor = 0;  // a chain of accumulating detectors sums energies or fluxes
+        R.halo = G.halo;
         for (int t = 0; t < tail; ++t) {
           const int a = h + t;
           R.q[t] = G.q[a]; R.slot[t] = G.slot[a]; R.dd[t] = G.dd[a];
@@ -1027,7 +1048,7 @@ static int forward_impl(const fdtdx_plan* p, const fdtdx_buffers* b, int32_t t0,
         if ((rc = flush())) return rc;
         G = R;
         for (int a = 0; a < G.count; ++a)
-          if (reduced_values(p->det[G.q[a]]) && !p->det[G.q[a]].accum) G.fin[G.nfin++] = a;
+          if (reduced_values(p->det[G.q[a]]) && !p->det[G.q[a]].accum && !deferred(G.q[a])) G.fin[G.nfin++] = a;
       }
       const int a = G.count;
       DetDyn& dd = G.dd[a];
@@ -1041,14 +1062,21 @@ static int forward_impl(const fdtdx_plan* p, const fdtdx_buffers* b, int32_t t0,
       dd.state = b->detector_state[q];
       dd.slot = p->det[q].kind == FDTDX_DET_PHASOR ? 0 : slot;
       dd.n = n;
-      dd.partial = (double*)(ws + p->ws_partial) + (size_t)q * kDetMaxValues * kDetMaxBlocks;
+      dd.partial = (double*)(ws + (ring ? p->ws_ring : p->ws_partial)) +
+                   ((size_t)(ring ? n - F.n0 : 0) * p->ndet + q) * kDetMaxValues * kDetMaxBlocks;
       G.q[a] = q;
       G.slot[a] = dd.slot;
       G.start[a + 1] = G.start[a] + detector_blocks(p->det[q]);
-      if (reduced_values(p->det[q]) && !p->det[q].accum) G.fin[G.nfin++] = a;
+      if (reduced_values(p->det[q]) && !p->det[q].accum && !deferred(q)) G.fin[G.nfin++] = a;
+      if (p->det[q].kind == FDTDX_DET_PHASOR && !p->det[q].reduce) G.phasor = 1;
+      if (needs_halo(p->P, p->det[q])) G.halo = 1;
       G.count = a + 1;
     }
     if (G.count > 0 && (rc = flush())) return rc;
+    if (ring && (n + 1 - F.n0 == kDetRing || n + 1 == t1)) {
+      HIP_TRY(launch_finalize_ring(p->P, p->det_dev, F, n + 1 - F.n0, s));
+      F.n0 = n + 1;
+    }
   }
   if (p->use_fused && ((t1 - t0) & 1)) {
     HIP_TRY(hipMemcpyAsync(b->E, Eb[1], 3 * (size_t)p->P.N * 4, hipMemcpyDeviceToDevice, s));

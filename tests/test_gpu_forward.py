@@ -470,6 +470,47 @@ def test_quad_sweeps_equal_one_cell_sweeps_bitwise(case, monkeypatch):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("T", [1, 15, 16, 17, 33])
+@pytest.mark.parametrize("halo", [False, True])
+def test_deferred_detector_sums_equal_a_launch_per_step(T, halo):
+    """Sums finalized for 16 steps at a time (one call) against step by step calls (one step each):
+    energy over the whole volume, flux with a switch, reduced field and phasor detectors and a closed
+    surface's accumulating faces agree bit for bit, with zero and periodic halos."""
+    import torch
+
+    from fdtdx_amd import fdtd as F
+    import scenarios
+
+    n = 20
+    full = ((0, n), (0, n), (0, n))
+    spec = W.scenario_c1(T=T, n=n, pml=4, cube=4)
+    spec["sources"][0]["profile"] = dict(kind="single", frequency=2e14, phase_shift=0.3)
+    if halo:
+        spec["pml"] = dict(spec["pml"], types={f: "periodic" for f in ("min_y", "max_y")})
+    spec["detectors"] = [
+        dict(name="energy", kind="energy", slc=full, reduce_volume=True),
+        dict(name="flux", kind="flux", slc=((14, 15), (0, n), (4, 16)), axis=0, reduce_volume=True,
+             switch={"interval": 3}),
+        dict(name="field", kind="field", slc=((6, 9), (5, 12), (4, 9)), components=("Ez", "Hx"), reduce_volume=True),
+        dict(name="phasor", kind="phasor", slc=((6, 9), (5, 12), (4, 9)), components=("Ez", "Hx"),
+             frequencies=[2e14], reduce_volume=True),
+        dict(name="box", kind="closed_flux", slc=((5, 15), (5, 15), (5, 15))),
+    ]
+    out = []
+    for stepwise in (False, True):
+        objects, arrays, params, config = scenarios.build(spec)
+        s = F.Solve(objects, config, arrays)
+        arrays.reset()
+        print(f"T={T} halo={halo} stepwise={stepwise}", flush=True)
+        for t in range(T if stepwise else 1):
+            s.forward(t if stepwise else 0, t + 1 if stepwise else T)
+        torch.cuda.synchronize()
+        out.append([t.cpu().numpy() for t in s.state_tensors()])
+    assert T == 1 or np.abs(out[0][0]).max() > 0  # the source's ramp starts from zero
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
 def _ragged_cases():
     """Rows of nz % 4 != 0 cells: the last quad of a row repeats cells of the quad before it."""
     c1 = W.scenario_c1(T=60, n=29, pml=5, cube=6)                                  # nz % 4 = 1
