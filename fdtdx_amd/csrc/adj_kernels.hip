@@ -915,6 +915,20 @@ __global__ __launch_bounds__(kBlock) void k_adj_B4(const StepStatic* __restrict_
   quad_transpose<false, 0, 0, RAG>(P, A.lpsi_in, A.lpsi_out, i, j, k0, sm, wy, wz, wy_ip, wz_ip, lh[0], lh[1], lh[2]);
   quad_transpose<false, 0, 1, RAG>(P, A.lpsi_in, A.lpsi_out, i, j, k0, sm, wz, wx, wz_jp, wx_jp, lh[0], lh[1], lh[2]);
   quad_transpose<false, 0, 2, RAG>(P, A.lpsi_in, A.lpsi_out, i, j, k0, sm, wx, wy, wx_kp, wy_kp, lh[0], lh[1], lh[2]);
+  if (A.nhalf && (P.vec_mask[lb] & kSnapBit)) {  // the detector boxes, grown by a cell
+#pragma unroll 1
+    for (int t = 0; t < A.nhalf; ++t) {
+      const AdjDyn::Half& B = A.half[t];
+      const long long by = B.hi[1] - B.lo[1], bz = B.hi[2] - B.lo[2], cells = (B.hi[0] - B.lo[0]) * by * bz;
+      const long long q = ((long long)(i - B.lo[0]) * by + (j - B.lo[1])) * bz + (k0 - B.lo[2]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (!in_box(i, j, k0 + e, B.lo, B.hi)) continue;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) lh[a][e] += B.v[a * cells + q + e];
+      }
+    }
+  }
 #pragma unroll
   for (int a = 0; a < 3; ++a) st4m<RAG>(A.lamH + a * N + o, lh[a], sm);
 }

@@ -709,7 +709,7 @@ hipError_t launch_snapshot(const StepStatic& P, const float* src, float* dst, co
 template <bool HALO>
 __global__ __launch_bounds__(kBlock) void k_det_adj_g(const StepStatic* __restrict__ Pp, const DetK K, const DetAdjDyn D) {
   const StepStatic& P = as_const(Pp);
-  const Src3 e = box3(D.E1, D.slo, D.shi, 0);
+  const Src3 e = D.E1full ? full3(P, D.E1, 0) : box3(D.E1, D.slo, D.shi, 0);
   const Src3 h1 = box3(D.H1, D.slo, D.shi, 1);
   const Src3 h0 = full3(P, D.H0, 1);
   for (long long q = (long long)blockIdx.x * kBlock + threadIdx.x; q < K.cells; q += (long long)gridDim.x * kBlock) {

@@ -227,6 +227,13 @@ struct AdjDyn {
   float* K;              // full-tensor permittivity: K^{n+1/2} of every cell, (3, N)
   float* Erev;           // fused reverse (non-null): E^{n+1} is reversed to E^n in place by pass A
   int n;                 // the step being undone (sources of the fused reverse)
+  // quad adjoint: the detectors' halves of the H cotangent that belong to H^n (DetAdjDyn::half_vH,
+  // over [lo, hi)), added to lam_H by pass B
+  int nhalf;
+  struct Half {
+    const float* v;
+    int lo[3], hi[3];
+  } half[FDTDX_MAX_DETECTORS];
 };
 
 hipError_t launch_adjoint(const StepStatic& P, const AdjDyn& A, int ec, int mc, hipStream_t s);
@@ -235,7 +242,8 @@ hipError_t launch_reverse_H(const StepStatic& P, const StepDyn& D, int mc, hipSt
 
 // Detector cotangent injection for reverse step n.
 struct DetAdjDyn {
-  const float* E1;     // E^{n+1} snapshot over the snapshot box
+  const float* E1;     // E^{n+1}: a snapshot over the snapshot box, or the whole field (E1full)
+  int E1full;
   const float* H1;     // H^{n+1} snapshot
   const float* H0;     // H^n (full field)
   int slo[3], shi[3];

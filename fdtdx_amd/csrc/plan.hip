@@ -1174,7 +1174,11 @@ int fdtdx_reverse_adjoint(const fdtdx_plan* p, const fdtdx_buffers* b, const fdt
       if (p->tti[q][n] < 0) continue;
       any = true;
     }
-    if (any) {
+    // E^{n+1} and H^{n+1} over the detector boxes: the quad adjoint reads E in place (pass A undoes it
+    // after the detector cotangents) and keeps H in its reverse H sweep
+    const bool quad = p->P.aquad && p->ec != 9 && p->mc != 9;
+    if (any && quad) D.snap = (float*)(ws + p->ws_snapH);
+    if (any && !quad) {
       HIP_TRY(launch_snapshot(p->P, b->E, (float*)(ws + p->ws_snapE), p->slo, p->shi, s, b->H,
                               (float*)(ws + p->ws_snapH)));
     }
@@ -1191,7 +1195,8 @@ int fdtdx_reverse_adjoint(const fdtdx_plan* p, const fdtdx_buffers* b, const fdt
       if (!on[q]) continue;
       DetAdjDyn& x = dd[q];
       memset(&x, 0, sizeof(x));
-      x.E1 = (const float*)(ws + p->ws_snapE);
+      x.E1 = quad ? b->E : (const float*)(ws + p->ws_snapE);
+      x.E1full = quad;
       x.H1 = (const float*)(ws + p->ws_snapH);
       x.H0 = b->H;
       for (int a = 0; a < 3; ++a) {
@@ -1216,10 +1221,17 @@ int fdtdx_reverse_adjoint(const fdtdx_plan* p, const fdtdx_buffers* b, const fdt
     A.W = (p->ec == 9 || p->mc == 9) ? (float*)(ws + p->ws_W) : nullptr;
     A.Erev = fuse ? b->E : nullptr;
     A.n = n;
+    A.nhalf = 0;
+    for (int q = 0; q < p->ndet; ++q) {
+      if (!on[q] || !quad) continue;
+      AdjDyn::Half& h = A.half[A.nhalf++];
+      h.v = dd[q].half_vH;
+      for (int a = 0; a < 3; ++a) { h.lo[a] = dd[q].elo[a]; h.hi[a] = dd[q].ehi[a]; }
+    }
     HIP_TRY(launch_adjoint(p->P, A, p->ec, p->mc, s));
     std::swap(lpsi_a, lpsi_b);
     for (int q = 0; q < p->ndet; ++q)
-      if (on[q]) HIP_TRY(launch_add_half_vH(p->P, dd[q], s));
+      if (on[q] && !quad) HIP_TRY(launch_add_half_vH(p->P, dd[q], s));
   }
   if (lpsi_a != adj->lam_psi && p->psi_floats)
     HIP_TRY(hipMemcpyAsync(adj->lam_psi, lpsi_a, p->psi_floats * 4, hipMemcpyDeviceToDevice, s));
