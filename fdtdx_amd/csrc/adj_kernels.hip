@@ -320,7 +320,7 @@ __device__ __forceinline__ void reverse_E_cell(const StepStatic& P, const AdjDyn
   float* Ey = A.Erev + P.N;
   float* Ez = A.Erev + 2 * P.N;
   float ex = Ex[o], ey = Ey[o], ez = Ez[o];
-  apply_sources<false>(P, m, A.ie, A.im, 0, A.n, true, i, j, k, o, EC, 0, ex, ey, ez);
+  apply_sources(P, m, A.ie, A.im, 0, A.n, true, i, j, k, o, EC, 0, ex, ey, ez);
   const float iex = A.ie[o];
   const float iey = EC == 3 ? A.ie[P.N + o] : iex;
   const float iez = EC == 3 ? A.ie[2 * P.N + o] : iex;

@@ -560,65 +560,81 @@ hipError_t launch_finalize_ring(const StepStatic& P, const DetK* Kdev, const Det
 // Batch detectors: the blocks of every (entry, detector) pair are concatenated; a persistent grid
 // strides over them. Each pair keeps the block count of the single-solve launch, so its partial
 // sums, and with them the reduced values, are bit-identical to a solve run alone.
-__global__ __launch_bounds__(kBlock) void k_batch_detector(const BatchTable* __restrict__ B,
+template <bool PH, bool HALO>
+__global__ __launch_bounds__(kBlock) void k_batch_detector(const BatchTable* __restrict__ Bp,
                                                            const int* __restrict__ base, int r) {
-  const int ni = B->ninst;
-  const int total = B->det_start[ni];
+  const BatchTable& B = as_const(Bp);
+  const int ni = B.ninst;
+  const int total = B.det_start[ni];
   int e = 0;
   for (int t = blockIdx.x; t < total; t += gridDim.x) {
-    while (t >= B->det_start[e + 1]) ++e;
-    const BatchInst& I = B->inst[e];
+    while (t >= B.det_start[e + 1]) ++e;
+    const BatchInst& I = B.inst[e];
     const int n = base[I.slot] + r;
     if (n >= I.stop) continue;
-    int b = t - B->det_start[e];
+    int b = t - B.det_start[e];
     int q = 0;
     while (q < I.ndet - 1 && b >= I.det_nb[q]) { b -= I.det_nb[q]; ++q; }
     const DetK& K = I.det[q];
     int slot = K.tti[n];
     if (slot < 0) continue;
     if (K.kind == FDTDX_DET_PHASOR) slot = 0;
-    detector_tile<false, true, true>(I.P, K, I.dd[q], n, slot, b, I.det_nb[q]);
+    DetDyn D = I.dd[q];
+    D.partial += (long long)(r % kDetRing) * I.ndet * kDetMaxValues * kDetMaxBlocks;
+    detector_tile<false, PH, HALO>(I.P, K, D, n, slot, b, I.det_nb[q]);
   }
 }
 
-__global__ __launch_bounds__(kBlock) void k_batch_finalize(const BatchTable* __restrict__ B,
-                                                           const int* __restrict__ base, int r) {
-  const int ni = B->ninst;
-  const int total = B->fin_start[ni];
+// The sums of chunk step r0 + blockIdx.y (reduced phasors, which add up over the steps: of all the
+// launch's steps in order, by the blocks of blockIdx.y = 0).
+__global__ __launch_bounds__(kBlock) void k_batch_finalize(const BatchTable* __restrict__ Bp,
+                                                           const int* __restrict__ base, int r0) {
+  const BatchTable& B = as_const(Bp);
+  const int ni = B.ninst;
+  const int total = B.fin_start[ni];
   int e = 0;
   for (int t = blockIdx.x; t < total; t += gridDim.x) {
-    while (t >= B->fin_start[e + 1]) ++e;
-    const BatchInst& I = B->inst[e];
-    const int n = base[I.slot] + r;
-    if (n >= I.stop) continue;
-    int want = t - B->fin_start[e];
-    for (int q = 0; q < I.ndet; ++q) {
-      const DetK& K = I.det[q];
-      if (!reduced_values(K) || K.accum) continue;
-      if (want-- != 0) continue;
+    while (t >= B.fin_start[e + 1]) ++e;
+    const BatchInst& I = B.inst[e];
+    int want = t - B.fin_start[e];
+    int q = 0;
+    for (; q < I.ndet; ++q)
+      if (reduced_values(I.det[q]) && !I.det[q].accum && want-- == 0) break;
+    if (q >= I.ndet) continue;
+    const DetK& K = I.det[q];
+    const bool ph = K.kind == FDTDX_DET_PHASOR;
+    if (ph && blockIdx.y) continue;
+    const int y0 = ph ? 0 : (int)blockIdx.y, y1 = ph ? (int)gridDim.y : y0 + 1;
+    for (int y = y0; y < y1; ++y) {
+      const int n = base[I.slot] + r0 + y;
+      if (n >= I.stop) break;
       int slot = K.tti[n];
-      if (slot >= 0) {
-        if (K.kind == FDTDX_DET_PHASOR) slot = 0;
-        float v = reduce_finalize_tile(I.P, K, I.dd[q].partial, I.det_nb[q], I.dd[q].state, slot, n);
-        // the detectors accumulating into this one's state follow it, in order, in this block
-        for (int a = q + 1; a < I.ndet && I.det[a].accum; ++a)
-          v = reduce_finalize_tile(I.P, I.det[a], I.dd[a].partial, I.det_nb[a], I.dd[a].state, slot, n);
-        if (threadIdx.x == 0 && (K.kind == FDTDX_DET_ENERGY || K.kind == FDTDX_DET_FLUX)) {
-          int f = 0;
-          if (!isfinite(v)) f = kFlagNonFinite;
-          else if (B->blowup > 0.f && fabsf(v) > B->blowup) f = kFlagBlowup;
-          if (f) B->flags[I.slot] = B->flags[I.slot] | f;
-        }
+      if (slot < 0) continue;
+      if (ph) slot = 0;
+      const long long ring = (long long)((r0 + y) % kDetRing) * I.ndet * kDetMaxValues * kDetMaxBlocks;
+      float v = reduce_finalize_tile(I.P, K, I.dd[q].partial + ring, I.det_nb[q], I.dd[q].state, slot, n);
+      // the detectors accumulating into this one's state follow it, in order, in this block
+      for (int a = q + 1; a < I.ndet && I.det[a].accum; ++a)
+        v = reduce_finalize_tile(I.P, I.det[a], I.dd[a].partial + ring, I.det_nb[a], I.dd[a].state, slot, n);
+      if (threadIdx.x == 0 && (K.kind == FDTDX_DET_ENERGY || K.kind == FDTDX_DET_FLUX)) {
+        int f = 0;
+        if (!isfinite(v)) f = kFlagNonFinite;
+        else if (B.blowup > 0.f && fabsf(v) > B.blowup) f = kFlagBlowup;
+        if (f) atomicOr(&B.flags[I.slot], f);
       }
-      break;
     }
   }
 }
 
-hipError_t launch_batch_detectors(const BatchTable* tab, const int* base, int r, int grid, bool finalize,
-                                  hipStream_t s) {
-  hipLaunchKernelGGL(k_batch_detector, dim3(grid), dim3(kBlock), 0, s, tab, base, r);
-  if (finalize) hipLaunchKernelGGL(k_batch_finalize, dim3(kMaxBatch), dim3(kBlock), 0, s, tab, base, r);
+hipError_t launch_batch_detectors(const BatchTable* tab, const int* base, int r, int mode, int grid, hipStream_t s) {
+  const auto f = mode & 1 ? (mode & 2 ? k_batch_detector<true, true> : k_batch_detector<true, false>)
+                          : (mode & 2 ? k_batch_detector<false, true> : k_batch_detector<false, false>);
+  hipLaunchKernelGGL(f, dim3(grid), dim3(kBlock), 0, s, tab, base, r);
+  return hipGetLastError();
+}
+
+hipError_t launch_batch_finalize(const BatchTable* tab, const int* base, int r0, int steps, hipStream_t s) {
+  hipLaunchKernelGGL(k_batch_finalize, dim3(kMaxBatch, (unsigned)steps), dim3(kBlock), 0, s, tab, base, r0);
   return hipGetLastError();
 }
 

@@ -122,7 +122,7 @@ __device__ __forceinline__ Deriv deriv_E(const StepStatic& P, const float* E, lo
 }
 
 // E half-step of step n for cell (i, j, k) at offset o; m is the mask of its tile.
-template <int EC, bool U, bool X>
+template <int EC, bool X>
 __device__ __forceinline__ void update_E_cell(const StepStatic& P, const StepDyn& D, int n, uint32_t m, int i, int j,
                                               int k, long long o) {
   float hx, hy, hz;
@@ -130,7 +130,7 @@ __device__ __forceinline__ void update_E_cell(const StepStatic& P, const StepDyn
   float cx = d.dy_z - d.dz_y;
   float cy = d.dz_x - d.dx_z;
   float cz = d.dx_y - d.dy_x;
-  apply_cpml<U>(P, m, D.psi, D.psi, 0, 1, i, j, k, d, cx, cy, cz);
+  apply_cpml(P, m, D.psi, D.psi, 0, 1, i, j, k, d, cx, cy, cz);
   const float iex = ldg(D.ie + o);
   const float iey = EC == 3 ? ldg(D.ie + P.N + o) : iex;
   const float iez = EC == 3 ? ldg(D.ie + 2 * P.N + o) : iex;
@@ -192,7 +192,7 @@ __device__ __forceinline__ void update_E_cell(const StepStatic& P, const StepDyn
     ny_ = ny_ / (1.0f + xl[1]);
     nz_ = nz_ / (1.0f + xl[2]);
   }
-  apply_sources<U>(P, m, D.ie, D.im, 0, n, false, i, j, k, o, EC, 0, nx_, ny_, nz_);
+  apply_sources(P, m, D.ie, D.im, 0, n, false, i, j, k, o, EC, 0, nx_, ny_, nz_);
   apply_walls(P, m, FDTDX_WALL_PEC, i, j, k, nx_, ny_, nz_);
   stg(Ex + o, nx_);
   stg(Ey + o, ny_);
@@ -208,20 +208,20 @@ __device__ __forceinline__ void update_E_cell(const StepStatic& P, const StepDyn
 }
 
 // E half-step of step n for the cells of tile lb.
-template <int EC, bool U, bool X>
+template <int EC, bool X>
 __device__ __forceinline__ void update_E_tile(const StepStatic& P, const StepDyn& D, int n, long long lb) {
   int i, j, k;
   long long o;
   if (!cell_of<true>(P, lb, i, j, k, o)) return;
   uint32_t m = tile_mask<true>(P, lb);
   if (X && D.cpart < 0) m &= ~(0xffu << kMaskSrc);  // real sources drive the real part only
-  update_E_cell<EC, U, X>(P, D, n, m, i, j, k, o);
+  update_E_cell<EC, X>(P, D, n, m, i, j, k, o);
 }
 
 // H half-step of step n for cell (i, j, k) at offset o (m: its tile's mask); record (step n's
 // record slot, or null) receives the CPML interface layers in float32 (records with narrow layers
 // are written by k_record).
-template <int MC, bool U, bool X>
+template <int MC, bool X>
 __device__ __forceinline__ void update_H_cell(const StepStatic& P, const StepDyn& D, int n, char* record, uint32_t m,
                                               int i, int j, int k, long long o) {
   float ex, ey, ez;
@@ -229,7 +229,7 @@ __device__ __forceinline__ void update_H_cell(const StepStatic& P, const StepDyn
   float cx = d.dy_z - d.dz_y;
   float cy = d.dz_x - d.dx_z;
   float cz = d.dx_y - d.dy_x;
-  apply_cpml<U>(P, m, D.psi, D.psi, 1, 1, i, j, k, d, cx, cy, cz);
+  apply_cpml(P, m, D.psi, D.psi, 1, 1, i, j, k, d, cx, cy, cz);
   float* Hx = D.H;
   float* Hy = D.H + P.N;
   float* Hz = D.H + 2 * P.N;
@@ -250,7 +250,7 @@ __device__ __forceinline__ void update_H_cell(const StepStatic& P, const StepDyn
     hy = hy0 - (c * cy) * imy;
     hz = hz0 - (c * cz) * imz;
   }
-  apply_sources<U>(P, m, D.ie, D.im, 1, n, false, i, j, k, o, 1, MC, hx, hy, hz);
+  apply_sources(P, m, D.ie, D.im, 1, n, false, i, j, k, o, 1, MC, hx, hy, hz);
   apply_walls(P, m, FDTDX_WALL_PMC, i, j, k, hx, hy, hz);
   stg(Hx + o, hx);
   stg(Hy + o, hy);
@@ -258,7 +258,7 @@ __device__ __forceinline__ void update_H_cell(const StepStatic& P, const StepDyn
   if (record && (m & 63u)) record_iface(P, m, record, i, j, k, ex, ey, ez, hx, hy, hz);
 }
 
-template <int MC, bool U, bool X>
+template <int MC, bool X>
 __device__ __forceinline__ void update_H_tile(const StepStatic& P, const StepDyn& D, int n, char* record,
                                               long long lb) {
   int i, j, k;
@@ -266,7 +266,7 @@ __device__ __forceinline__ void update_H_tile(const StepStatic& P, const StepDyn
   if (!cell_of<true>(P, lb, i, j, k, o)) return;
   uint32_t m = tile_mask<true>(P, lb);
   if (X && D.cpart < 0) m &= ~(0xffu << kMaskSrc);
-  update_H_cell<MC, U, X>(P, D, n, record, m, i, j, k, o);
+  update_H_cell<MC, X>(P, D, n, record, m, i, j, k, o);
 }
 
 // ---------------------------------------------------------------- full-tensor materials
@@ -412,7 +412,7 @@ __global__ __launch_bounds__(kBlock) void k_tensor_curl(const StepStatic* __rest
   float cx = d.dy_z - d.dz_y;
   float cy = d.dz_x - d.dx_z;
   float cz = d.dx_y - d.dy_x;
-  apply_cpml<false>(P, m, D.psi, D.psi, field, update, i, j, k, d, cx, cy, cz);
+  apply_cpml(P, m, D.psi, D.psi, field, update, i, j, k, d, cx, cy, cz);
   if (field == 0 && update && P.nade) {  // ADE poles: curl + delta / c (update.py:416-423)
 #pragma unroll
     for (int b = 0; b < FDTDX_MAX_ADE; ++b) {
@@ -435,8 +435,8 @@ __global__ __launch_bounds__(kBlock) void k_tensor_curl(const StepStatic* __rest
     const float* F = field == 0 ? D.E : D.H;
     float v0 = F[o], v1 = F[P.N + o], v2 = F[2 * P.N + o];
     if (!update) {
-      if (field == 0) apply_sources<false>(P, m, D.ie, D.im, 0, D.n, true, i, j, k, o, 9, 0, v0, v1, v2);
-      else apply_sources<false>(P, m, D.ie, D.im, 1, D.n, true, i, j, k, o, 1, 9, v0, v1, v2);
+      if (field == 0) apply_sources(P, m, D.ie, D.im, 0, D.n, true, i, j, k, o, 9, 0, v0, v1, v2);
+      else apply_sources(P, m, D.ie, D.im, 1, D.n, true, i, j, k, o, 1, 9, v0, v1, v2);
     }
     D.Fo[o] = v0;
     D.Fo[P.N + o] = v1;
@@ -497,14 +497,14 @@ __global__ __launch_bounds__(kBlock) void k_tensor_E(const StepStatic* __restric
   if (tensor_sigma_rows<X, false>(P, D, 0, reverse, reverse ? -1.f : 1.f, o, i, j, k, v)) {
     // the reverse run's sources are already in Fo
   } else {
-    if (reverse) apply_sources<false>(P, m, D.ie, D.im, 0, D.n, true, i, j, k, o, 9, 0, v[0], v[1], v[2]);
+    if (reverse) apply_sources(P, m, D.ie, D.im, 0, D.n, true, i, j, k, o, 9, 0, v[0], v[1], v[2]);
 #pragma unroll
     for (int r = 0; r < 3; ++r) {
       const float t = tensor_row<X, false>(P, D.ie, D.K, o, i, j, k, r);
       v[r] = reverse ? v[r] - t : v[r] + t;
     }
   }
-  if (!reverse) apply_sources<false>(P, m, D.ie, D.im, 0, D.n, false, i, j, k, o, 9, 0, v[0], v[1], v[2]);
+  if (!reverse) apply_sources(P, m, D.ie, D.im, 0, D.n, false, i, j, k, o, 9, 0, v[0], v[1], v[2]);
   apply_walls(P, m, FDTDX_WALL_PEC, i, j, k, v[0], v[1], v[2]);
   D.E[o] = v[0];
   D.E[P.N + o] = v[1];
@@ -524,14 +524,14 @@ __global__ __launch_bounds__(kBlock) void k_tensor_H(const StepStatic* __restric
   float v[3] = {D.H[o], D.H[P.N + o], D.H[2 * P.N + o]};
   if (tensor_sigma_rows<X, true>(P, D, 1, reverse, reverse ? 1.f : -1.f, o, i, j, k, v)) {
   } else {
-    if (reverse) apply_sources<false>(P, m, D.ie, D.im, 1, D.n, true, i, j, k, o, 1, 9, v[0], v[1], v[2]);
+    if (reverse) apply_sources(P, m, D.ie, D.im, 1, D.n, true, i, j, k, o, 1, 9, v[0], v[1], v[2]);
 #pragma unroll
     for (int r = 0; r < 3; ++r) {
       const float t = tensor_row<X, true>(P, D.im, D.K, o, i, j, k, r);
       v[r] = reverse ? v[r] + t : v[r] - t;
     }
   }
-  if (!reverse) apply_sources<false>(P, m, D.ie, D.im, 1, D.n, false, i, j, k, o, 1, 9, v[0], v[1], v[2]);
+  if (!reverse) apply_sources(P, m, D.ie, D.im, 1, D.n, false, i, j, k, o, 1, 9, v[0], v[1], v[2]);
   apply_walls(P, m, FDTDX_WALL_PMC, i, j, k, v[0], v[1], v[2]);
   D.H[o] = v[0];
   D.H[P.N + o] = v[1];
@@ -544,13 +544,13 @@ __global__ __launch_bounds__(kBlock) void k_tensor_H(const StepStatic* __restric
 template <int EC, bool X>
 __global__ __launch_bounds__(kBlock) void k_update_E(const StepStatic* __restrict__ Pp, const StepDyn D) {
   const StepStatic& P = as_const(Pp);
-  update_E_tile<EC, false, X>(P, D, D.n, logical_block(P.xorder, P.nblocks_pad));
+  update_E_tile<EC, X>(P, D, D.n, logical_block(P.xorder, P.nblocks_pad));
 }
 
 template <int MC, bool X>
 __global__ __launch_bounds__(kBlock) void k_update_H(const StepStatic* __restrict__ Pp, const StepDyn D) {
   const StepStatic& P = as_const(Pp);
-  update_H_tile<MC, false, X>(P, D, D.n, D.record, logical_block(P.xorder, P.nblocks_pad));
+  update_H_tile<MC, X>(P, D, D.n, D.record, logical_block(P.xorder, P.nblocks_pad));
 }
 
 // ---------------------------------------------------------------- quad sweeps
@@ -629,17 +629,11 @@ __device__ __forceinline__ void cpml_quad(const StepStatic& P, uint32_t mask, fl
   }
 }
 
-// The E half-step of quad tiles that meet an ADE box (listed in vslow) runs one cell per thread in a
-// launch of its own, four blocks per listed tile: the polarisation update would cost the quad
-// kernel its register budget. Cell of block b: false past the last listed tile.
-__device__ __forceinline__ bool slow_cell(const StepStatic& P, long long b, int& i, int& j, int& k, long long& o,
-                                          uint32_t& m) {
-  const long long s = b >> 2;
-  if (s >= P.vnslow) return false;
-  const long long lb = P.vslow[s];
-  m = P.vec_mask[lb];
+// Cell of this lane in quarter `part` of quad tile lb, one cell per lane.
+__device__ __forceinline__ bool tile_cell(const StepStatic& P, long long lb, int part, int& i, int& j, int& k,
+                                          long long& o) {
   i = (int)(lb / P.vbpp);
-  const int c = (int)(b & 3) * kBlock + threadIdx.x;  // cell of the quad tile, four per quad
+  const int c = part * kBlock + threadIdx.x;  // cell of the quad tile, four per quad
   const int p = (int)(lb - (long long)i * P.vbpp) * kBlock + (c >> 2);
   if (p >= P.ny * P.nzq) return false;
   int k0, sm;
@@ -650,25 +644,32 @@ __device__ __forceinline__ bool slow_cell(const StepStatic& P, long long b, int&
   return true;
 }
 
+// The E half-step of quad tiles that meet an ADE box (listed in vslow) runs one cell per thread in a
+// launch of its own, four blocks per listed tile: the polarisation update would cost the quad
+// kernel its register budget. Cell of block b: false past the last listed tile.
+__device__ __forceinline__ bool slow_cell(const StepStatic& P, long long b, int& i, int& j, int& k, long long& o,
+                                          uint32_t& m) {
+  const long long s = b >> 2;
+  if (s >= P.vnslow) return false;
+  const long long lb = P.vslow[s];
+  m = P.vec_mask[lb];
+  return tile_cell(P, lb, (int)(b & 3), i, j, k, o);
+}
+
 template <int EC, bool X>
 __global__ __launch_bounds__(kBlock) void k_update_E4s(const StepStatic* __restrict__ Pp, const StepDyn D) {
   const StepStatic& P = as_const(Pp);
   int i, j, k;
   long long o;
   uint32_t ms;
-  if (slow_cell(P, (long long)blockIdx.x, i, j, k, o, ms)) update_E_cell<EC, false, X>(P, D, D.n, ms, i, j, k, o);
+  if (slow_cell(P, (long long)blockIdx.x, i, j, k, o, ms)) update_E_cell<EC, X>(P, D, D.n, ms, i, j, k, o);
 }
 
+// The E and H half-steps of step n for one quad (m: its tile's mask, ADE tiles excepted).
 // CAX: the per-axis CPML (plans with StepStatic::cax), else the slab loop of cpml_quad.
 template <int EC, bool X, bool CAX, bool RAG>
-__global__ __launch_bounds__(kBlock) void k_update_E4(const StepStatic* __restrict__ Pp, const StepDyn D) {
-  const StepStatic& P = as_const(Pp);
-  int i, j, k0, sm;
-  long long o;
-  const long long lb = logical_block(P.xorder, P.vnblocks_pad);
-  if (!quad_of(P, lb, i, j, k0, sm, o)) return;
-  const uint32_t m = P.vec_mask[lb];
-  if (m & P.vlistE) return;  // a listed tile: its cells run in k_update_E4s
+__device__ __forceinline__ void quad_E(const StepStatic& P, const StepDyn& D, int n, uint32_t m, int i, int j, int k0,
+                                       int sm, long long o) {
   QuadSlabs S;
   S.in[0] = S.in[1] = S.in[2] = false;
   S.hi[0] = S.hi[1] = S.hi[2] = false;
@@ -717,7 +718,7 @@ __global__ __launch_bounds__(kBlock) void k_update_E4(const StepStatic* __restri
   st4m<RAG>(Ex + o, en[0], sm);
   st4m<RAG>(Ey + o, en[1], sm);
   st4m<RAG>(Ez + o, en[2], sm);
-  if (m & P.vpoint[0]) quad_points<0>(P, m, D.ie, D.im, D.E, D.n, i, j, k0, sm, o, EC, 0);
+  if (m & P.vpoint[0]) quad_points<0>(P, m, D.ie, D.im, D.E, n, i, j, k0, sm, o, EC, 0);
   if ((m & kSnapBit) && D.snap) {  // H_prev of the detector boxes, as update_E_cell
     const long long sy = D.shi[1] - D.slo[1], sz = D.shi[2] - D.slo[2];
     const long long sc = (long long)(D.shi[0] - D.slo[0]) * sy * sz;
@@ -733,13 +734,8 @@ __global__ __launch_bounds__(kBlock) void k_update_E4(const StepStatic* __restri
 }
 
 template <int MC, bool X, bool CAX, bool RAG>
-__global__ __launch_bounds__(kBlock) void k_update_H4(const StepStatic* __restrict__ Pp, const StepDyn D) {
-  const StepStatic& P = as_const(Pp);
-  int i, j, k0, sm;
-  long long o;
-  const long long lb = logical_block(P.xorder, P.vnblocks_pad);
-  if (!quad_of(P, lb, i, j, k0, sm, o)) return;
-  const uint32_t m = P.vec_mask[lb];
+__device__ __forceinline__ void quad_H(const StepStatic& P, const StepDyn& D, int n, char* record, uint32_t m, int i,
+                                       int j, int k0, int sm, long long o) {
   QuadSlabs S;
   S.in[0] = S.in[1] = S.in[2] = false;
   S.hi[0] = S.hi[1] = S.hi[2] = false;
@@ -790,17 +786,39 @@ __global__ __launch_bounds__(kBlock) void k_update_H4(const StepStatic* __restri
   st4m<RAG>(Hy + o, hn[1], sm);
   st4m<RAG>(Hz + o, hn[2], sm);
   if (m & P.vpoint[1]) {
-    quad_points<1>(P, m, D.ie, D.im, D.H, D.n, i, j, k0, sm, o, 1, MC);
-    if (D.record) {  // the recorded layers hold the sources
+    quad_points<1>(P, m, D.ie, D.im, D.H, n, i, j, k0, sm, o, 1, MC);
+    if (record) {  // the recorded layers hold the sources
       hn[0] = ld4<RAG>(Hx + o);
       hn[1] = ld4<RAG>(Hy + o);
       hn[2] = ld4<RAG>(Hz + o);
     }
   }
-  if (D.record && (m & kSlabBits)) {
+  if (record && (m & kSlabBits)) {
 #pragma unroll 1
-    for (int e = RAG ? sm : 0; e < 4; ++e) record_iface(P, m, D.record, i, j, k0 + e, ex[e], ey[e], ez[e], hn[0][e], hn[1][e], hn[2][e]);
+    for (int e = RAG ? sm : 0; e < 4; ++e) record_iface(P, m, record, i, j, k0 + e, ex[e], ey[e], ez[e], hn[0][e], hn[1][e], hn[2][e]);
   }
+}
+
+template <int EC, bool X, bool CAX, bool RAG>
+__global__ __launch_bounds__(kBlock) void k_update_E4(const StepStatic* __restrict__ Pp, const StepDyn D) {
+  const StepStatic& P = as_const(Pp);
+  int i, j, k0, sm;
+  long long o;
+  const long long lb = logical_block(P.xorder, P.vnblocks_pad);
+  if (!quad_of(P, lb, i, j, k0, sm, o)) return;
+  const uint32_t m = P.vec_mask[lb];
+  if (m & P.vlistE) return;  // a listed tile: its cells run in k_update_E4s
+  quad_E<EC, X, CAX, RAG>(P, D, D.n, m, i, j, k0, sm, o);
+}
+
+template <int MC, bool X, bool CAX, bool RAG>
+__global__ __launch_bounds__(kBlock, 5) void k_update_H4(const StepStatic* __restrict__ Pp, const StepDyn D) {
+  const StepStatic& P = as_const(Pp);
+  int i, j, k0, sm;
+  long long o;
+  const long long lb = logical_block(P.xorder, P.vnblocks_pad);
+  if (!quad_of(P, lb, i, j, k0, sm, o)) return;
+  quad_H<MC, X, CAX, RAG>(P, D, D.n, D.record, P.vec_mask[lb], i, j, k0, sm, o);
 }
 
 // ---------------------------------------------------------------- reverse reconstruction
@@ -829,12 +847,12 @@ __global__ __launch_bounds__(kBlock) void k_reverse_H(const StepStatic* __restri
   float cy = d.dz_x - d.dx_z;
   float cz = d.dx_y - d.dy_x;
   if constexpr (AXS) cpml_axes_frozen(ax, d, cx, cy, cz);
-  else apply_cpml<false>(P, m, D.psi, D.psi, 1, 0, i, j, k, d, cx, cy, cz);
+  else apply_cpml(P, m, D.psi, D.psi, 1, 0, i, j, k, d, cx, cy, cz);
   float* Hx = D.H;
   float* Hy = D.H + P.N;
   float* Hz = D.H + 2 * P.N;
   float hx = Hx[o], hy = Hy[o], hz = Hz[o];
-  apply_sources<false>(P, m, D.ie, D.im, 1, D.n, true, i, j, k, o, 1, MC, hx, hy, hz);
+  apply_sources(P, m, D.ie, D.im, 1, D.n, true, i, j, k, o, 1, MC, hx, hy, hz);
   const float c = P.c;
   const float imx = MC ? D.im[o] : 1.0f;
   const float imy = MC == 3 ? D.im[P.N + o] : imx;
@@ -922,12 +940,12 @@ __global__ __launch_bounds__(kBlock) void k_reverse_E(const StepStatic* __restri
   float cx = d.dy_z - d.dz_y;
   float cy = d.dz_x - d.dx_z;
   float cz = d.dx_y - d.dy_x;
-  apply_cpml<false>(P, m, D.psi, D.psi, 0, 0, i, j, k, d, cx, cy, cz);
+  apply_cpml(P, m, D.psi, D.psi, 0, 0, i, j, k, d, cx, cy, cz);
   float* Ex = D.E;
   float* Ey = D.E + P.N;
   float* Ez = D.E + 2 * P.N;
   float ex = Ex[o], ey = Ey[o], ez = Ez[o];
-  apply_sources<false>(P, m, D.ie, D.im, 0, D.n, true, i, j, k, o, EC, 0, ex, ey, ez);
+  apply_sources(P, m, D.ie, D.im, 0, D.n, true, i, j, k, o, EC, 0, ex, ey, ez);
   const float iex = D.ie[o];
   const float iey = EC == 3 ? D.ie[P.N + o] : iex;
   const float iez = EC == 3 ? D.ie[2 * P.N + o] : iex;
@@ -1143,14 +1161,14 @@ hipError_t launch_update_H(const StepStatic& P, const StepDyn& D, int mc, hipStr
 // Kernel of a quad sweep: x (periodic axes or conductivity), the per-axis CPML c, rows of nz % 4 != 0
 // cells rag (which always have the per-axis CPML).
 template <int EC>
-static SweepKernel quad_E(bool x, bool c, bool rag) {
+static SweepKernel quad_E_kernel(bool x, bool c, bool rag) {
   if (rag) return x ? k_update_E4<EC, true, true, true> : k_update_E4<EC, false, true, true>;
   if (c) return x ? k_update_E4<EC, true, true, false> : k_update_E4<EC, false, true, false>;
   return x ? k_update_E4<EC, true, false, false> : k_update_E4<EC, false, false, false>;
 }
 
 template <int MC>
-static SweepKernel quad_H(bool x, bool c, bool rag) {
+static SweepKernel quad_H_kernel(bool x, bool c, bool rag) {
   if (rag) return x ? k_update_H4<MC, true, true, true> : k_update_H4<MC, false, true, true>;
   if (c) return x ? k_update_H4<MC, true, true, false> : k_update_H4<MC, false, true, false>;
   return x ? k_update_H4<MC, true, false, false> : k_update_H4<MC, false, false, false>;
@@ -1158,7 +1176,7 @@ static SweepKernel quad_H(bool x, bool c, bool rag) {
 
 hipError_t launch_update_E4(const StepStatic& P, const StepDyn& D, int ec, hipStream_t s) {
   const bool x = extras(P), c = P.cax != 0, rag = P.nz % 4 != 0;
-  const SweepKernel f = ec == 3 ? quad_E<3>(x, c, rag) : quad_E<1>(x, c, rag);
+  const SweepKernel f = ec == 3 ? quad_E_kernel<3>(x, c, rag) : quad_E_kernel<1>(x, c, rag);
   const SweepKernel fs = ec == 3 ? (x ? k_update_E4s<3, true> : k_update_E4s<3, false>)
                                  : (x ? k_update_E4s<1, true> : k_update_E4s<1, false>);
   hipLaunchKernelGGL(f, dim3((unsigned)P.vnblocks_pad), dim3(kBlock), 0, s, P.self, D);
@@ -1168,7 +1186,7 @@ hipError_t launch_update_E4(const StepStatic& P, const StepDyn& D, int ec, hipSt
 
 hipError_t launch_update_H4(const StepStatic& P, const StepDyn& D, int mc, hipStream_t s) {
   const bool x = extras(P), c = P.cax != 0, rag = P.nz % 4 != 0;
-  const SweepKernel f = mc == 3 ? quad_H<3>(x, c, rag) : (mc == 1 ? quad_H<1>(x, c, rag) : quad_H<0>(x, c, rag));
+  const SweepKernel f = mc == 3 ? quad_H_kernel<3>(x, c, rag) : (mc == 1 ? quad_H_kernel<1>(x, c, rag) : quad_H_kernel<0>(x, c, rag));
   hipLaunchKernelGGL(f, dim3((unsigned)P.vnblocks_pad), dim3(kBlock), 0, s, P.self, D);
   return hipGetLastError();
 }
@@ -1225,9 +1243,9 @@ hipError_t launch_reverse(const StepStatic& P, const StepDyn& D, int ec, int mc,
 // One tile per block over the concatenated tile space of the batch. Block h serves XCD h % 8 and
 // takes tile (h % 8) * per + h / 8, so each XCD sweeps a contiguous eighth and neighbouring planes
 // of one instance share an L2; blocks past the tile count (the grid is rounded up) exit.
-__device__ __forceinline__ bool batch_tile(const BatchTable* __restrict__ B, long long& t, int& e) {
-  const int ni = B->ninst;
-  const long long total = B->tile_start[ni];
+__device__ __forceinline__ bool batch_tile(const BatchTable& B, long long& t, int& e) {
+  const int ni = B.ninst;
+  const long long total = B.tile_start[ni];
   const long long per = (total + kXcds - 1) / kXcds;
   const long long w = blockIdx.x / kXcds;
   t = (long long)(blockIdx.x % kXcds) * per + w;
@@ -1235,37 +1253,67 @@ __device__ __forceinline__ bool batch_tile(const BatchTable* __restrict__ B, lon
   int lo = 0, hi = ni - 1;  // the entry e with tile_start[e] <= t < tile_start[e + 1]
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
-    if (B->tile_start[mid] <= t) lo = mid;
+    if (B.tile_start[mid] <= t) lo = mid;
     else hi = mid - 1;
   }
   e = lo;
   return true;
 }
 
+// (Two 128x128x64, three 96^3 and three 64^3 solves, 5.5M cells: E / H sweep 53.2 / 54.0 us one cell per
+// lane, 37.7 / 37.2 us four, with the table's scalar loads through the constant address space.)
+// A batch tile is a quad tile of an instance with the per-axis quad sweeps (BatchInst::quad; rows of
+// any length, so with 4-byte aligned accesses), else a tile of the one-cell sweeps. Quad tiles that
+// meet an ADE box run their E half-step one cell per lane, a quarter at a time.
 template <int EC>
-__global__ __launch_bounds__(kBlock) void k_batch_E(const BatchTable* __restrict__ B, const int* __restrict__ base,
+__global__ __launch_bounds__(kBlock) void k_batch_E(const BatchTable* __restrict__ Bp, const int* __restrict__ base,
                                                     int r) {
+  const BatchTable& B = as_const(Bp);
   long long t;
   int e;
   if (!batch_tile(B, t, e)) return;
-  const BatchInst& I = B->inst[e];
+  const BatchInst& I = B.inst[e];
+  const StepStatic& P = I.P;
   const int n = base[I.slot] + r;
   if (n >= I.stop) return;
-  update_E_tile<EC, true, true>(I.P, I.D, n, t - B->tile_start[e]);
+  const long long lb = t - B.tile_start[e];
+  if (!I.quad) {
+    update_E_tile<EC, true>(P, I.D, n, lb);
+    return;
+  }
+  const uint32_t m = P.vec_mask[lb];
+  int i, j, k, sm;
+  long long o;
+  if (m & P.vlistE) {
+#pragma unroll 1
+    for (int part = 0; part < 4; ++part)
+      if (tile_cell(P, lb, part, i, j, k, o)) update_E_cell<EC, true>(P, I.D, n, m, i, j, k, o);
+    return;
+  }
+  if (quad_of(P, lb, i, j, k, sm, o)) quad_E<EC, true, true, true>(P, I.D, n, m, i, j, k, sm, o);
 }
 
 template <int MC>
-__global__ __launch_bounds__(kBlock) void k_batch_H(const BatchTable* __restrict__ B, const int* __restrict__ base,
+__global__ __launch_bounds__(kBlock) void k_batch_H(const BatchTable* __restrict__ Bp, const int* __restrict__ base,
                                                     int r) {
+  const BatchTable& B = as_const(Bp);
   long long t;
   int e;
   if (!batch_tile(B, t, e)) return;
-  const BatchInst& I = B->inst[e];
+  const BatchInst& I = B.inst[e];
+  const StepStatic& P = I.P;
   const int n = base[I.slot] + r;
   if (n >= I.stop) return;
-  const int rs = I.P.rec_slot ? I.P.rec_slot[n] : n;
-  char* record = (I.rec_base && rs >= 0) ? I.rec_base + (long long)rs * I.P.rec_slot_bytes : nullptr;
-  update_H_tile<MC, true, true>(I.P, I.D, n, record, t - B->tile_start[e]);
+  const int rs = P.rec_slot ? P.rec_slot[n] : n;
+  char* record = (I.rec_base && rs >= 0) ? I.rec_base + (long long)rs * P.rec_slot_bytes : nullptr;
+  const long long lb = t - B.tile_start[e];
+  if (!I.quad) {
+    update_H_tile<MC, true>(P, I.D, n, record, lb);
+    return;
+  }
+  int i, j, k, sm;
+  long long o;
+  if (quad_of(P, lb, i, j, k, sm, o)) quad_H<MC, true, true, true>(P, I.D, n, record, P.vec_mask[lb], i, j, k, sm, o);
 }
 
 __global__ void k_batch_set(int* base, int* flags, const BatchSet set) {

@@ -110,6 +110,7 @@ struct BatchInst {
   StepStatic P;
   StepDyn D;             // snap is set whenever the instance has detectors
   char* rec_base;        // interface record slot 0 (null: off); step n at slot P.rec_slot[n]
+  int quad;              // its tiles are quad tiles
   int stop;              // first step index not to run
   int slot;              // index into the step counter array
   int ec, mc;
@@ -125,7 +126,8 @@ struct BatchTable {
   int* flags;                           // per-slot health flags (device)
   long long tile_start[kMaxBatch + 1];  // sweep tiles, prefix over entries
   int det_start[kMaxBatch + 1];         // detector blocks, prefix over entries
-  int fin_start[kMaxBatch + 1];         // reducing detectors, prefix over entries
+  int fin_start[kMaxBatch + 1];         // reducing detectors, prefix over entries (sums of a step at
+                                        // dd.partial + (step in the chunk % kDetRing) * its ring stride)
   BatchInst inst[kMaxBatch];
 };
 
@@ -143,8 +145,10 @@ int batch_sweep_grid(long long tiles);  // blocks of a batch sweep over `tiles` 
 hipError_t launch_batch_set(int* base, int* flags, const BatchSet& set, hipStream_t s);
 hipError_t launch_batch_sweeps(const BatchTable* tab, const int* base, int r, int ec, int mc, int grid,
                                hipStream_t s);
-hipError_t launch_batch_detectors(const BatchTable* tab, const int* base, int r, int grid, bool finalize,
-                                  hipStream_t s);
+// Detectors of chunk step r (mode bit 0: some detector keeps per-cell phasors, bit 1: some needs_halo),
+// and the sums of chunk steps [r0, r0 + steps), at most kDetRing of them.
+hipError_t launch_batch_detectors(const BatchTable* tab, const int* base, int r, int mode, int grid, hipStream_t s);
+hipError_t launch_batch_finalize(const BatchTable* tab, const int* base, int r0, int steps, hipStream_t s);
 hipError_t launch_batch_advance(const BatchTable* tab, int* base, int steps, hipStream_t s);
 
 // Fused single-pass step (fused_kernels.hip): kFusedThreads threads, kFusedM positions per thread

@@ -212,7 +212,7 @@ __global__ __launch_bounds__(kMarchThreads) void k_march(const StepStatic* __res
           float cy = d.dz_x - d.dx_z;
           float cz = d.dx_y - d.dy_x;
           const bool st = own_k && own_row && ownE;
-          if (!plain) apply_cpml<false>(P, kMaskAll, D.psi_in, D.psi_out, 0, st ? 1 : 2, i, j, k, d, cx, cy, cz);
+          if (!plain) apply_cpml(P, kMaskAll, D.psi_in, D.psi_out, 0, st ? 1 : 2, i, j, k, d, cx, cy, cz);
           const float iex = cur.ie[r][0];
           const float iey = EC == 3 ? cur.ie[r][EC == 3 ? 1 : 0] : iex;
           const float iez = EC == 3 ? cur.ie[r][EC == 3 ? 2 : 0] : iex;
@@ -252,7 +252,7 @@ __global__ __launch_bounds__(kMarchThreads) void k_march(const StepStatic* __res
               eyn = eyn + iey * dl[1];
               ezn = ezn + iez * dl[2];
             }
-            apply_sources<false>(P, kMaskAll, D.ie, D.im, 0, n, false, i, j, k, o, EC, 0, exn, eyn, ezn);
+            apply_sources(P, kMaskAll, D.ie, D.im, 0, n, false, i, j, k, o, EC, 0, exn, eyn, ezn);
           }
           if (st) {
             stb(Ex_out, ob, exn);
@@ -279,7 +279,7 @@ __global__ __launch_bounds__(kMarchThreads) void k_march(const StepStatic* __res
         float cx = d.dy_z - d.dz_y;
         float cy = d.dz_x - d.dx_z;
         float cz = d.dx_y - d.dy_x;
-        if (!plain) apply_cpml<false>(P, kMaskAll, D.psi_in, D.psi_out, 1, 1, ip, j, k, d, cx, cy, cz);
+        if (!plain) apply_cpml(P, kMaskAll, D.psi_in, D.psi_out, 1, 1, ip, j, k, d, cx, cy, cz);
         const int o = (ip * Ny + j) * Nz + k;
         const unsigned ob = (unsigned)o * 4u;
         const float imx = MC ? D.im[o] : 1.0f;
@@ -288,7 +288,7 @@ __global__ __launch_bounds__(kMarchThreads) void k_march(const StepStatic* __res
         float hxn = hp[r][0] - (c * cx) * imx;
         float hyn = hp[r][1] - (c * cy) * imy;
         float hzn = hp[r][2] - (c * cz) * imz;
-        if (!plain) apply_sources<false>(P, kMaskAll, D.ie, D.im, 1, n, false, ip, j, k, o, 1, MC, hxn, hyn, hzn);
+        if (!plain) apply_sources(P, kMaskAll, D.ie, D.im, 1, n, false, ip, j, k, o, 1, MC, hxn, hyn, hzn);
         stb(Hx_out, ob, hxn);
         stb(Hy_out, ob, hyn);
         stb(Hz_out, ob, hzn);

@@ -715,7 +715,7 @@ static int plan_create(const fdtdx_plan_desc* d, fdtdx_plan** out) {
   pl->ws_partial = off; off = align256(off + (size_t)pl->ndet * kDetMaxValues * kDetMaxBlocks * 8);
   pl->ws_fwd_end = off;  // the forward (two-sweep schedules) touches nothing past this offset
   for (int q = 0; q < pl->ndet; ++q)
-    if (reduced_values(pl->det[q]) && pl->det[q].kind != FDTDX_DET_PHASOR) pl->ws_ring = off;
+    if (reduced_values(pl->det[q])) pl->ws_ring = off;
   if (pl->ws_ring) off = align256(off + (size_t)kDetRing * pl->ndet * kDetMaxValues * kDetMaxBlocks * 8);
   for (int q = 0; q < pl->ndet; ++q) { pl->g_off[q] = off; off = align256(off + 6 * (size_t)pl->det[q].cells * 4); }
   for (int q = 0; q < pl->ndet; ++q) {
@@ -1260,7 +1260,7 @@ struct fdtdx_batch {
     bool pending_set = false;      // counter must be initialised before the next chunk
   };
   Slot slot[kMaxBatch];
-  std::map<std::tuple<int, int, int>, hipGraphExec_t> graphs;  // (steps, with detectors, grid) -> executable
+  std::map<std::tuple<int, int, int>, hipGraphExec_t> graphs;  // (steps, detector mode, grid) -> executable
 
   ~fdtdx_batch() {
     for (auto& g : graphs) (void)hipGraphExecDestroy(g.second);
@@ -1391,9 +1391,10 @@ static int batch_upload(fdtdx_batch* b, hipStream_t s) {
       for (int a = 0; a < 3; ++a) { dd.slo[a] = p->slo[a]; dd.shi[a] = p->shi[a]; }
       dd.ie = S.buf.inv_eps; dd.im = S.buf.inv_mu; dd.ec = p->ec; dd.mc = p->mc;
       dd.state = S.det_state[q];
-      dd.partial = (double*)(ws + p->ws_partial) + (size_t)q * kDetMaxValues * kDetMaxBlocks;
+      dd.partial = (double*)(ws + (p->ws_ring ? p->ws_ring : p->ws_partial)) + (size_t)q * kDetMaxValues * kDetMaxBlocks;
     }
-    T->tile_start[e + 1] = T->tile_start[e] + p->P.nblocks;
+    I.quad = p->P.vq && p->P.cax;
+    T->tile_start[e + 1] = T->tile_start[e] + (I.quad ? p->P.vnblocks : p->P.nblocks);
     T->det_start[e + 1] = T->det_start[e] + nb;
     T->fin_start[e + 1] = T->fin_start[e] + nf;
     ++e;
@@ -1409,10 +1410,15 @@ static int batch_upload(fdtdx_batch* b, hipStream_t s) {
   return FDTDX_OK;
 }
 
-static int batch_chunk(fdtdx_batch* b, int steps, bool det, hipStream_t s) {
+// det: -1 no detectors, else the launch mode of launch_batch_detectors (bits 0, 1) and bit 2: some sums.
+static int batch_chunk(fdtdx_batch* b, int steps, int det, hipStream_t s) {
   for (int r = 0; r < steps; ++r) {
     HIP_TRY(launch_batch_sweeps(b->dtab, b->dbase, r, b->ec, b->mc, b->grid, s));
-    if (det) HIP_TRY(launch_batch_detectors(b->dtab, b->dbase, r, b->det_grid, true, s));
+    if (det >= 0) HIP_TRY(launch_batch_detectors(b->dtab, b->dbase, r, det, b->det_grid, s));
+    if (det >= 0 && (det & 4) && ((r + 1) % kDetRing == 0 || r + 1 == steps)) {
+      const int r0 = r / kDetRing * kDetRing;
+      HIP_TRY(launch_batch_finalize(b->dtab, b->dbase, r0, r + 1 - r0, s));
+    }
   }
   HIP_TRY(launch_batch_advance(b->dtab, b->dbase, steps, s));
   return FDTDX_OK;
@@ -1427,12 +1433,19 @@ int fdtdx_batch_advance(fdtdx_batch* b, int32_t steps, int32_t use_graph, void* 
   if (b->dirty && (rc = batch_upload(b, s))) return rc;
   BatchSet set;
   memset(&set, 0, sizeof(set));
-  bool det = false, any = false;
+  int det = -1;
+  bool any = false;
   for (int sl = 0; sl < kMaxBatch; ++sl) {
     fdtdx_batch::Slot& S = b->slot[sl];
     if (!S.plan) continue;
     any = true;
-    det = det || S.plan->ndet > 0;
+    if (S.plan->ndet > 0 && det < 0) det = 0;
+    for (int q = 0; q < S.plan->ndet; ++q) {
+      const DetK& K = S.plan->det[q];
+      if (K.kind == FDTDX_DET_PHASOR && !K.reduce) det |= 1;
+      if (needs_halo(S.plan->P, K)) det |= 2;
+      if (reduced_values(K)) det |= 4;
+    }
     if (S.pending_set) {
       set.slot[set.count] = sl;
       set.value[set.count] = S.t0;
@@ -1443,7 +1456,7 @@ int fdtdx_batch_advance(fdtdx_batch* b, int32_t steps, int32_t use_graph, void* 
   if (!any) return FDTDX_OK;
   HIP_TRY(launch_batch_set(b->dbase, b->dflags, set, s));
   if (use_graph) {
-    const auto key = std::make_tuple((int)steps, det ? 1 : 0, b->grid);
+    const auto key = std::make_tuple((int)steps, det, b->grid);
     auto it = b->graphs.find(key);
     if (it == b->graphs.end()) {
       hipGraph_t g = nullptr;

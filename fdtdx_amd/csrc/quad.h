@@ -316,7 +316,7 @@ __device__ __forceinline__ void quad_points(const StepStatic& P, uint32_t m, con
 #pragma unroll 1
   for (int e = sm; e < 4; ++e) {
     float x = p[e], y = p[P.N + e], z = p[2 * P.N + e];
-    apply_sources<false>(P, m, ie, im, W, n, INV, i, j, k0 + e, o + e, ec, mc, x, y, z);
+    apply_sources(P, m, ie, im, W, n, INV, i, j, k0 + e, o + e, ec, mc, x, y, z);
     if (!INV) apply_walls(P, m, W ? FDTDX_WALL_PMC : FDTDX_WALL_PEC, i, j, k0 + e, x, y, z);
     p[e] = x;
     p[P.N + e] = y;

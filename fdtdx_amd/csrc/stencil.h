@@ -4,10 +4,8 @@
 #pragma once
 #include "engine_common.h"
 
-// Descriptor loops (slabs, sources) are rolled or fully unrolled per kernel through the template
-// flag U. Measured on the 400x400x200 forward: the single-solve sweeps (descriptors then passed by
-// value) run 0.66 ms/step rolled against 1.12 ms/step unrolled, while the batch sweeps
-// (descriptors read from the device table) run 0.68 ms/step unrolled against 0.90 rolled.
+// Descriptor loops (slabs, sources) are rolled: on the 400x400x200 forward the single-solve sweeps
+// (descriptors then passed by value) measured 0.66 ms per step rolled against 1.12 unrolled.
 
 namespace fdtdx {
 
@@ -154,25 +152,15 @@ __device__ __forceinline__ void cpml_axes_frozen(const AxCell* ax, const Deriv& 
 }
 
 // `mask`: tile mask (bit s = slab s may touch the tile); slabs in object order.
-template <bool U>
 __device__ __forceinline__ void apply_cpml(const StepStatic& P, uint32_t mask, const float* psi_in, float* psi_out,
                                            int which, int update, int i, int j, int k, const Deriv& d, float& cx,
                                            float& cy, float& cz) {
   if (!(mask & ((1u << FDTDX_MAX_CPML) - 1u))) return;
-  if constexpr (U) {
-#pragma unroll
-    for (int s = 0; s < FDTDX_MAX_CPML; ++s) {
-      if (s >= P.nslab) break;
-      if (!((mask >> s) & 1u)) continue;
-      cpml_slab(P.slab[s], psi_in, psi_out, which, update, i, j, k, d, cx, cy, cz);
-    }
-  } else {
-    uint32_t m = mask & ((1u << P.nslab) - 1u);
-    while (m) {
-      const int s = __builtin_ctz(m);
-      m &= m - 1u;
-      cpml_slab(P.slab[s], psi_in, psi_out, which, update, i, j, k, d, cx, cy, cz);
-    }
+  uint32_t m = mask & ((1u << P.nslab) - 1u);
+  while (m) {
+    const int s = __builtin_ctz(m);
+    m &= m - 1u;
+    cpml_slab(P.slab[s], psi_in, psi_out, which, update, i, j, k, d, cx, cy, cz);
   }
 }
 
@@ -206,27 +194,16 @@ __device__ __forceinline__ void source_one(const StepStatic& P, const SrcK& sr, 
 }
 
 // `mask`: tile mask (bit kMaskSrc + s = source s may touch the tile); sources in list order.
-template <bool U>
 __device__ __forceinline__ void apply_sources(const StepStatic& P, uint32_t mask, const float* ie, const float* im,
                                               int field, int n, bool inverse, int i, int j, int k,
                                               long long o, int ec, int mc, float& vx, float& vy, float& vz) {
-  if constexpr (U) {
-#pragma unroll
-    for (int s = 0; s < FDTDX_MAX_SOURCES; ++s) {
-      if (s >= P.nsrc) break;
-      if (!((mask >> (kMaskSrc + s)) & 1u)) continue;
-      source_one(P, P.src[s], ie, im, field, n, inverse, i, j, k, o, ec, mc, vx, vy, vz);
-    }
-  } else {
-    uint32_t m = (mask >> kMaskSrc) & ((1u << P.nsrc) - 1u);
-    while (m) {
-      const int s = __builtin_ctz(m);
-      m &= m - 1u;
-      source_one(P, P.src[s], ie, im, field, n, inverse, i, j, k, o, ec, mc, vx, vy, vz);
-    }
+  uint32_t m = (mask >> kMaskSrc) & ((1u << P.nsrc) - 1u);
+  while (m) {
+    const int s = __builtin_ctz(m);
+    m &= m - 1u;
+    source_one(P, P.src[s], ie, im, field, n, inverse, i, j, k, o, ec, mc, vx, vy, vz);
   }
 }
-
 
 // PEC / PMC faces of kind `kind` (update.py:48-89): zero the components tangential to the face on
 // its layer. `mask` is the tile mask.

@@ -158,3 +158,74 @@ def test_blowup_limit_flags_every_solve(plain):
     fwd = sorted([r for r in reqs if not r.gradient], key=lambda r: -r.steps)[:2]
     res, stats = _serve(fwd, chunk=6, blowup=1e-30)
     assert all(res[r.rid].status == "failed" and "blow-up" in res[r.rid].reason for r in fwd)
+
+
+@pytest.mark.parametrize("eps_comps", [1, 3])
+def test_batch_of_mixed_schedules_equals_single_solves(eps_comps):
+    """One batch of solves whose tiles differ (quads over aligned and ragged rows, one cell per lane,
+    ADE tiles, conductivity with a conducting face, periodic axes) and whose detectors need per-cell
+    phasors, halos, reduced phasors and accumulating faces, advanced 21 steps per chunk (sums finalized
+    for 16, then 5): every state equals the single solve's bit for bit."""
+    import torch
+
+    from fdtdx_amd import engine
+    from fdtdx_amd import fdtd as F
+    from fdtdx_amd import scenarios as W
+    import scenarios
+
+    n = 24
+    f0 = 1.9e14
+    if eps_comps == 3:
+        specs = [W.scenario_c4(T=45, n=28, pml=5, slab=(10, 10, 8), cube=4),
+                 W.scenario_c4(T=50, n=31, pml=5, slab=(10, 10, 8), cube=4)]
+    else:
+        ragged = W.scenario_c2(T=45, shape=(44, 30, 27), pml=5, slab=(10, 12, 8))
+        lossy = W.scenario_c1(T=50, n=26, pml=4, cube=6)
+        lossy["pml"] = dict(lossy["pml"], types={"max_x": "pec"})
+        lossy["boxes"] = lossy["boxes"] + [dict(slc=((5, 12), (5, 12), (6, 20)), eps=2.0, sigma_E=3e4)]
+        per = W.scenario_c1(T=40, n=n, pml=4, cube=4)
+        per["pml"] = dict(per["pml"], types={f: "periodic" for f in ("min_y", "max_y", "min_z", "max_z")})
+        per["detectors"].append(dict(name="box", kind="closed_flux", slc=((8, 16), (8, 16), (8, 16))))
+        per["detectors"].append(dict(name="ph", kind="phasor", slc=((8, 12), (8, 12), (8, 12)), components=("Ez", "Hy"),
+                                     frequencies=[f0, 2 * f0], reduce_volume=True))
+        flat = W.scenario_c1(T=30, n=n, pml=4, cube=4)  # three cells in z: one cell per lane
+        flat["shape"] = (n, n, 3)
+        flat["pml"] = dict(flat["pml"], types={"min_z": "pec", "max_z": "pec"})
+        flat["boxes"] = [dict(slc=((8, 12), (8, 12), (0, 3)), eps=2.25)]
+        flat["sources"][0]["cell"] = (12, 12, 1)
+        flat["detectors"] = []
+        specs = [ragged, lossy, per, flat]
+
+    def solves():
+        out = []
+        for spec in specs:
+            objects, arrays, params, config = scenarios.build(spec)
+            s = F.Solve(objects, config, arrays)
+            arrays.reset()
+            out.append(s)
+        return out
+
+    def state(s):
+        a = s.arrays
+        return [t.cpu().numpy() for t in (a.fields.E, a.fields.H, a.psi, *s.state_tensors())]
+
+    single = solves()
+    for s, spec in zip(single, specs):
+        s.forward(0, spec["T"])
+    torch.cuda.synchronize()
+    batched = solves()
+    stream = torch.cuda.Stream()
+    handle = engine.c_void_p(stream.cuda_stream)
+    torch.cuda.synchronize()
+    batch = engine.Batch(eps_comps, 0)
+    for i, (s, spec) in enumerate(zip(batched, specs)):
+        print("attach", i, spec["shape"], flush=True)
+        batch.attach(i, s.plan, s.buffers(), s._keep, 0, spec["T"])
+    for _ in range(3):
+        batch.advance(21, handle)
+    stream.synchronize()
+    for i, (a, b) in enumerate(zip(single, batched)):
+        for x, y in zip(state(a), state(b)):
+            assert np.array_equal(x, y), i
+    assert not batch.flags().any()
+    batch.close()
