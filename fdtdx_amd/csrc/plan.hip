@@ -516,32 +516,13 @@ static int plan_create(const fdtdx_plan_desc* d, fdtdx_plan** out) {
         if ((g * W) % kBlock == 0 && (g * Wz) % kBlock == 0) { P.zg = g; break; }
       P.zg = std::min(P.zg, P.ny);
     }
-    std::vector<uint32_t> tm((size_t)P.nblocks, 0u), fm((size_t)P.nblocks, 0u);
+    std::vector<uint32_t> tm((size_t)P.nblocks, 0u);
     for (long long lb = 0; lb < P.nblocks; ++lb) {
       const int i = (int)(lb / P.bpp);
       const long long p0 = (lb - (long long)i * P.bpp) * kBlock;
-      const long long p1 = std::min(p0 + kBlock, P.plane) - 1;
-      tm[(size_t)lb] = span_mask(i, p0, p1, P.nz, true);
-      if (!perm) {
-        fm[(size_t)lb] = span_mask(i, p0, p1, P.nz, false);
-        continue;
-      }
-      // footprints of the tile's z-interior and z-slab cells, from the sweeps' own mapping
-      int lo[2][2] = {{P.ny, P.nz}, {P.ny, P.nz}}, hi[2][2] = {{-1, -1}, {-1, -1}};
-      for (long long p = p0; p <= p1; ++p) {
-        int j, k;
-        perm_cell(P, (int)p, j, k);
-        const int c = (k < P.zlo || k >= P.zhi) ? 1 : 0;
-        lo[c][0] = std::min(lo[c][0], j); hi[c][0] = std::max(hi[c][0], j);
-        lo[c][1] = std::min(lo[c][1], k); hi[c][1] = std::max(hi[c][1], k);
-      }
-      uint32_t m = 0;
-      for (int c = 0; c < 2; ++c)
-        if (hi[c][0] >= 0) m |= box_mask(i, lo[c][0], hi[c][0], lo[c][1], hi[c][1], false);
-      fm[(size_t)lb] = m;
+      tm[(size_t)lb] = span_mask(i, p0, std::min(p0 + kBlock, P.plane) - 1, P.nz, true);
     }
     if ((rc = pl->upload(tm.data(), tm.size(), &P.tile_mask))) return bail(rc);
-    if ((rc = pl->upload(fm.data(), fm.size(), &P.fwd_mask))) return bail(rc);
     // quad sweeps: 4 z cells per lane
     P.vq = 0;
     P.cax = 0;
@@ -608,6 +589,33 @@ static int plan_create(const fdtdx_plan_desc* d, fdtdx_plan** out) {
           x.aligned = (sl.lo % 4 == 0 && sl.L % 4 == 0) ? 1 : 0;
           x.cells = sl.cells; x.psi_off = sl.psi_off; x.coef = sl.coef;
         }
+    }
+    // masks of the one-cell forward sweeps' tiles, which plans with the per-axis quad sweeps never run
+    if (!(quad_ok && P.cax)) {
+      std::vector<uint32_t> fm((size_t)P.nblocks, 0u);
+      for (long long lb = 0; lb < P.nblocks; ++lb) {
+        const int i = (int)(lb / P.bpp);
+        const long long p0 = (lb - (long long)i * P.bpp) * kBlock;
+        const long long p1 = std::min(p0 + kBlock, P.plane) - 1;
+        if (!perm) {
+          fm[(size_t)lb] = span_mask(i, p0, p1, P.nz, false);
+          continue;
+        }
+        // footprints of the tile's z-interior and z-slab cells, from the sweeps' own mapping
+        int lo[2][2] = {{P.ny, P.nz}, {P.ny, P.nz}}, hi[2][2] = {{-1, -1}, {-1, -1}};
+        for (long long p = p0; p <= p1; ++p) {
+          int j, k;
+          perm_cell(P, (int)p, j, k);
+          const int c = (k < P.zlo || k >= P.zhi) ? 1 : 0;
+          lo[c][0] = std::min(lo[c][0], j); hi[c][0] = std::max(hi[c][0], j);
+          lo[c][1] = std::min(lo[c][1], k); hi[c][1] = std::max(hi[c][1], k);
+        }
+        uint32_t m = 0;
+        for (int c = 0; c < 2; ++c)
+          if (hi[c][0] >= 0) m |= box_mask(i, lo[c][0], hi[c][0], lo[c][1], hi[c][1], false);
+        fm[(size_t)lb] = m;
+      }
+      if ((rc = pl->upload(fm.data(), fm.size(), &P.fwd_mask))) return bail(rc);
     }
     if (quad_ok) {
       // Without the per-axis CPML the quads of a plane run in the row-grouped order (z-interior
