@@ -132,9 +132,6 @@ struct StepStatic {
   int vbpp;                // quad tiles per x-plane
   long long vnblocks, vnblocks_pad;
   const uint32_t* vec_mask;  // per quad tile, as fwd_mask
-  long long vnslow;          // quad tiles whose E half-step runs one cell per thread (vlistE bits) ...
-  const int* vslow;          // ... and their indices
-  uint32_t vlistE;           // the mask bits that list a quad tile for the E half-step (ADE boxes)
   uint32_t vpoint[2];        // the mask bits of E sources and PEC faces, of H sources and PMC faces
   // Per-axis CPML (acax = 1): every slab spans its face, at most one slab per side of an axis and
   // no two overlapping, and the x slabs before the y slabs before the z slabs in object order (the

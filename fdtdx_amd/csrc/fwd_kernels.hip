@@ -644,30 +644,10 @@ __device__ __forceinline__ bool tile_cell(const StepStatic& P, long long lb, int
   return true;
 }
 
-// The E half-step of quad tiles that meet an ADE box (listed in vslow) runs one cell per thread in a
-// launch of its own, four blocks per listed tile: the polarisation update would cost the quad
-// kernel its register budget. Cell of block b: false past the last listed tile.
-__device__ __forceinline__ bool slow_cell(const StepStatic& P, long long b, int& i, int& j, int& k, long long& o,
-                                          uint32_t& m) {
-  const long long s = b >> 2;
-  if (s >= P.vnslow) return false;
-  const long long lb = P.vslow[s];
-  m = P.vec_mask[lb];
-  return tile_cell(P, lb, (int)(b & 3), i, j, k, o);
-}
-
-template <int EC, bool X>
-__global__ __launch_bounds__(kBlock) void k_update_E4s(const StepStatic* __restrict__ Pp, const StepDyn D) {
-  const StepStatic& P = as_const(Pp);
-  int i, j, k;
-  long long o;
-  uint32_t ms;
-  if (slow_cell(P, (long long)blockIdx.x, i, j, k, o, ms)) update_E_cell<EC, X>(P, D, D.n, ms, i, j, k, o);
-}
-
-// The E and H half-steps of step n for one quad (m: its tile's mask, ADE tiles excepted).
+// The E and H half-steps of step n for one quad (m: its tile's mask; ADE: the plan has
+// poles).
 // CAX: the per-axis CPML (plans with StepStatic::cax), else the slab loop of cpml_quad.
-template <int EC, bool X, bool CAX, bool RAG>
+template <int EC, bool X, bool CAX, bool RAG, bool ADE>
 __device__ __forceinline__ void quad_E(const StepStatic& P, const StepDyn& D, int n, uint32_t m, int i, int j, int k0,
                                        int sm, long long o) {
   QuadSlabs S;
@@ -711,8 +691,13 @@ __device__ __forceinline__ void quad_E(const StepStatic& P, const StepDyn& D, in
   const f4v eo[3] = {ld4<RAG>(Ex + o), ld4<RAG>(Ey + o), ld4<RAG>(Ez + o)};
   const f4v t[3] = {(c * cx) * iex, (c * cy) * iey, (c * cz) * iez};
   f4v en[3] = {eo[0] + t[0], eo[1] + t[1], eo[2] + t[2]};
-  if (X && ((m >> kMaskLoss) & 1u)) {
-    const f4v inv[3] = {iex, iey, iez};
+  const f4v inv[3] = {iex, iey, iez};
+  const bool lossy = X && ((m >> kMaskLoss) & 1u);
+  if (ADE && (m & kAdeBits)) {
+    if (lossy) quad_loss<0, 1>(P, i, j, k0, inv, eo, t, en);
+    quad_ade<EC>(P, D.ade, D.ie + o, m, n, i, j, k0, sm, eo, en);
+    if (lossy) quad_loss<0, 2>(P, i, j, k0, inv, eo, t, en);
+  } else if (lossy) {
     quad_loss<0>(P, i, j, k0, inv, eo, t, en);
   }
   st4m<RAG>(Ex + o, en[0], sm);
@@ -799,16 +784,15 @@ __device__ __forceinline__ void quad_H(const StepStatic& P, const StepDyn& D, in
   }
 }
 
-template <int EC, bool X, bool CAX, bool RAG>
-__global__ __launch_bounds__(kBlock) void k_update_E4(const StepStatic* __restrict__ Pp, const StepDyn D) {
+template <int EC, bool X, bool CAX, bool RAG, bool ADE>
+__global__ __launch_bounds__(kBlock, ADE && X ? 4 : 5) void k_update_E4(const StepStatic* __restrict__ Pp, const StepDyn D) {
   const StepStatic& P = as_const(Pp);
   int i, j, k0, sm;
   long long o;
   const long long lb = logical_block(P.xorder, P.vnblocks_pad);
   if (!quad_of(P, lb, i, j, k0, sm, o)) return;
   const uint32_t m = P.vec_mask[lb];
-  if (m & P.vlistE) return;  // a listed tile: its cells run in k_update_E4s
-  quad_E<EC, X, CAX, RAG>(P, D, D.n, m, i, j, k0, sm, o);
+  quad_E<EC, X, CAX, RAG, ADE>(P, D, D.n, m, i, j, k0, sm, o);
 }
 
 template <int MC, bool X, bool CAX, bool RAG>
@@ -1160,11 +1144,11 @@ hipError_t launch_update_H(const StepStatic& P, const StepDyn& D, int mc, hipStr
 
 // Kernel of a quad sweep: x (periodic axes or conductivity), the per-axis CPML c, rows of nz % 4 != 0
 // cells rag (which always have the per-axis CPML).
-template <int EC>
+template <int EC, bool ADE>
 static SweepKernel quad_E_kernel(bool x, bool c, bool rag) {
-  if (rag) return x ? k_update_E4<EC, true, true, true> : k_update_E4<EC, false, true, true>;
-  if (c) return x ? k_update_E4<EC, true, true, false> : k_update_E4<EC, false, true, false>;
-  return x ? k_update_E4<EC, true, false, false> : k_update_E4<EC, false, false, false>;
+  if (rag) return x ? k_update_E4<EC, true, true, true, ADE> : k_update_E4<EC, false, true, true, ADE>;
+  if (c) return x ? k_update_E4<EC, true, true, false, ADE> : k_update_E4<EC, false, true, false, ADE>;
+  return x ? k_update_E4<EC, true, false, false, ADE> : k_update_E4<EC, false, false, false, ADE>;
 }
 
 template <int MC>
@@ -1176,11 +1160,9 @@ static SweepKernel quad_H_kernel(bool x, bool c, bool rag) {
 
 hipError_t launch_update_E4(const StepStatic& P, const StepDyn& D, int ec, hipStream_t s) {
   const bool x = extras(P), c = P.cax != 0, rag = P.nz % 4 != 0;
-  const SweepKernel f = ec == 3 ? quad_E_kernel<3>(x, c, rag) : quad_E_kernel<1>(x, c, rag);
-  const SweepKernel fs = ec == 3 ? (x ? k_update_E4s<3, true> : k_update_E4s<3, false>)
-                                 : (x ? k_update_E4s<1, true> : k_update_E4s<1, false>);
+  const SweepKernel f = P.nade ? (ec == 3 ? quad_E_kernel<3, true>(x, c, rag) : quad_E_kernel<1, true>(x, c, rag))
+                              : (ec == 3 ? quad_E_kernel<3, false>(x, c, rag) : quad_E_kernel<1, false>(x, c, rag));
   hipLaunchKernelGGL(f, dim3((unsigned)P.vnblocks_pad), dim3(kBlock), 0, s, P.self, D);
-  if (P.vnslow) hipLaunchKernelGGL(fs, dim3((unsigned)(4 * P.vnslow)), dim3(kBlock), 0, s, P.self, D);
   return hipGetLastError();
 }
 
@@ -1284,13 +1266,13 @@ __global__ __launch_bounds__(kBlock) void k_batch_E(const BatchTable* __restrict
   const uint32_t m = P.vec_mask[lb];
   int i, j, k, sm;
   long long o;
-  if (m & P.vlistE) {
+  if (m & kAdeBits) {
 #pragma unroll 1
     for (int part = 0; part < 4; ++part)
       if (tile_cell(P, lb, part, i, j, k, o)) update_E_cell<EC, true>(P, I.D, n, m, i, j, k, o);
     return;
   }
-  if (quad_of(P, lb, i, j, k, sm, o)) quad_E<EC, true, true, true>(P, I.D, n, m, i, j, k, sm, o);
+  if (quad_of(P, lb, i, j, k, sm, o)) quad_E<EC, true, true, true, false>(P, I.D, n, m, i, j, k, sm, o);
 }
 
 template <int MC>

@@ -669,20 +669,9 @@ static int plan_create(const fdtdx_plan_desc* d, fdtdx_plan** out) {
         vm[(size_t)lb] = m;
       }
       if ((rc = pl->upload(vm.data(), vm.size(), &P.vec_mask))) return bail(rc);
-      // listed tiles, one cell per thread: those whose E half-step meets an ADE box (a
-      // quad-vectorised ADE sweep measured slower than the one-cell one: 0.245 against 0.236 ms per
-      // E sweep of the 256^3 dispersive case); conductivity, sources and conducting faces run in the
-      // quad sweeps
-      P.vlistE = ((1u << FDTDX_MAX_ADE) - 1u) << kMaskAde;
       P.vpoint[0] = P.vpoint[1] = 0u;
       for (int q = 0; q < P.nsrc; ++q) P.vpoint[P.src[q].field] |= 1u << (kMaskSrc + q);
       for (int w = 0; w < P.nwall; ++w) P.vpoint[P.wall[w].kind == FDTDX_WALL_PEC ? 0 : 1] |= 1u << (kMaskWall + w);
-      std::vector<int> slow;
-      for (long long lb = 0; lb < P.vnblocks; ++lb)
-        if (vm[(size_t)lb] & P.vlistE) slow.push_back((int)lb);
-      P.vnslow = (long long)slow.size();
-      P.vslow = nullptr;
-      if (!slow.empty() && (rc = pl->upload(slow.data(), slow.size(), &P.vslow))) return bail(rc);
       P.vq = 1;
     }
   }

@@ -40,6 +40,7 @@ __device__ __forceinline__ void st4m(float* p, f4v v, int sm) {
 }
 
 constexpr uint32_t kSlabBits = (1u << FDTDX_MAX_CPML) - 1u;
+constexpr uint32_t kAdeBits = ((1u << FDTDX_MAX_ADE) - 1u) << kMaskAde;
 constexpr uint32_t kSnapBit = 1u << kMaskSnap;
 
 // Quad of this lane in quad tile lb: cells (i, j, k0 .. k0 + 3) at offsets o .. o + 3, the first sm
@@ -268,23 +269,98 @@ __device__ __forceinline__ void quad_slab_frozen(const StepStatic& P, const Quad
   quad_frozen_axis<W, 2, RAG>(P, S, i, j, k0, d, cx, cy, cz);
 }
 
+// The cells [a0, a1) of a quad, as one access where that is all of it.
+__device__ __forceinline__ f4v ld4p(const float* p, int a0, int a1) {
+  if (a1 - a0 == 4) return ld4<true>(p);
+  f4v v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (e >= a0 && e < a1) v[e] = p[e];
+  return v;
+}
+
+__device__ __forceinline__ void st4p(float* p, f4v v, int a0, int a1) {
+  if (a1 - a0 == 4) {
+    *reinterpret_cast<f4u*>(p) = v;
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (e >= a0 && e < a1) p[e] = v[e];
+}
+
 // Conductivity of a quad (loss_x and the update of update_E_cell / update_H_cell): f the field before
-// the step, t = (c curl) inv, n the lossless result, replaced for the cells inside the box.
-template <int W>
+// the step, t = (c curl) inv, n the lossless result, replaced for the cells inside the box. PART 1 leaves
+// out the division by 1 + x and PART 2 is that division alone, so that poles come between them.
+template <int W, int PART = 0>
 __device__ __forceinline__ void quad_loss(const StepStatic& P, int i, int j, int k0, const f4v* inv, const f4v* f,
                                           const f4v* t, f4v* n) {
   const LossK& L = P.loss[W];
   if (i < L.lo[0] || i >= L.hi[0] || j < L.lo[1] || j >= L.hi[1] || k0 + 3 < L.lo[2] || k0 >= L.hi[2]) return;
   const long long q = ((long long)(i - L.lo[0]) * L.by + (j - L.lo[1])) * L.bz + (k0 - L.lo[2]);
+  // cells outside the box: zero conductivity, which leaves n as it is
+  const int a0 = max(0, L.lo[2] - k0), a1 = min(4, L.hi[2] - k0);
+  const f4v c = {P.c, P.c, P.c, P.c}, one = {1.f, 1.f, 1.f, 1.f};
+  f4v sg;
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
+    if (a == 0 || L.comps == 3) sg = ld4p(L.sig + a * L.cells + q, a0, a1);
+    f4v x = (W == 0 ? ((c * sg) * P.eta0) * inv[a] : ((c * sg) / P.eta0) * inv[a]) / 2.0f;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      if (k0 + e < L.lo[2] || k0 + e >= L.hi[2]) continue;
-      const float sg = L.sig[(L.comps == 3 ? a : 0) * L.cells + q + e];
-      const float x = W == 0 ? (((P.c * sg) * P.eta0) * inv[a][e]) / 2.0f : (((P.c * sg) / P.eta0) * inv[a][e]) / 2.0f;
-      const float g = (1.0f - x) * f[a][e];
-      n[a][e] = (W == 0 ? g + t[a][e] : g - t[a][e]) / (1.0f + x);
+    for (int e = 0; e < 4; ++e) x[e] = e >= a0 && e < a1 ? x[e] : 0.f;  // also where inv is not finite
+    if (PART != 2) {
+      const f4v g = (one - x) * f[a];
+      n[a] = W == 0 ? g + t[a] : g - t[a];
+    }
+    if (PART != 1) n[a] = n[a] / (one + x);
+  }
+}
+
+// Lorentz and Drude poles of a quad (the recurrence of update_E_cell): en += ie sum_p (P^n - P_hat) for
+// the cells e >= sm inside each box; eo is E^n. ie (at the quad) is read again here: few quads have
+// poles, and twelve registers held for them would cost every other quad a wave. Box edges and widths
+// have no alignment, so whole quads move with 4-byte aligned accesses.
+template <int EC>
+__device__ __forceinline__ void quad_ade(const StepStatic& P, float* ade, const float* ie, uint32_t m, int n, int i,
+                                         int j, int k0, int sm, const f4v* eo, f4v* en) {
+#pragma unroll 1
+  for (uint32_t mm = (m >> kMaskAde) & ((1u << P.nade) - 1u); mm; mm &= mm - 1u) {
+    const AdeK& A = P.ade[__builtin_ctz(mm)];
+    if (i < A.lo[0] || i >= A.hi[0] || j < A.lo[1] || j >= A.hi[1]) continue;
+    const int a0 = max(sm, A.lo[2] - k0), a1 = min(4, A.hi[2] - k0);
+    if (a0 >= a1) continue;
+    const long long q = ((long long)(i - A.lo[0]) * A.by + (j - A.lo[1])) * A.bz + (k0 - A.lo[2]);
+    // three slots: P^n in slot n%3, P^{n-1} in (n+2)%3, P^{n+1} written to (n+1)%3
+    const long long cells = A.cells, slot = (long long)A.poles * 3 * cells;
+    const long long coef = (long long)A.poles * A.ccomp * cells;
+    const float* cur = ade + A.state_off + (long long)(n % 3) * slot + q;
+    const float* prv = ade + A.state_off + (long long)((n + 2) % 3) * slot + q;
+    float* nxt = ade + A.state_off + (long long)((n + 1) % 3) * slot + q;
+    f4v dl[3];
+#pragma unroll 1
+    for (int p = 0; p < A.poles; ++p) {
+      f4v c1, c2, c3;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        if (a == 0 || A.ccomp == 3) {
+          const float* cf = A.coef + ((long long)p * A.ccomp + a) * cells + q;
+          c1 = ld4p(cf, a0, a1);
+          c2 = ld4p(cf + coef, a0, a1);
+          c3 = ld4p(cf + 2 * coef, a0, a1);
+        }
+        const long long si = ((long long)p * 3 + a) * cells;
+        const f4v pc = ld4p(cur + si, a0, a1), pp = ld4p(prv + si, a0, a1);
+        const f4v ph = (c1 * pc + c2 * pp) + c3 * eo[a];
+        dl[a] = p == 0 ? pc - ph : dl[a] + (pc - ph);
+        st4p(nxt + si, ph, a0, a1);
+      }
+    }
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const f4v inv = ld4<true>(ie + (EC == 3 ? a * P.N : 0));
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (e >= a0 && e < a1) en[a][e] = en[a][e] + inv[e] * dl[a][e];
     }
   }
 }

@@ -119,6 +119,39 @@ def test_quad_ade_tiles_match_the_one_cell_path(monkeypatch):
     assert rel(out["quad"][1], st.E) < 1e-5 and rel(out["quad"][4], ds[0]) < 1e-5
 
 
+@pytest.mark.parametrize("nz,types", [(36, {}), (37, {}), (39, {}), (38, {"min_z": "periodic", "max_z": "periodic"})])
+@pytest.mark.parametrize("sigma", [0.0, 2e4])
+def test_quad_poles_equal_the_one_cell_poles_bitwise(nz, types, sigma, monkeypatch):
+    """Poles inside the quad E sweep against one cell per lane: boxes with edges inside quads, one of
+    them up to the row's last quad, isotropic and diagonal permittivity, one and two poles, with and
+    without conductivity in the same cells. Fields, psi, poles and phasors agree bit for bit."""
+    import scenarios
+
+    from fdtdx_amd import fdtd as F
+
+    spec = W.scenario_c4(T=41, n=36, pml=5, slab=(12, 12, 8), cube=6)
+    spec["shape"] = (36, 34, nz)
+    spec["pml"] = dict(spec["pml"], types=types)
+    spec["detectors"] = [dict(d, slc=((26, 27), (0, 34), (0, nz))) for d in spec["detectors"]]
+    poles = spec["boxes"][0]["poles"]
+    spec["boxes"] = [dict(slc=((12, 25), (9, 22), (15, 26)), eps=(2.0, 4.0, 9.0), poles=poles, sigma_E=sigma),
+                     dict(slc=((20, 29), (14, 23), (22, nz if types else nz - 5)), eps=4.0, poles=poles[:1],
+                          sigma_E=sigma),
+                     dict(slc=((9, 11), (9, 20), (18, 21)), eps=3.0, poles=[("drude", 2e15, 1e14)])]
+    out = {}
+    for mode in ("quad", "two"):
+        _set_mode(monkeypatch, mode)
+        objects, arrays, params, config = scenarios.build(spec)
+        F.run_fdtd(arrays, objects, config)
+        solve = F._solve_for(objects, config, arrays)
+        assert solve.plan.quad == (mode == "quad")
+        out[mode] = [arrays.fields.E.cpu().numpy(), arrays.fields.H.cpu().numpy(), arrays.psi.cpu().numpy(),
+                     arrays.ade_state.cpu().numpy()] + [t.cpu().numpy() for t in solve.det_tensors()]
+    assert np.abs(out["two"][0]).max() > 0 and np.abs(out["two"][3]).max() > 0
+    for a, b in zip(out["quad"], out["two"]):
+        np.testing.assert_array_equal(a, b)
+
+
 def test_single_pass_equals_two_sweep_bitwise(monkeypatch):
     """The single-pass kernels perform the two-sweep kernels' float operations in the same order:
     fields, psi, detector states and the interface record agree bit for bit (z split into two
