@@ -132,6 +132,8 @@ struct StepStatic {
   int vbpp;                // quad tiles per x-plane
   long long vnblocks, vnblocks_pad;
   const uint32_t* vec_mask;  // per quad tile, as fwd_mask
+  long long vnslow;          // quad tiles with poles and conductivity (k_update_E4s) ...
+  const int* vslow;          // ... and their indices
   uint32_t vpoint[2];        // the mask bits of E sources and PEC faces, of H sources and PMC faces
   // Per-axis CPML (acax = 1): every slab spans its face, at most one slab per side of an axis and
   // no two overlapping, and the x slabs before the y slabs before the z slabs in object order (the
@@ -243,6 +245,12 @@ struct StepDyn {
   // sweep updates one part: cpart = +1 the real part (the imaginary part lies 3 N floats after the
   // pointers above), -1 the imaginary part (the real part 3 N floats before), 0 a real plan.
   int cpart;
+};
+
+// Where the imaginary part of a complex-field plan's state lies (quad sweeps, both parts in one launch).
+struct PartDyn {
+  long long psi, ade;      // floats from the real part's psi and poles to the imaginary part's
+  float* snap;             // the imaginary part's H_prev snapshot
 };
 
 // The value a complex-field sweep reads across the min (side 0) or max (side 1) face of periodic

@@ -209,6 +209,8 @@ hipError_t launch_update_H(const StepStatic& P, const StepDyn& D, int mc, hipStr
 hipError_t launch_tensor_ab(const StepStatic& P, const StepDyn& D, hipStream_t s);
 hipError_t launch_update_E4(const StepStatic& P, const StepDyn& D, int ec, hipStream_t s);
 hipError_t launch_update_H4(const StepStatic& P, const StepDyn& D, int mc, hipStream_t s);
+hipError_t launch_update_E4c(const StepStatic& P, const StepDyn& D, const PartDyn& C, int ec, hipStream_t s);
+hipError_t launch_update_H4c(const StepStatic& P, const StepDyn& D, const PartDyn& C, int mc, hipStream_t s);
 hipError_t launch_restore(const StepStatic& P, const StepDyn& D, long long iface_cells, hipStream_t s);
 hipError_t launch_record(const StepStatic& P, const StepDyn& D, long long iface_cells, hipStream_t s);
 hipError_t launch_reverse(const StepStatic& P, const StepDyn& D, int ec, int mc, hipStream_t s);

@@ -528,7 +528,7 @@ static int plan_create(const fdtdx_plan_desc* d, fdtdx_plan** out) {
     P.cax = 0;
     P.acax = 0;
     const char* qenv = getenv("FDTDX_SWEEP");
-    bool quad_ok = P.nz >= 4 && d->eps_comps <= 3 && d->mu_comps <= 3 && !pl->cplx &&
+    bool quad_ok = P.nz >= 4 && d->eps_comps <= 3 && d->mu_comps <= 3 &&
                    !(qenv && strcmp(qenv, "quad") != 0 && strcmp(qenv, "default") != 0);
     // per-axis CPML: every slab spans its face, at most one slab per side of an axis, the two sides
     // apart, and the x slabs before the y slabs before the z slabs in object order (the order in
@@ -565,8 +565,10 @@ static int plan_create(const fdtdx_plan_desc* d, fdtdx_plan** out) {
         zq = (zhi0 - 1) / 4 < zlo1 / 4 && (P.nz % 4 == 0 || P.nz - 4 >= zhi0);
       }
       // rows of nz % 4 != 0 cells only with the per-axis CPML: the slab loop's vector path needs
-      // aligned quads
-      if (P.nz % 4 && !(xyz && zq)) quad_ok = false;
+      // aligned quads. Complex fields too, to keep the kernels few. Neither with poles and
+      // conductivity: their tiles run one cell per lane (200x200x101: 101 us per step against 93 with
+      // every tile one cell per lane; 128x120x100, 56 against 57, has them listed)
+      if ((P.nz % 4 || pl->cplx) && (!(xyz && zq) || (P.nade && P.loss[0].comps))) quad_ok = false;
       P.cax = quad_ok && xyz && zq ? 1 : 0;
       bool gap = true;
       for (int a = 0; a < 3; ++a)
@@ -672,6 +674,14 @@ static int plan_create(const fdtdx_plan_desc* d, fdtdx_plan** out) {
       P.vpoint[0] = P.vpoint[1] = 0u;
       for (int q = 0; q < P.nsrc; ++q) P.vpoint[P.src[q].field] |= 1u << (kMaskSrc + q);
       for (int w = 0; w < P.nwall; ++w) P.vpoint[P.wall[w].kind == FDTDX_WALL_PEC ? 0 : 1] |= 1u << (kMaskWall + w);
+      std::vector<int> slow;  // tiles with poles and conductivity
+      const uint32_t ade = ((1u << FDTDX_MAX_ADE) - 1u) << kMaskAde;
+      if (P.nade && P.loss[0].comps)
+        for (long long lb = 0; lb < P.vnblocks; ++lb)
+          if ((vm[(size_t)lb] & ade) && ((vm[(size_t)lb] >> kMaskLoss) & 1u)) slow.push_back((int)lb);
+      P.vnslow = (long long)slow.size();
+      P.vslow = nullptr;
+      if (!slow.empty() && (rc = pl->upload(slow.data(), slow.size(), &P.vslow))) return bail(rc);
       P.vq = 1;
     }
   }
@@ -991,13 +1001,16 @@ static int forward_impl(const fdtdx_plan* p, const fdtdx_buffers* b, int32_t t0,
       D.record = p->P.rec_narrow ? nullptr : recp;  // narrow layers are encoded by k_record
       Di.n = n;
       Di.snap = snap ? (float*)(ws + p->ws_snapE) : nullptr;  // H_prev of the imaginary part
-      if (p->P.vq) HIP_TRY(launch_update_E4(p->P, D, p->ec, s));
+      const PartDyn C = {(long long)p->psi_floats, (long long)p->ade_floats, Di.snap};
+      if (p->P.vq && p->cplx) HIP_TRY(launch_update_E4c(p->P, D, C, p->ec, s));
+      else if (p->P.vq) HIP_TRY(launch_update_E4(p->P, D, p->ec, s));
       else HIP_TRY(launch_update_E(p->P, D, p->ec, s));
-      if (p->cplx) HIP_TRY(launch_update_E(p->P, Di, p->ec, s));
+      if (p->cplx && !p->P.vq) HIP_TRY(launch_update_E(p->P, Di, p->ec, s));
       if (ev) HIP_TRY(hipEventRecord(ev[3 * (n - t0) + 1], s));
-      if (p->P.vq) HIP_TRY(launch_update_H4(p->P, D, p->mc, s));
+      if (p->P.vq && p->cplx) HIP_TRY(launch_update_H4c(p->P, D, C, p->mc, s));
+      else if (p->P.vq) HIP_TRY(launch_update_H4(p->P, D, p->mc, s));
       else HIP_TRY(launch_update_H(p->P, D, p->mc, s));
-      if (p->cplx) HIP_TRY(launch_update_H(p->P, Di, p->mc, s));
+      if (p->cplx && !p->P.vq) HIP_TRY(launch_update_H(p->P, Di, p->mc, s));
       if (p->P.rec_narrow && recp) {
         D.record = recp;
         HIP_TRY(launch_record(p->P, D, p->iface_cells, s));

@@ -290,9 +290,8 @@ __device__ __forceinline__ void st4p(float* p, f4v v, int a0, int a1) {
 }
 
 // Conductivity of a quad (loss_x and the update of update_E_cell / update_H_cell): f the field before
-// the step, t = (c curl) inv, n the lossless result, replaced for the cells inside the box. PART 1 leaves
-// out the division by 1 + x and PART 2 is that division alone, so that poles come between them.
-template <int W, int PART = 0>
+// the step, t = (c curl) inv, n the lossless result, replaced for the cells inside the box.
+template <int W>
 __device__ __forceinline__ void quad_loss(const StepStatic& P, int i, int j, int k0, const f4v* inv, const f4v* f,
                                           const f4v* t, f4v* n) {
   const LossK& L = P.loss[W];
@@ -308,11 +307,8 @@ __device__ __forceinline__ void quad_loss(const StepStatic& P, int i, int j, int
     f4v x = (W == 0 ? ((c * sg) * P.eta0) * inv[a] : ((c * sg) / P.eta0) * inv[a]) / 2.0f;
 #pragma unroll
     for (int e = 0; e < 4; ++e) x[e] = e >= a0 && e < a1 ? x[e] : 0.f;  // also where inv is not finite
-    if (PART != 2) {
-      const f4v g = (one - x) * f[a];
-      n[a] = W == 0 ? g + t[a] : g - t[a];
-    }
-    if (PART != 1) n[a] = n[a] / (one + x);
+    const f4v g = (one - x) * f[a];
+    n[a] = (W == 0 ? g + t[a] : g - t[a]) / (one + x);
   }
 }
 
