@@ -108,46 +108,45 @@ __device__ __forceinline__ long long src_index(const Src3& s, int i, int j, int 
   return ((long long)(i - s.lo[0]) * s.sy + (j - s.lo[1])) * s.sz + (k - s.lo[2]);
 }
 
-// interp where no halo of a periodic axis or symmetry plane is needed (needs_halo): the stencil reads
-// i-1, j-1 and k+1, which a source's box holds unless they lie beyond the domain (the zero halo; then the cell itself is
-// read and dropped). Plain offsets and no branches: all loads are in flight together, and a wavefront
-// with one cell on a face costs no second pass. The expressions and their order are those of the
-// general path.
-__device__ __forceinline__ void interp_open(const StepStatic& P, const Src3& e, const Src3& hp, const Src3& h, int i,
-                                            int j, int k, float* Ei, float* Hi) {
+// Component c (Ex Ey Ez Hx Hy Hz) of interp where no halo of a periodic axis or symmetry plane is needed
+// (needs_halo): the stencil reads i-1, j-1 and k+1, which a source's box holds unless they lie beyond the
+// domain (the zero halo; then the cell itself is read and dropped). Plain offsets and no branches: all
+// loads are in flight together, and a wavefront with one cell on a face costs no second pass. The
+// expressions and their order are those of the general path.
+__device__ __forceinline__ float interp_open(const StepStatic& P, const Src3& e, const Src3& hp, const Src3& h, int i,
+                                             int j, int k, int c) {
   const bool vi = i > 0, vj = j > 0, vk = k + 1 < P.nz;
-  const long long oe = src_index(e, i, j, k);
-  const long long xe = vi ? -(long long)e.sy * e.sz : 0, ye = vj ? -(long long)e.sz : 0, ze = vk ? 1 : 0;
   auto z = [](bool v, float x) { return v ? x : 0.f; };
-  const float* ex = e.p;
-  const float* ey = e.p + e.stride;
-  const float* ez = e.p + 2 * e.stride;
-  const float lo_x = 0.5f * (ex[oe] + z(vi, ex[oe + xe]));
-  const float up_x = 0.5f * (z(vk, ex[oe + ze]) + z(vi && vk, ex[oe + xe + ze]));
-  Ei[0] = (lo_x + up_x) / 2.0f;
-  const float lo_y = 0.5f * (ey[oe] + z(vj, ey[oe + ye]));
-  const float up_y = 0.5f * (z(vk, ey[oe + ze]) + z(vj && vk, ey[oe + ye + ze]));
-  Ei[1] = (lo_y + up_y) / 2.0f;
-  Ei[2] = ez[oe];
-  const long long op = src_index(hp, i, j, k), oh = src_index(h, i, j, k);
+  if (c < 3) {
+    const float* f = e.p + c * e.stride;
+    const long long o = src_index(e, i, j, k);
+    if (c == 2) return f[o];
+    // back along x for Ex, along y for Ey
+    const bool v = c == 0 ? vi : vj;
+    const long long d = v ? -(c == 0 ? (long long)e.sy * e.sz : (long long)e.sz) : 0, ze = vk ? 1 : 0;
+    const float lo = 0.5f * (f[o] + z(v, f[o + d]));
+    const float up = 0.5f * (z(vk, f[o + ze]) + z(v && vk, f[o + d + ze]));
+    return (lo + up) / 2.0f;
+  }
+  const long long op = src_index(hp, i, j, k), oh = src_index(h, i, j, k), ze = vk ? 1 : 0;
   const long long xp = vi ? -(long long)hp.sy * hp.sz : 0, yp = vj ? -(long long)hp.sz : 0;
   const long long xh = vi ? -(long long)h.sy * h.sz : 0, yh = vj ? -(long long)h.sz : 0;
   // time-centred H at the offset (-dx, -dy, +dz)
-  auto hcq = [&](int c, int dx, int dy, int dz) {
-    const float a = hp.p[c * hp.stride + op + dx * xp + dy * yp + dz * ze];
-    const float b = h.p[c * h.stride + oh + dx * xh + dy * yh + dz * ze];
+  auto hcq = [&](int dx, int dy, int dz) {
+    const float a = hp.p[(c - 3) * hp.stride + op + dx * xp + dy * yp + dz * ze];
+    const float b = h.p[(c - 3) * h.stride + oh + dx * xh + dy * yh + dz * ze];
     return z((!dx || vi) && (!dy || vj) && (!dz || vk), (a + b) / 2.0f);
   };
-  Hi[0] = 0.5f * (hcq(0, 0, 0, 0) + hcq(0, 0, 1, 0));
-  Hi[1] = 0.5f * (hcq(1, 0, 0, 0) + hcq(1, 1, 0, 0));
+  if (c == 3) return 0.5f * (hcq(0, 0, 0) + hcq(0, 1, 0));
+  if (c == 4) return 0.5f * (hcq(0, 0, 0) + hcq(1, 0, 0));
   float zz[2];
 #pragma unroll
   for (int dz = 0; dz < 2; ++dz) {
-    const float a = 0.5f * (hcq(2, 0, 0, dz) + hcq(2, 1, 0, dz));
-    const float b = 0.5f * (hcq(2, 0, 1, dz) + hcq(2, 1, 1, dz));
+    const float a = 0.5f * (hcq(0, 0, dz) + hcq(1, 0, dz));
+    const float b = 0.5f * (hcq(0, 1, dz) + hcq(1, 1, dz));
     zz[dz] = 0.5f * (a + b);
   }
-  Hi[2] = (zz[0] + zz[1]) / 2.0f;
+  return (zz[0] + zz[1]) / 2.0f;
 }
 
 // Where that halo is needed, cells whose stencil stays inside every source's box read plain offsets.
@@ -155,30 +154,55 @@ __device__ __forceinline__ bool stencil_inside(const Src3& s, int i, int j, int 
   return i - 1 >= s.lo[0] && j - 1 >= s.lo[1] && k + 1 < s.hi[2] && i < s.hi[0] && j < s.hi[1] && k >= s.lo[2];
 }
 
-// interpolate_fields (curl.py:86-224) at cell (i,j,k) on a uniform grid. HALO: see needs_halo.
-template <bool HALO>
-__device__ __forceinline__ void interp(const StepStatic& P, const Src3& e, const Src3& hp, const Src3& h, int i, int j, int k,
-                       float* Ei, float* Hi) {
-  if (!HALO || (stencil_inside(e, i, j, k) && stencil_inside(hp, i, j, k) && stencil_inside(h, i, j, k))) {
-    interp_open(P, e, hp, h, i, j, k, Ei, Hi);
-    return;
+// Component c of interpolate_fields (curl.py:86-224) at cell (i,j,k) on a uniform grid, in general.
+__device__ __forceinline__ float interp_halo(const StepStatic& P, const Src3& e, const Src3& hp, const Src3& h, int i,
+                                             int j, int k, int c) {
+  if (c == 2) return at(P, e, 2, i, j, k);
+  if (c < 2) {
+    const int i1 = c == 0 ? i - 1 : i, j1 = c == 1 ? j - 1 : j;
+    const float lo = 0.5f * (at(P, e, c, i, j, k) + at(P, e, c, i1, j1, k));
+    const float up = 0.5f * (at(P, e, c, i, j, k + 1) + at(P, e, c, i1, j1, k + 1));
+    return (lo + up) / 2.0f;
   }
-  const float lo_x = 0.5f * (at(P, e, 0, i, j, k) + at(P, e, 0, i - 1, j, k));
-  const float up_x = 0.5f * (at(P, e, 0, i, j, k + 1) + at(P, e, 0, i - 1, j, k + 1));
-  Ei[0] = (lo_x + up_x) / 2.0f;
-  const float lo_y = 0.5f * (at(P, e, 1, i, j, k) + at(P, e, 1, i, j - 1, k));
-  const float up_y = 0.5f * (at(P, e, 1, i, j, k + 1) + at(P, e, 1, i, j - 1, k + 1));
-  Ei[1] = (lo_y + up_y) / 2.0f;
-  Ei[2] = at(P, e, 2, i, j, k);
-  Hi[0] = 0.5f * (hc(P, hp, h, 0, i, j, k) + hc(P, hp, h, 0, i, j - 1, k));
-  Hi[1] = 0.5f * (hc(P, hp, h, 1, i, j, k) + hc(P, hp, h, 1, i - 1, j, k));
+  if (c == 3) return 0.5f * (hc(P, hp, h, 0, i, j, k) + hc(P, hp, h, 0, i, j - 1, k));
+  if (c == 4) return 0.5f * (hc(P, hp, h, 1, i, j, k) + hc(P, hp, h, 1, i - 1, j, k));
   float zz[2];
   for (int dz = 0; dz < 2; ++dz) {
     const float a = 0.5f * (hc(P, hp, h, 2, i, j, k + dz) + hc(P, hp, h, 2, i - 1, j, k + dz));
     const float b = 0.5f * (hc(P, hp, h, 2, i, j - 1, k + dz) + hc(P, hp, h, 2, i - 1, j - 1, k + dz));
     zz[dz] = 0.5f * (a + b);
   }
-  Hi[2] = (zz[0] + zz[1]) / 2.0f;
+  return (zz[0] + zz[1]) / 2.0f;
+}
+
+template <bool HALO>
+__device__ __forceinline__ bool open_stencil(const Src3& e, const Src3& hp, const Src3& h, int i, int j, int k) {
+  return !HALO || (stencil_inside(e, i, j, k) && stencil_inside(hp, i, j, k) && stencil_inside(h, i, j, k));
+}
+
+// One component, and all six. HALO: see needs_halo.
+template <bool HALO>
+__device__ __forceinline__ float interp1(const StepStatic& P, const Src3& e, const Src3& hp, const Src3& h, int i,
+                                         int j, int k, int c) {
+  if (open_stencil<HALO>(e, hp, h, i, j, k)) return interp_open(P, e, hp, h, i, j, k, c);
+  return interp_halo(P, e, hp, h, i, j, k, c);
+}
+
+template <bool HALO>
+__device__ __forceinline__ void interp(const StepStatic& P, const Src3& e, const Src3& hp, const Src3& h, int i, int j,
+                                       int k, float* Ei, float* Hi) {
+  const bool open = open_stencil<HALO>(e, hp, h, i, j, k);
+  if (open) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) Ei[c] = interp_open(P, e, hp, h, i, j, k, c);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) Hi[c] = interp_open(P, e, hp, h, i, j, k, 3 + c);
+    return;
+  }
+#pragma unroll
+  for (int c = 0; c < 3; ++c) Ei[c] = interp_halo(P, e, hp, h, i, j, k, c);
+#pragma unroll
+  for (int c = 0; c < 3; ++c) Hi[c] = interp_halo(P, e, hp, h, i, j, k, 3 + c);
 }
 
 __device__ __forceinline__ float pick6(int c, const float* E, const float* H) {
@@ -298,15 +322,70 @@ __device__ __forceinline__ void energy_mean_tile(const StepStatic& P, const DetK
   }
 }
 
+// PhasorDetector per cell (phasor.py:190-235): state += EH * exp(i w t) * scale * window. One lane per cell
+// and component (detector_blocks): a plane detector has few cells, and one lane each of all six
+// components left most CUs idle and its loads in one long chain (one-frequency complex plane of 94x94 cells normal to z
+// 16.8 us, 8.4 here; 398x198 three-frequency with a flux plane 13.5, 13 to 14). The state words of up to four
+// frequencies are loaded ahead of the field reads, so that all are in flight together.
+template <bool CX, bool HALO>
+__device__ __forceinline__ void phasor_tile(const StepStatic& P, const DetK& K, const DetDyn& D, int n, int blk,
+                                            int nblk, const Src3& e, const Src3& hp, const Src3& h, const Src3& e2,
+                                            const Src3& hp2, const Src3& h2) {
+  float2* st = (float2*)D.state;
+  const float w = K.window[n];
+  const long long row = (long long)K.ncomp * K.cells;  // state words per frequency, t of each this lane's
+  for (long long t = (long long)blk * kBlock + threadIdx.x; t < row; t += (long long)nblk * kBlock) {
+    const int c = (int)(t / K.cells);
+    int i, j, k;
+    region_cell(K, t - c * K.cells, i, j, k);
+    const int cc = K.comps[c];
+    float2 old[4];
+    auto load = [&](int f0) {
+#pragma unroll
+      for (int df = 0; df < 4; ++df)
+        if (f0 + df < K.nfreq) old[df] = st[(f0 + df) * row + t];
+    };
+    load(0);
+    float v, vi = 0.f;
+    if (K.exact) {
+      v = interp1<HALO>(P, e, hp, h, i, j, k, cc);
+      if (CX) vi = interp1<HALO>(P, e2, hp2, h2, i, j, k, cc);
+    } else {
+      const long long o = ((long long)i * P.ny + j) * P.nz + k + (cc % 3) * P.N;
+      v = (cc < 3 ? D.E : D.H)[o];
+      if (CX) vi = (cc < 3 ? D.Ei : D.Hi)[o];
+    }
+    for (int f0 = 0; f0 < K.nfreq; f0 += 4) {
+      if (f0) load(f0);
+#pragma unroll
+      for (int df = 0; df < 4; ++df) {
+        const int f = f0 + df;
+        if (f >= K.nfreq) break;
+        const float cs = K.cos_t[(long long)f * P.T + n];
+        const float sn = K.sin_t[(long long)f * P.T + n];
+        float re = ((v * cs) * K.scale) * w;
+        float im = ((v * sn) * K.scale) * w;
+        if (CX) {  // (v + i vi)(cos + i sin)
+          re = re - ((vi * sn) * K.scale) * w;
+          im = ((vi * cs) * K.scale) * w + im;
+        }
+        float2 s = old[df];
+        if (K.sign < 0.f) { s.x = s.x - re; s.y = s.y - im; }
+        else { s.x = s.x + re; s.y = s.y + im; }
+        st[f * row + t] = s;
+      }
+    }
+  }
+}
+
 // One detector update at step n into record slot `slot`, computed by block blk of nblk blocks
 // that stride over the detector's cells. A reducing detector leaves one partial sum per block and
 // value: the weighted energy or flux, or the sum of each recorded component (field and phasor
 // detectors with reduce_volume, whose box mean is formed in reduce_finalize_tile).
-// PH: the launch has a detector with per-cell phasors, HALO: one that needs_halo. Without them
-// the kernel takes 76 (119 with phasors) instead of 199 (232) registers and more blocks run at a time:
-// the full-volume energy of the 64^3 cube measured 6.2 us against 25.5, the flux and three-frequency
-// phasor planes of 400x400x200 13.5 against 17.2.
-template <bool CX, bool PH, bool HALO>
+// HALO: the launch has a detector that needs_halo. Without one the kernel takes 76 instead of 199
+// registers and more blocks run at a time: the full-volume energy of the 64^3 cube measured 6.2 us
+// against 25.5.
+template <bool CX, bool HALO>
 __device__ __forceinline__ void detector_tile(const StepStatic& P, const DetK& K, const DetDyn& D, int n, int slot,
                                               int blk, int nblk) {
   // CX: a complex-field plan (D.Ei set): e, hp, h view the real part and e2, hp2, h2 the imaginary one
@@ -326,25 +405,16 @@ __device__ __forceinline__ void detector_tile(const StepStatic& P, const DetK& K
     return;
   }
   const int nv = reduced_values(K);
+  if (K.kind == FDTDX_DET_PHASOR && !nv) {
+    phasor_tile<CX, HALO>(P, K, D, n, blk, nblk, e, hp, h, e2, hp2, h2);
+    return;
+  }
   double acc[kDetMaxValues] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   for (long long q = (long long)blk * kBlock + threadIdx.x; q < K.cells; q += (long long)nblk * kBlock) {
     int i, j, k;
     region_cell(K, q, i, j, k);
     const long long o = ((long long)i * P.ny + j) * P.nz + k;
     float Ei[3], Hi[3], Ej[3] = {0.f, 0.f, 0.f}, Hj[3] = {0.f, 0.f, 0.f};
-    // per-cell phasors: the state words of up to three frequencies are loaded before any is updated,
-    // those of the first three ahead of the field reads, so that all are in flight together (a plane
-    // detector launches too few waves to hide them one by one)
-    float2 old[3][6];
-    auto load_phasor = [&](int f0) {
-      const float2* st = (const float2*)D.state;
-#pragma unroll
-      for (int df = 0; df < 3; ++df)
-#pragma unroll
-        for (int c = 0; c < 6; ++c)
-          if (f0 + df < K.nfreq && c < K.ncomp) old[df][c] = st[((long long)(f0 + df) * K.ncomp + c) * K.cells + q];
-    };
-    if (PH && K.kind == FDTDX_DET_PHASOR && !nv) load_phasor(0);
     if (K.exact) {
       interp<HALO>(P, e, hp, h, i, j, k, Ei, Hi);
       if (cx) interp<HALO>(P, e2, hp2, h2, i, j, k, Ej, Hj);
@@ -382,43 +452,10 @@ __device__ __forceinline__ void detector_tile(const StepStatic& P, const DetK& K
         if (nv) acc[t] += (double)(pf * K.weight);
         else ((float*)D.state)[((long long)slot * na + t) * K.cells + q] = pf;
       }
-    } else if (nv) {  // reduced PHASOR: the phase factor is uniform over the box, so sum EH first
+    } else {  // reduced PHASOR: the phase factor is uniform over the box, so sum EH first
       for (int c = 0; c < K.ncomp; ++c) acc[c] += (double)pick6(K.comps[c], Ei, Hi);
       if (cx)  // the imaginary parts' sums follow the real parts'
         for (int c = 0; c < K.ncomp; ++c) acc[K.ncomp + c] += (double)pick6(K.comps[c], Ej, Hj);
-    } else if constexpr (PH) {  // PHASOR (phasor.py:190-235): state += EH * exp(i w t) * scale * window
-      float2* st = (float2*)D.state;
-      const float w = K.window[n];
-      float v[6], vi[6];
-#pragma unroll
-      for (int c = 0; c < 6; ++c) {
-        v[c] = c < K.ncomp ? pick6(K.comps[c], Ei, Hi) : 0.f;
-        vi[c] = c < K.ncomp ? pick6(K.comps[c], Ej, Hj) : 0.f;
-      }
-      for (int f0 = 0; f0 < K.nfreq; f0 += 3) {
-        if (f0) load_phasor(f0);
-#pragma unroll
-        for (int df = 0; df < 3; ++df) {
-          const int f = f0 + df;
-          if (f >= K.nfreq) break;
-          const float cs = K.cos_t[(long long)f * P.T + n];
-          const float sn = K.sin_t[(long long)f * P.T + n];
-#pragma unroll
-          for (int c = 0; c < 6; ++c) {
-            if (c >= K.ncomp) break;
-            float re = ((v[c] * cs) * K.scale) * w;
-            float im = ((v[c] * sn) * K.scale) * w;
-            if (cx) {  // (v + i vi)(cos + i sin)
-              re = re - ((vi[c] * sn) * K.scale) * w;
-              im = ((vi[c] * cs) * K.scale) * w + im;
-            }
-            float2 s = old[df][c];
-            if (K.sign < 0.f) { s.x = s.x - re; s.y = s.y - im; }
-            else { s.x = s.x + re; s.y = s.y + im; }
-            st[((long long)f * K.ncomp + c) * K.cells + q] = s;
-          }
-        }
-      }
     }
   }
   for (int v = 0; v < kDetMaxValues; ++v) {  // nv is uniform over the block
@@ -498,7 +535,7 @@ __device__ __forceinline__ float reduce_finalize_tile(const StepStatic& P, const
 template <bool CX>
 __global__ __launch_bounds__(kBlock) void k_detector(const StepStatic* __restrict__ Pp, const DetK K, const DetDyn D) {
   const StepStatic& P = as_const(Pp);
-  detector_tile<CX, true, true>(P, K, D, D.n, D.slot, blockIdx.x, gridDim.x);
+  detector_tile<CX, true>(P, K, D, D.n, D.slot, blockIdx.x, gridDim.x);
 }
 
 __global__ __launch_bounds__(kBlock) void k_reduce_finalize(const StepStatic* __restrict__ Pp, const DetK K, const double* partial,
@@ -509,7 +546,7 @@ __global__ __launch_bounds__(kBlock) void k_reduce_finalize(const StepStatic* __
 
 static_assert(2 * sizeof(void*) + sizeof(DetGroup) <= 4096, "grouped detector kernel arguments exceed 4 KB");
 
-template <bool CX, bool PH, bool HALO>
+template <bool CX, bool HALO>
 __global__ __launch_bounds__(kBlock) void k_detector_group(const StepStatic* __restrict__ Pp, const DetK* __restrict__ Kd,
                                                            const DetGroup G) {
   const StepStatic& P = as_const(Pp);
@@ -517,7 +554,7 @@ __global__ __launch_bounds__(kBlock) void k_detector_group(const StepStatic* __r
   while (a + 1 < G.count && (int)blockIdx.x >= G.start[a + 1]) ++a;
   const DetK& K = Kd[G.q[a]];
   const DetDyn& D = G.dd[a];
-  detector_tile<CX, PH, HALO>(P, K, D, D.n, G.slot[a], (int)blockIdx.x - G.start[a], G.start[a + 1] - G.start[a]);
+  detector_tile<CX, HALO>(P, K, D, D.n, G.slot[a], (int)blockIdx.x - G.start[a], G.start[a + 1] - G.start[a]);
 }
 
 __global__ __launch_bounds__(kBlock) void k_finalize_group(const StepStatic* __restrict__ Pp, const DetK* __restrict__ Kd,
@@ -560,7 +597,7 @@ hipError_t launch_finalize_ring(const StepStatic& P, const DetK* Kdev, const Det
 // Batch detectors: the blocks of every (entry, detector) pair are concatenated; a persistent grid
 // strides over them. Each pair keeps the block count of the single-solve launch, so its partial
 // sums, and with them the reduced values, are bit-identical to a solve run alone.
-template <bool PH, bool HALO>
+template <bool HALO>
 __global__ __launch_bounds__(kBlock) void k_batch_detector(const BatchTable* __restrict__ Bp,
                                                            const int* __restrict__ base, int r) {
   const BatchTable& B = as_const(Bp);
@@ -581,7 +618,7 @@ __global__ __launch_bounds__(kBlock) void k_batch_detector(const BatchTable* __r
     if (K.kind == FDTDX_DET_PHASOR) slot = 0;
     DetDyn D = I.dd[q];
     D.partial += (long long)(r % kDetRing) * I.ndet * kDetMaxValues * kDetMaxBlocks;
-    detector_tile<false, PH, HALO>(I.P, K, D, n, slot, b, I.det_nb[q]);
+    detector_tile<false, HALO>(I.P, K, D, n, slot, b, I.det_nb[q]);
   }
 }
 
@@ -627,8 +664,7 @@ __global__ __launch_bounds__(kBlock) void k_batch_finalize(const BatchTable* __r
 }
 
 hipError_t launch_batch_detectors(const BatchTable* tab, const int* base, int r, int mode, int grid, hipStream_t s) {
-  const auto f = mode & 1 ? (mode & 2 ? k_batch_detector<true, true> : k_batch_detector<true, false>)
-                          : (mode & 2 ? k_batch_detector<false, true> : k_batch_detector<false, false>);
+  const auto f = mode & 1 ? k_batch_detector<true> : k_batch_detector<false>;
   hipLaunchKernelGGL(f, dim3(grid), dim3(kBlock), 0, s, tab, base, r);
   return hipGetLastError();
 }
@@ -652,9 +688,8 @@ hipError_t launch_detector_group(const StepStatic& P, const DetK* Kdev, const De
   const dim3 g((unsigned)G.start[G.count]);
   using GroupKernel = void (*)(const StepStatic*, const DetK*, const DetGroup);
   const bool hl = G.halo != 0;
-  const GroupKernel f = G.dd[0].Ei ? (hl ? k_detector_group<true, true, true> : k_detector_group<true, true, false>)
-                        : G.phasor ? (hl ? k_detector_group<false, true, true> : k_detector_group<false, true, false>)
-                                   : (hl ? k_detector_group<false, false, true> : k_detector_group<false, false, false>);
+  const GroupKernel f = G.dd[0].Ei ? (hl ? k_detector_group<true, true> : k_detector_group<true, false>)
+                                   : (hl ? k_detector_group<false, true> : k_detector_group<false, false>);
   hipLaunchKernelGGL(f, g, dim3(kBlock), 0, s, P.self, Kdev, G);
   if (G.nfin > 0) hipLaunchKernelGGL(k_finalize_group, dim3(G.nfin), dim3(kBlock), 0, s, P.self, Kdev, G);
   return hipGetLastError();

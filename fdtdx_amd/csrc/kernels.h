@@ -44,7 +44,7 @@ struct DetDyn {
   const float* Hprevi;
 };
 
-constexpr int kDetMaxBlocks = 1024;  // blocks of one detector launch (detector_blocks)
+constexpr int kDetMaxBlocks = 1024;  // blocks of a summing detector's launch (detector_blocks)
 constexpr int kDetGroup = 8;         // detectors of one grouped launch (the kernel arguments stay below 4 KB)
 
 // The detectors updated at one step, in one launch: detector a of the group is entry q[a] of the
@@ -54,7 +54,6 @@ constexpr int kDetGroup = 8;         // detectors of one grouped launch (the ker
 // which then also finalizes the accumulating detectors that follow it.
 struct DetGroup {
   int count, nfin;
-  int phasor;  // some detector of the group keeps per-cell phasors
   int halo;    // some detector of the group needs_halo
   int q[kDetGroup];
   int slot[kDetGroup];
@@ -62,10 +61,12 @@ struct DetGroup {
   int fin[kDetGroup];
   DetDyn dd[kDetGroup];
 };
-// Blocks of one detector's launch.
+// Blocks of one detector's launch: a lane per cell, per cell and component for per-cell phasors.
 __host__ __device__ inline int detector_blocks(const DetK& K) {
-  const long long b = (K.cells + kBlock - 1) / kBlock;
-  return (int)(b > kDetMaxBlocks ? kDetMaxBlocks : (b < 1 ? 1 : b));
+  const bool phasor = K.kind == FDTDX_DET_PHASOR && !K.reduce;  // leaves no partial sums
+  const long long b = ((phasor ? K.cells * K.ncomp : K.cells) + kBlock - 1) / kBlock;
+  const long long most = phasor ? 4 * kDetMaxBlocks : kDetMaxBlocks;
+  return (int)(b > most ? most : (b < 1 ? 1 : b));
 }
 
 // The interpolation stencil of some cell of the detector reads beyond a periodic face or below a

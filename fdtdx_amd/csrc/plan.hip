@@ -1023,11 +1023,11 @@ static int forward_impl(const fdtdx_plan* p, const fdtdx_buffers* b, int32_t t0,
     // the detectors of step n in grouped launches of up to kDetGroup (a chain of accumulating
     // detectors stays in one group); one finalize launch per group for the reduced values
     DetGroup G;
-    G.count = G.nfin = G.phasor = G.halo = 0;
+    G.count = G.nfin = G.halo = 0;
     G.start[0] = 0;
     auto flush = [&]() -> int {
       const hipError_t e = launch_detector_group(p->P, p->det_dev, G, s);
-      G.count = G.nfin = G.phasor = G.halo = 0;
+      G.count = G.nfin = G.halo = 0;
       return e == hipSuccess ? FDTDX_OK : fail(FDTDX_EHIP, "detector launch: %s", hipGetErrorString(e));
     };
     for (int q = 0; q < p->ndet; ++q) {
@@ -1043,7 +1043,6 @@ static int forward_impl(const fdtdx_plan* p, const fdtdx_buffers* b, int32_t t0,
         const int tail = G.count - h;
         DetGroup R;
         R.count = 0; R.nfin = 0; R.start[0] = 0;
-        R.phasor = 0;  // a chain of accumulating detectors sums energies or fluxes
         R.halo = G.halo;
         for (int t = 0; t < tail; ++t) {
           const int a = h + t;
@@ -1078,7 +1077,6 @@ static int forward_impl(const fdtdx_plan* p, const fdtdx_buffers* b, int32_t t0,
       G.slot[a] = dd.slot;
       G.start[a + 1] = G.start[a] + detector_blocks(p->det[q]);
       if (reduced_values(p->det[q]) && !p->det[q].accum && !deferred(q)) G.fin[G.nfin++] = a;
-      if (p->det[q].kind == FDTDX_DET_PHASOR && !p->det[q].reduce) G.phasor = 1;
       if (needs_halo(p->P, p->det[q])) G.halo = 1;
       G.count = a + 1;
     }
@@ -1420,12 +1418,12 @@ static int batch_upload(fdtdx_batch* b, hipStream_t s) {
   return FDTDX_OK;
 }
 
-// det: -1 no detectors, else the launch mode of launch_batch_detectors (bits 0, 1) and bit 2: some sums.
+// det: -1 no detectors, else bit 0: some detector needs_halo, bit 1: some sums.
 static int batch_chunk(fdtdx_batch* b, int steps, int det, hipStream_t s) {
   for (int r = 0; r < steps; ++r) {
     HIP_TRY(launch_batch_sweeps(b->dtab, b->dbase, r, b->ec, b->mc, b->grid, s));
     if (det >= 0) HIP_TRY(launch_batch_detectors(b->dtab, b->dbase, r, det, b->det_grid, s));
-    if (det >= 0 && (det & 4) && ((r + 1) % kDetRing == 0 || r + 1 == steps)) {
+    if (det >= 0 && (det & 2) && ((r + 1) % kDetRing == 0 || r + 1 == steps)) {
       const int r0 = r / kDetRing * kDetRing;
       HIP_TRY(launch_batch_finalize(b->dtab, b->dbase, r0, r + 1 - r0, s));
     }
@@ -1452,9 +1450,8 @@ int fdtdx_batch_advance(fdtdx_batch* b, int32_t steps, int32_t use_graph, void* 
     if (S.plan->ndet > 0 && det < 0) det = 0;
     for (int q = 0; q < S.plan->ndet; ++q) {
       const DetK& K = S.plan->det[q];
-      if (K.kind == FDTDX_DET_PHASOR && !K.reduce) det |= 1;
-      if (needs_halo(S.plan->P, K)) det |= 2;
-      if (reduced_values(K)) det |= 4;
+      if (needs_halo(S.plan->P, K)) det |= 1;
+      if (reduced_values(K)) det |= 2;
     }
     if (S.pending_set) {
       set.slot[set.count] = sl;
