@@ -9,7 +9,7 @@ FDTD time step (E sweep, H sweep, detectors) of that grid; the timed region runs
 with all state resident in HBM.
 
 Prints one JSON line: Mcell-updates/s (median and best of --reps repetitions), the HBM roofline of
-the dominant kernel (the E sweep, k_update_E4, with k_update_E4s for ADE tiles, timed with HIP events on
+the dominant kernel (the E sweep, k_update_E4, timed with HIP events on
 the engine's stream), a CPU baseline (the oracle's C/OpenMP forward loop on every host thread
 OMP_NUM_THREADS allows, over a bounded sample of steps), the 256^3 dispersive forward, the seconds
 per gradient of the 200x200x100 differentiation case, and served-vs-serial throughput with p50/p99
@@ -298,10 +298,8 @@ def time_forward(spec, steps, warmup, reps):
     e_b, h_b, det_b, n_slab = algorithmic_bytes(solve.spec, snapshot_cells(solve.spec))
     sched = {0: "one cell per lane", 1: "four z cells per lane (dwordx4)", 2: "fused", 3: "march"}[solve.plan.schedule]
     kname = ("k_update_E4", "k_update_H4") if solve.plan.schedule == 1 else ("k_update_E", "k_update_H")
-    # the E half-step of tiles with ADE poles runs in a second launch (k_update_E4s); the HIP events
-    # bracket both launches of a sweep
-    sweep = {"k_update_E4": "E sweep: k_update_E4" + (" + k_update_E4s" if solve.spec["ade"] else ""),
-             "k_update_H4": "H sweep: k_update_H4"}
+    # the HIP events bracket all launches of a sweep
+    sweep = {"k_update_E4": "E sweep: k_update_E4", "k_update_H4": "H sweep: k_update_H4"}
     e_launch, h_launch = e_ms / ksteps, h_ms / ksteps
     wl = "x".join(str(v) for v in spec["shape"])
     roof = {
