@@ -569,6 +569,10 @@ static int plan_create(const fdtdx_plan_desc* d, fdtdx_plan** out) {
       // conductivity: their tiles run one cell per lane (200x200x101: 101 us per step against 93 with
       // every tile one cell per lane; 128x120x100, 56 against 57, has them listed)
       if ((P.nz % 4 || pl->cplx) && (!(xyz && zq) || (P.nade && P.loss[0].comps))) quad_ok = false;
+      // Poles in a grid of few wavefronts: one cell per lane (a quad's chain of pole loads is four cells
+      // long and little runs beside it). us per step, one cell / quads: 64x56x60 20 / 27, 88x80x84
+      // 29 / 32, 100x95x101 37 / 37; the other way from about two million cells (200x200x101 89 / 85).
+      if (P.nade && P.N < (1ll << 20) && !(qenv && strcmp(qenv, "quad") == 0)) quad_ok = false;
       P.cax = quad_ok && xyz && zq ? 1 : 0;
       bool gap = true;
       for (int a = 0; a < 3; ++a)
