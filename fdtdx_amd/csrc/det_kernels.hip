@@ -622,8 +622,8 @@ __global__ __launch_bounds__(kBlock) void k_batch_detector(const BatchTable* __r
   }
 }
 
-// The sums of chunk step r0 + blockIdx.y (reduced phasors, which add up over the steps: of all the
-// launch's steps in order, by the blocks of blockIdx.y = 0).
+// The sums of chunk step r0 + blockIdx.y (reduced phasors, which add up over the steps, and detectors whose
+// steps share slots: of all the launch's steps in order, by the blocks of blockIdx.y = 0).
 __global__ __launch_bounds__(kBlock) void k_batch_finalize(const BatchTable* __restrict__ Bp,
                                                            const int* __restrict__ base, int r0) {
   const BatchTable& B = as_const(Bp);
@@ -639,9 +639,9 @@ __global__ __launch_bounds__(kBlock) void k_batch_finalize(const BatchTable* __r
       if (reduced_values(I.det[q]) && !I.det[q].accum && want-- == 0) break;
     if (q >= I.ndet) continue;
     const DetK& K = I.det[q];
-    const bool ph = K.kind == FDTDX_DET_PHASOR;
-    if (ph && blockIdx.y) continue;
-    const int y0 = ph ? 0 : (int)blockIdx.y, y1 = ph ? (int)gridDim.y : y0 + 1;
+    const bool ph = K.kind == FDTDX_DET_PHASOR, ordered = ph || K.ordered;
+    if (ordered && blockIdx.y) continue;
+    const int y0 = ordered ? 0 : (int)blockIdx.y, y1 = ordered ? (int)gridDim.y : y0 + 1;
     for (int y = y0; y < y1; ++y) {
       const int n = base[I.slot] + r0 + y;
       if (n >= I.stop) break;

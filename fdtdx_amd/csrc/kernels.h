@@ -1,5 +1,7 @@
 // Launchers shared between the kernel translation units and the C-ABI in plan.hip.
 #pragma once
+#include <map>
+
 #include "engine_common.h"
 
 namespace fdtdx {
@@ -24,6 +26,7 @@ struct DetK {
   const float* window; // device T
   const int* tti;      // device time_to_idx (T): record slot of step n, or -1
   int cplx;            // complex fields: a reduced phasor sums the real, then the imaginary parts
+  int ordered;         // its sums are finalized step by step, in order (slots_repeat)
 };
 
 struct DetDyn {
@@ -79,8 +82,24 @@ inline bool needs_halo(const StepStatic& P, const DetK& K) {
 }
 
 // Deferred sums (k_finalize_ring): the partial sums of up to kDetRing steps, and the chain heads
-// (reducing energy, flux and field detectors that do not accumulate).
+// (reducing energy, flux and field detectors that do not accumulate). Their steps are finalized by
+// concurrent blocks, so detectors whose slots_repeat are left out.
 constexpr int kDetRing = 16;
+
+// True when two steps less than `window` apart share a record slot (time_to_idx tti of T steps, -1: off).
+// A launch that finalizes `window` steps at a time must then store them in step order: the last one's value
+// stays in the slot, and the faces accumulating into it belong to one step.
+inline bool slots_repeat(const int32_t* tti, int T, int window) {
+  std::map<int32_t, int> last;
+  for (int n = 0; n < T; ++n) {
+    if (tti[n] < 0) continue;
+    const auto it = last.find(tti[n]);
+    if (it != last.end() && n - it->second < window) return true;
+    last[tti[n]] = n;
+  }
+  return false;
+}
+
 struct DetRing {
   int n0, ndet, count;
   int q[FDTDX_MAX_DETECTORS];

@@ -417,6 +417,7 @@ static int plan_create(const fdtdx_plan_desc* d, fdtdx_plan** out) {
                      reduced_values(pl->det[q - 1]) == reduced_values(k) && pl->tti[q - 1] == pl->tti[q]))
       return bail(fail(FDTDX_EINVAL, "detector %d: accumulate needs a reducing energy or flux detector after one "
                                      "of the same kind, value count and time_to_idx", q));
+    k.ordered = slots_repeat(c.time_to_idx, P.T, kDetRing) ? 1 : 0;
     if ((rc = pl->upload((const int*)c.time_to_idx, (size_t)P.T, &k.tti))) return bail(rc);
     if (c.kind == FDTDX_DET_PHASOR) {
       if (k.nfreq < 1) return bail(fail(FDTDX_EINVAL, "detector %d: no frequencies", q));
@@ -956,21 +957,22 @@ static int forward_impl(const fdtdx_plan* p, const fdtdx_buffers* b, int32_t t0,
   float* Eb[2] = {b->E, p->use_fused ? (float*)(ws + p->ws_Ealt) : b->E};
   float* Hb[2] = {b->H, p->use_fused ? (float*)(ws + p->ws_Halt) : b->H};
   float* Pb[2] = {b->psi, p->use_fused ? (float*)(ws + p->ws_psialt) : b->psi};
-  // sums of energy, flux and field detectors: finalized for kDetRing steps at a time
+  // sums of energy, flux and field detectors: finalized for kDetRing steps at a time, unless steps of one
+  // launch would share a slot
   DetRing F;
   memset(&F, 0, sizeof(F));
   ring = ring && p->ws_ring;
+  auto deferred = [&](int q) { return ring && p->det[q].kind != FDTDX_DET_PHASOR && !p->det[q].ordered; };
   if (ring) {
     F.n0 = t0;
     F.ndet = p->ndet;
     F.partial = (const double*)(ws + p->ws_ring);
     for (int q = 0; q < p->ndet; ++q) {
       F.state[q] = b->detector_state[q];
-      if (reduced_values(p->det[q]) && p->det[q].kind != FDTDX_DET_PHASOR && !p->det[q].accum && !p->det[q].inv)
+      if (reduced_values(p->det[q]) && deferred(q) && !p->det[q].accum && !p->det[q].inv)
         F.q[F.count++] = q;
     }
   }
-  auto deferred = [&](int q) { return ring && p->det[q].kind != FDTDX_DET_PHASOR; };
   for (int n = t0; n < t1; ++n) {
     bool any = false;
     for (int q = 0; q < p->ndet; ++q) any = any || p->tti[q][n] >= 0;

@@ -123,7 +123,8 @@ enum { FDTDX_DET_ENERGY = 0, FDTDX_DET_FIELD = 1, FDTDX_DET_FLUX = 2, FDTDX_DET_
  *         (re, im pairs)
  * reduce_volume sums energy and flux over the box with the weight, and averages field and phasor
  * values over it (the volume-weighted mean of detector.py:95-109 on a uniform grid).
- * time_to_idx[n] is the record slot of step n or -1 when the detector is off. */
+ * time_to_idx[n] is the record slot of step n or -1 when the detector is off; where steps share a slot,
+ * the last of them leaves its value there (PHASOR ignores the slot). */
 typedef struct fdtdx_detector_desc {
   int32_t kind;
   int32_t lo[3], hi[3];

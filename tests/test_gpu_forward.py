@@ -544,6 +544,67 @@ def test_deferred_detector_sums_equal_a_launch_per_step(T, halo):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("slots", ["last", "pairs", "wrapped"])
+def test_detector_steps_that_share_a_slot_are_stored_in_order(slots):
+    """Energy, flux, reduced field and a closed surface's accumulating faces whose time_to_idx maps several
+    steps to one slot (keep the last value; two steps per slot; a ring of 7 slots, some steps off): one call and
+    one batch leave what step by step calls leave, the last step's values of each slot."""
+    import torch
+
+    from fdtdx_amd import engine
+    from fdtdx_amd import fdtd as F
+    import scenarios
+
+    n, T = 20, 41
+    spec = W.scenario_c1(T=T, n=n, pml=4, cube=4)
+    spec["sources"][0]["profile"] = dict(kind="single", frequency=2e14, phase_shift=0.3)
+    spec["detectors"] = [
+        dict(name="energy", kind="energy", slc=((0, n),) * 3, reduce_volume=True),
+        dict(name="flux", kind="flux", slc=((14, 15), (0, n), (4, 16)), axis=0, reduce_volume=True),
+        dict(name="box", kind="closed_flux", slc=((5, 15), (5, 15), (5, 15))),
+        dict(name="field", kind="field", slc=((6, 9), (5, 12), (4, 9)), components=("Ez", "Hx"), reduce_volume=True),
+    ]
+    step = np.arange(T)
+    tti = {"last": 0 * step, "pairs": step // 2, "wrapped": np.where(step % 5 == 3, -1, step % 7)}[slots]
+
+    def solve(shared=True):
+        objects, arrays, params, config = scenarios.build(spec)
+        s = F.Solve(objects, config, arrays)
+        if shared:
+            low = F.lower(objects, config, arrays)
+            for d in low["detectors"]:
+                d["time_to_idx"] = tti.astype(np.int32)
+            s.plan = engine.Plan(low)
+        arrays.reset()
+        return s
+
+    def states(s):
+        torch.cuda.synchronize()
+        return [t.cpu().numpy() for t in s.state_tensors()]
+
+    own, whole, stepwise, batched = solve(False), solve(), solve(), solve()
+    print(f"slots {slots}", flush=True)
+    own.forward(0, T)  # a slot per step
+    whole.forward(0, T)
+    for t in range(T):
+        stepwise.forward(t, t + 1)
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    batch = engine.Batch(1, 0)
+    batch.attach(0, batched.plan, batched.buffers(), batched._keep, 0, T)
+    for _ in range(2):
+        batch.advance(21, engine.c_void_p(stream.cuda_stream))
+    stream.synchronize()
+    batch.close()
+    last = {int(s): t for t, s in enumerate(tti) if s >= 0}  # the last step of each slot
+    ref = states(own)
+    assert np.abs(ref[0]).max() > 0 and np.abs(ref[2]).max() > 0
+    for got in (stepwise, whole, batched):
+        for a, r in zip(states(got), ref):
+            for slot, t in last.items():
+                assert np.array_equal(a[slot], r[t]), (slot, t)
+
+
 def _ragged_cases():
     """Rows of nz % 4 != 0 cells: the last quad of a row repeats cells of the quad before it."""
     c1 = W.scenario_c1(T=60, n=29, pml=5, cube=6)                                  # nz % 4 = 1

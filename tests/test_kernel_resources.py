@@ -69,6 +69,22 @@ def test_forward_sweeps_keep_full_occupancy(resources):
         assert v["VGPRs"] <= 96 and v["Occupancy [waves/SIMD]"] >= 5, (k, v)
 
 
+def test_detector_slots_that_repeat(tmp_path):
+    """Which detectors may have the sums of 16 steps finalized at once: those none of whose steps less
+    than 16 apart share a record slot (-1: off)."""
+    from fdtdx_amd import build as B
+
+    exe = str(tmp_path / "slots")
+    r = subprocess.run([B.hipcc(), "-std=c++17", "-O1", "-I", os.path.join(ROOT, "include"), "-o", exe,
+                        os.path.join(ROOT, "tests", "det_slots_harness.cpp")], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    for tti, want in (([], 0), ([-1] * 40, 0), (list(range(40)), 0), ([3, 3], 1), ([0] + [-1] * 14 + [0], 1),
+                      ([0] + [-1] * 15 + [0], 0), ([n // 3 for n in range(20)], 1),
+                      ([n % 16 for n in range(64)], 0), ([n % 15 for n in range(64)], 1)):
+        out = subprocess.run([exe, "16", *map(str, tti)], capture_output=True, text=True)
+        assert int(out.stdout) == want, tti
+
+
 @pytest.mark.parametrize("ny,nz,zlo,zhi,zg", [(400, 200, 12, 188, 32), (45, 70, 5, 65, 7), (30, 24, 0, 19, 32),
                                               (17, 33, 6, 33, 4), (20, 16, 0, 16, 20)])
 def test_forward_plane_order_is_a_permutation(ny, nz, zlo, zhi, zg, tmp_path):
