@@ -134,7 +134,8 @@ struct StepStatic {
   const uint32_t* vec_mask;  // per quad tile, as fwd_mask
   long long vnslow;          // quad tiles with poles and conductivity (k_update_E4s) ...
   const int* vslow;          // ... and their indices
-  uint32_t vpoint[2];        // the mask bits of E sources and PEC faces, of H sources and PMC faces
+  uint32_t vpoint[2];        // the mask bits of E sources, of H sources ...
+  uint32_t vwall[2];         // ... of PEC faces, of PMC faces
   // Per-axis CPML (acax = 1): every slab spans its face, at most one slab per side of an axis and
   // no two overlapping, and the x slabs before the y slabs before the z slabs in object order (the
   // order in which the corrections are added); the one-cell reverse and adjoint sweeps then find

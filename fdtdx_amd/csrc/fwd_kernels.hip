@@ -734,6 +734,7 @@ __device__ __forceinline__ void quad_E(const StepStatic& P, const StepDyn& D, in
   const f4v inv[3] = {iex, iey, iez};
   if (X && ((m >> kMaskLoss) & 1u)) quad_loss<0>(P, i, j, k0, inv, eo, t, en);
   if (ADE && (m & kAdeBits)) quad_ade<EC>(P, D.ade, D.ie + o, m, n, i, j, k0, sm, eo, en);
+  if (m & P.vwall[0]) quad_walls<0>(P, m, i, j, k0, en);
   st4m<RAG>(Ex + o, en[0], sm);
   st4m<RAG>(Ey + o, en[1], sm);
   st4m<RAG>(Ez + o, en[2], sm);
@@ -816,6 +817,7 @@ __device__ __forceinline__ void quad_H(const StepStatic& P, const StepDyn& D, in
     const f4v inv[3] = {imx, imy, imz};
     quad_loss<1>(P, i, j, k0, inv, ho, t, hn);
   }
+  if (m & P.vwall[1]) quad_walls<1>(P, m, i, j, k0, hn);
   st4m<RAG>(Hx + o, hn[0], sm);
   st4m<RAG>(Hy + o, hn[1], sm);
   st4m<RAG>(Hz + o, hn[2], sm);

@@ -678,7 +678,8 @@ static int plan_create(const fdtdx_plan_desc* d, fdtdx_plan** out) {
       if ((rc = pl->upload(vm.data(), vm.size(), &P.vec_mask))) return bail(rc);
       P.vpoint[0] = P.vpoint[1] = 0u;
       for (int q = 0; q < P.nsrc; ++q) P.vpoint[P.src[q].field] |= 1u << (kMaskSrc + q);
-      for (int w = 0; w < P.nwall; ++w) P.vpoint[P.wall[w].kind == FDTDX_WALL_PEC ? 0 : 1] |= 1u << (kMaskWall + w);
+      P.vwall[0] = P.vwall[1] = 0u;
+      for (int w = 0; w < P.nwall; ++w) P.vwall[P.wall[w].kind == FDTDX_WALL_PEC ? 0 : 1] |= 1u << (kMaskWall + w);
       std::vector<int> slow;  // tiles with poles and conductivity
       const uint32_t ade = ((1u << FDTDX_MAX_ADE) - 1u) << kMaskAde;
       if (P.nade && P.loss[0].comps)

@@ -361,7 +361,27 @@ __device__ __forceinline__ void quad_ade(const StepStatic& P, float* ade, const 
   }
 }
 
-// Sources and conducting faces of field W (0: E, PEC; 1: H, PMC) over a quad, after its update has
+// Conducting faces of field W (0: E, PEC; 1: H, PMC) in the updated quad f (apply_walls). In registers
+// ahead of the store: a face normal to z meets the end of every row, where the rounds of quad_points, which
+// held the faces before, cost more than the sweep itself. us per step of a grid between two PEC faces normal
+// to z, quad_points / here / one cell per lane: 800x800x20 240 / 179 / 190, 400x400x8 26.6 / 20.3 / 21.6,
+// 300x300x150 (four faces, y and z) 225 / 207 / 216.
+template <int W>
+__device__ __forceinline__ void quad_walls(const StepStatic& P, uint32_t m, int i, int j, int k0, f4v* f) {
+#pragma unroll 1
+  for (uint32_t mm = (m & P.vwall[W]) >> kMaskWall; mm; mm &= mm - 1u) {
+    const WallK& w = P.wall[__builtin_ctz(mm)];
+    const int d = w.index - (w.axis == 0 ? i : (w.axis == 1 ? j : k0));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const bool on = w.axis == 2 ? d == e : d == 0;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) f[a][e] = on && w.axis != a ? 0.f : f[a][e];
+    }
+  }
+}
+
+// Sources of field W (0: E; 1: H) over a quad, after its update (with quad_walls) has
 // been stored: the cells e >= sm are read back, changed and stored one by one (rolled, so that the
 // few quads that hold one cost the others no registers). m: the tile's mask. Before, such tiles
 // ran one cell per lane in launches of their own: 6 to 9 us each whatever the grid, against no
@@ -377,11 +397,6 @@ __device__ __forceinline__ void quad_points(const StepStatic& P, uint32_t m, con
     const SrcK& sr = P.src[__builtin_ctz(mm)];
     hit = hit || (sr.field == W && i >= sr.lo[0] && i < sr.hi[0] && j >= sr.lo[1] && j < sr.hi[1] &&
                   k0 + 3 >= sr.lo[2] && k0 < sr.hi[2]);
-  }
-  for (uint32_t mm = (m >> kMaskWall) & ((1u << P.nwall) - 1u); mm; mm &= mm - 1u) {
-    const WallK& w = P.wall[__builtin_ctz(mm)];
-    const int c = w.axis == 0 ? i : (w.axis == 1 ? j : k0);
-    hit = hit || (w.kind == (W ? FDTDX_WALL_PMC : FDTDX_WALL_PEC) && w.index >= c && w.index <= (w.axis == 2 ? c + 3 : c));
   }
   if (!hit) return;
   float* p = F + o;

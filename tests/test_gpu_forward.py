@@ -544,6 +544,43 @@ def test_deferred_detector_sums_equal_a_launch_per_step(T, halo):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("nz", [24, 25, 26, 27])
+@pytest.mark.parametrize("kind", ["pec", "pmc"])
+def test_conducting_faces_in_quads_equal_one_cell_sweeps_bitwise(nz, kind, monkeypatch):
+    """Conducting faces on all three axes inside the quad sweeps against one cell per lane, with sources in the
+    face cells: a plane wave that spans the cross-section (E and H sources up to the y and z faces) and a dipole
+    tangential to the upper z face in its layer. Fields, psi, the interface record and the energy agree bit for
+    bit, and the tangential field of a face stays zero."""
+    import torch
+
+    from fdtdx_amd import fdtd as F
+    import scenarios
+
+    spec = W.scenario_c1(T=45, n=24, pml=4, cube=6)
+    spec["shape"] = (24, 22, nz)
+    spec["boxes"] = [dict(slc=((8, 20), (5, 22), (9, nz)), eps=(2.0, 3.0, 4.0))]
+    spec["pml"] = dict(spec["pml"], types={f: kind for f in ("max_x", "min_y", "max_y", "min_z", "max_z")})
+    prof = dict(kind="single", frequency=2e14, phase_shift=0.3)
+    spec["sources"] = [dict(kind="plane", axis=0, index=7, direction="+", e_pol=(0, 1, 0), profile=prof),
+                       dict(kind="dipole", cell=(12, 11, nz - 1), polarization=0, profile=prof)]
+    spec["detectors"] = [dict(name="energy", kind="energy", slc=((0, 24), (0, 22), (0, nz)), reduce_volume=True)]
+    out = {}
+    for mode in ("two", "quad"):
+        _set_mode(monkeypatch, mode)
+        objects, arrays, params, config = scenarios.build(spec)
+        s = F.Solve(objects, config, arrays, record_steps=spec["T"])
+        assert s.plan.quad == (mode == "quad")
+        arrays.reset()
+        print(f"nz {nz} {kind} {mode}", flush=True)
+        s.forward(0, spec["T"], record=True)
+        torch.cuda.synchronize()
+        out[mode] = [t.cpu().numpy() for t in (arrays.fields.E, arrays.fields.H, arrays.psi, s.record, *s.det_tensors())]
+    f = out["quad"][0 if kind == "pec" else 1]
+    assert np.abs(f).max() > 0 and not f[:2, :, :, 0].any() and not f[:2, :, :, -1].any() and not f[0, :, 0].any()
+    for a, b in zip(out["quad"], out["two"]):
+        assert np.array_equal(a, b)
+
+
 @pytest.mark.parametrize("slots", ["last", "pairs", "wrapped"])
 def test_detector_steps_that_share_a_slot_are_stored_in_order(slots):
     """Energy, flux, reduced field and a closed surface's accumulating faces whose time_to_idx maps several
