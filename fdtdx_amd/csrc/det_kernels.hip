@@ -298,7 +298,14 @@ __device__ __forceinline__ void energy_mean_tile(const StepStatic& P, const DetK
   const int na = K.hi[K.axis] - K.lo[K.axis];
   const int d1 = K.hi[b1] - K.lo[b1];
   const long long pc = K.cells / na;
-  for (long long q = (long long)blk * kBlock + threadIdx.x; q < pc; q += (long long)nblk * kBlock) {
+  // The launch has a lane per cell of the box (detector_blocks) and few of them are plane cells, whose
+  // lanes read box cells one row apart (uncoalesced where the axis is z): bound by a CU's loads. One
+  // wavefront of a block takes plane cells where the blocks are enough, which spreads them over four times
+  // the CUs. Steps of 128^3 with the three means of a 64^3 box: 368 us with whole blocks (322 when the
+  // stencil's k + 1 loads still joined those of k), 142 so; 128x128x32 box 375 -> 223.
+  const int per = (long long)nblk * 64 >= pc ? 64 : kBlock;
+  if ((int)threadIdx.x >= per) return;
+  for (long long q = (long long)blk * per + threadIdx.x; q < pc; q += (long long)nblk * per) {
     const int u = (int)(q / d1), v = (int)(q - (long long)u * d1);
     int c[3];
     c[b0] = K.lo[b0] + u;

@@ -544,6 +544,34 @@ def test_deferred_detector_sums_equal_a_launch_per_step(T, halo):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("box", [((5, 8), (2, 22), (1, 22)), ((2, 22), (7, 11), (3, 22)), ((9, 10), (4, 13), (0, 24)),
+                                 ((0, 24), (0, 24), (0, 24))])
+def test_energy_slice_means_equal_the_means_of_per_cell_energies(box):
+    """The collapsed-axis means of a box (one wavefront of a block where a plane has at most a quarter of
+    the box's cells, whole blocks else) against the float64 sums, in order, of the per-cell energies."""
+    import torch
+
+    from fdtdx_amd import fdtd as F
+    import scenarios
+
+    spec = W.scenario_c1(T=30, n=24, pml=4, cube=6)
+    on = {"fixed_on_time_steps": [11, 29]}
+    spec["detectors"] = [dict(name="s", kind="energy", slc=box, as_slices=True, aggregate="mean", switch=on),
+                         dict(name="c", kind="energy", slc=box, switch=on)]
+    objects, arrays, params, config = scenarios.build(spec)
+    F.run_fdtd(arrays, objects, config)
+    torch.cuda.synchronize()
+    cells = arrays.detector_states["c"]["energy"].cpu().numpy()
+    assert cells.shape == (2, *(b - a for a, b in box)) and np.abs(cells[1]).max() > 0
+    got = arrays.detector_states["s"]
+    assert len(got) == 3
+    for a, plane in enumerate(("YZ Plane", "XZ Plane", "XY Plane")):
+        ref = np.zeros(np.delete(np.array(cells.shape), a + 1))
+        for t in range(cells.shape[a + 1]):
+            ref = ref + np.take(cells, t, a + 1).astype(np.float64)
+        assert np.array_equal(got[plane].cpu().numpy(), (ref / cells.shape[a + 1]).astype(np.float32)), plane
+
+
 @pytest.mark.parametrize("nz", [24, 25, 26, 27])
 @pytest.mark.parametrize("kind", ["pec", "pmc"])
 def test_conducting_faces_in_quads_equal_one_cell_sweeps_bitwise(nz, kind, monkeypatch):
