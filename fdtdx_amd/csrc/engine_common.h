@@ -117,7 +117,7 @@ struct StepStatic {
   // group's cells with zlo <= k < zhi (row by row), then its cells of the z-normal CPML slabs
   // (k < zlo or k >= zhi, row by row), so a wavefront runs the CPML code for all or none of its
   // lanes while both parts of a row are written close together in time. fwd_mask holds the tile
-  // masks of that order (null in plans with the per-axis quad sweeps). zlo = 0, zhi = nz is the plain
+  // masks of that order (null where only the per-axis quad sweeps run). zlo = 0, zhi = nz is the plain
   // row-major order.
   int zlo, zhi, zg;
   const uint32_t* fwd_mask;

@@ -78,6 +78,7 @@ struct fdtdx_plan {
   // single-pass paths (1: LDS-tiled fused kernel, 2: register-march kernel): tile configuration
   // and ping-pong copies of E, H and psi in the workspace
   int cplx = 0;                // complex fields: every field array holds the real, then the imaginary part
+  int alone_one = 0;           // the plan's quad sweeps run in batches only; alone it runs one cell per lane
   int use_fused = 0;
   FusedDyn fd;
   MarchDyn md;
@@ -99,6 +100,9 @@ struct fdtdx_plan {
     return FDTDX_OK;
   }
 };
+
+// Plans with poles of fewer cells run one cell per lane when alone (plan_create).
+constexpr long long kAlonePoles = 700000;
 
 static bool box_ok(const int32_t* lo, const int32_t* hi, const StepStatic& P) {
   const int n[3] = {P.nx, P.ny, P.nz};
@@ -570,10 +574,13 @@ static int plan_create(const fdtdx_plan_desc* d, fdtdx_plan** out) {
       // conductivity: their tiles run one cell per lane (200x200x101: 101 us per step against 93 with
       // every tile one cell per lane; 128x120x100, 56 against 57, has them listed)
       if ((P.nz % 4 || pl->cplx) && (!(xyz && zq) || (P.nade && P.loss[0].comps))) quad_ok = false;
-      // Poles in a grid of few wavefronts: one cell per lane (a quad's chain of pole loads is four cells
-      // long and little runs beside it). us per step, one cell / quads: 64x56x60 20 / 27, 88x80x84
-      // 29 / 32, 100x95x101 37 / 37; the other way from about two million cells (200x200x101 89 / 85).
-      if (P.nade && P.N < (1ll << 20) && !(qenv && strcmp(qenv, "quad") == 0)) quad_ok = false;
+      // Poles in a grid of few wavefronts, run alone: one cell per lane (a quad's chain of pole loads is four
+      // cells long and little runs beside it). us per step with a two-pole slab, one cell / quads: 48^3
+      // 16.1 / 20.4, 64x56x60 17.5 / 19.8, 80^3 22.2 / 23.7, 88^3 27.1 / 27.7; the other way from there (92^3
+      // 29.5 / 28.6, 100^3 32.6 / 28.6; with a 10^3 particle from 84^3, 21.7 / 21.5, 96^3 27.1 / 24.0).
+      // Complex fields have both parts in a launch and fewer launches with quads (24x24x36 25.3 / 21.6,
+      // 96x96x100 50 / 40), batches many solves in one (eight of 64^3 78 / 52, of 64^3 with the slab 80 / 68).
+      pl->alone_one = quad_ok && P.nade && P.N < kAlonePoles && !pl->cplx && !(qenv && strcmp(qenv, "quad") == 0);
       P.cax = quad_ok && xyz && zq ? 1 : 0;
       bool gap = true;
       for (int a = 0; a < 3; ++a)
@@ -597,8 +604,8 @@ static int plan_create(const fdtdx_plan_desc* d, fdtdx_plan** out) {
           x.cells = sl.cells; x.psi_off = sl.psi_off; x.coef = sl.coef;
         }
     }
-    // masks of the one-cell forward sweeps' tiles, which plans with the per-axis quad sweeps never run
-    if (!(quad_ok && P.cax)) {
+    // masks of the one-cell forward sweeps' tiles, where those may run
+    if (!(quad_ok && P.cax) || pl->alone_one) {
       std::vector<uint32_t> fm((size_t)P.nblocks, 0u);
       for (long long lb = 0; lb < P.nblocks; ++lb) {
         const int i = (int)(lb / P.bpp);
@@ -849,6 +856,9 @@ static StepDyn make_dyn(const fdtdx_plan* p, const fdtdx_buffers* b) {
 static int forward_impl(const fdtdx_plan* p, const fdtdx_buffers* b, int32_t t0, int32_t t1, int32_t rec,
                         void* stream, hipEvent_t* ev, bool ring = true);
 
+// The tiles of a plan in a batch are quad tiles.
+static bool batch_quad(const fdtdx_plan* p) { return p->P.vq && p->P.cax; }
+
 // ---------------------------------------------------------------- forward without allocation
 // fdtdx_forward_noalloc runs fdtdx_forward with its workspace (the H_prev snapshot of the detector
 // boxes and the detectors' per-block partial sums) in a static device array instead of a caller
@@ -896,8 +906,16 @@ int fdtdx_forward_noalloc(const fdtdx_plan* p, const fdtdx_buffers* b, int32_t t
 
 int fdtdx_plan_schedule(const fdtdx_plan* p, int32_t* out) {
   if (!p || !out) return fail(FDTDX_EINVAL, "null argument");
-  *out = p->use_fused == 2 ? FDTDX_SCHED_MARCH : p->use_fused ? FDTDX_SCHED_FUSED : p->P.vq ? FDTDX_SCHED_QUAD
-                                                                                           : FDTDX_SCHED_ONE;
+  *out = p->use_fused == 2               ? FDTDX_SCHED_MARCH
+         : p->use_fused                  ? FDTDX_SCHED_FUSED
+         : p->P.vq && !p->alone_one      ? FDTDX_SCHED_QUAD
+                                         : FDTDX_SCHED_ONE;
+  return FDTDX_OK;
+}
+
+int fdtdx_plan_batch_schedule(const fdtdx_plan* p, int32_t* out) {
+  if (!p || !out) return fail(FDTDX_EINVAL, "null argument");
+  *out = batch_quad(p) ? FDTDX_SCHED_QUAD : FDTDX_SCHED_ONE;
   return FDTDX_OK;
 }
 
@@ -958,6 +976,7 @@ static int forward_impl(const fdtdx_plan* p, const fdtdx_buffers* b, int32_t t0,
   float* Eb[2] = {b->E, p->use_fused ? (float*)(ws + p->ws_Ealt) : b->E};
   float* Hb[2] = {b->H, p->use_fused ? (float*)(ws + p->ws_Halt) : b->H};
   float* Pb[2] = {b->psi, p->use_fused ? (float*)(ws + p->ws_psialt) : b->psi};
+  const bool vq = p->P.vq && !p->alone_one;
   // sums of energy, flux and field detectors: finalized for kDetRing steps at a time, unless steps of one
   // launch would share a slot
   DetRing F;
@@ -1009,15 +1028,15 @@ static int forward_impl(const fdtdx_plan* p, const fdtdx_buffers* b, int32_t t0,
       Di.n = n;
       Di.snap = snap ? (float*)(ws + p->ws_snapE) : nullptr;  // H_prev of the imaginary part
       const PartDyn C = {(long long)p->psi_floats, (long long)p->ade_floats, Di.snap};
-      if (p->P.vq && p->cplx) HIP_TRY(launch_update_E4c(p->P, D, C, p->ec, s));
-      else if (p->P.vq) HIP_TRY(launch_update_E4(p->P, D, p->ec, s));
+      if (vq && p->cplx) HIP_TRY(launch_update_E4c(p->P, D, C, p->ec, s));
+      else if (vq) HIP_TRY(launch_update_E4(p->P, D, p->ec, s));
       else HIP_TRY(launch_update_E(p->P, D, p->ec, s));
-      if (p->cplx && !p->P.vq) HIP_TRY(launch_update_E(p->P, Di, p->ec, s));
+      if (p->cplx && !vq) HIP_TRY(launch_update_E(p->P, Di, p->ec, s));
       if (ev) HIP_TRY(hipEventRecord(ev[3 * (n - t0) + 1], s));
-      if (p->P.vq && p->cplx) HIP_TRY(launch_update_H4c(p->P, D, C, p->mc, s));
-      else if (p->P.vq) HIP_TRY(launch_update_H4(p->P, D, p->mc, s));
+      if (vq && p->cplx) HIP_TRY(launch_update_H4c(p->P, D, C, p->mc, s));
+      else if (vq) HIP_TRY(launch_update_H4(p->P, D, p->mc, s));
       else HIP_TRY(launch_update_H(p->P, D, p->mc, s));
-      if (p->cplx && !p->P.vq) HIP_TRY(launch_update_H(p->P, Di, p->mc, s));
+      if (p->cplx && !vq) HIP_TRY(launch_update_H(p->P, Di, p->mc, s));
       if (p->P.rec_narrow && recp) {
         D.record = recp;
         HIP_TRY(launch_record(p->P, D, p->iface_cells, s));
@@ -1408,7 +1427,7 @@ static int batch_upload(fdtdx_batch* b, hipStream_t s) {
       dd.state = S.det_state[q];
       dd.partial = (double*)(ws + (p->ws_ring ? p->ws_ring : p->ws_partial)) + (size_t)q * kDetMaxValues * kDetMaxBlocks;
     }
-    I.quad = p->P.vq && p->P.cax;
+    I.quad = batch_quad(p);
     T->tile_start[e + 1] = T->tile_start[e] + (I.quad ? p->P.vnblocks : p->P.nblocks);
     T->det_start[e + 1] = T->det_start[e] + nb;
     T->fin_start[e + 1] = T->fin_start[e] + nf;

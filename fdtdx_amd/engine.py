@@ -93,7 +93,7 @@ EXPORTED = ("fdtdx_plan_create", "fdtdx_plan_destroy", "fdtdx_psi_floats", "fdtd
             "fdtdx_workspace_bytes", "fdtdx_forward", "fdtdx_forward_timed",
             "fdtdx_reverse_adjoint", "fdtdx_reverse", "fdtdx_last_error", "fdtdx_batch_create", "fdtdx_batch_destroy",
             "fdtdx_batch_attach", "fdtdx_batch_detach", "fdtdx_batch_advance", "fdtdx_batch_step_index",
-            "fdtdx_batch_flags", "fdtdx_stream_probe", "fdtdx_plan_schedule",
+            "fdtdx_batch_flags", "fdtdx_stream_probe", "fdtdx_plan_schedule", "fdtdx_plan_batch_schedule",
             "fdtdx_forward_noalloc", "fdtdx_stencil_probe")
 
 FDTDX_MAX_BATCH = 64
@@ -126,8 +126,9 @@ def load_library(path: Path | None = None):
                "fdtdx_record_slots", "fdtdx_workspace_bytes"):
         getattr(lib, nm).argtypes = [c_void_p, POINTER(c_size_t)]
         getattr(lib, nm).restype = c_int32
-    lib.fdtdx_plan_schedule.argtypes = [c_void_p, POINTER(c_int32)]
-    lib.fdtdx_plan_schedule.restype = c_int32
+    for nm in ("fdtdx_plan_schedule", "fdtdx_plan_batch_schedule"):
+        getattr(lib, nm).argtypes = [c_void_p, POINTER(c_int32)]
+        getattr(lib, nm).restype = c_int32
     lib.fdtdx_record_slot_of.argtypes = [c_void_p, c_int32, POINTER(c_int32)]
     lib.fdtdx_record_slot_of.restype = c_int32
     lib.fdtdx_forward.argtypes = [c_void_p, POINTER(Buffers), c_int32, c_int32, c_int32, c_void_p]
@@ -316,14 +317,22 @@ class Plan:
     @property
     def schedule(self) -> int:
         """The forward sweep schedule of the plan (SCHED_ONE, SCHED_QUAD, SCHED_FUSED, SCHED_MARCH)."""
+        return self._schedule("fdtdx_plan_schedule")
+
+    def _schedule(self, nm) -> int:
         out = c_int32()
-        _check(self._lib, self._lib.fdtdx_plan_schedule(self._h, ctypes.byref(out)), "fdtdx_plan_schedule")
+        _check(self._lib, getattr(self._lib, nm)(self._h, ctypes.byref(out)), nm)
         return int(out.value)
 
     @property
     def quad(self) -> bool:
         """True when the forward sweeps update four z cells per lane."""
         return self.schedule == SCHED_QUAD
+
+    @property
+    def batch_quad(self) -> bool:
+        """True when the plan's tiles in a batch are of four z cells per lane."""
+        return self._schedule("fdtdx_plan_batch_schedule") == SCHED_QUAD
 
     def _query(self, nm):
         out = c_size_t()

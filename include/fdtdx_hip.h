@@ -280,10 +280,15 @@ int fdtdx_record_slot_of(const fdtdx_plan* plan, int32_t step, int32_t* out);
 int fdtdx_workspace_bytes(const fdtdx_plan* plan, size_t* out);
 /* The forward sweep schedule chosen at plan creation (no counterpart in the reference; for tests
  * and measurement): FDTDX_SCHED_ONE (E and H sweeps, one cell per lane), FDTDX_SCHED_QUAD (E and H
- * sweeps, four z cells per lane; the default for real fields without full tensors, except rows of
- * fewer than 4 cells, or of nz % 4 != 0 cells where the CPML slabs do not each span a face), FDTDX_SCHED_FUSED or FDTDX_SCHED_MARCH (single-pass, opted in by FDTDX_SWEEP). */
+ * sweeps, four z cells per lane), FDTDX_SCHED_FUSED or FDTDX_SCHED_MARCH (single-pass, opted in by
+ * FDTDX_SWEEP). Quads are the default; one cell per lane run full tensors, rows of fewer than 4 cells,
+ * rows of nz % 4 != 0 cells and complex fields where the CPML slabs do not each span a face or where there
+ * are both poles and conductivity, and small grids of real fields with poles. All give the same bits.
+ * fdtdx_plan_batch_schedule: the schedule of the plan's tiles in a batch (fdtdx_batch_attach), where the
+ * size of one grid does not count. */
 enum { FDTDX_SCHED_ONE = 0, FDTDX_SCHED_QUAD = 1, FDTDX_SCHED_FUSED = 2, FDTDX_SCHED_MARCH = 3 };
 int fdtdx_plan_schedule(const fdtdx_plan* plan, int32_t* out);
+int fdtdx_plan_batch_schedule(const fdtdx_plan* plan, int32_t* out);
 
 /* Advance steps n = t0 .. t1-1 in place (forward.py:83-156 per step). When rec != 0 the PML
  * interface layers of each kept step are written, compressed, to its slot of buffers->record

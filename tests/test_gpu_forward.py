@@ -670,6 +670,30 @@ def test_detector_steps_that_share_a_slot_are_stored_in_order(slots):
                 assert np.array_equal(a[slot], r[t]), (slot, t)
 
 
+@pytest.mark.parametrize("shape,poles,quad", [((40, 40, 40), False, True), ((40, 40, 40), True, False),
+                                              ((88, 88, 88), True, False), ((92, 92, 92), True, True)])
+def test_schedule_of_small_grids_with_poles(shape, poles, quad, monkeypatch):
+    """Small grids with poles run one cell per lane alone and in quads in a batch or under
+    FDTDX_SWEEP=quad; larger ones and those without poles in quads."""
+    import scenarios
+
+    from fdtdx_amd import fdtd as F
+
+    spec = W.scenario_c1(T=3, n=40, pml=5, cube=8)
+    spec["shape"] = shape
+    spec["detectors"] = []
+    if poles:
+        spec["boxes"][0]["poles"] = [("drude", 2e15, 1e14)]
+    for mode in (None, "quad"):
+        if mode:
+            monkeypatch.setenv("FDTDX_SWEEP", mode)
+        else:
+            monkeypatch.delenv("FDTDX_SWEEP", raising=False)
+        objects, arrays, params, config = scenarios.build(spec)
+        plan = F.Solve(objects, config, arrays).plan
+        assert plan.quad == (quad or mode == "quad") and plan.batch_quad
+
+
 def _ragged_cases():
     """Rows of nz % 4 != 0 cells: the last quad of a row repeats cells of the quad before it."""
     c1 = W.scenario_c1(T=60, n=29, pml=5, cube=6)                                  # nz % 4 = 1

@@ -163,9 +163,10 @@ def test_blowup_limit_flags_every_solve(plain):
 @pytest.mark.parametrize("eps_comps", [1, 3])
 def test_batch_of_mixed_schedules_equals_single_solves(eps_comps):
     """One batch of solves whose tiles differ (quads over aligned and ragged rows, one cell per lane,
-    ADE tiles, conductivity with a conducting face, periodic axes) and whose detectors need per-cell
-    phasors, halos, reduced phasors and accumulating faces, advanced 21 steps per chunk (sums finalized
-    for 16, then 5): every state equals the single solve's bit for bit."""
+    ADE tiles with and without conductivity, conductivity with a conducting face, periodic axes) and whose
+    detectors need per-cell phasors, halos, reduced phasors and accumulating faces, advanced 21 steps per
+    chunk (sums finalized for 16, then 5): every state equals the single solve's bit for bit. Each solve's
+    tiles are of the kind it stands for: small grids with poles run one cell per lane alone, in quads here."""
     import torch
 
     from fdtdx_amd import engine
@@ -176,8 +177,14 @@ def test_batch_of_mixed_schedules_equals_single_solves(eps_comps):
     n = 24
     f0 = 1.9e14
     if eps_comps == 3:
+        lossy = W.scenario_c4(T=35, n=28, pml=5, slab=(10, 10, 8), cube=4)
+        lossy["boxes"][0]["sigma_E"] = 2e4  # poles and conductivity in the same tiles
+        plain = W.scenario_c4(T=40, n=30, pml=5, slab=(10, 10, 8), cube=4)
+        for b in plain["boxes"]:
+            del b["poles"]
         specs = [W.scenario_c4(T=45, n=28, pml=5, slab=(10, 10, 8), cube=4),
-                 W.scenario_c4(T=50, n=31, pml=5, slab=(10, 10, 8), cube=4)]
+                 W.scenario_c4(T=50, n=31, pml=5, slab=(10, 10, 8), cube=4), lossy, plain]
+        alone, quads = [False, False, False, True], [True, True, True, True]
     else:
         ragged = W.scenario_c2(T=45, shape=(44, 30, 27), pml=5, slab=(10, 12, 8))
         lossy = W.scenario_c1(T=50, n=26, pml=4, cube=6)
@@ -195,6 +202,7 @@ def test_batch_of_mixed_schedules_equals_single_solves(eps_comps):
         flat["sources"][0]["cell"] = (12, 12, 1)
         flat["detectors"] = []
         specs = [ragged, lossy, per, flat]
+        alone, quads = [True, True, True, False], [True, True, True, False]
 
     def solves():
         out = []
@@ -210,6 +218,7 @@ def test_batch_of_mixed_schedules_equals_single_solves(eps_comps):
         return [t.cpu().numpy() for t in (a.fields.E, a.fields.H, a.psi, *s.state_tensors())]
 
     single = solves()
+    assert [s.plan.quad for s in single] == alone and [s.plan.batch_quad for s in single] == quads
     for s, spec in zip(single, specs):
         s.forward(0, spec["T"])
     torch.cuda.synchronize()
