@@ -134,6 +134,7 @@ struct StepStatic {
   const uint32_t* vec_mask;  // per quad tile, as fwd_mask
   long long vnslow;          // quad tiles with poles and conductivity (k_update_E4s) ...
   const int* vslow;          // ... and their indices
+  const int* btile;          // batch blocks of a plan with such tiles, four for each: 4 * tile + quarter (or null)
   uint32_t vpoint[2];        // the mask bits of E sources, of H sources ...
   uint32_t vwall[2];         // ... of PEC faces, of PMC faces
   // Per-axis CPML (acax = 1): every slab spans its face, at most one slab per side of an axis and

@@ -1369,9 +1369,20 @@ __device__ __forceinline__ bool batch_tile(const BatchTable& B, long long& t, in
 // (Two 128x128x64, three 96^3 and three 64^3 solves, 5.5M cells: E / H sweep 53.2 / 54.0 us one cell per
 // lane, 37.7 / 37.2 us four, with the table's scalar loads through the constant address space.)
 // A batch tile is a quad tile of an instance with the per-axis quad sweeps (BatchInst::quad; rows of
-// any length, so with 4-byte aligned accesses), else a tile of the one-cell sweeps. Quad tiles that
-// meet an ADE box run their E half-step one cell per lane, a quarter at a time.
-template <int EC>
+// any length, so with 4-byte aligned accesses), else a tile of the one-cell sweeps. Quad tiles
+// with poles and conductivity run their E half-step one cell per lane, a quarter in each of four consecutive
+// blocks (StepStatic::btile). ADE: some solve with quad tiles has poles (us per step with
+// the tiles that hold poles one cell per lane, their quarters in turn / with poles in the quads:
+// 128x128x72 with a two-pole slab 48 / 36, four of them 102 / 88, eight of 64^3 68 / 51).
+// Quarter of its tile that batch block lb of a solve has (0 where tiles are not split), lb becoming the tile.
+__device__ __forceinline__ int batch_part(const StepStatic& P, long long& lb) {
+  if (!P.btile) return 0;
+  const int v = P.btile[lb];
+  lb = v >> 2;
+  return v & 3;
+}
+
+template <int EC, bool ADE>
 __global__ __launch_bounds__(kBlock) void k_batch_E(const BatchTable* __restrict__ Bp, const int* __restrict__ base,
                                                     int r) {
   const BatchTable& B = as_const(Bp);
@@ -1382,21 +1393,20 @@ __global__ __launch_bounds__(kBlock) void k_batch_E(const BatchTable* __restrict
   const StepStatic& P = I.P;
   const int n = base[I.slot] + r;
   if (n >= I.stop) return;
-  const long long lb = t - B.tile_start[e];
+  long long lb = t - B.tile_start[e];
   if (!I.quad) {
     update_E_tile<EC, true>(P, I.D, n, lb);
     return;
   }
-  const uint32_t m = P.vec_mask[lb];
   int i, j, k, sm;
   long long o;
-  if (m & kAdeBits) {
-#pragma unroll 1
-    for (int part = 0; part < 4; ++part)
-      if (tile_cell(P, lb, part, i, j, k, o)) update_E_cell<EC, true>(P, I.D, n, m, i, j, k, o);
+  const int part = batch_part(P, lb);
+  const uint32_t m = P.vec_mask[lb];
+  if (ADE && poles_and_loss(m)) {
+    if (tile_cell(P, lb, part, i, j, k, o)) update_E_cell<EC, true>(P, I.D, n, m, i, j, k, o);
     return;
   }
-  if (quad_of(P, lb, i, j, k, sm, o)) quad_E<EC, true, true, true, false>(P, I.D, n, m, i, j, k, sm, o);
+  if (quad_of(P, lb, i, j, k, sm, o)) quad_E<EC, true, true, true, ADE>(P, I.D, n, m, i, j, k, sm, o);
 }
 
 template <int MC>
@@ -1412,11 +1422,12 @@ __global__ __launch_bounds__(kBlock) void k_batch_H(const BatchTable* __restrict
   if (n >= I.stop) return;
   const int rs = P.rec_slot ? P.rec_slot[n] : n;
   char* record = (I.rec_base && rs >= 0) ? I.rec_base + (long long)rs * P.rec_slot_bytes : nullptr;
-  const long long lb = t - B.tile_start[e];
+  long long lb = t - B.tile_start[e];
   if (!I.quad) {
     update_H_tile<MC, true>(P, I.D, n, record, lb);
     return;
   }
+  if (batch_part(P, lb)) return;
   int i, j, k, sm;
   long long o;
   if (quad_of(P, lb, i, j, k, sm, o)) quad_H<MC, true, true, true>(P, I.D, n, record, P.vec_mask[lb], i, j, k, sm, o);
@@ -1455,10 +1466,10 @@ hipError_t launch_batch_set(int* base, int* flags, const BatchSet& set, hipStrea
   return hipGetLastError();
 }
 
-hipError_t launch_batch_sweeps(const BatchTable* tab, const int* base, int r, int ec, int mc, int grid,
+hipError_t launch_batch_sweeps(const BatchTable* tab, const int* base, int r, int ec, int mc, bool ade, int grid,
                                hipStream_t s) {
-  if (ec == 3) hipLaunchKernelGGL(k_batch_E<3>, dim3(grid), dim3(kBlock), 0, s, tab, base, r);
-  else hipLaunchKernelGGL(k_batch_E<1>, dim3(grid), dim3(kBlock), 0, s, tab, base, r);
+  const auto fe = ec == 3 ? (ade ? k_batch_E<3, true> : k_batch_E<3, false>) : (ade ? k_batch_E<1, true> : k_batch_E<1, false>);
+  hipLaunchKernelGGL(fe, dim3(grid), dim3(kBlock), 0, s, tab, base, r);
   if (mc == 3) hipLaunchKernelGGL(k_batch_H<3>, dim3(grid), dim3(kBlock), 0, s, tab, base, r);
   else if (mc == 1) hipLaunchKernelGGL(k_batch_H<1>, dim3(grid), dim3(kBlock), 0, s, tab, base, r);
   else hipLaunchKernelGGL(k_batch_H<0>, dim3(grid), dim3(kBlock), 0, s, tab, base, r);

@@ -163,7 +163,8 @@ struct BatchSet {               // counters to (re)initialise (and flags to clea
 
 int batch_sweep_grid(long long tiles);  // blocks of a batch sweep over `tiles` tiles
 hipError_t launch_batch_set(int* base, int* flags, const BatchSet& set, hipStream_t s);
-hipError_t launch_batch_sweeps(const BatchTable* tab, const int* base, int r, int ec, int mc, int grid,
+// ade: some solve of the batch has poles
+hipError_t launch_batch_sweeps(const BatchTable* tab, const int* base, int r, int ec, int mc, bool ade, int grid,
                                hipStream_t s);
 // Detectors of chunk step r (mode bit 0: some detector keeps per-cell phasors, bit 1: some needs_halo),
 // and the sums of chunk steps [r0, r0 + steps), at most kDetRing of them.

@@ -695,6 +695,17 @@ static int plan_create(const fdtdx_plan_desc* d, fdtdx_plan** out) {
       P.vnslow = (long long)slow.size();
       P.vslow = nullptr;
       if (!slow.empty() && (rc = pl->upload(slow.data(), slow.size(), &P.vslow))) return bail(rc);
+      P.btile = nullptr;
+      if (!slow.empty()) {
+        std::vector<int> bt;
+        size_t q = 0;
+        for (long long lb = 0; lb < P.vnblocks; ++lb) {
+          const bool split = q < slow.size() && slow[q] == lb;
+          if (split) ++q;
+          for (int part = 0; part < (split ? 4 : 1); ++part) bt.push_back((int)(4 * lb + part));
+        }
+        if ((rc = pl->upload(bt.data(), bt.size(), &P.btile))) return bail(rc);
+      }
       P.vq = 1;
     }
   }
@@ -1276,6 +1287,7 @@ int fdtdx_reverse_adjoint(const fdtdx_plan* p, const fdtdx_buffers* b, const fdt
 struct fdtdx_batch {
   int ec = 1, mc = 0;
   int grid = 0, det_grid = 1024;
+  bool ade = false;                // some solve with quad tiles has poles
   BatchTable* dtab = nullptr;      // device table
   int* dbase = nullptr;            // device step counters, one per slot
   int* dflags = nullptr;           // device health flags, one per slot
@@ -1294,7 +1306,7 @@ struct fdtdx_batch {
     bool pending_set = false;      // counter must be initialised before the next chunk
   };
   Slot slot[kMaxBatch];
-  std::map<std::tuple<int, int, int>, hipGraphExec_t> graphs;  // (steps, detector mode, grid) -> executable
+  std::map<std::tuple<int, int, int, bool>, hipGraphExec_t> graphs;  // (steps, detector mode, grid, ade) -> executable
 
   ~fdtdx_batch() {
     for (auto& g : graphs) (void)hipGraphExecDestroy(g.second);
@@ -1399,6 +1411,7 @@ static int batch_upload(fdtdx_batch* b, hipStream_t s) {
   T->tile_start[0] = 0;
   T->det_start[0] = 0;
   T->fin_start[0] = 0;
+  b->ade = false;
   for (int sl = 0; sl < kMaxBatch; ++sl) {
     const fdtdx_batch::Slot& S = b->slot[sl];
     if (!S.plan) continue;
@@ -1428,7 +1441,8 @@ static int batch_upload(fdtdx_batch* b, hipStream_t s) {
       dd.partial = (double*)(ws + (p->ws_ring ? p->ws_ring : p->ws_partial)) + (size_t)q * kDetMaxValues * kDetMaxBlocks;
     }
     I.quad = batch_quad(p);
-    T->tile_start[e + 1] = T->tile_start[e] + (I.quad ? p->P.vnblocks : p->P.nblocks);
+    b->ade = b->ade || (I.quad && p->P.nade);
+    T->tile_start[e + 1] = T->tile_start[e] + (I.quad ? p->P.vnblocks + 3 * p->P.vnslow : p->P.nblocks);
     T->det_start[e + 1] = T->det_start[e] + nb;
     T->fin_start[e + 1] = T->fin_start[e] + nf;
     ++e;
@@ -1447,7 +1461,7 @@ static int batch_upload(fdtdx_batch* b, hipStream_t s) {
 // det: -1 no detectors, else bit 0: some detector needs_halo, bit 1: some sums.
 static int batch_chunk(fdtdx_batch* b, int steps, int det, hipStream_t s) {
   for (int r = 0; r < steps; ++r) {
-    HIP_TRY(launch_batch_sweeps(b->dtab, b->dbase, r, b->ec, b->mc, b->grid, s));
+    HIP_TRY(launch_batch_sweeps(b->dtab, b->dbase, r, b->ec, b->mc, b->ade, b->grid, s));
     if (det >= 0) HIP_TRY(launch_batch_detectors(b->dtab, b->dbase, r, det, b->det_grid, s));
     if (det >= 0 && (det & 2) && ((r + 1) % kDetRing == 0 || r + 1 == steps)) {
       const int r0 = r / kDetRing * kDetRing;
@@ -1489,7 +1503,7 @@ int fdtdx_batch_advance(fdtdx_batch* b, int32_t steps, int32_t use_graph, void* 
   if (!any) return FDTDX_OK;
   HIP_TRY(launch_batch_set(b->dbase, b->dflags, set, s));
   if (use_graph) {
-    const auto key = std::make_tuple((int)steps, det, b->grid);
+    const auto key = std::make_tuple((int)steps, det, b->grid, b->ade);
     auto it = b->graphs.find(key);
     if (it == b->graphs.end()) {
       hipGraph_t g = nullptr;

@@ -201,8 +201,10 @@ def test_batch_of_mixed_schedules_equals_single_solves(eps_comps):
         flat["boxes"] = [dict(slc=((8, 12), (8, 12), (0, 3)), eps=2.25)]
         flat["sources"][0]["cell"] = (12, 12, 1)
         flat["detectors"] = []
-        specs = [ragged, lossy, per, flat]
-        alone, quads = [True, True, True, False], [True, True, True, False]
+        poles = W.scenario_c1(T=35, n=27, pml=4, cube=7)
+        poles["boxes"][0]["poles"] = [("drude", 2e15, 1e14)]
+        specs = [ragged, lossy, per, flat, poles]
+        alone, quads = [True, True, True, False, False], [True, True, True, False, True]
 
     def solves():
         out = []
