@@ -826,7 +826,6 @@ __global__ __launch_bounds__(kBlock) void k_adj_A4(const StepStatic* __restrict_
   const long long lb = logical_block(P.xorder, P.vnblocks_pad);
   if (!quad_of(P, lb, i, j, k0, sm, o)) return;
   const uint32_t m = P.vec_mask[lb];
-  if (m & P.vpoint[0]) quad_points<0, true>(P, m, A.ie, A.im, A.Erev, A.n, i, j, k0, sm, o, EC, 0);
   const long long N = P.N;
   const bool vj = j > 0, vi = i > 0, vk = k0 > 0;
   const f4v z4 = {0.f, 0.f, 0.f, 0.f}, c = {P.c, P.c, P.c, P.c};
@@ -848,11 +847,13 @@ __global__ __launch_bounds__(kBlock) void k_adj_A4(const StepStatic* __restrict_
       quad_two_curls<1, RAG>(P, A.psi, i, j, k0, dyx, dyz, K, Kr);
       quad_two_curls<2, RAG>(P, A.psi, i, j, k0, dzy, dzx, K, Kr);
     }
+    f4v E1[3];
 #pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      float* Ea = A.Erev + a * N + o;
-      st4m<RAG>(Ea, ld4<RAG>(Ea) - (c * Kr[a]) * ld4<RAG>(A.ie + (EC == 3 ? a : 0) * N + o), sm);
-    }
+    for (int a = 0; a < 3; ++a) E1[a] = ld4<RAG>(A.Erev + a * N + o);
+    if (m & P.vpoint[0]) quad_sources<0, true>(P, m, A.ie + o, EC, A.n, i, j, k0, E1);
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+      st4m<RAG>(A.Erev + a * N + o, E1[a] - (c * Kr[a]) * ld4<RAG>(A.ie + (EC == 3 ? a : 0) * N + o), sm);
   }
   const f4v wx = w_h4<MC, RAG>(P, A, 0, o), wy = w_h4<MC, RAG>(P, A, 1, o), wz = w_h4<MC, RAG>(P, A, 2, o);
   const f4v wx_jm = vj ? w_h4<MC, RAG>(P, A, 0, o - P.nz) : z4, wz_jm = vj ? w_h4<MC, RAG>(P, A, 2, o - P.nz) : z4;

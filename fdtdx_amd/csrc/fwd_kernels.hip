@@ -734,11 +734,11 @@ __device__ __forceinline__ void quad_E(const StepStatic& P, const StepDyn& D, in
   const f4v inv[3] = {iex, iey, iez};
   if (X && ((m >> kMaskLoss) & 1u)) quad_loss<0>(P, i, j, k0, inv, eo, t, en);
   if (ADE && (m & kAdeBits)) quad_ade<EC>(P, D.ade, D.ie + o, m, n, i, j, k0, sm, eo, en);
+  if (m & P.vpoint[0]) quad_sources<0>(P, m, D.ie + o, EC, n, i, j, k0, en);
   if (m & P.vwall[0]) quad_walls<0>(P, m, i, j, k0, en);
   st4m<RAG>(Ex + o, en[0], sm);
   st4m<RAG>(Ey + o, en[1], sm);
   st4m<RAG>(Ez + o, en[2], sm);
-  if (m & P.vpoint[0]) quad_points<0>(P, m, D.ie, D.im, D.E, n, i, j, k0, sm, o, EC, 0);
   if ((m & kSnapBit) && D.snap) {  // H_prev of the detector boxes, as update_E_cell
     const long long sy = D.shi[1] - D.slo[1], sz = D.shi[2] - D.slo[2];
     const long long sc = (long long)(D.shi[0] - D.slo[0]) * sy * sz;
@@ -817,18 +817,11 @@ __device__ __forceinline__ void quad_H(const StepStatic& P, const StepDyn& D, in
     const f4v inv[3] = {imx, imy, imz};
     quad_loss<1>(P, i, j, k0, inv, ho, t, hn);
   }
+  if (m & P.vpoint[1]) quad_sources<1>(P, m, MC ? D.im + o : nullptr, MC, n, i, j, k0, hn);
   if (m & P.vwall[1]) quad_walls<1>(P, m, i, j, k0, hn);
   st4m<RAG>(Hx + o, hn[0], sm);
   st4m<RAG>(Hy + o, hn[1], sm);
   st4m<RAG>(Hz + o, hn[2], sm);
-  if (m & P.vpoint[1]) {
-    quad_points<1>(P, m, D.ie, D.im, D.H, n, i, j, k0, sm, o, 1, MC);
-    if (record) {  // the recorded layers hold the sources
-      hn[0] = ld4<RAG>(Hx + o);
-      hn[1] = ld4<RAG>(Hy + o);
-      hn[2] = ld4<RAG>(Hz + o);
-    }
-  }
   if (record && (m & kSlabBits)) {
 #pragma unroll 1
     for (int e = RAG ? sm : 0; e < 4; ++e) record_iface(P, m, record, i, j, k0 + e, ex[e], ey[e], ez[e], hn[0][e], hn[1][e], hn[2][e]);
@@ -974,7 +967,6 @@ __global__ __launch_bounds__(kBlock) void k_reverse_H4(const StepStatic* __restr
       for (int a = 0; a < 3; ++a) D.snap[a * sc + q] = D.H[a * P.N + o + e];
     }
   }
-  if (m & P.vpoint[1]) quad_points<1, true>(P, m, D.ie, D.im, D.H, D.n, i, j, k0, sm, o, 1, MC);
   const long long N = P.N;
   QuadSlabs S;
   S.in[0] = S.in[1] = S.in[2] = false;
@@ -988,7 +980,7 @@ __global__ __launch_bounds__(kBlock) void k_reverse_H4(const StepStatic* __restr
   const f4v exj = vj ? ld4<RAG>(Ex + P.nz) : z4, ezj = vj ? ld4<RAG>(Ez + P.nz) : z4;
   const f4v eyi = vi ? ld4<RAG>(Ey + P.plane) : z4, ezi = vi ? ld4<RAG>(Ez + P.plane) : z4;
   const float exk = vk ? Ex[4] : 0.f, eyk = vk ? Ey[4] : 0.f;
-  const f4v ho[3] = {ld4<RAG>(Hx), ld4<RAG>(Hy), ld4<RAG>(Hz)};
+  f4v ho[3] = {ld4<RAG>(Hx), ld4<RAG>(Hy), ld4<RAG>(Hz)};
   const f4v exn = {ex[1], ex[2], ex[3], exk}, eyn = {ey[1], ey[2], ey[3], eyk};
   QuadDeriv d;
   d.x1 = ezi - ez;
@@ -999,6 +991,7 @@ __global__ __launch_bounds__(kBlock) void k_reverse_H4(const StepStatic* __restr
   d.z2 = exn - ex;
   f4v cx = d.y2 - d.z1, cy = d.z2 - d.x1, cz = d.x2 - d.y1;
   if (m & kSlabBits) quad_slab_frozen<1, RAG>(P, S, i, j, k0, d, cx, cy, cz);
+  if (m & P.vpoint[1]) quad_sources<1, true>(P, m, MC ? D.im + o : nullptr, MC, D.n, i, j, k0, ho);
   const f4v one = {1.f, 1.f, 1.f, 1.f}, c = {P.c, P.c, P.c, P.c};
   const f4v imx = MC ? ld4<RAG>(D.im + o) : one;
   const f4v imy = MC == 3 ? ld4<RAG>(D.im + N + o) : imx;

@@ -362,9 +362,9 @@ __device__ __forceinline__ void quad_ade(const StepStatic& P, float* ade, const 
 }
 
 // Conducting faces of field W (0: E, PEC; 1: H, PMC) in the updated quad f (apply_walls). In registers
-// ahead of the store: a face normal to z meets the end of every row, where the rounds of quad_points, which
-// held the faces before, cost more than the sweep itself. us per step of a grid between two PEC faces normal
-// to z, quad_points / here / one cell per lane: 800x800x20 240 / 179 / 190, 400x400x8 26.6 / 20.3 / 21.6,
+// ahead of the store: a face normal to z meets the end of every row, where reading the stored quad back in
+// four rounds cost more than the sweep itself. us per step of a grid between two PEC faces normal
+// to z, rounds / here / one cell per lane: 800x800x20 240 / 179 / 190, 400x400x8 26.6 / 20.3 / 21.6,
 // 300x300x150 (four faces, y and z) 225 / 207 / 216.
 template <int W>
 __device__ __forceinline__ void quad_walls(const StepStatic& P, uint32_t m, int i, int j, int k0, f4v* f) {
@@ -381,33 +381,43 @@ __device__ __forceinline__ void quad_walls(const StepStatic& P, uint32_t m, int 
   }
 }
 
-// Sources of field W (0: E; 1: H) over a quad, after its update (with quad_walls) has
-// been stored: the cells e >= sm are read back, changed and stored one by one (rolled, so that the
-// few quads that hold one cost the others no registers). m: the tile's mask. Before, such tiles
-// ran one cell per lane in launches of their own: 6 to 9 us each whatever the grid, against no
-// measurable time here (steps of the 64^3 dipole 49.5 -> 44.6 us, the 128x128x64 plane wave 45.2
-// -> 37.8, the 200x200x100 dipole 77.7 -> 70.4, the 400x400x200 plane wave 529 -> 511).
-// INV: the reverse run's sources (negated), added before the half-step is undone.
+// Sources of field W (0: E; 1: H) in the updated quad f (source_one, in list order), ahead of quad_walls and
+// the store: profile and inverse material move as vectors, inv (at the quad, comps components; null: 1) is
+// read again here rather than held. m: the tile's mask. INV: the reverse run's sources (negated),
+// added before the half-step is undone. Tiles with sources ran one cell per lane in launches of their own
+// at first (6 to 9 us each whatever the grid), then read the quad back after the store in four rounds, the
+// end of a launch of one wave of blocks. us per step, launches / rounds / here: two plane waves in 128x120x100
+// 60 / 45 / 41; rounds / here: 128x128x64 plane wave 35.1 / 30.6, 301x277x150 236 / 229. Rows of nz % 4 != 0
+// cells, one cell per lane / rounds / here: four plane waves in 128x120x99 47 / 54 / 47.5, 141^3 53 / 54.6 / 52.
 template <int W, bool INV = false>
-__device__ __forceinline__ void quad_points(const StepStatic& P, uint32_t m, const float* ie, const float* im,
-                                            float* F, int n, int i, int j, int k0, int sm, long long o, int ec,
-                                            int mc) {
-  bool hit = false;
-  for (uint32_t mm = (m >> kMaskSrc) & ((1u << P.nsrc) - 1u); mm; mm &= mm - 1u) {
-    const SrcK& sr = P.src[__builtin_ctz(mm)];
-    hit = hit || (sr.field == W && i >= sr.lo[0] && i < sr.hi[0] && j >= sr.lo[1] && j < sr.hi[1] &&
-                  k0 + 3 >= sr.lo[2] && k0 < sr.hi[2]);
-  }
-  if (!hit) return;
-  float* p = F + o;
+__device__ __forceinline__ void quad_sources(const StepStatic& P, uint32_t m, const float* inv, int comps, int n,
+                                             int i, int j, int k0, f4v* f) {
 #pragma unroll 1
-  for (int e = sm; e < 4; ++e) {
-    float x = p[e], y = p[P.N + e], z = p[2 * P.N + e];
-    apply_sources(P, m, ie, im, W, n, INV, i, j, k0 + e, o + e, ec, mc, x, y, z);
-    if (!INV) apply_walls(P, m, W ? FDTDX_WALL_PMC : FDTDX_WALL_PEC, i, j, k0 + e, x, y, z);
-    p[e] = x;
-    p[P.N + e] = y;
-    p[2 * P.N + e] = z;
+  for (uint32_t mm = (m & P.vpoint[W]) >> kMaskSrc; mm; mm &= mm - 1u) {
+    const SrcK& S = P.src[__builtin_ctz(mm)];
+    if (i < S.lo[0] || i >= S.hi[0] || j < S.lo[1] || j >= S.hi[1] || k0 + 3 < S.lo[2] || k0 >= S.hi[2]) continue;
+    const int a0 = max(0, S.lo[2] - k0), a1 = min(4, S.hi[2] - k0);
+    auto add = [&](int c, f4v v) {  // as source_one: zero is added to the other components
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bool in = e >= a0 && e < a1;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) f[a][e] = in ? f[a][e] + (a == c ? v[e] : 0.f) : f[a][e];
+      }
+    };
+    if (S.kind == FDTDX_SRC_POINT) {
+      const float v = INV ? -S.table[n] : S.table[n];
+      add(S.comp, f4v{v, v, v, v});
+      continue;
+    }
+    const long long q = ((long long)(i - S.lo[0]) * S.py + (j - S.lo[1])) * S.pz + (k0 - S.lo[2]);
+#pragma unroll 1
+    for (int t = 0; t < 2; ++t) {
+      const int tc = S.target[t], sc = S.src[t];
+      f4v x = (ld4p(S.profile + sc * S.pcells + q, a0, a1) * S.table[sc * P.T + n]) * P.c;
+      if (inv) x = x * ld4<true>(inv + (comps == 3 ? tc : 0) * P.N);
+      add(tc, (INV ? -S.sign[t] : S.sign[t]) * x);
+    }
   }
 }
 

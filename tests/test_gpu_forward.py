@@ -544,6 +544,43 @@ def test_deferred_detector_sums_equal_a_launch_per_step(T, halo):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("nz", [28, 30, 31])
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_sources_in_quads_equal_one_cell_sweeps_bitwise(nz, axis, monkeypatch):
+    """Plane sources normal to each axis (one normal to z holds one cell of its quads) and dipoles in
+    overlapping quads, one in the cells a ragged row's last quad repeats, over diagonal permittivity and
+    permeability: fields, psi, the interface record and the flux equal one cell per lane bit for bit."""
+    import torch
+
+    from fdtdx_amd import fdtd as F
+    import scenarios
+
+    spec = W.scenario_c1(T=45, n=28, pml=4, cube=6)
+    spec["shape"] = (26, 25, nz)
+    spec["boxes"] = [dict(slc=((0, 26), (0, 25), (0, nz)), eps=(2.0, 3.0, 4.0), mu=(1.2, 1.5, 1.7))]
+    prof = dict(kind="single", frequency=2e14, phase_shift=0.3)
+    e_pol = [0, 0, 0]
+    e_pol[(axis + 1) % 3] = 1
+    spec["sources"] = [dict(kind="plane", axis=axis, index=6, direction="+", e_pol=tuple(e_pol), profile=prof),
+                       dict(kind="dipole", cell=(12, 11, 13), polarization=axis, profile=prof),
+                       dict(kind="dipole", cell=(13, 11, nz - 3), polarization=(axis + 1) % 3, profile=prof)]
+    spec["detectors"] = [dict(name="flux", kind="flux", slc=((17, 18), (5, 20), (5, 20)), axis=0, reduce_volume=True)]
+    out = {}
+    for mode in ("two", "quad"):
+        _set_mode(monkeypatch, mode)
+        objects, arrays, params, config = scenarios.build(spec)
+        s = F.Solve(objects, config, arrays, record_steps=spec["T"])
+        assert s.plan.quad == (mode == "quad")
+        arrays.reset()
+        print(f"nz {nz} axis {axis} {mode}", flush=True)
+        s.forward(0, spec["T"], record=True)
+        torch.cuda.synchronize()
+        out[mode] = [t.cpu().numpy() for t in (arrays.fields.E, arrays.fields.H, arrays.psi, s.record, *s.det_tensors())]
+    assert np.abs(out["quad"][0]).max() > 0
+    for a, b in zip(out["quad"], out["two"]):
+        assert np.array_equal(a, b)
+
+
 @pytest.mark.parametrize("box", [((5, 8), (2, 22), (1, 22)), ((2, 22), (7, 11), (3, 22)), ((9, 10), (4, 13), (0, 24)),
                                  ((0, 24), (0, 24), (0, 24))])
 def test_energy_slice_means_equal_the_means_of_per_cell_energies(box):
