@@ -101,8 +101,9 @@ struct fdtdx_plan {
   }
 };
 
-// Plans with poles of fewer cells run one cell per lane when alone (plan_create).
-constexpr long long kAlonePoles = 700000;
+// Plans of fewer cells run one cell per lane when alone (plan_create): with poles, with poles and rows of
+// nz % 4 != 0 cells and CPML normal to z, with such rows.
+constexpr long long kAlonePoles = 700000, kAlonePolesRagged = 3000000, kAloneRagged = 400000;
 
 static bool box_ok(const int32_t* lo, const int32_t* hi, const StepStatic& P) {
   const int n[3] = {P.nx, P.ny, P.nz};
@@ -574,13 +575,22 @@ static int plan_create(const fdtdx_plan_desc* d, fdtdx_plan** out) {
       // conductivity: their tiles run one cell per lane (200x200x101: 101 us per step against 93 with
       // every tile one cell per lane; 128x120x100, 56 against 57, has them listed)
       if ((P.nz % 4 || pl->cplx) && (!(xyz && zq) || (P.nade && P.loss[0].comps))) quad_ok = false;
-      // Poles in a grid of few wavefronts, run alone: one cell per lane (a quad's chain of pole loads is four
-      // cells long and little runs beside it). us per step with a two-pole slab, one cell / quads: 48^3
-      // 16.1 / 20.4, 64x56x60 17.5 / 19.8, 80^3 22.2 / 23.7, 88^3 27.1 / 27.7; the other way from there (92^3
-      // 29.5 / 28.6, 100^3 32.6 / 28.6; with a 10^3 particle from 84^3, 21.7 / 21.5, 96^3 27.1 / 24.0).
-      // Complex fields have both parts in a launch and fewer launches with quads (24x24x36 25.3 / 21.6,
-      // 96x96x100 50 / 40), batches many solves in one (eight of 64^3 78 / 52, of 64^3 with the slab 80 / 68).
-      pl->alone_one = quad_ok && P.nade && P.N < kAlonePoles && !pl->cplx && !(qenv && strcmp(qenv, "quad") == 0);
+      // Grids of few wavefronts, run alone: one cell per lane. A quad's chain of loads is four cells long and
+      // little runs beside it; unaligned rows (nz % 4 != 0) and poles lengthen it, quads across the edges of
+      // CPML normal to z too. us per step, one cell / quads. Poles (a two-pole slab): 48^3 16.1 / 20.4,
+      // 64x56x60 17.5 / 19.8, 80^3 22.2 / 23.7, 88^3 27.1 / 27.7; the other way from there (92^3 29.5 / 28.6,
+      // 100^3 32.6 / 28.6; with a 10^3 particle from 84^3, 21.7 / 21.5, 96^3 27.1 / 24.0). Poles and unaligned
+      // rows: with CPML normal to z 73x72x71 20.8 / 24.6, 111^3 39 / 42.6, 141^3 58 / 62, 200x200x101 79 / 74;
+      // without it 61^3 18.5 / 19.8, 97^3 30.7 / 27.4. Unaligned rows alone: 41^3 11.7 / 13.4,
+      // 71^3 15.0 / 15.7; the other way 81^3 16.9 / 15.8, 95^3 29.0 / 26.2 (a plane wave), 301x277x150 218 / 204.
+      // Rows of one quad and a few cells, whose second quad does less than half the work of its lane: 400x400x7
+      // 18.9 / 22.4, 400x400x5 15.8 / 17.6 (400x400x9 24.4 / 22.9).
+      // Complex fields have both parts in a launch and fewer launches with quads (24x24x36 with poles
+      // 25.3 / 21.6, 61^3 30 / 23), batches many solves in one (eight of 64^3 with the slab 80 / 51, of 47^3
+      // 27 / 22).
+      const bool rag = P.nz % 4 != 0, zslab = P.axs[2][0] >= 0 || P.axs[2][1] >= 0;
+      const bool one = (P.nade && P.N < (rag && zslab ? kAlonePolesRagged : kAlonePoles)) || (rag && (P.N < kAloneRagged || P.nz < 8));
+      pl->alone_one = quad_ok && one && !pl->cplx && !(qenv && strcmp(qenv, "quad") == 0);
       P.cax = quad_ok && xyz && zq ? 1 : 0;
       bool gap = true;
       for (int a = 0; a < 3; ++a)
@@ -606,27 +616,33 @@ static int plan_create(const fdtdx_plan_desc* d, fdtdx_plan** out) {
     }
     // masks of the one-cell forward sweeps' tiles, where those may run
     if (!(quad_ok && P.cax) || pl->alone_one) {
+      // footprints of a tile's z-interior and z-slab cells, from the sweeps' own mapping (the same in every
+      // x-plane)
+      struct Footprint {
+        int lo[2][2], hi[2][2];
+      };
+      std::vector<Footprint> fp(perm ? (size_t)P.bpp : 0, Footprint{{{P.ny, P.nz}, {P.ny, P.nz}}, {{-1, -1}, {-1, -1}}});
+      for (long long p = 0; perm && p < P.plane; ++p) {
+        int j, k;
+        perm_cell(P, (int)p, j, k);
+        const int c = (k < P.zlo || k >= P.zhi) ? 1 : 0;
+        Footprint& f = fp[(size_t)(p / kBlock)];
+        f.lo[c][0] = std::min(f.lo[c][0], j); f.hi[c][0] = std::max(f.hi[c][0], j);
+        f.lo[c][1] = std::min(f.lo[c][1], k); f.hi[c][1] = std::max(f.hi[c][1], k);
+      }
       std::vector<uint32_t> fm((size_t)P.nblocks, 0u);
       for (long long lb = 0; lb < P.nblocks; ++lb) {
         const int i = (int)(lb / P.bpp);
-        const long long p0 = (lb - (long long)i * P.bpp) * kBlock;
-        const long long p1 = std::min(p0 + kBlock, P.plane) - 1;
+        const long long b = lb - (long long)i * P.bpp;
+        const long long p0 = b * kBlock, p1 = std::min(p0 + kBlock, P.plane) - 1;
         if (!perm) {
           fm[(size_t)lb] = span_mask(i, p0, p1, P.nz, false);
           continue;
         }
-        // footprints of the tile's z-interior and z-slab cells, from the sweeps' own mapping
-        int lo[2][2] = {{P.ny, P.nz}, {P.ny, P.nz}}, hi[2][2] = {{-1, -1}, {-1, -1}};
-        for (long long p = p0; p <= p1; ++p) {
-          int j, k;
-          perm_cell(P, (int)p, j, k);
-          const int c = (k < P.zlo || k >= P.zhi) ? 1 : 0;
-          lo[c][0] = std::min(lo[c][0], j); hi[c][0] = std::max(hi[c][0], j);
-          lo[c][1] = std::min(lo[c][1], k); hi[c][1] = std::max(hi[c][1], k);
-        }
+        const Footprint& f = fp[(size_t)b];
         uint32_t m = 0;
         for (int c = 0; c < 2; ++c)
-          if (hi[c][0] >= 0) m |= box_mask(i, lo[c][0], hi[c][0], lo[c][1], hi[c][1], false);
+          if (f.hi[c][0] >= 0) m |= box_mask(i, f.lo[c][0], f.hi[c][0], f.lo[c][1], f.hi[c][1], false);
         fm[(size_t)lb] = m;
       }
       if ((rc = pl->upload(fm.data(), fm.size(), &P.fwd_mask))) return bail(rc);

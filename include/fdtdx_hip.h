@@ -283,7 +283,8 @@ int fdtdx_workspace_bytes(const fdtdx_plan* plan, size_t* out);
  * sweeps, four z cells per lane), FDTDX_SCHED_FUSED or FDTDX_SCHED_MARCH (single-pass, opted in by
  * FDTDX_SWEEP). Quads are the default; one cell per lane run full tensors, rows of fewer than 4 cells,
  * rows of nz % 4 != 0 cells and complex fields where the CPML slabs do not each span a face or where there
- * are both poles and conductivity, and small grids of real fields with poles. All give the same bits.
+ * are both poles and conductivity, and small grids of real fields with poles or with rows of nz % 4 != 0
+ * cells. All give the same bits.
  * fdtdx_plan_batch_schedule: the schedule of the plan's tiles in a batch (fdtdx_batch_attach), where the
  * size of one grid does not count. */
 enum { FDTDX_SCHED_ONE = 0, FDTDX_SCHED_QUAD = 1, FDTDX_SCHED_FUSED = 2, FDTDX_SCHED_MARCH = 3 };

@@ -707,11 +707,16 @@ def test_detector_steps_that_share_a_slot_are_stored_in_order(slots):
                 assert np.array_equal(a[slot], r[t]), (slot, t)
 
 
-@pytest.mark.parametrize("shape,poles,quad", [((40, 40, 40), False, True), ((40, 40, 40), True, False),
-                                              ((88, 88, 88), True, False), ((92, 92, 92), True, True)])
-def test_schedule_of_small_grids_with_poles(shape, poles, quad, monkeypatch):
-    """Small grids with poles run one cell per lane alone and in quads in a batch or under
-    FDTDX_SWEEP=quad; larger ones and those without poles in quads."""
+@pytest.mark.parametrize("shape,kind,quad", [
+    ((40, 40, 40), "", True), ((40, 40, 40), "poles", False), ((88, 88, 88), "poles", False),
+    ((92, 92, 92), "poles", True), ((92, 92, 93), "poles", False), ((144, 144, 146), "poles", True),
+    ((92, 92, 93), "poles open_z", True), ((40, 40, 41), "", False), ((73, 73, 74), "", False),
+    ((74, 74, 74), "", True), ((300, 200, 7), "open_z", False), ((300, 200, 9), "open_z", True),
+    ((40, 40, 8), "open_z", True), ((40, 40, 41), "bloch", True), ((40, 40, 41), "bloch poles", True)])
+def test_schedule_of_grids_run_alone(shape, kind, quad, monkeypatch):
+    """Small grids with poles (with rows of nz % 4 != 0 cells and CPML normal to z, larger ones too) or with
+    such rows, and those with such rows of under 8 cells, run one cell per lane alone and in quads in a batch or under FDTDX_SWEEP=quad; larger ones,
+    complex fields and other grids in quads."""
     import scenarios
 
     from fdtdx_amd import fdtd as F
@@ -719,8 +724,16 @@ def test_schedule_of_small_grids_with_poles(shape, poles, quad, monkeypatch):
     spec = W.scenario_c1(T=3, n=40, pml=5, cube=8)
     spec["shape"] = shape
     spec["detectors"] = []
-    if poles:
+    if shape[2] < 16:
+        spec["boxes"] = []
+        spec["sources"][0]["cell"] = (20, 20, 4)
+    if "poles" in kind:
         spec["boxes"][0]["poles"] = [("drude", 2e15, 1e14)]
+    if "open_z" in kind:
+        spec["pml"] = dict(spec["pml"], types={"min_z": "pec", "max_z": "pec"})
+    if "bloch" in kind:
+        spec["pml"] = dict(spec["pml"], types={"min_x": "bloch", "max_x": "bloch"})
+        spec["bloch_vector"] = (1e5, 0.0, 0.0)
     for mode in (None, "quad"):
         if mode:
             monkeypatch.setenv("FDTDX_SWEEP", mode)

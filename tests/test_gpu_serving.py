@@ -184,7 +184,7 @@ def test_batch_of_mixed_schedules_equals_single_solves(eps_comps):
             del b["poles"]
         specs = [W.scenario_c4(T=45, n=28, pml=5, slab=(10, 10, 8), cube=4),
                  W.scenario_c4(T=50, n=31, pml=5, slab=(10, 10, 8), cube=4), lossy, plain]
-        alone, quads = [False, False, False, True], [True, True, True, True]
+        alone, quads = [False, False, False, False], [True, True, True, True]
     else:
         ragged = W.scenario_c2(T=45, shape=(44, 30, 27), pml=5, slab=(10, 12, 8))
         lossy = W.scenario_c1(T=50, n=26, pml=4, cube=6)
@@ -204,7 +204,7 @@ def test_batch_of_mixed_schedules_equals_single_solves(eps_comps):
         poles = W.scenario_c1(T=35, n=27, pml=4, cube=7)
         poles["boxes"][0]["poles"] = [("drude", 2e15, 1e14)]
         specs = [ragged, lossy, per, flat, poles]
-        alone, quads = [True, True, True, False, False], [True, True, True, False, True]
+        alone, quads = [False, False, True, False, False], [True, True, True, False, True]
 
     def solves():
         out = []
