@@ -719,7 +719,7 @@ __device__ __forceinline__ void quad_E(const StepStatic& P, const StepDyn& D, in
   f4v cx = d.y2 - d.z1;  // dy Hz - dz Hy
   f4v cy = d.z2 - d.x1;  // dz Hx - dx Hz
   f4v cz = d.x2 - d.y1;  // dx Hy - dy Hx
-  if (fast_slabs) quad_slab_apply<0, RAG>(P, S, D.psi, i, j, k0, sm, true, d, cx, cy, cz);
+  if (fast_slabs) quad_slab_apply<0, RAG>(P, S, D.psi, i, j, k0, sm, d, cx, cy, cz);
   else if (!CAX && (m & kSlabBits)) cpml_quad(P, m, D.psi, 0, i, j, k0, d, cx, cy, cz);
   const f4v iex = ld4<RAG>(D.ie + o);
   const f4v iey = EC == 3 ? ld4<RAG>(D.ie + N + o) : iex;
@@ -800,7 +800,7 @@ __device__ __forceinline__ void quad_H(const StepStatic& P, const StepDyn& D, in
   f4v cx = d.y2 - d.z1;  // dy Ez - dz Ey
   f4v cy = d.z2 - d.x1;  // dz Ex - dx Ez
   f4v cz = d.x2 - d.y1;  // dx Ey - dy Ex
-  if (fast_slabs) quad_slab_apply<1, RAG>(P, S, D.psi, i, j, k0, sm, true, d, cx, cy, cz);
+  if (fast_slabs) quad_slab_apply<1, RAG>(P, S, D.psi, i, j, k0, sm, d, cx, cy, cz);
   else if (!CAX && (m & kSlabBits)) cpml_quad(P, m, D.psi, 1, i, j, k0, d, cx, cy, cz);
   float* Hx = D.H;
   float* Hy = D.H + N;

@@ -166,7 +166,7 @@ hipError_t launch_batch_set(int* base, int* flags, const BatchSet& set, hipStrea
 // ade: some solve of the batch has poles
 hipError_t launch_batch_sweeps(const BatchTable* tab, const int* base, int r, int ec, int mc, bool ade, int grid,
                                hipStream_t s);
-// Detectors of chunk step r (mode bit 0: some detector keeps per-cell phasors, bit 1: some needs_halo),
+// Detectors of chunk step r (mode bit 0: some detector needs_halo),
 // and the sums of chunk steps [r0, r0 + steps), at most kDetRing of them.
 hipError_t launch_batch_detectors(const BatchTable* tab, const int* base, int r, int mode, int grid, hipStream_t s);
 hipError_t launch_batch_finalize(const BatchTable* tab, const int* base, int r0, int steps, hipStream_t s);

@@ -946,6 +946,12 @@ int fdtdx_plan_batch_schedule(const fdtdx_plan* p, int32_t* out) {
   return FDTDX_OK;
 }
 
+int fdtdx_plan_reverse_schedule(const fdtdx_plan* p, int32_t* out) {
+  if (!p || !out) return fail(FDTDX_EINVAL, "null argument");
+  *out = p->P.aquad ? FDTDX_SCHED_QUAD : FDTDX_SCHED_ONE;
+  return FDTDX_OK;
+}
+
 int fdtdx_forward(const fdtdx_plan* p, const fdtdx_buffers* b, int32_t t0, int32_t t1, int32_t rec,
                   void* stream) {
   return forward_impl(p, b, t0, t1, rec, stream, nullptr);

@@ -1,12 +1,14 @@
-// Device helpers of the kernels that update four consecutive z cells (a quad) per lane: the two
-// sweeps of fwd_kernels.hip and the single-pass step of fused_kernels.hip. Every field array moves
-// as dwordx4, the z neighbours inside a quad come from the lane's own registers. Per cell the
+// Device helpers of the kernels that update four consecutive z cells (a quad) per lane: the forward,
+// batch and reverse sweeps of fwd_kernels.hip and the adjoint passes of adj_kernels.hip. Every field
+// array moves as dwordx4, the z neighbours inside a quad come from the lane's own registers. Per cell the
 // arithmetic is that of the one-cell sweeps, in the same order, so results are bit-identical.
 //
 // Rows of nz cells with nz not a multiple of 4 (RAG): the row's last quad starts at nz - 4 and so
-// repeats up to 3 cells of the quad before it. Both lanes compute these cells from the same
-// inputs (a sweep reads only its own cells of the field it writes), only the first stores them:
-// `sm` is the number of leading cells a lane leaves out of its stores. Accesses are then aligned to
+// repeats up to 3 cells of the quad before it, the `sm` leading cells that its lane leaves out of its
+// stores. Of the arrays a sweep writes the lane may read these cells before or after the other lane has
+// stored them, so their values are unspecified: nothing computed from them may reach a cell that the lane
+// stores, nor a record, a snapshot of a written field or the state of a pole. (A sweep reads only a lane's own
+// cells of the arrays it writes, so kept cells never depend on them.) Accesses are then aligned to
 // 4 bytes only, which global dwordx4 accesses allow.
 #pragma once
 #include "engine_common.h"
@@ -144,11 +146,10 @@ __device__ __forceinline__ void quad_slab_loads(const StepStatic& P, const float
   quad_slab_load<W, 2, RAG>(P, psi, i, j, k0, S);
 }
 
-// store: write the advanced psi of the cells e >= sm to psi_out (false: a recomputed halo quad).
+// Writes the advanced psi of the cells e >= sm to psi_out.
 template <int W, int AX, bool RAG>
 __device__ __forceinline__ void quad_slab_axis(const StepStatic& P, const QuadSlabs& S, float* psi_out, int i, int j,
-                                               int k0, int sm, bool store, const QuadDeriv& d, f4v& cx, f4v& cy,
-                                               f4v& cz) {
+                                               int k0, int sm, const QuadDeriv& d, f4v& cx, f4v& cy, f4v& cz) {
   if (!S.in[AX]) return;
   int dep, L, kap, aligned;
   long long cells;
@@ -188,10 +189,8 @@ __device__ __forceinline__ void quad_slab_axis(const StepStatic& P, const QuadSl
     r2 = k * d2 + n2;
   }
   if (AX != 2 || zvec) {
-    if (store) {
-      st4m<RAG>(psi_out + q, n1, sm);
-      st4m<RAG>(psi_out + q + cells, n2, sm);
-    }
+    st4m<RAG>(psi_out + q, n1, sm);
+    st4m<RAG>(psi_out + q + cells, n2, sm);
   } else {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -200,7 +199,7 @@ __device__ __forceinline__ void quad_slab_axis(const StepStatic& P, const QuadSl
         r2[e] = 0.f;
         continue;
       }
-      if (store && e >= sm) {
+      if (e >= sm) {
         psi_out[q + e] = n1[e];
         psi_out[q + e + cells] = n2[e];
       }
@@ -221,11 +220,10 @@ __device__ __forceinline__ void quad_slab_axis(const StepStatic& P, const QuadSl
 
 template <int W, bool RAG>
 __device__ __forceinline__ void quad_slab_apply(const StepStatic& P, const QuadSlabs& S, float* psi_out, int i, int j,
-                                                int k0, int sm, bool store, const QuadDeriv& d, f4v& cx, f4v& cy,
-                                                f4v& cz) {
-  quad_slab_axis<W, 0, RAG>(P, S, psi_out, i, j, k0, sm, store, d, cx, cy, cz);
-  quad_slab_axis<W, 1, RAG>(P, S, psi_out, i, j, k0, sm, store, d, cx, cy, cz);
-  quad_slab_axis<W, 2, RAG>(P, S, psi_out, i, j, k0, sm, store, d, cx, cy, cz);
+                                                int k0, int sm, const QuadDeriv& d, f4v& cx, f4v& cy, f4v& cz) {
+  quad_slab_axis<W, 0, RAG>(P, S, psi_out, i, j, k0, sm, d, cx, cy, cz);
+  quad_slab_axis<W, 1, RAG>(P, S, psi_out, i, j, k0, sm, d, cx, cy, cz);
+  quad_slab_axis<W, 2, RAG>(P, S, psi_out, i, j, k0, sm, d, cx, cy, cz);
 }
 
 // The correction with psi frozen (the reverse run, PML.py:181-182) of the preloaded slabs, x, y, z.

@@ -94,7 +94,7 @@ EXPORTED = ("fdtdx_plan_create", "fdtdx_plan_destroy", "fdtdx_psi_floats", "fdtd
             "fdtdx_reverse_adjoint", "fdtdx_reverse", "fdtdx_last_error", "fdtdx_batch_create", "fdtdx_batch_destroy",
             "fdtdx_batch_attach", "fdtdx_batch_detach", "fdtdx_batch_advance", "fdtdx_batch_step_index",
             "fdtdx_batch_flags", "fdtdx_stream_probe", "fdtdx_plan_schedule", "fdtdx_plan_batch_schedule",
-            "fdtdx_forward_noalloc", "fdtdx_stencil_probe")
+            "fdtdx_plan_reverse_schedule", "fdtdx_forward_noalloc", "fdtdx_stencil_probe")
 
 FDTDX_MAX_BATCH = 64
 SCHED_ONE, SCHED_QUAD, SCHED_FUSED, SCHED_MARCH = 0, 1, 2, 3
@@ -126,7 +126,7 @@ def load_library(path: Path | None = None):
                "fdtdx_record_slots", "fdtdx_workspace_bytes"):
         getattr(lib, nm).argtypes = [c_void_p, POINTER(c_size_t)]
         getattr(lib, nm).restype = c_int32
-    for nm in ("fdtdx_plan_schedule", "fdtdx_plan_batch_schedule"):
+    for nm in ("fdtdx_plan_schedule", "fdtdx_plan_batch_schedule", "fdtdx_plan_reverse_schedule"):
         getattr(lib, nm).argtypes = [c_void_p, POINTER(c_int32)]
         getattr(lib, nm).restype = c_int32
     lib.fdtdx_record_slot_of.argtypes = [c_void_p, c_int32, POINTER(c_int32)]
@@ -333,6 +333,11 @@ class Plan:
     def batch_quad(self) -> bool:
         """True when the plan's tiles in a batch are of four z cells per lane."""
         return self._schedule("fdtdx_plan_batch_schedule") == SCHED_QUAD
+
+    @property
+    def reverse_quad(self) -> bool:
+        """True when the reverse and adjoint sweeps update four z cells per lane."""
+        return self._schedule("fdtdx_plan_reverse_schedule") == SCHED_QUAD
 
     def _query(self, nm):
         out = c_size_t()

@@ -286,10 +286,13 @@ int fdtdx_workspace_bytes(const fdtdx_plan* plan, size_t* out);
  * are both poles and conductivity, and small grids of real fields with poles or with rows of nz % 4 != 0
  * cells. All give the same bits.
  * fdtdx_plan_batch_schedule: the schedule of the plan's tiles in a batch (fdtdx_batch_attach), where the
- * size of one grid does not count. */
+ * size of one grid does not count. fdtdx_plan_reverse_schedule: the schedule of the sweeps of
+ * fdtdx_reverse_adjoint; quads for CPML slabs that each span a face, a cell apart (five along z), and neither
+ * conducting faces, conductivity nor periodic axes. */
 enum { FDTDX_SCHED_ONE = 0, FDTDX_SCHED_QUAD = 1, FDTDX_SCHED_FUSED = 2, FDTDX_SCHED_MARCH = 3 };
 int fdtdx_plan_schedule(const fdtdx_plan* plan, int32_t* out);
 int fdtdx_plan_batch_schedule(const fdtdx_plan* plan, int32_t* out);
+int fdtdx_plan_reverse_schedule(const fdtdx_plan* plan, int32_t* out);
 
 /* Advance steps n = t0 .. t1-1 in place (forward.py:83-156 per step). When rec != 0 the PML
  * interface layers of each kept step are written, compressed, to its slot of buffers->record

@@ -187,6 +187,7 @@ def test_quad_adjoint_equals_one_cell_adjoint_bitwise(case, monkeypatch):
 
     import fdtdx_amd as fx
     import scenarios
+    from fdtdx_amd import fdtd
 
     spec = _quad_adjoint_cases()[case]
     out = {}
@@ -197,6 +198,7 @@ def test_quad_adjoint_equals_one_cell_adjoint_bitwise(case, monkeypatch):
             monkeypatch.delenv("FDTDX_REVERSE_CPML", raising=False)
         print("case", case, mode, spec["shape"], flush=True)
         objects, arrays, params, config = scenarios.build(spec, gradient=True)
+        assert fdtd.Solve(objects, config, arrays).plan.reverse_quad == (mode == "quad")
         ie = arrays.inv_permittivities.detach().clone().requires_grad_(True)
         arrays.inv_permittivities = ie
         _, arrays = fx.run_fdtd(arrays, objects, config)
