@@ -556,7 +556,7 @@ __global__ __launch_bounds__(kBlock) void k_update_H(const StepStatic* __restric
 // ---------------------------------------------------------------- quad sweeps
 // The forward sweeps with four consecutive z cells per lane (quad.h); a quad tile covers kBlock
 // quads. RAG: rows of nz % 4 != 0 cells (a sweep with 4-byte aligned accesses). Measured on the
-// 301x277x150 plane wave: E / H sweep 119 / 113 us against 128 / 122 us one cell per lane (an aligned
+// 301x277x150 plane wave: E / H sweep 116 / 108 us against 128 / 122 us one cell per lane (an aligned
 // grid of that many cells would take about 101 / 90).
 
 // CPML of the four cells of a quad, slab by slab in object order (per cell the order of
@@ -852,7 +852,7 @@ __global__ __launch_bounds__(kBlock, 5) void k_update_H4(const StepStatic* __res
 
 // The sweeps of complex fields (periodic axes with Bloch phases): both parts in one launch, the part
 // in blockIdx.y. A part's half-step reads the other part of the field it does not write. 96x96x160, E / H
-// half-step of both parts: 22.9 / 20.8 us, a launch per part and one cell per lane 30 / 28 (118 / 106 MB
+// half-step of both parts: 23.1 / 21.0 us, a launch per part and one cell per lane 30 / 28 (118 / 106 MB
 // from the last-level cache, 17 / 15 us at its rate); step 74 -> 62 us.
 __device__ __forceinline__ StepDyn part_of(const StepStatic& P, const StepDyn& D, const PartDyn& C, uint32_t& m) {
   StepDyn S = D;

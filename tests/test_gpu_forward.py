@@ -16,8 +16,8 @@ def rel(a, b):
     return float(np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-300))
 
 
-# Sweep schedules: the two in-place sweeps with four z cells per lane (the default when nz is a
-# multiple of 4) and with one, the LDS-tiled fused kernel and the register-march kernel with 4
+# Sweep schedules: the two in-place sweeps with four z cells per lane (the default but for small grids,
+# which the setting overrides) and with one, the LDS-tiled fused kernel and the register-march kernel with 4
 # and 2 rows per wavefront (short x chunks so chunk halos are exercised).
 MODES = {
     "quad": {"FDTDX_SWEEP": "quad"},
