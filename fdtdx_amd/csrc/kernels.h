@@ -1,7 +1,5 @@
 // Launchers shared between the kernel translation units and the C-ABI in plan.hip.
 #pragma once
-#include <map>
-
 #include "engine_common.h"
 
 namespace fdtdx {
@@ -90,13 +88,9 @@ constexpr int kDetRing = 16;
 // A launch that finalizes `window` steps at a time must then store them in step order: the last one's value
 // stays in the slot, and the faces accumulating into it belong to one step.
 inline bool slots_repeat(const int32_t* tti, int T, int window) {
-  std::map<int32_t, int> last;
-  for (int n = 0; n < T; ++n) {
-    if (tti[n] < 0) continue;
-    const auto it = last.find(tti[n]);
-    if (it != last.end() && n - it->second < window) return true;
-    last[tti[n]] = n;
-  }
+  for (int n = 0; n < T; ++n)
+    for (int m = n < window ? 0 : n - window + 1; m < n && tti[n] >= 0; ++m)
+      if (tti[m] == tti[n]) return true;
   return false;
 }
 
