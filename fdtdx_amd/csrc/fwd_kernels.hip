@@ -1045,15 +1045,16 @@ __global__ __launch_bounds__(kBlock) void k_reverse_E(const StepStatic* __restri
 // n's slot, or interpolate between the slots around it, and write it back into E and H. Where
 // interface planes of two slabs cross, the later slab's value is the one restored, as in the
 // reference's loop over PML objects. PLAIN: float32 layers and a kept step, so the six values are read
-// before any is written (200x200x100: 18.0 -> 13.5 us, most of it the two z faces' single floats).
+// before any is written (200x200x100: 18.0 -> 13.5 us, most of it the two z faces' single floats). The slab loop
+// is rolled: unrolled, its code is read cold by every launch, and the same instructions took 12.0 or
+// 13.4 us by where the linker had put them (11.3 rolled).
 template <bool PLAIN>
 __global__ __launch_bounds__(kBlock) void k_restore(const StepStatic* __restrict__ Pp, const StepDyn D) {
   const StepStatic& P = as_const(Pp);
   const long long t = (long long)blockIdx.x * kBlock + threadIdx.x;
   long long acc = 0;
-#pragma unroll
-  for (int s = 0; s < FDTDX_MAX_CPML; ++s) {
-    if (s >= P.nslab) break;
+#pragma unroll 1
+  for (int s = 0; s < P.nslab; ++s) {
     const SlabK& sl = P.slab[s];
     const long long pc = (long long)sl.pn0 * sl.pn1;
     if (t < acc + pc) {
